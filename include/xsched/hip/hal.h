@@ -84,17 +84,13 @@ XResult HipAxpyCommandCreate(HwCommandHandle *cmd, float alpha, const void *x, v
                              size_t n, int guard);
 
 /* C[M,N] = A[M,K] * B[K,N]; A, B, C row-major bf16, fp32 accumulation in ascending
- * k, round-to-nearest-even on store. Any M, N, K >= 1 (at most 2^18 tiles). The fast MFMA
- * kernel takes M, N in multiples of 128, K in multiples of 64 (K, N <= 2^22) and matrices
- * aligned to 16 bytes: it works on 256x256 tiles of C, or on 128x128 tiles when M or N is no
- * multiple of 256 or the large tiles would cover at most half of the compute units
- * (XSCHED_HIP_GEMM_TILE=128|256 overrides that). Where only M is not as the fast kernel wants
- * it, the fast kernel takes the rows up to the last multiple of 128 and the kernel below the
- * rest, in one command. Every other shape or alignment runs on a
- * bounds-checked kernel with 64x64 tiles (XSCHED_HIP_GEMM_TILE=64 forces it): correct and
- * guarded like the others, 5-20 times slower (180-230 TFLOP/s where rows are 16-byte aligned,
- * 60 where they are not). Every element is summed in the same order
- * in all three. */
+ * k, round-to-nearest-even on store. Any M, N, K >= 1 (at most 2^18 tiles), any alignment to
+ * the element. The work is cut into tiles of C of 256x256 (M and N multiples of 256, K of 64,
+ * enough of them to cover half of the compute units), 128x128 or 64x64, whichever keeps the
+ * compute units busy (XSCHED_HIP_GEMM_TILE=64|128|256 overrides that where the shape allows).
+ * Fastest where the rows of all three matrices start on 16-byte boundaries (N and K multiples
+ * of 8, matrices aligned to 16 bytes); up to twice as long where they do not. Every element is
+ * summed in the same order on all paths. */
 XResult HipGemmBf16CommandCreate(HwCommandHandle *cmd, const void *A, const void *B, void *C,
                                  int M, int N, int K, int guard);
 

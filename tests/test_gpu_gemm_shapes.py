@@ -1,0 +1,57 @@
+"""GPU parity of the GEMM's tile kernels at the sizes where they change their ways: the number
+of K steps around the length of their pipelines and of their polls of the preempt word, the last
+step full and not, edges of tiles, and rows that start on 16-byte boundaries or do not."""
+from ctypes import byref, c_uint64
+
+import numpy as np
+import pytest
+
+import oracle
+from test_gpu_kernels import Queue
+
+pytestmark = pytest.mark.gpu
+
+NAN = 0x7FC0
+
+
+def _shape(fit, tile, steps):
+    if fit == "exact":
+        return tile, 2 * tile, 64 * steps
+    if fit == "edges":      # one row and eight columns in the second tile; 8 to 56 values in the last step
+        return tile + 1, tile + 8, 64 * steps - 8 * (1 + (steps - 1) % 7)
+    return tile + 3, tile + 1, 64 * steps - (2 * steps + 1) % 64   # odd sizes
+
+
+@pytest.mark.parametrize("level,guard", [(1, 0), (2, 1)])
+@pytest.mark.parametrize("steps", [1, 2, 3, 4, 5, 6, 7, 9, 10, 13, 14, 18])
+@pytest.mark.parametrize("fit", ["exact", "edges", "unaligned"])
+@pytest.mark.parametrize("tile", [64, 128])
+def test_gemm_pipeline_lengths_and_edges(xs, gpu, monkeypatch, tile, fit, steps, level, guard):
+    """Integers in [-4, 4]: at most 18 x 64 x 16 < 2^24, so every sum is exact and the result is
+    determined. The matrices lie between NaNs, which must not get into a sum, and C between
+    values that must come back untouched."""
+    torch = gpu
+    monkeypatch.setenv("XSCHED_HIP_GEMM_TILE", str(tile))
+    M, N, K = _shape(fit, tile, steps)
+    pad = 3 if fit == "unaligned" else 8     # elements in front of each matrix
+    print(f"case gemm-pipeline tile={tile} {fit} M={M} N={N} K={K} level={level} guard={guard}", flush=True)
+    rng = np.random.default_rng(100 * steps + tile)
+
+    def between_nans(bits):
+        return np.concatenate([np.full(pad, NAN, np.uint16), bits.ravel(), np.full(64, NAN, np.uint16)])
+    a_bits = oracle.f32_to_bf16_bits(rng.integers(-4, 5, (M, K)).astype(np.float32))
+    b_bits = oracle.f32_to_bf16_bits(rng.integers(-4, 5, (K, N)).astype(np.float32))
+    a = torch.from_numpy(between_nans(a_bits).view(np.int16)).cuda()
+    b = torch.from_numpy(between_nans(b_bits).view(np.int16)).cuda()
+    c = torch.full((pad + M * N + 64,), 0x1234, dtype=torch.int16, device="cuda")
+    q = Queue(xs, torch, level)
+    cmd = c_uint64()
+    xs.check(xs.halhip().HipGemmBf16CommandCreate(byref(cmd), a.data_ptr() + 2 * pad, b.data_ptr() + 2 * pad,
+                                                  c.data_ptr() + 2 * pad, M, N, K, guard))
+    q.submit(cmd.value)
+    q.wait()
+    got = c.cpu().numpy().view(np.uint16)
+    q.close()
+    want = oracle.gemm_bf16(a_bits.ravel(), b_bits.ravel(), M, N, K)
+    assert np.array_equal(got[pad:pad + M * N].reshape(M, N), want.reshape(M, N))
+    assert np.all(got[:pad] == 0x1234) and np.all(got[pad + M * N:] == 0x1234)

@@ -36,6 +36,7 @@
 // Work-group ids are remapped so that the 32 CUs of one XCD (ids equal modulo 8 land on one
 // XCD) work on neighbouring tiles and share A/B panels in that XCD's L2.
 #include <type_traits>
+#include <utility>
 
 #include "hip_hal.h"
 #include "xsched/hip/hal.h"
@@ -62,6 +63,7 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kLargeTile = 256;     // edge of the large tile of C (M and N)
 constexpr int kSmallTile = 128;     // edge of the small one
+constexpr int kTinyTile = 64;       // and of the smallest
 constexpr int kStepK = 64;          // K per step
 constexpr int kPollSteps = 4;       // K steps between two looks at the preempt word
 constexpr int kXcds = 8;
@@ -85,11 +87,8 @@ __device__ __forceinline__ void TileOf(uint32_t wg, uint32_t tiles_m, uint32_t t
                                        uint32_t &tm, uint32_t &tn)
 {
     const uint32_t n_tiles = tiles_m * tiles_n;
-    uint32_t t = wg;
-    if (n_tiles % kXcds == 0) {
-        const uint32_t per_xcd = n_tiles / kXcds;
-        t = (wg % kXcds) * per_xcd + wg / kXcds;
-    }
+    const uint32_t xcd = wg % kXcds, whole = n_tiles / kXcds, more = n_tiles % kXcds;   // `more` XCDs get one tile more
+    const uint32_t t = xcd * whole + min(xcd, more) + wg / kXcds;
     const uint32_t band = kGroupRows * tiles_n;
     const uint32_t band_id = t / band;
     const uint32_t first_row = band_id * kGroupRows;
@@ -405,29 +404,497 @@ void GemmBf16Kernel(const uint16_t *__restrict__ A, const uint16_t *__restrict__
 }
 
 
-// Any shape: M, N, K >= 1, any alignment of the three matrices to two bytes. 64 x 64 tiles of
-// C, four waves of one 32x32 block each, K in steps of 32 (two slices of 16 through the same
-// MFMA as above and in the same order, so an element is summed as the kernels above sum it;
-// what lies beyond K is zero). Every load and store is checked against the matrix; a thread's
-// eight neighbouring elements come as one 16-byte load where they lie inside the matrix and
-// are aligned, one by one otherwise. The loads of the next step are on their way while the
-// current one is multiplied. This kernel is the fall-back for the shapes the fast kernels do
-// not take, 5-20 times slower than they are. The guard is at entry only: a tile is short.
+// ---- smaller tiles, any shape ------------------------------------------------------------
+//
+// 128 x 128 or 64 x 64 tiles of C, four waves in a 2 x 2 grid, for outputs of too few large
+// tiles to fill the device and for every shape the large tiles do not fit. One such work-group
+// sits on a compute unit with one wave per SIMD, so nothing but its own instruction stream
+// hides latencies; what bounds it is the round trip to memory (0.8-1 us, several K steps) and
+// then LDS bandwidth (a 64 x 64 wave tile reads 16 KiB per 16 MFMAs of 32 cycles). Hence:
+//   - kStages tiles of A and B are in LDS or on their way (4 x 32 KiB or 4 x 16 KiB), and the
+//     waits count loads instead of draining them: s_waitcnt vmcnt leaves the newer tiles in
+//     flight;
+//   - the fragments of a WHOLE step are read from LDS into registers one step ahead, so a step
+//     is one wait, one barrier and then MFMAs with an LDS read and a load next to each: the
+//     buffer of tile t is free as soon as step t begins, and no MFMA waits for LDS.
+// Layouts in LDS, fragments and the order of the additions are those of the kernel above; the
+// results are bit-identical.
+//
+// Measured, per guarded command in a stream of them (before: 128 x 128 tiles with one tile of
+// lead, or a bounds-checked kernel of 64 x 64 tiles for what is not a multiple of the tiles):
+//   1024^3            10.8 -> 5.8 us (64 x 64: 256 work-groups instead of 64)
+//   2048^3            23.7 -> 17.8 us = 0.96 PFLOP/s
+//   2000^3            86.5 -> 21.8 us      2000 x 1999 x 2047   254 -> 31.0 us
+//   128 x 128 x 8192  76.0 -> 19.7 us      4097 x 4095 x 4097   2122 -> 243 us
+//
+// What the matrices have to be like is kFit:
+//   kExact      M, N multiples of the tile, K of kStepK, matrices aligned to 16 bytes
+//   kEdges      M any; N and K multiples of 8, matrices aligned to 16 bytes: every 16-byte piece
+//               lies inside the matrix or outside. Pieces outside are fetched from somewhere
+//               inside (their row or column of C is not stored); behind K the fragments are
+//               masked to zero, which adds nothing to a sum
+//   kUnaligned  any N >= 8, any alignment to the element: pieces start at any multiple of two
+//               bytes, which the loads into LDS do not take: they come through registers
+//               (kRegTiles tiles of them in flight) and are stored to the same places. Only
+//               the last K step can reach behind the end of a matrix: its pieces are checked
+//               one by one and fetched element by element where they do.
+enum class Fit { kExact, kEdges, kUnaligned };
+
+/// What a K step does besides its MFMAs (see GemmDeepBody).
+enum LoadKind { kNothing, kWholeTile, kLastTile };
+template <int kLoad_, bool kPut_, bool kRead_, int kNewer_>
+struct Step
+{
+    static constexpr int kLoad = kLoad_;     // request a tile
+    static constexpr bool kPut = kPut_;      // kUnaligned: store a tile that has arrived to LDS
+    static constexpr bool kRead = kRead_;    // read the next tile's fragments
+    static constexpr int kNewer = kNewer_;   // tiles in flight behind the one waited for
+};
+
+typedef u32x4 u32x4_any __attribute__((aligned(2)));
+typedef s16x8 s16x8_any __attribute__((aligned(2)));
+
+/// s_waitcnt vmcnt(n) lgkmcnt(0)
+template <int kVm>
+__device__ __forceinline__ void WaitLoadsAndLds()
+{
+    static_assert(kVm >= 0 && kVm < 64, "vmcnt has six bits");
+    __builtin_amdgcn_s_waitcnt((kVm & 15) | (7 << 4) | ((kVm >> 4) << 14));
+}
+
+/// The 16 bytes of v moved down by d (0..15) bytes, zeroes behind them.
+__device__ __forceinline__ u32x4 ShiftDownBytes(u32x4 v, uint32_t d)
+{
+    const u32x4 zero = { 0, 0, 0, 0 };
+    v = d & 8 ? __builtin_shufflevector(v, zero, 2, 3, 4, 4) : v;
+    v = d & 4 ? __builtin_shufflevector(v, zero, 1, 2, 3, 4) : v;
+    return u32x4 { __builtin_amdgcn_alignbyte(v.y, v.x, d & 3), __builtin_amdgcn_alignbyte(v.z, v.y, d & 3),
+                   __builtin_amdgcn_alignbyte(v.w, v.z, d & 3), __builtin_amdgcn_alignbyte(0u, v.w, d & 3) };
+}
+
+/// s_waitcnt as above with at most `newer` tiles of kLoads loads in flight (`newer` is uniform, at most kMost).
+template <int kMost, int kLoads>
+__device__ __forceinline__ void WaitNewer(int newer)
+{
+    if constexpr (kMost == 0) WaitLoadsAndLds<0>();
+    else if (newer >= kMost) WaitLoadsAndLds<kMost * kLoads>();
+    else WaitNewer<kMost - 1, kLoads>(newer);
+}
+
+template <bool kGuard, Fit kFit, int kTile, int kStages>
+__device__ __forceinline__
+void GemmDeepBody(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B,
+                  uint16_t *__restrict__ C, int M, int N, int K, const XGuardArgs &g)
+{
+    constexpr bool kDirect = kFit != Fit::kUnaligned;      // loads go straight into LDS
+    constexpr int kWaves = 4;
+    constexpr int kBlocks = kTile / 64;                    // 32x32 blocks per wave in each direction
+    constexpr int kSlices = kStepK / 16;
+    constexpr int kMfmas = kSlices * kBlocks * kBlocks;    // per wave and step
+    constexpr int kFrags = kSlices * kBlocks;              // fragments of A (and of B) per wave and step
+    constexpr int kTileBytes = kTile * kStepK * 2;         // A or B tile in LDS
+    constexpr int kHalfLoads = kTileBytes / 1024 / kWaves; // 1 KiB loads per wave of one of them
+    constexpr int kLoads = 2 * kHalfLoads;
+    constexpr int kRegTiles = 2;                           // kUnaligned: tiles in flight in registers
+    constexpr int kBuffers = kDirect ? kStages : 2;
+    constexpr int kBRowBytes = kTile * 2;
+    constexpr int kBSlotsPerRow = kBRowBytes / 16;
+    constexpr int kBRowsPerLoad = 64 / kBSlotsPerRow;
+    static_assert(2 * kFrags % kMfmas == 0 || 2 * kFrags <= kMfmas, "reads pair up with the MFMAs of a step");
+    static_assert((kStages & (kStages - 1)) == 0 && kStages >= 4, "stages are numbered modulo a power of two");
+    // one LDS object (see above): the tiles, then two slots for the preempt word and the guard's own word
+    constexpr int kFlagAt = 2 * kBuffers * kTileBytes;
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[kFlagAt + 2 * 256 + 16];
+    uint32_t &guard_word = *(uint32_t *)(lds + kFlagAt + 2 * 256);
+    uint8_t *const As0 = lds;
+    uint8_t *const Bs0 = lds + kBuffers * kTileBytes;
+
+    const uint32_t tid = threadIdx.x;
+    const uint32_t lane = tid & 63;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t wm = wave >> 1, wn = wave & 1;
+
+    uint32_t tm, tn;
+    TileOf(blockIdx.x, ((uint32_t)M + kTile - 1) / kTile, ((uint32_t)N + kTile - 1) / kTile, tm, tn);
+    const size_t m0 = (size_t)tm * kTile, n0 = (size_t)tn * kTile;
+    const int steps = kFit == Fit::kExact ? K / kStepK : (K + kStepK - 1) / kStepK;
+    const int rest = K - (steps - 1) * kStepK;             // K values of the last step
+
+    // ---- what each lane fetches: byte offsets from the tile's first element, as above ----
+    uint32_t off[kLoads];
+    uint32_t k_of[kLoads];                                 // the piece's first k within the step
+#pragma unroll
+    for (int i = 0; i < kHalfLoads; ++i) {
+        const uint32_t q = wave * kHalfLoads + i;
+        const uint32_t line = 4 * q + (lane >> 4);
+        const uint32_t piece = (lane & 15) ^ (line & 15);
+        uint32_t row = 2 * line + (piece >> 3);
+        const uint32_t kc = piece & 7;
+        if (kFit != Fit::kExact && m0 + row >= (size_t)M) row = (uint32_t)((size_t)M - 1 - m0);
+        off[i] = (row * (uint32_t)K + kc * 8) * 2;
+        k_of[i] = kc * 8;
+    }
+#pragma unroll
+    for (int i = 0; i < kHalfLoads; ++i) {
+        const uint32_t q = wave * kHalfLoads + i;
+        const uint32_t k = kBRowsPerLoad * q + lane / kBSlotsPerRow;
+        const uint32_t slot = lane % kBSlotsPerRow;
+        const uint32_t swz = kTile == 64 ? (k >> 1) & 1 : k & 3;
+        uint32_t col = ((slot >> 2) ^ swz) * 32 + (slot & 3) * 8;
+        if (kFit != Fit::kExact && n0 + col >= (size_t)N) col = 0;
+        off[kHalfLoads + i] = (k * (uint32_t)N + col) * 2;
+        k_of[kHalfLoads + i] = k;
+    }
+    const uint16_t *const a_tile = A + m0 * (size_t)K;     // + kStepK columns per step
+    const uint16_t *const b_tile = B + n0;                 // + kStepK rows per step
+
+    // Offset of piece idx in the last step: pieces behind K come from k = 0 of the step instead.
+    auto last_off = [&](int idx) -> uint32_t {
+        if (kFit == Fit::kExact || k_of[idx] < (uint32_t)rest) return off[idx];
+        return idx < kHalfLoads ? off[idx] - k_of[idx] * 2 : off[idx] - k_of[idx] * (uint32_t)N * 2;
+    };
+    auto load_direct = [&](int step, int idx, uint32_t at) {
+        const int buf = step & (kBuffers - 1);
+        if (idx < kHalfLoads) {
+            const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void *)(a_tile + (size_t)step * kStepK), 0, 0x7fffffff, 0x00020000);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (LdsVoid *)(As0 + buf * kTileBytes + (wave * kHalfLoads + idx) * 1024), 16, at, 0, 0, 0);
+        } else {
+            const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void *)(b_tile + (size_t)step * kStepK * N), 0, 0x7fffffff, 0x00020000);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (LdsVoid *)(Bs0 + buf * kTileBytes + (wave * kHalfLoads + idx - kHalfLoads) * 1024), 16, at, 0, 0, 0);
+        }
+    };
+    // kUnaligned: the pieces of kRegTiles tiles on their way through registers
+    u32x4 held[kDirect ? 1 : kRegTiles][kDirect ? 1 : kLoads];
+    auto load_held = [&](int set, int step, int idx) {
+        const uint8_t *base = idx < kHalfLoads ? (const uint8_t *)(a_tile + (size_t)step * kStepK)
+                                               : (const uint8_t *)(b_tile + (size_t)step * kStepK * N);
+        held[set][idx] = *(const u32x4_any *)(base + off[idx]);
+    };
+    auto load_held_last = [&](int set, int step, int idx) {
+        const uint8_t *base = idx < kHalfLoads ? (const uint8_t *)(a_tile + (size_t)step * kStepK)
+                                               : (const uint8_t *)(b_tile + (size_t)step * kStepK * N);
+        const uint8_t *const end = idx < kHalfLoads ? (const uint8_t *)(A + (size_t)M * K) : (const uint8_t *)(B + (size_t)K * N);
+        // A piece that would reach behind the matrix is fetched from its last 16 bytes instead and
+        // shifted into place; what is then missing lies behind K or in columns behind N.
+        const uint8_t *const p = base + last_off(idx);
+        const uint8_t *const inside = p + 16 <= end ? p : end - 16;
+        held[set][idx] = ShiftDownBytes(*(const u32x4_any *)inside, (uint32_t)(p - inside));
+    };
+    auto put_held = [&](int set, int step, int idx) {
+        const int buf = step & (kBuffers - 1);
+        uint8_t *const at = idx < kHalfLoads ? As0 + buf * kTileBytes + (wave * kHalfLoads + idx) * 1024
+                                             : Bs0 + buf * kTileBytes + (wave * kHalfLoads + idx - kHalfLoads) * 1024;
+        *(u32x4 *)(at + lane * 16) = held[set][idx];
+    };
+
+    // ---- LDS -> fragments, as above ----
+    const uint32_t a_row0 = 32 * kBlocks * wm + (lane & 31);
+    const uint32_t a_line = a_row0 >> 1;
+    const uint32_t a_base = a_line * 256 + (((((lane & 1) << 3) | (lane >> 5)) ^ (a_line & 15)) << 4);
+    const uint32_t b_row = 8 * (lane >> 5) + ((lane & 15) >> 2);
+    const uint32_t b_swz = kTile == 64 ? (b_row >> 1) & 1 : b_row & 3;
+    const uint32_t b_base = b_row * kBRowBytes + (((kBlocks * wn) ^ b_swz) << 6) + (16 * ((lane >> 4) & 1) + 4 * (lane & 3)) * 2;
+    bf16x8 fa[2][kFrags], fb[2][kFrags];                   // [parity of the step][slice * kBlocks + block]
+    // Fragment unit n of tile `step` into set `set`: A and B of a slice next to each other.
+    auto read_unit = [&](int set, int step, int n) {
+        const int buf = step & (kBuffers - 1);
+        const int ks = n / (2 * kBlocks), r = n % (2 * kBlocks);
+        if (r < kBlocks) {
+            fa[set][ks * kBlocks + r] = *(const bf16x8 *)(As0 + buf * kTileBytes + (a_base ^ (ks << 5)) + r * 4096);
+        } else {
+            const int j = r - kBlocks;
+            const uint8_t *p = Bs0 + buf * kTileBytes + ks * 16 * kBRowBytes + (b_base ^ (j << 6));
+            const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsS16x4 *)p);
+            const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsS16x4 *)(p + 4 * kBRowBytes));
+            fb[set][ks * kBlocks + j] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+        }
+    };
+
+    f32x16 acc[kBlocks][kBlocks];
+#pragma unroll
+    for (int i = 0; i < kBlocks; ++i)
+#pragma unroll
+        for (int j = 0; j < kBlocks; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+    auto mfma = [&](int set, int n) {
+        const int ks = n / (kBlocks * kBlocks), i = n / kBlocks % kBlocks, j = n % kBlocks;
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[set][ks * kBlocks + i], fb[set][ks * kBlocks + j], acc[i][j], 0, 0, 0);
+    };
+    // A lane's fragment of slice ks holds k = 16 ks + 8 (lane / 32) + 0..7 of the step, for A and
+    // for B alike: everything from `rest` on becomes zero.
+    auto mask_behind_k = [&](int set) {
+#pragma unroll
+        for (int ks = 0; ks < kSlices; ++ks) {
+            const int valid = rest - (16 * ks + 8 * (int)(lane >> 5));
+            u32x4 m;
+#pragma unroll
+            for (int d = 0; d < 4; ++d) m[d] = valid >= 2 * d + 2 ? 0xFFFFFFFFu : valid == 2 * d + 1 ? 0xFFFFu : 0u;
+#pragma unroll
+            for (int i = 0; i < kBlocks; ++i) {
+                fa[set][ks * kBlocks + i] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, fa[set][ks * kBlocks + i]) & m);
+                fb[set][ks * kBlocks + i] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, fb[set][ks * kBlocks + i]) & m);
+            }
+        }
+    };
+#define XS_BARRIER do { asm volatile("" ::: "memory"); XS_PIN; __builtin_amdgcn_s_barrier(); XS_PIN; asm volatile("" ::: "memory"); } while (0)
+
+    // ---- prologue: the first tiles on their way, the guard's reads beside them ----
+    constexpr int kAhead = kDirect ? kStages : kRegTiles;
+#pragma unroll
+    for (int t = 0; t < kAhead; ++t) {
+        if (t >= steps) break;
+#pragma unroll
+        for (int idx = 0; idx < kLoads; ++idx) {
+            if constexpr (kDirect) load_direct(t, idx, t == steps - 1 ? last_off(idx) : off[idx]);
+            else if (t == steps - 1) load_held_last(t, t, idx);
+            else load_held(t, t, idx);
+        }
+    }
+    if (kGuard) {
+        XGuardBlock guard(g, blockIdx.x, &guard_word);
+        if (!guard.Enter()) {
+            XS_WAIT_GLOBAL_LOADS; // nothing may still be on its way into LDS when the group is gone
+            return;
+        }
+    }
+    // Waits until tile t has landed, i.e. all but the `newer` tiles requested behind it.
+    auto wait_tile = [&](int newer) { WaitNewer<kStages - 1, kLoads>(newer); };
+    if constexpr (kDirect) {
+        wait_tile(min(kStages, steps) - 1);
+    } else {
+        // tile 0, then tile 1, into their LDS buffers; the next ones into the registers they leave
+#pragma unroll
+        for (int t = 0; t < kRegTiles; ++t) {
+            if (t < steps) {
+#pragma unroll
+                for (int idx = 0; idx < kLoads; ++idx) put_held(t, t, idx);
+            }
+            const int next = t + kRegTiles;
+            if (next < steps - 1) {
+#pragma unroll
+                for (int idx = 0; idx < kLoads; ++idx) load_held(t, next, idx);
+            } else if (next == steps - 1) {
+#pragma unroll
+                for (int idx = 0; idx < kLoads; ++idx) load_held_last(t, next, idx);
+            }
+        }
+        static_assert(kDirect || kRegTiles == kBuffers, "tiles 0 .. kRegTiles - 1 each have a buffer");
+        __builtin_amdgcn_s_waitcnt(0xC07F); // lgkmcnt(0): the stores to LDS are done
+    }
+    XS_BARRIER;
+
+    // The preempt word travels like a tile: wave 0 has it loaded into LDS (one more wave-wide
+    // load, in order with the tiles'), and kPollSteps steps later, when that load has landed
+    // because loads requested behind it have been waited for in front of a barrier, every wave
+    // reads it there. (A load into a register would have to be waited for with all tiles
+    // requested before it; a scalar load with all LDS reads.) Two slots in turn: between two
+    // writes of one slot lie the barriers of eight steps and one look at it.
+    auto request_flag = [&](int slot) {
+        if (wave == 0) {
+            const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void *)xguard_flag_copy(g, blockIdx.x), 0, 4, 0x00020000);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (LdsVoid *)(lds + kFlagAt + slot * 256), 4, 0, 0, 0, 0x11 /* sc0 sc1: system scope */);
+        }
+    };
+    auto flag_is_current = [&](int slot) -> bool {
+        return (uint32_t)__builtin_amdgcn_readfirstlane((int)*(LdsVolatileWord *)(lds + kFlagAt + slot * 256)) == g.epoch;
+    };
+
+    // One step. Tile t + 1 is waited for (kNewer tiles requested behind it stay in flight), then
+    // come the MFMAs on the fragments of tile t, next to them the fragment reads of tile t + 1 and
+    // the loads of the tile that goes into the buffer that has just become free. `what` says what
+    // is left to do besides the MFMAs; all of it is known where a step is written down, for the
+    // last steps too: a branch in a step would make its MFMAs wait for its reads.
+    auto step = [&](int t, auto parity, auto what) {
+        constexpr int p = decltype(parity)::value;
+        using Do = decltype(what);
+        XS_PIN;
+        if constexpr (kDirect) WaitLoadsAndLds<Do::kNewer * kLoads>();
+        else __builtin_amdgcn_s_waitcnt(0xC07F);
+        XS_BARRIER;
+        if constexpr (kFit != Fit::kExact && !Do::kRead) {
+            if (rest != kStepK) mask_behind_k(p);
+        }
+#pragma unroll
+        for (int n = 0; n < kMfmas; ++n) {
+            mfma(p, n);
+            constexpr int kReads = 2 * kFrags >= kMfmas ? 2 * kFrags / kMfmas : 1;
+#pragma unroll
+            for (int r = n * kReads; Do::kRead && r < (n + 1) * kReads && r < 2 * kFrags; ++r) read_unit(p ^ 1, t + 1, r);
+#pragma unroll
+            for (int idx = n * kLoads / kMfmas; idx < (n + 1) * kLoads / kMfmas; ++idx) {
+                if constexpr (kDirect) {
+                    if constexpr (Do::kLoad == kWholeTile) load_direct(t + kStages, idx, off[idx]);
+                    if constexpr (Do::kLoad == kLastTile) load_direct(t + kStages, idx, last_off(idx));
+                } else {
+                    if constexpr (Do::kPut) put_held(p, t + 2, idx);
+                    if constexpr (Do::kLoad == kWholeTile) load_held(p, t + 2 + kRegTiles, idx);
+                    if constexpr (Do::kLoad == kLastTile) load_held_last(p, t + 2 + kRegTiles, idx);
+                }
+            }
+            XS_PIN;
+        }
+    };
+    constexpr std::integral_constant<int, 0> even {};
+    constexpr std::integral_constant<int, 1> odd {};
+    using Main = Step<kWholeTile, true, true, kStages - 2>;
+
+    // The main steps load whole tiles; the kTail steps behind them load the last tile (kExact: it
+    // is like the others) or nothing, and the last reads no fragments.
+    constexpr int kTail = kDirect ? (kFit == Fit::kExact ? kStages : kStages + 1) : 3 + kRegTiles;
+    if (steps >= kTail) {
+        const int main_steps = steps - kTail;
+        int t = 0;
+#pragma unroll
+        for (int n = 0; n < 2 * kFrags; ++n) read_unit(0, 0, n);
+        if constexpr (kGuard) {
+            static_assert(kPollSteps == 4 && kStages <= kPollSteps + 2, "a request has landed by the last barrier in front of its look");
+            uint32_t slot = 0;
+            if (main_steps >= kPollSteps) request_flag(0);
+            for (; t + kPollSteps <= main_steps; t += kPollSteps) {
+                step(t, even, Main {}); step(t + 1, odd, Main {});
+                step(t + 2, even, Main {}); step(t + 3, odd, Main {});
+                if (!flag_is_current(slot)) {   // the same word in every wave: the group leaves together
+                    XS_WAIT_GLOBAL_LOADS;
+                    if (tid == 0) xguard_note_flush(g);
+                    return;
+                }
+                slot ^= 1;
+                request_flag(slot);
+            }
+        }
+        for (; t + 2 <= main_steps; t += 2) { step(t, even, Main {}); step(t + 1, odd, Main {}); }
+        auto tail = [&](auto first_parity) {
+            constexpr int p = decltype(first_parity)::value;
+            auto at = [&]<int j>(std::integral_constant<int, j>) {
+                constexpr int left = kTail - 1 - j;                              // steps behind this one
+                constexpr bool loads_last = kFit != Fit::kExact && j == 0;
+                constexpr int newer = left - 1 < 0 ? 0 : left - 1 < kStages - 2 ? left - 1 : kStages - 2;
+                using Do = Step<loads_last ? kLastTile : kNothing, (left >= 2), (left >= 1), newer>;
+                step(main_steps + j, std::integral_constant<int, (p + j) & 1> {}, Do {});
+            };
+            [&]<int... j>(std::integer_sequence<int, j...>) { (at(std::integral_constant<int, j> {}), ...); }(std::make_integer_sequence<int, kTail> {});
+        };
+        if (t < main_steps) {
+            step(t, even, Main {});
+            tail(odd);
+        } else {
+            tail(even);
+        }
+    } else {
+        // K of a few steps: everything is on its way (or here) already, and the fragments are
+        // read in front of their MFMAs.
+        if constexpr (kDirect) WaitLoadsAndLds<0>();
+        XS_BARRIER;
+        for (int t = 0; t < steps; ++t) {
+#pragma unroll
+            for (int n = 0; n < 2 * kFrags; ++n) read_unit(0, t, n);
+            if (kFit != Fit::kExact && t == steps - 1) mask_behind_k(0);
+#pragma unroll
+            for (int n = 0; n < kMfmas; ++n) mfma(0, n);
+            if constexpr (!kDirect) {
+                // the buffer just read takes the tile after the next one
+                WaitLoadsAndLds<0>();
+                XS_BARRIER;
+#pragma unroll
+                for (int idx = 0; idx < kLoads; ++idx) {
+                    if (t + 2 < steps) { if (t & 1) put_held(1, t + 2, idx); else put_held(0, t + 2, idx); }
+                }
+                WaitLoadsAndLds<0>();
+                XS_BARRIER;
+            }
+        }
+        XS_PIN;
+        WaitLoadsAndLds<0>();
+        XS_BARRIER;
+    }
+    if (kGuard) XS_WAIT_GLOBAL_LOADS;                      // the last look at the preempt word that nobody took
+
+    // ---- write-out, as above: strips of 32 rows x 32 kBlocks columns turned over in LDS ----
+    // (behind the last step's barrier nobody reads the tile buffers any more, and nothing is on
+    // its way into them)
+    constexpr int kStripColumnBytes = 64 + 8;
+    constexpr int kStripBytes = 32 * kBlocks * kStripColumnBytes;
+    static_assert(kBuffers * kTileBytes >= kWaves * kStripBytes, "the A buffers hold one strip per wave");
+    uint8_t *const strip = As0 + wave * kStripBytes;
+    const uint32_t put_at = (lane & 31) * kStripColumnBytes + 4 * (lane >> 5) * 2;
+    const uint32_t l16 = lane & 15, patch = lane >> 4;     // a patch: 4 rows x 32 columns per 16 lanes
+    constexpr int kRowsPerStore = 16 / kBlocks;
+    const uint32_t get_row = 4 * (patch / kBlocks), get_col = 32 * (patch % kBlocks);
+    const uint32_t get_at = (get_col + 8 * (l16 & 3) + (l16 >> 2)) * kStripColumnBytes + get_row * 2;
+#pragma unroll
+    for (int i = 0; i < kBlocks; ++i) {
+#pragma unroll
+        for (int j = 0; j < kBlocks; ++j) {
+#pragma unroll
+            for (int run = 0; run < 4; ++run) {
+                const uint32_t lo = f32x2_to_bf16x2_rne(acc[i][j][4 * run], acc[i][j][4 * run + 1]);
+                const uint32_t hi = f32x2_to_bf16x2_rne(acc[i][j][4 * run + 2], acc[i][j][4 * run + 3]);
+                *(u32x2 *)(strip + 32 * j * kStripColumnBytes + put_at + 8 * run * 2) = u32x2 { lo, hi };
+            }
+        }
+        const size_t row0 = m0 + 32 * kBlocks * wm + 32 * i;
+        const size_t col0 = n0 + 32 * kBlocks * wn + get_col + 8 * (l16 >> 2);
+#pragma unroll
+        for (int q = 0; q < 32 / kRowsPerStore; ++q) {
+            const uint8_t *p = strip + get_at + kRowsPerStore * q * 2;
+            const s16x4 left = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsS16x4 *)p);
+            const s16x4 right = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsS16x4 *)(p + 4 * kStripColumnBytes));
+            const s16x8 eight = __builtin_shufflevector(left, right, 0, 1, 2, 3, 4, 5, 6, 7);
+            const size_t row = row0 + kRowsPerStore * q + get_row + (l16 & 3);
+            uint16_t *const at = C + row * (size_t)N + col0;
+            if constexpr (kFit == Fit::kExact) {
+                __builtin_nontemporal_store(eight, (s16x8 *)at);
+            } else if (row < (size_t)M) {
+                if constexpr (kFit == Fit::kEdges) {
+                    if (col0 < (size_t)N) __builtin_nontemporal_store(eight, (s16x8 *)at);
+                } else if (col0 + 8 <= (size_t)N) {
+                    *(s16x8_any *)at = eight;
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) if (col0 + e < (size_t)N) at[e] = (uint16_t)eight[e];
+                }
+            }
+        }
+    }
+
+    if (kGuard) {
+        XGuardBlock guard(g, blockIdx.x, &guard_word);
+        guard.Commit();
+    }
+}
+#undef XS_BARRIER
+
+template <bool kGuard, Fit kFit, int kTile, int kStages>
+__global__ __launch_bounds__(256)
+void GemmDeepKernel(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B,
+                    uint16_t *__restrict__ C, int M, int N, int K, XGuardArgs g)
+{
+    GemmDeepBody<kGuard, kFit, kTile, kStages>(A, B, C, M, N, K, g);
+}
+
+
+// What the kernels above do not take: fewer than eight columns or fewer than eight elements of A
+// (less than one 16-byte piece to fetch), K or N above kMaxK (their 32-bit offsets). Any M, N, K >= 1,
+// any alignment of the three matrices to two bytes. 64 x 64 tiles of C, four waves of one 32x32
+// block each, K in steps of 32 (two slices of 16 through the same MFMA as above and in the same
+// order; what lies beyond K is zero). Every load and store is checked against the matrix; a
+// thread's eight neighbouring elements come as one 16-byte load where they lie inside the matrix
+// and are aligned, one by one otherwise. The guard is at entry only: a tile is short.
 constexpr int kAnyTile = 64;
 constexpr int kAnyK = 32;
 
 template <bool kGuard>
 __global__ __launch_bounds__(256)
 void GemmBf16AnyShapeKernel(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B,
-                            uint16_t *__restrict__ C, int M, int N, int K, uint32_t tiles_n, uint32_t first_wg,
-                            XGuardArgs g)
+                            uint16_t *__restrict__ C, int M, int N, int K, uint32_t tiles_n, XGuardArgs g)
 {
     // a row of 32 k values padded to 40: 80-byte rows, every 16-byte fragment aligned
     __shared__ __attribute__((aligned(16))) uint16_t a_rows[kAnyTile][kAnyK + 8];
     __shared__ __attribute__((aligned(16))) uint16_t b_cols[kAnyTile][kAnyK + 8];   // B transposed: [column][k]
     __shared__ uint32_t guard_word;
 
-    XGuardBlock guard(g, first_wg + blockIdx.x, &guard_word);   // its progress bytes follow the fast kernel's
+    XGuardBlock guard(g, blockIdx.x, &guard_word);
     if (kGuard && !guard.Enter()) return;
 
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -489,87 +956,104 @@ void GemmBf16AnyShapeKernel(const uint16_t *__restrict__ A, const uint16_t *__re
     if (kGuard) guard.Commit();
 }
 
-/// Rows [0, rows_fast) of C go to the fast kernel with tiles of fast_tile (rows_fast is then a
-/// multiple of it and the shape one the fast kernel takes), rows [rows_fast, M) to the any-shape
-/// kernel; either part may be empty. The progress map holds the fast kernel's tiles first.
+/// How a command computes its product: which kernel, on tiles of which size, and what it may
+/// assume about the matrices.
+struct Plan
+{
+    int tile;       // edge of a tile of C
+    Fit fit;        // of the kernels with 256, 128 and 64 tiles
+    bool narrow;    // the kernel without requirements
+    uint64_t tiles; // work-groups = bytes of the progress map
+};
+
 class HipGemmCommand final : public HipGuardedCommand
 {
 public:
-    HipGemmCommand(const void *A, const void *B, void *C, int M, int N, int K, int rows_fast, int fast_tile, int guard_mode)
-        : HipGuardedCommand(FastTiles(rows_fast, N, fast_tile) + AnyTiles(M - rows_fast, N), guard_mode)
-        , A_((const uint16_t *)A), B_((const uint16_t *)B), C_((uint16_t *)C), M_(M), N_(N), K_(K)
-        , rows_fast_(rows_fast), fast_tile_(fast_tile) {}
-
-    static uint32_t FastTiles(int rows, int N, int tile) { return rows > 0 ? (uint32_t)(rows / tile) * (uint32_t)(N / tile) : 0u; }
-    static uint32_t AnyTiles(int rows, int N)
-    {
-        return rows > 0 ? (uint32_t)((rows + kAnyTile - 1) / kAnyTile) * (uint32_t)((N + kAnyTile - 1) / kAnyTile) : 0u;
-    }
+    HipGemmCommand(const void *A, const void *B, void *C, int M, int N, int K, const Plan &plan, int guard_mode)
+        : HipGuardedCommand((uint32_t)plan.tiles, guard_mode)
+        , A_((const uint16_t *)A), B_((const uint16_t *)B), C_((uint16_t *)C), M_(M), N_(N), K_(K), plan_(plan) {}
 
 protected:
     virtual hipError_t LaunchKernel(hipStream_t stream, bool guarded, const XGuardArgs &g) override
     {
-        const uint32_t fast_tiles = FastTiles(rows_fast_, N_, fast_tile_), any_tiles = AnyTiles(M_ - rows_fast_, N_);
-        const hipEvent_t stop = TakeStopEvent();   // for the command's last kernel
-        if (fast_tiles != 0) {
-            const hipEvent_t mine = any_tiles == 0 ? stop : nullptr;
-            const dim3 grid(fast_tiles);
-            if (fast_tile_ == kLargeTile) {
-                const dim3 block(512);
-                if (guarded) LaunchWithStop(mine, (GemmBf16Kernel<true, kLargeTile, 2, 4>), grid, block, stream, A_, B_, C_, rows_fast_, N_, K_, g);
-                else         LaunchWithStop(mine, (GemmBf16Kernel<false, kLargeTile, 2, 4>), grid, block, stream, A_, B_, C_, rows_fast_, N_, K_, g);
-            } else {
-                const dim3 block(256);
-                if (guarded) LaunchWithStop(mine, (GemmBf16Kernel<true, kSmallTile, 2, 2>), grid, block, stream, A_, B_, C_, rows_fast_, N_, K_, g);
-                else         LaunchWithStop(mine, (GemmBf16Kernel<false, kSmallTile, 2, 2>), grid, block, stream, A_, B_, C_, rows_fast_, N_, K_, g);
-            }
-            const hipError_t err = hipGetLastError();
-            if (err != hipSuccess || any_tiles == 0) return err;
+        if (plan_.narrow) {
+            const uint32_t tiles_n = (uint32_t)((N_ + kAnyTile - 1) / kAnyTile);
+            const dim3 grid((uint32_t)plan_.tiles), block(256);
+            const hipEvent_t stop = TakeStopEvent();
+            if (guarded) LaunchWithStop(stop, GemmBf16AnyShapeKernel<true>, grid, block, stream, A_, B_, C_, M_, N_, K_, tiles_n, g);
+            else         LaunchWithStop(stop, GemmBf16AnyShapeKernel<false>, grid, block, stream, A_, B_, C_, M_, N_, K_, tiles_n, g);
+        } else if (plan_.tile == kLargeTile) {
+            Launch(guarded ? GemmBf16Kernel<true, kLargeTile, 2, 4> : GemmBf16Kernel<false, kLargeTile, 2, 4>, 512, stream, g);
+        } else if (plan_.tile == kSmallTile) {
+            LaunchDeep<kSmallTile, 4>(stream, guarded, g);
+        } else {
+            LaunchDeep<kTinyTile, 4>(stream, guarded, g);
         }
-        const dim3 grid(any_tiles), block(256);
-        const uint32_t tiles_n = (uint32_t)((N_ + kAnyTile - 1) / kAnyTile);
-        const uint16_t *a = A_ + (size_t)rows_fast_ * (size_t)K_;
-        uint16_t *c = C_ + (size_t)rows_fast_ * (size_t)N_;
-        const int rows = M_ - rows_fast_;
-        if (guarded) LaunchWithStop(stop, GemmBf16AnyShapeKernel<true>, grid, block, stream, a, B_, c, rows, N_, K_, tiles_n, fast_tiles, g);
-        else         LaunchWithStop(stop, GemmBf16AnyShapeKernel<false>, grid, block, stream, a, B_, c, rows, N_, K_, tiles_n, fast_tiles, g);
         return hipGetLastError();
     }
 
 private:
+    using Kernel = void (*)(const uint16_t *, const uint16_t *, uint16_t *, int, int, int, XGuardArgs);
+    void Launch(Kernel kernel, unsigned threads, hipStream_t stream, const XGuardArgs &g)
+    {
+        LaunchWithStop(TakeStopEvent(), kernel, dim3((uint32_t)plan_.tiles), dim3(threads), stream, A_, B_, C_, M_, N_, K_, g);
+    }
+    template <int kTile, int kStages>
+    void LaunchDeep(hipStream_t stream, bool guarded, const XGuardArgs &g)
+    {
+        switch (plan_.fit) {
+        case Fit::kExact:
+            return Launch(guarded ? GemmDeepKernel<true, Fit::kExact, kTile, kStages> : GemmDeepKernel<false, Fit::kExact, kTile, kStages>, 256, stream, g);
+        case Fit::kEdges:
+            return Launch(guarded ? GemmDeepKernel<true, Fit::kEdges, kTile, kStages> : GemmDeepKernel<false, Fit::kEdges, kTile, kStages>, 256, stream, g);
+        case Fit::kUnaligned:
+            return Launch(guarded ? GemmDeepKernel<true, Fit::kUnaligned, kTile, kStages> : GemmDeepKernel<false, Fit::kUnaligned, kTile, kStages>, 256, stream, g);
+        }
+    }
+
     const uint16_t *A_, *B_;
     uint16_t *C_;
     const int M_, N_, K_;
-    const int rows_fast_, fast_tile_;
+    const Plan plan_;
 };
 
-/// The tile edge for an M x N output: large tiles do more arithmetic per byte read from LDS,
-/// but each one keeps a single compute unit busy, so an output of few large tiles leaves most
-/// of the device idle. Small tiles when the large ones would cover at most half of the compute
-/// units, or when M or N is no multiple of the large edge. XSCHED_HIP_GEMM_TILE=128|256
-/// overrides the choice where the shape allows.
-inline int TileFor(int M, int N);
-
-/// Whether the fast kernels take the shape and the pointers.
-inline bool FastKernelsTake(const void *A, const void *B, const void *C, int M, int N, int K)
+inline uint64_t TilesOf(int M, int N, int tile)
 {
-    return M % kSmallTile == 0 && N % kSmallTile == 0 && K % kStepK == 0 && K <= kMaxK && N <= kMaxK &&
-           (((uintptr_t)A | (uintptr_t)B | (uintptr_t)C) & 15) == 0;
+    return ((uint64_t)M + (unsigned)tile - 1) / (unsigned)tile * (((uint64_t)N + (unsigned)tile - 1) / (unsigned)tile);
 }
 
-inline int TileFor(int M, int N)
+inline uint32_t ComputeUnits()
 {
-    const bool large_fits = M % kLargeTile == 0 && N % kLargeTile == 0;
-    if (!large_fits) return kSmallTile;
-    int64_t forced = 0;
-    if (GetEnvInt64("XSCHED_HIP_GEMM_TILE", forced) && (forced == kSmallTile || forced == kLargeTile)) return (int)forced;
-    static const int cus = []() {
+    static const uint32_t cus = []() {
         int dev = 0, n = 256;
         if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev);
-        return n > 0 ? n : 256;
+        return (uint32_t)(n > 0 ? n : 256);
     }();
-    const int64_t large_tiles = (int64_t)(M / kLargeTile) * (N / kLargeTile);
-    return large_tiles * 2 <= cus ? kSmallTile : kLargeTile;
+    return cus;
+}
+
+/// The plan for a shape. Large tiles do more arithmetic per byte read from LDS, but each keeps one
+/// compute unit busy, and so does a small one: large tiles when they cover more than half of the
+/// compute units (4096^3: 101 us against 119 on small tiles; 2048^3, a quarter covered: 41 against
+/// 17.8), small ones when they cover more than half (2048^3: 17.8 us against 27.7 on tiny tiles;
+/// 1024^3, a quarter covered: 9.4 against 5.8), else tiny ones. The large tiles take exact
+/// multiples only. XSCHED_HIP_GEMM_TILE=64|128|256 overrides the tile where the shape allows.
+inline Plan PlanFor(const void *A, const void *B, const void *C, int M, int N, int K)
+{
+    if (N < 8 || (int64_t)M * K < 8 || K > kMaxK || N > kMaxK) return Plan { kAnyTile, Fit::kUnaligned, true, TilesOf(M, N, kAnyTile) };
+    const bool aligned = (((uintptr_t)A | (uintptr_t)B | (uintptr_t)C) & 15) == 0 && N % 8 == 0 && K % 8 == 0;
+    auto exact = [&](int tile) { return aligned && M % tile == 0 && N % tile == 0 && K % kStepK == 0; };
+    int tile = kSmallTile;
+    int64_t forced = 0;
+    if (GetEnvInt64("XSCHED_HIP_GEMM_TILE", forced) &&
+        (forced == kTinyTile || forced == kSmallTile || (forced == kLargeTile && exact(kLargeTile)))) {
+        tile = (int)forced;
+    } else if (exact(kLargeTile) && TilesOf(M, N, kLargeTile) * 2 > ComputeUnits()) {
+        tile = kLargeTile;
+    } else if (TilesOf(M, N, kSmallTile) * 2 <= ComputeUnits()) {
+        tile = kTinyTile;
+    }
+    return Plan { tile, exact(tile) ? Fit::kExact : aligned ? Fit::kEdges : Fit::kUnaligned, false, TilesOf(M, N, tile) };
 }
 
 } // namespace gemm
@@ -588,23 +1072,13 @@ EXPORT_C_FUNC XResult HipGemmBf16CommandCreate(HwCommandHandle *cmd, const void 
         XWARN("HipGemmBf16CommandCreate: M, N and K must be positive and the matrices aligned to their elements (got %d %d %d)", M, N, K);
         return kXSchedErrorInvalidValue;
     }
-    // The fast kernels take M and N in multiples of 128, K in multiples of 64 (K and N at most
-    // 2^22) and matrices aligned to 16 bytes. Where only M stands in the way, they take the
-    // rows up to the last multiple of 128 and the any-shape kernel the rest (the rows of a
-    // row-major matrix can be cut anywhere); every other shape goes to the any-shape kernel whole.
-    int64_t forced = 0;
-    const bool force_any = GetEnvInt64("XSCHED_HIP_GEMM_TILE", forced) && forced == gemm::kAnyTile;
-    const int whole_rows = M / gemm::kSmallTile * gemm::kSmallTile;
-    int rows_fast = 0;
-    if (!force_any && whole_rows > 0 && gemm::FastKernelsTake(A, B, C, whole_rows, N, K)) rows_fast = whole_rows;
-    const int fast_tile = rows_fast > 0 ? gemm::TileFor(rows_fast, N) : gemm::kSmallTile;
-    // one progress-map byte per tile
-    const uint64_t tiles = (uint64_t)gemm::HipGemmCommand::FastTiles(rows_fast, N, fast_tile) +
-                           (uint64_t)((M - rows_fast + gemm::kAnyTile - 1) / gemm::kAnyTile) * (uint64_t)((N + gemm::kAnyTile - 1) / gemm::kAnyTile);
+    const gemm::Plan plan = gemm::PlanFor(A, B, C, M, N, K);
+    // one progress-map byte per tile; a shape without alignment is held to the limit in 64 x 64 tiles
+    const uint64_t tiles = plan.fit == gemm::Fit::kUnaligned ? gemm::TilesOf(M, N, gemm::kAnyTile) : plan.tiles;
     if (tiles > GuardState::kMaxWorkGroups) {
         XWARN("HipGemmBf16CommandCreate: %d x %d needs more than 2^18 tiles", M, N);
         return kXSchedErrorInvalidValue;
     }
-    *cmd = HwCommandManager::Add(std::make_shared<gemm::HipGemmCommand>(A, B, C, M, N, K, rows_fast, fast_tile, guard));
+    *cmd = HwCommandManager::Add(std::make_shared<gemm::HipGemmCommand>(A, B, C, M, N, K, plan, guard));
     return kXSchedSuccess;
 }
