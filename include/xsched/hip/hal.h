@@ -100,7 +100,7 @@ XResult HipHistogramCommandCreate(HwCommandHandle *cmd, const void *keys, size_t
                                   uint32_t n_bins, int guard);
 
 /* The same histogram (bins[keys[i]] += 1, bins not cleared) enqueued on `stream` (a
- * hipStream_t; NULL = the default stream) directly, as two plain kernel launches, by an entry
+ * hipStream_t; NULL = the default stream) directly, as one or two plain kernel launches, by an entry
  * point that allocates nothing: no hipMalloc / hipFree, no pool, no XQueue, no command object.
  * No counterpart in the reference. It is for callers that cannot allocate device memory where
  * they call it: code under HIP graph capture, tight serving loops, harnesses that forbid

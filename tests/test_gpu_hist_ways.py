@@ -1,0 +1,37 @@
+"""GPU parity of the histogram where it changes its ways by itself: few keys, one kernel or two,
+whole-word, half-word and byte counters, and key arrays at any multiple of four bytes."""
+import numpy as np
+import pytest
+
+import oracle
+from test_gpu_kernels import Queue, hist_cmd
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n_bins", [1, 255, 256, 257, 16383, 16384, 16385, 32768, 32769, 49153, 65536])
+@pytest.mark.parametrize("n,offset", [(1, 0), (1023, 1), (1024, 0), (1025, 3), (1 << 16, 0), ((1 << 16) + 1, 2), (1 << 18, 1),
+                                      ((1 << 21) + 4099, 0)])
+@pytest.mark.parametrize("level,guard", [(1, 0), (2, 1)])
+def test_histogram_ways_by_size_and_bins(xs, gpu, n, offset, n_bins, level, guard):
+    """Counts are whole numbers: bit for bit the oracle's. One key in eight is the last bin (it
+    fills a byte counter several times over from 2048 keys of a group on), a few lie outside
+    the bins and count nowhere; twice, since bins are added to."""
+    torch = gpu
+    print(f"case hist-ways n={n} offset={offset} bins={n_bins} level={level} guard={guard}", flush=True)
+    rng = np.random.default_rng(n + n_bins)
+    keys_h = rng.integers(0, n_bins, n).astype(np.int32)
+    keys_h[rng.random(n) < 0.125] = n_bins - 1
+    outside = rng.random(n) < 0.01
+    keys_h[outside] = rng.choice(np.array([-1, n_bins, n_bins + 16384, 1 << 30], np.int32), int(outside.sum()))
+    keys = torch.from_numpy(np.concatenate([np.zeros(offset, np.int32), keys_h])).cuda()[offset:]
+    bins = torch.zeros(n_bins + 1, dtype=torch.int32, device="cuda")
+    q = Queue(xs, torch, level)
+    for _ in range(2):
+        q.submit(hist_cmd(xs, keys, n, bins, n_bins, guard))
+    q.wait()
+    got = bins.cpu().numpy().view(np.uint32)
+    q.close()
+    want = oracle.histogram(keys_h[~outside], n_bins)
+    assert np.array_equal(got[:n_bins], 2 * want)
+    assert got[n_bins] == 0, "wrote beyond the bins array"

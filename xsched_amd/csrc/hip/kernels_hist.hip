@@ -12,43 +12,39 @@
 //
 // One work-group of 1024 threads per compute unit owns a contiguous chunk of keys
 // (sized so that a launch has about one work-group per CU) and keeps everything it
-// counts on chip until the end. Keys < kHotBins are counted by wave ballot + popcount
-// into scalar registers: for skewed (Zipf-like) keys these few bins take a quarter of
-// all keys and would otherwise serialise the LDS atomics of a wave on one address.
-// The other keys go to LDS counters, in one of two layouts:
+// counts on chip until the end, in 128 KiB of LDS counters split in two. Bins below 256 (two
+// thirds of all Zipf(1.1) keys, a fifth of them in bins 0 and 1) have one 32-bit counter PER
+// LANE: 256 bins x 64 lanes, so the lanes of a wave never add to the same address for them, no
+// vote and no popcount is needed, and they cannot overflow. Every other bin shares one of 16384
+// words with the bins 16384, 32768 and 49152 above it, as far as there are such bins: a BYTE
+// each when n_bins > 32768, a half word each when n_bins > 16384, the whole word otherwise; one
+// ds_add of 1 << (width * (key >> 14)) per key. One vote per iteration tells whether every key
+// of the wave is below n_bins, so the add needs no branch.
 //
-// Two kernels (kMerge; the layout in use up to 2^28 keys). The group's 128 KiB of LDS
-// counters are split in two. Bins below 256 (two thirds of all Zipf(1.1) keys, a fifth of
-// them in bins 0 and 1) have one 32-bit counter PER LANE: 256 bins x 64 lanes, so the lanes of
-// a wave never add to the same address for them, no vote and no popcount is needed, and they
-// cannot overflow. Every other bin is a BYTE: 16384 words shared by the group, word w counts
-// bins w, w + 16384, w + 32768, w + 49152 in its bytes 0..3, one ds_add of
-// 1 << 8 * (key >> 14) per key. One vote per iteration tells whether every key of the wave is
-// below n_bins, so the add needs no branch. The group then stores a partial histogram of
-// 65 KiB (the byte words as they are, the per-lane counters summed) into a scratch buffer,
-// and a second kernel sums the partials column by column and adds the totals to the result
-// with one 64-bit atomic per pair of bins. A byte overflows only when one bin outside the
-// first 256 takes 256 keys of a chunk (0.1 % of it; the hottest such bin of a Zipf(1.1)
-// chunk takes 80). Every overflow lowers the sum of all counters by at least 255 and nothing
-// raises it, so "sum of counters == keys that must be in them" (all key slots of the chunk
-// minus the invalid ones) proves there was none; a group that fails the test stores an
-// all-zero partial and recounts its chunk the slow way (32-bit counters, two passes over its
-// keys, atomic sweep into the result). The first version of this layout kept 16-bit halves
-// for every bin and ballot counters for bins 0 and 1: partials of 128 KiB (32 MiB written
-// and read back per 2^26 keys, now 16.25 MiB), 14 vector instructions per key (now 10), and
-// LDS adds that serialised on the hot bins.
+// A byte overflows only when one bin outside the first 256 takes 256 keys of a chunk (0.1 % of
+// it; the hottest such bin of a Zipf(1.1) chunk takes 80), a half when it takes 65536. Every
+// overflow lowers the sum of all counters by at least 255 and nothing raises it, so "sum of
+// counters == keys that must be in them" (all key slots of the chunk minus the invalid ones)
+// proves there was none; a group that fails the test recounts its chunk the slow way (32-bit
+// counters, two passes over its keys, atomic sweep into the result). Whole words need no test:
+// with bytes for any n_bins, 2^26 evenly spread keys over 1000 bins overflowed in every group
+// (262 keys of a chunk to a bin) and took 182 us instead of 49.
 //
-// One kernel (above 2^28 keys, where the partials would need more than 128 MiB of
-// scratch, when the scratch buffer cannot be allocated, or on request through
-// XSCHED_HIP_HIST_MERGE_MIN_KEYS). The group keeps 32-bit counters for bins < 32768,
-// appends the rarer keys above that as 16-bit values to an LDS list (one list
-// reservation per wave and iteration), and merges by itself: a sweep of atomic adds
-// over its non-zero counters (a wave covers 256 consecutive bins, so the adds arrive
-// line by line; each group starts its sweep at a different segment because atomics on
-// ONE cache line retire at only ~0.1 G/s); then the same 128 KiB are cleared, the
-// listed keys are counted into them and swept out the same way. If the list
-// overflows (an adversarial distribution), the group re-reads its chunk for those
-// keys instead.
+// What becomes of a group's counts (PlanFor() chooses, with the figures):
+//   few keys over many bins: another kernel, HistogramFewKeysKernel below.
+//   one kernel (few bins, or few groups): the group adds its non-zero counters to the result itself, the 64
+//       lanes of a wave to 64 neighbouring bins, each group from another place on because
+//       atomics on ONE cache line retire at only ~0.1 G/s. Also above 2^28 keys, where the
+//       partials would need more than 128 MiB of scratch, and when the scratch buffer cannot
+//       be allocated.
+//   two kernels (kMerge): the group stores a partial histogram of 65 KiB (less when n_bins is
+//       below 16384; the words as they are, the per-lane counters summed) into a scratch
+//       buffer, and a second kernel sums the partials column by column and adds the totals to
+//       the result with one atomic per bin.
+// The first version of this layout kept 16-bit halves for every bin and ballot counters for
+// bins 0 and 1: partials of 128 KiB (32 MiB written and read back per 2^26 keys, now
+// 16.25 MiB), 14 vector instructions per key (now 10), and LDS adds that serialised on the hot
+// bins.
 //
 // Guard: entry check, and because a group has no side effects before its write-out,
 // every wave re-reads the preempt word every 32768 keys of the group and the group abandons
@@ -61,6 +57,8 @@
 // their entry check on a copy of the preempt word that has not been rewritten yet while
 // this command is already flushed). Integer adds commute, so the result does not depend on the order in which work-groups (or
 // replays) run.
+#include <cmath>
+
 #include "hip_hal.h"
 #include "xsched/hip/hal.h"
 
@@ -73,13 +71,7 @@ namespace hist
 {
 
 constexpr uint32_t kThreads = 1024;
-constexpr uint32_t kWaves = kThreads / 64;
-#ifndef XSCHED_HIST_HOT_BINS
-#define XSCHED_HIST_HOT_BINS 2
-#endif
-constexpr uint32_t kHotBins = XSCHED_HIST_HOT_BINS;
 constexpr uint32_t kLdsBins = 1u << 15;       // 128 KiB of counters
-constexpr uint32_t kTailCap = 14336;          // 16-bit entries, 28 KiB
 #ifndef XSCHED_HIST_UNITS
 #define XSCHED_HIST_UNITS 1
 #endif
@@ -97,25 +89,24 @@ constexpr uint32_t kIterKeys = kUnitKeys * kUnits;
 constexpr uint32_t kMinChunk = kUnitKeys;
 constexpr uint32_t kMaxChunk = 1u << 18;
 constexpr uint32_t kTargetGroups = 256;       // compute units of an MI355X
-constexpr uint32_t kSegBins = 256;            // bins one wave sweeps per step
-constexpr uint32_t kSegs = kLdsBins / kSegBins;
-// merge layout
-constexpr uint32_t kColdWords = 1u << 14;           // byte counters: word w, byte b = bin w + b * 16384
+constexpr uint32_t kFewThreads = 256;         // HistogramFewKeysKernel: threads
+constexpr uint32_t kFewKeys = kFewThreads * 4;        // keys per work-group
+constexpr uint64_t kFewMaxKeys = 1u << 16;            // and the most keys it is used for
+constexpr uint32_t kColdWords = 1u << 14;           // word w counts bins w + i * 16384
 constexpr uint32_t kWarmBins = 256;                 // bins below this have 32-bit counters of their own
-constexpr uint32_t kCountWords = kColdWords + kWarmBins * 64;   // LDS words in use: byte words, then a counter per warm bin and lane
-static_assert(kCountWords <= kLdsBins, "the merge layout's counters fit the group's LDS array");
+static_assert(kColdWords + kWarmBins * 64 <= kLdsBins, "the cold words, then a counter per warm bin and lane");
 // The partial histograms of a launch in memory, n_part of them (one per counting group): the
-// byte words column by column, one column per merge group, and within a column partial by
+// cold words column by column, one column per merge group, and within a column partial by
 // partial: column c of partial p is the 64 words (256 bytes, two whole cache lines) at
 // ((c * n_part) + p) * 64. A merge group therefore reads ONE contiguous run of n_part * 256
 // bytes, and a counting group stores its partial as 256 pieces of two lines each. (Partial by
 // partial, column by column inside, a merge group read 272 bytes out of every 68 KiB: three
-// lines touched for two and a bit used, 1.41 times its bytes in traffic.) Behind the byte
-// words: the counts of bins 0..255, which are kept outside the bytes, partial by partial
-// (1 KiB each).
+// lines touched for two and a bit used, 1.41 times its bytes in traffic.) Behind the cold
+// words: the counts of bins 0..255, which are kept outside them, partial by partial
+// (1 KiB each). Columns that n_bins leaves empty are neither stored nor read.
 constexpr uint32_t kMergeGroups = 256;
 constexpr uint32_t kMergeThreads = 256;             // threads of a merge group
-constexpr uint32_t kMergeWords = kColdWords / kMergeGroups;          // byte words per column (64)
+constexpr uint32_t kMergeWords = kColdWords / kMergeGroups;          // cold words per column (64)
 constexpr uint32_t kPartialWords = kColdWords + kWarmBins;           // 65 KiB of scratch per counting group
 
 /// Where column `column` of partial `p` lies, and where that partial's 256 outside counts do.
@@ -128,12 +119,18 @@ __host__ __device__ inline size_t OutsideAt(uint32_t p, uint32_t n_part)
     return (size_t)n_part * kColdWords + (size_t)p * kWarmBins;
 }
 constexpr uint32_t kMaxPartials = 1024;
-static_assert(kWarmBins == kMergeGroups && kHotBins <= kWarmBins, "column j carries the outside count of bin j");
-constexpr uint64_t kMergeMinKeys = 1;             // the two-kernel layout wins at every size measured
-constexpr uint32_t kMergeMinChunk = 16384;        // fewer, fuller partials for small inputs
-
+static_assert(kWarmBins == kMergeGroups, "column j carries the outside count of bin j");
 typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef i32x4 i32x4_any __attribute__((aligned(4)));   // keys may start at any int32
+
+/// How many cold words n_bins bins use: whole columns.
+__host__ __device__ inline uint32_t ColdWordsOf(uint32_t n_bins)
+{
+    return n_bins >= kColdWords ? kColdWords : (n_bins + kMergeWords - 1) / kMergeWords * kMergeWords;
+}
+/// log2 of a cold counter's bits; with at most 16384 bins nothing is ever shifted by it.
+__host__ __device__ inline uint32_t ColdWidthLog2(uint32_t n_bins) { return n_bins > 2 * kColdWords ? 3 : 4; }
 
 /// Keys per work-group for a histogram of n keys: a multiple of kMinChunk, at least
 /// `floor` (rounded up to one).
@@ -147,15 +144,44 @@ inline uint32_t ChunkFor(uint64_t n, uint64_t floor = kMinChunk)
     return (uint32_t)c;
 }
 
+/// The least keys per work-group: a launch takes as long as its longest group (the more keys
+/// the longer) plus what all groups together write out (the more groups the longer), which balances
+/// where the keys of a group grow with the square root of all. Measured best: 2^18 keys 8192
+/// (10.6 us; 16384: 10.8, 4096: 11.1), 2^20 16384 (12.1; 13.0, 13.4), 2^22 32768 to 65536 (16.5;
+/// 16384: 17.5), and about the same with few bins (2^20 over 1000 bins: 8192 6.3 us, 16384 5.8,
+/// 32768 6.5).
+inline uint64_t ChunkFloor(uint64_t n) { return (uint64_t)(16.0 * std::sqrt((double)n)); }
+
+enum class Way { kFew, kSweep, kMerge };
+
+/// How n keys are counted (see the head of this file), in work-groups of `chunk` keys.
+struct Plan { Way way; uint32_t chunk; uint64_t groups; };
+
+/// - Few keys and many bins: HistogramFewKeysKernel. 16384 Zipf keys over 65536 bins take 3.8 us
+///   (two kernels: 10.4), 65536 take 7.2, evenly spread 5.4 (10.5); 131072 take 11.8 (10.7).
+/// - One kernel while the groups' sweeps are short, in wave-wide atomics of 64 neighbouring bins:
+///   at most 768 per group (7 ns each; a whole 65536 bins is 1024: 12.5 us against 10.5 for two
+///   kernels at 65536 keys), and 2^16 of all groups together (2^24 keys over 16000 bins, 2^16:
+///   22.8 us against 23.8; over 20000 bins, 2^17: 28.8 against 24.6; over 1000 bins: 15.8
+///   against 16.7; 2^18 keys over 1000 bins: 4.6 against 8.5).
+/// - Two kernels otherwise.
+inline Plan PlanFor(uint64_t n, uint32_t n_bins)
+{
+    if (n <= kFewMaxKeys && n_bins > kColdWords) return Plan { Way::kFew, kFewKeys, (n + kFewKeys - 1) / kFewKeys };
+    const uint32_t chunk = ChunkFor(n, ChunkFloor(n));
+    const uint64_t groups = (n + chunk - 1) / chunk;
+    const uint64_t atomics = n_bins < kColdWords ? (n_bins + 63) / 64 : (uint64_t)((n_bins + kColdWords - 1) / kColdWords) * (kColdWords / 64);
+    const bool sweep = (atomics <= 768 && groups * atomics <= (1u << 16)) || groups > kMaxPartials;
+    return Plan { sweep ? Way::kSweep : Way::kMerge, chunk, groups };
+}
+
 struct Shared
 {
     uint32_t bins[kLdsBins];
-    uint16_t tail[kTailCap];
-    uint32_t tail_count;
     uint32_t bailed;
     uint32_t guard_word;
-    uint32_t invalid;       // merge layout: keys outside [0, n_bins), absent ones included
-    uint32_t sum;           // merge layout: sum of all packed counters
+    uint32_t invalid;       // keys outside [0, n_bins), absent ones included
+    uint32_t sum;           // sum of all counters
 };
 
 __device__ __forceinline__ void LdsAdd(uint32_t *p, uint32_t v)
@@ -168,99 +194,40 @@ __device__ __forceinline__ void GlobalAdd(uint32_t *p, uint32_t v)
     __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-/// dst[0] += lo, dst[1] += hi with ONE 64-bit atomic (dst is 8-byte aligned): the
-/// write-out is bound by the number of atomic operations, and this halves it. The two
-/// counters stay independent 32-bit values: should the low one wrap, the returned old
-/// value shows it and the carry that leaked into the high one is taken back (PairFix).
-/// Issue and check are separate calls so that a sweep has all its atomics in flight
-/// before it looks at the first returned value.
-__device__ __forceinline__ uint32_t PairAdd(uint32_t *dst, uint32_t lo, uint32_t hi)
+__device__ __forceinline__ void ClearBins(Shared &sh, uint32_t first, uint32_t end)
 {
-    return (uint32_t)__hip_atomic_fetch_add((unsigned long long *)dst, ((unsigned long long)hi << 32) | lo,
-                                            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (uint32_t i = first + threadIdx.x * 4; i < end; i += kThreads * 4) *(u32x4 *)&sh.bins[i] = u32x4 { 0, 0, 0, 0 };
 }
 
-__device__ __forceinline__ void PairFix(uint32_t *dst, uint32_t old_lo, uint32_t lo)
-{
-    if ((uint32_t)(old_lo + lo) < lo) GlobalAdd(dst + 1, 0xFFFFFFFFu);
-}
-
-/// acc += popcount(mask), issued where it is written. Left to the compiler, the
-/// popcounts of a whole iteration sink below the per-key branches and their 64-bit
-/// lane masks are spilled and reloaded.
-__device__ __forceinline__ void AddPopcount(uint32_t &acc, uint64_t mask)
-{
-    uint32_t tmp;
-    asm volatile("s_bcnt1_i32_b64 %1, %2\n\ts_add_u32 %0, %0, %1" : "+s"(acc), "=&s"(tmp) : "s"(mask) : "scc");
-}
-
-/// Adds the non-zero counters of sh.bins[0, count) to dst[0, count), never touching
-/// memory at or beyond dst + count. Wave q of the group sweeps segments rot + q,
-/// rot + q + 16, ... (mod kSegs), so groups that write out at the same time start on
-/// different cache lines.
-__device__ __forceinline__ void SweepOut(Shared &sh, uint32_t *dst, uint32_t count, uint32_t rot)
-{
-    constexpr uint32_t kSteps = kSegs / kWaves;
-    const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const bool pair_ok = (((uintptr_t)dst) & 7) == 0; // segment starts are even indices
-    uint32_t low[kSteps][2], old[kSteps][2];
-#pragma unroll
-    for (uint32_t step = 0; step < kSteps; ++step) {
-        const uint32_t seg = (rot + step * kWaves + wave) & (kSegs - 1);
-        const uint32_t b4 = seg * kSegBins + lane * 4;
-        // counters at or beyond `count` are never incremented, so they read zero
-        const u32x4 c = b4 < count ? *(const u32x4 *)&sh.bins[b4] : u32x4 { 0, 0, 0, 0 };
-        const uint32_t v[4] = { c.x, c.y, c.z, c.w };
-#pragma unroll
-        for (uint32_t p = 0; p < 2; ++p) {
-            const uint32_t i = b4 + p * 2, lo = v[p * 2], hi = v[p * 2 + 1];
-            low[step][p] = 0;
-            old[step][p] = 0;
-            if ((lo | hi) == 0) continue;
-            if (pair_ok && i + 1 < count) {
-                low[step][p] = lo;
-                old[step][p] = PairAdd(dst + i, lo, hi);
-            } else {
-                if (lo != 0 && i < count) GlobalAdd(dst + i, lo);
-                if (hi != 0 && i + 1 < count) GlobalAdd(dst + i + 1, hi);
-            }
-        }
-    }
-#pragma unroll
-    for (uint32_t step = 0; step < kSteps; ++step) {
-        const uint32_t seg = (rot + step * kWaves + wave) & (kSegs - 1);
-        const uint32_t b4 = seg * kSegBins + lane * 4;
-#pragma unroll
-        for (uint32_t p = 0; p < 2; ++p) PairFix(dst + b4 + p * 2, old[step][p], low[step][p]);
-    }
-}
-
-__device__ __forceinline__ void ClearBins(Shared &sh, uint32_t words = kLdsBins)
-{
-    for (uint32_t i = threadIdx.x * 4; i < words; i += kThreads * 4) *(u32x4 *)&sh.bins[i] = u32x4 { 0, 0, 0, 0 };
-}
-
-/// Merge layout: where a valid key is counted, and by how much. Bins below kWarmBins (two
-/// thirds of all Zipf(1.1) keys) have one 32-bit counter PER LANE, so the lanes of a wave never
-/// add to the same address for them; every other bin is a byte of a word shared by the group.
-__device__ __forceinline__ void PackedSlot(uint32_t key, uint32_t lane, uint32_t &word, uint32_t &inc)
+/// Where a valid key is counted, and by how much (see the head of this file).
+__device__ __forceinline__ void PackedSlot(uint32_t key, uint32_t lane, uint32_t width_log2, uint32_t &word, uint32_t &inc)
 {
     const bool warm = key < kWarmBins;
     word = warm ? kColdWords + key * 64 + lane : key & (kColdWords - 1);
-    inc = warm ? 1u : 1u << ((key >> 11) & 24u);
+    inc = 1u << ((key >> 14) << width_log2);
 }
 
-/// Sum of the four byte counters of each of four packed words.
-__device__ __forceinline__ uint32_t ByteSum(const u32x4 &w)
+/// Sum of the counters (bytes or halves) of four cold words.
+__device__ __forceinline__ uint32_t ColdSum(const u32x4 &w, bool bytes)
 {
+    if (!bytes) {
+        return (w.x & 0xFFFFu) + (w.x >> 16) + (w.y & 0xFFFFu) + (w.y >> 16) + (w.z & 0xFFFFu) + (w.z >> 16) + (w.w & 0xFFFFu) + (w.w >> 16);
+    }
     const uint32_t even = (w.x & 0x00FF00FFu) + (w.y & 0x00FF00FFu) + (w.z & 0x00FF00FFu) + (w.w & 0x00FF00FFu);
     const uint32_t odd = ((w.x >> 8) & 0x00FF00FFu) + ((w.y >> 8) & 0x00FF00FFu) + ((w.z >> 8) & 0x00FF00FFu) +
                          ((w.w >> 8) & 0x00FF00FFu);
     return (even & 0xFFFFu) + (even >> 16) + (odd & 0xFFFFu) + (odd >> 16);
 }
 
-/// kMerge: the group stores a packed partial histogram at partials + blockIdx.x *
-/// kPartialWords instead of adding its counts to bins itself (HistogramMergeKernel does).
+__device__ __forceinline__ uint32_t WaveSum(uint32_t v)
+{
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) v += __shfl_xor(v, d);
+    return v;
+}
+
+/// kMerge: the group stores its partial histogram (ColumnAt(), OutsideAt()) instead of adding its
+/// counts to bins itself; HistogramMergeKernel does.
 template <bool kGuard, bool kMerge>
 __global__ __launch_bounds__(kThreads)
 void HistogramKernel(const int32_t *__restrict__ keys, uint64_t n, uint32_t *__restrict__ bins,
@@ -270,26 +237,22 @@ void HistogramKernel(const int32_t *__restrict__ keys, uint64_t n, uint32_t *__r
 
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = tid & 63;
-    const uint32_t lds_used = n_bins < kLdsBins ? n_bins : kLdsBins;
-    // unsigned "k - lo < range" tests: one subtract and one compare per tier, and the
-    // sentinel 0xFFFFFFFF of an absent key fails all of them
-    const uint32_t main_range = kMerge ? (n_bins > kHotBins ? n_bins - kHotBins : 0)
-                                       : (lds_used > kHotBins ? lds_used - kHotBins : 0);
-    const uint32_t tail_range = !kMerge && n_bins > kLdsBins ? n_bins - kLdsBins : 0;
+    const uint32_t cold_words = ColdWordsOf(n_bins), width_log2 = ColdWidthLog2(n_bins);
     XGuardBlock guard(g, blockIdx.x, &sh.guard_word);
 
-    ClearBins(sh, kMerge ? kCountWords : kLdsBins);   // the same number today; the layouts differ
-    if (tid == 0) { sh.tail_count = 0; sh.bailed = 0; sh.invalid = 0; sh.sum = 0; }
+    ClearBins(sh, 0, cold_words);
+    ClearBins(sh, kColdWords, kColdWords + kWarmBins * 64);
+    if (tid == 0) { sh.bailed = 0; sh.invalid = 0; sh.sum = 0; }
 
     const uint64_t begin = (uint64_t)blockIdx.x * chunk;
     const uint64_t end = begin + chunk < n ? begin + chunk : n;
-    const bool vec_ok = (((uintptr_t)keys) & 15) == 0; // chunk starts are multiples of 4 keys
-    const uint64_t full_end = vec_ok ? begin + (end - begin) / kIterKeys * kIterKeys : begin;
+    const uint64_t full_end = begin + (end - begin) / kIterKeys * kIterKeys;
 
+    // 128-bit loads whatever the array's alignment: a global load takes any multiple of four bytes.
     auto load_iter = [&](i32x4 *v, uint64_t base) {
 #pragma unroll
         for (uint32_t u = 0; u < kUnits; ++u) {
-            v[u] = __builtin_nontemporal_load((const i32x4 *)(keys + base + ((uint64_t)u * kThreads + tid) * 4));
+            v[u] = __builtin_nontemporal_load((const i32x4_any *)(keys + base + ((uint64_t)u * kThreads + tid) * 4));
             if (u + 1 < kUnits) asm volatile("" ::: "memory");
         }
     };
@@ -319,31 +282,7 @@ void HistogramKernel(const int32_t *__restrict__ keys, uint64_t n, uint32_t *__r
         __syncthreads();
     }
 
-    uint32_t hot[kHotBins];
-#pragma unroll
-    for (uint32_t b = 0; b < kHotBins; ++b) hot[b] = 0;
-    uint32_t invalid = 0; // merge layout: keys of this thread outside [0, n_bins), absent ones included
-
-    // Lists the tail keys among k[0, count) one key vector at a time: one reservation for
-    // the wave, each key placed by its rank among the wave's tail lanes of that vector.
-    // Used when some thread holds more than four tail keys in one iteration.
-    auto list_tail_per_key = [&](const uint32_t *k, uint32_t count) {
-        uint32_t total = 0;
-        for (uint32_t j = 0; j < count; ++j) AddPopcount(total, __ballot(k[j] - kLdsBins < tail_range));
-        uint32_t slot = 0;
-        if (lane == 0) slot = __hip_atomic_fetch_add(&sh.tail_count, total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        slot = __builtin_amdgcn_readfirstlane(slot);
-        for (uint32_t j = 0; j < count; ++j) {
-            const bool is_tail = k[j] - kLdsBins < tail_range;
-            const uint64_t m = __ballot(is_tail);
-            if (is_tail) {
-                const uint32_t at = slot + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
-                                           __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-                if (at < kTailCap) sh.tail[at] = (uint16_t)k[j];
-            }
-            AddPopcount(slot, m);
-        }
-    };
+    uint32_t invalid = 0; // keys of this thread outside [0, n_bins), absent ones included
 
     // Counts kUnitsNow * 4 keys per thread.
     auto process = [&](const i32x4 *v, auto units_tag) {
@@ -354,81 +293,28 @@ void HistogramKernel(const int32_t *__restrict__ keys, uint64_t n, uint32_t *__r
             k[u * 4 + 0] = (uint32_t)v[u].x; k[u * 4 + 1] = (uint32_t)v[u].y;
             k[u * 4 + 2] = (uint32_t)v[u].z; k[u * 4 + 3] = (uint32_t)v[u].w;
         }
-        if (kMerge) {
-            // Are all keys of the wave below n_bins (the usual case)? One max per key and one
-            // vote per iteration decide it; then nothing has to be tallied per key and the
-            // LDS add needs no branch.
-            uint32_t largest = k[0];
+        // Are all keys of the wave below n_bins (the usual case)? One max per key and one
+        // vote per iteration decide it; then nothing has to be tallied per key and the
+        // LDS add needs no branch.
+        uint32_t largest = k[0];
 #pragma unroll
-            for (uint32_t j = 1; j < kN; ++j) largest = largest > k[j] ? largest : k[j];
-            if (__ballot(largest >= n_bins) == 0) {
+        for (uint32_t j = 1; j < kN; ++j) largest = largest > k[j] ? largest : k[j];
+        if (__ballot(largest >= n_bins) == 0) {
 #pragma unroll
-                for (uint32_t j = 0; j < kN; ++j) {
-                    uint32_t word, inc;
-                    PackedSlot(k[j], lane, word, inc);
-                    LdsAdd(&sh.bins[word], inc);
-                }
-            } else {
-#pragma unroll
-                for (uint32_t j = 0; j < kN; ++j) {
-                    if (k[j] >= n_bins) {
-                        invalid += 1;
-                    } else {
-                        uint32_t word, inc;
-                        PackedSlot(k[j], lane, word, inc);
-                        LdsAdd(&sh.bins[word], inc);
-                    }
-                }
+            for (uint32_t j = 0; j < kN; ++j) {
+                uint32_t word, inc;
+                PackedSlot(k[j], lane, width_log2, word, inc);
+                LdsAdd(&sh.bins[word], inc);
             }
         } else {
 #pragma unroll
             for (uint32_t j = 0; j < kN; ++j) {
-#pragma unroll
-                for (uint32_t b = 0; b < kHotBins; ++b) AddPopcount(hot[b], __ballot(k[j] == b));
-                if (k[j] - kHotBins < main_range) LdsAdd(&sh.bins[k[j]], 1u);
-            }
-        }
-        if (!kMerge && tail_range != 0) {
-            // Tail keys are rare for skewed inputs, and VALU issue is what bounds this loop:
-            // each thread first gathers its own tail keys (up to four 16-bit values in two
-            // registers, newest in the low half of `lo`), then the wave places them with at
-            // most four list writes per iteration instead of one per key.
-            uint32_t cnt = 0, lo = 0, hi = 0;
-#pragma unroll
-            for (uint32_t j = 0; j < kN; ++j) {
-                if (k[j] - kLdsBins < tail_range) {
-                    // asm so that the body stays under the branch (three instructions that
-                    // run only for key vectors with a tail lane) instead of becoming selects
-                    asm volatile("v_alignbit_b32 %0, %0, %1, 16\n\t"
-                                 "v_lshl_or_b32 %1, %1, 16, %3\n\t"
-                                 "v_add_u32 %2, 1, %2"
-                                 : "+v"(hi), "+v"(lo), "+v"(cnt) : "v"(k[j]));
-                }
-            }
-            if (kN > 4 && __ballot(cnt > 4) != 0) {
-                list_tail_per_key(k, kN);
-            } else {
-                const uint64_t l1 = __ballot(cnt >= 1);
-                if (l1 != 0) {
-                    const uint64_t l2 = __ballot(cnt >= 2), l3 = __ballot(cnt >= 3), l4 = __ballot(cnt >= 4);
-                    const uint32_t n1 = (uint32_t)__popcll(l1), n2 = (uint32_t)__popcll(l2);
-                    const uint32_t n3 = (uint32_t)__popcll(l3), n4 = (uint32_t)__popcll(l4);
-                    const uint32_t total = n1 + n2 + n3 + n4;
-                    uint32_t slot = 0;
-                    if (lane == 0) slot = __hip_atomic_fetch_add(&sh.tail_count, total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                    slot = __builtin_amdgcn_readfirstlane(slot);
-                    if (slot + total <= kTailCap) {
-                        auto rank = [](uint64_t m) {
-                            return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-                        };
-                        if (cnt >= 1) sh.tail[slot + rank(l1)] = (uint16_t)lo;
-                        if (cnt >= 2) sh.tail[slot + n1 + rank(l2)] = (uint16_t)(lo >> 16);
-                        if (l3 != 0) {
-                            if (cnt >= 3) sh.tail[slot + n1 + n2 + rank(l3)] = (uint16_t)hi;
-                            if (cnt >= 4) sh.tail[slot + n1 + n2 + n3 + rank(l4)] = (uint16_t)(hi >> 16);
-                        }
-                    }
-                    // else: tail_count has passed the capacity, the write-out re-reads the chunk
+                if (k[j] >= n_bins) {
+                    invalid += 1;
+                } else {
+                    uint32_t word, inc;
+                    PackedSlot(k[j], lane, width_log2, word, inc);
+                    LdsAdd(&sh.bins[word], inc);
                 }
             }
         }
@@ -476,13 +362,12 @@ void HistogramKernel(const int32_t *__restrict__ keys, uint64_t n, uint32_t *__r
             load_iter(v, base);
             process(v, Units {});
         }
-        // Ragged remainder (and unaligned key arrays): one unit at a time, absent keys read
-        // as the sentinel.
+        // Ragged remainder: one unit at a time, absent keys read as the sentinel.
         for (; base < end; base += kUnitKeys) {
             const uint64_t idx = base + (uint64_t)tid * 4;
             i32x4 v = { -1, -1, -1, -1 };
-            if (vec_ok && idx + 3 < end) {
-                v = __builtin_nontemporal_load((const i32x4 *)(keys + idx));
+            if (idx + 3 < end) {
+                v = __builtin_nontemporal_load((const i32x4_any *)(keys + idx));
             } else {
                 if (idx + 0 < end) v.x = keys[idx + 0];
                 if (idx + 1 < end) v.y = keys[idx + 1];
@@ -495,14 +380,7 @@ void HistogramKernel(const int32_t *__restrict__ keys, uint64_t n, uint32_t *__r
     };
     if (!count_chunk() && lane == 0) sh.bailed = 1;
 
-    // Ballot counters are per wave: lane 0 of each wave folds them into the group's.
-    if (!kMerge && lane == 0) {
-#pragma unroll
-        for (uint32_t b = 0; b < kHotBins; ++b) {
-            if (hot[b] != 0 && b < lds_used) LdsAdd(&sh.bins[b], hot[b]);
-        }
-    }
-    if (kMerge && invalid != 0) LdsAdd(&sh.invalid, invalid);
+    if (invalid != 0) LdsAdd(&sh.invalid, invalid);
     __syncthreads();
 
     if (kGuard) {
@@ -514,93 +392,167 @@ void HistogramKernel(const int32_t *__restrict__ keys, uint64_t n, uint32_t *__r
         if (sh.bailed != 0) return;
     }
 
-    const uint32_t rot = (blockIdx.x * 37u) & (kSegs - 1);
+    const uint32_t me = blockIdx.x, n_part = gridDim.x;
+    uint32_t *const outside = kMerge ? partials + OutsideAt(me, n_part) : nullptr;
+    const bool may_overflow = n_bins > kColdWords;
+    uint32_t counted = 0;
+    // the 64 per-lane counters of warm bin tid / 4: four threads sum 16 each
+    uint32_t warm = 0;
+    {
+        const uint32_t *mine = &sh.bins[kColdWords + (tid / 4) * 64 + (tid % 4) * 16];
+#pragma unroll
+        for (uint32_t q = 0; q < 4; ++q) {
+            const u32x4 w = *(const u32x4 *)&mine[q * 4];
+            warm += w.x + w.y + w.z + w.w;
+        }
+        counted += warm;
+        warm += __shfl_xor(warm, 1);
+        warm += __shfl_xor(warm, 2);
+    }
     if (kMerge) {
-        const uint32_t me = blockIdx.x, n_part = gridDim.x;
-        uint32_t *const outside = partials + OutsideAt(me, n_part);
-        uint32_t counted = 0;
         // Every group starts at a column of its own: column c of all partials is one run of
         // n_part * 256 bytes, and groups that all wrote column 0 first, then column 1, would
         // all be storing into the same few DRAM pages at any moment.
-        const uint32_t turn = ((me * 37u) & (kMergeGroups - 1)) * kMergeWords;
-        for (uint32_t k = tid * 4; k < kColdWords; k += kThreads * 4) {
-            const uint32_t i = (k + turn) & (kColdWords - 1);
+        const uint32_t turn = me * 37u % (cold_words / kMergeWords) * kMergeWords;
+        for (uint32_t k = tid * 4; k < cold_words; k += kThreads * 4) {
+            const uint32_t i = k + turn < cold_words ? k + turn : k + turn - cold_words;
             const u32x4 w = *(const u32x4 *)&sh.bins[i];
             // (a plain store: non-temporal ones make the command 1.5 us slower, the counting
             // kernel and the merge kernel's reads both)
             *(u32x4 *)&partials[ColumnAt(i / kMergeWords, me, n_part) + i % kMergeWords] = w;
-            counted += ByteSum(w);
+            if (may_overflow) counted += ColdSum(w, width_log2 == 3);
         }
-        {
-            // the 64 per-lane counters of warm bin tid / 4: four threads sum 16 each
-            const uint32_t *mine = &sh.bins[kColdWords + (tid / 4) * 64 + (tid % 4) * 16];
-            uint32_t warm = 0;
-#pragma unroll
-            for (uint32_t q = 0; q < 4; ++q) {
-                const u32x4 w = *(const u32x4 *)&mine[q * 4];
-                warm += w.x + w.y + w.z + w.w;
-            }
-            counted += warm;
-            warm += __shfl_xor(warm, 1);
-            warm += __shfl_xor(warm, 2);
-            if (tid % 4 == 0) outside[tid / 4] = warm;
-        }
-        LdsAdd(&sh.sum, counted);
+        if (tid % 4 == 0) outside[tid / 4] = warm;
+    } else if (may_overflow) {
+        for (uint32_t k = tid * 4; k < cold_words; k += kThreads * 4) counted += ColdSum(*(const u32x4 *)&sh.bins[k], width_log2 == 3);
+    }
+
+    bool exact = true;
+    if (may_overflow) {
+        // One LDS add per wave: 1024 lanes adding to this one address took 3.4 us of every launch.
+        counted = WaveSum(counted);
+        if (lane == 0) LdsAdd(&sh.sum, counted);
         __syncthreads();
         // every key slot the group went through (absent keys of the ragged end included) is
         // an invalid key or in the counters
         const uint32_t expected = (uint32_t)(full_end - begin)
                                 + (uint32_t)((end - full_end + kUnitKeys - 1) / kUnitKeys) * kUnitKeys - sh.invalid;
-        if (__builtin_amdgcn_readfirstlane(sh.sum) != __builtin_amdgcn_readfirstlane(expected)) {
-            // A byte counter overflowed: this group's partial counts nothing, and the chunk
-            // is counted again with 32-bit counters, one half of the bins at a time.
-            __syncthreads();
-            for (uint32_t i = tid * 4; i < kColdWords; i += kThreads * 4) {
+        exact = __builtin_amdgcn_readfirstlane(sh.sum) == __builtin_amdgcn_readfirstlane(expected);
+    }
+    if (!exact) {
+        // A counter overflowed: this group's partial counts nothing, and the chunk is counted
+        // again with 32-bit counters, one half of the bins at a time.
+        __syncthreads();
+        if (kMerge) {
+            for (uint32_t i = tid * 4; i < cold_words; i += kThreads * 4) {
                 *(u32x4 *)&partials[ColumnAt(i / kMergeWords, me, n_part) + i % kMergeWords] = u32x4 { 0, 0, 0, 0 };
             }
             if (tid < kWarmBins) outside[tid] = 0;
-            for (uint32_t first = 0; first < n_bins; first += kLdsBins) {
-                const uint32_t count = n_bins - first < kLdsBins ? n_bins - first : kLdsBins;
-                ClearBins(sh);
-                __syncthreads();
-                for (uint64_t idx = begin + tid; idx < end; idx += kThreads) {
-                    const uint32_t key = (uint32_t)keys[idx];
-                    if (key - first < count) LdsAdd(&sh.bins[key - first], 1u);
-                }
-                __syncthreads();
-                SweepOut(sh, bins + first, count, rot);
-                __syncthreads();
-            }
         }
-    } else {
-        SweepOut(sh, bins, lds_used, rot);
-
-        if (tail_range != 0) {
-            const uint32_t listed = sh.tail_count;
+        for (uint32_t first = 0; first < n_bins; first += kLdsBins) {
+            const uint32_t count = n_bins - first < kLdsBins ? n_bins - first : kLdsBins;
+            ClearBins(sh, 0, kLdsBins);
             __syncthreads();
-            ClearBins(sh);
-            __syncthreads();
-            if (listed <= kTailCap) {
-                for (uint32_t i = tid; i < listed; i += kThreads) LdsAdd(&sh.bins[sh.tail[i] - kLdsBins], 1u);
-            } else {
-                // The list overflowed: count the chunk's tail keys from memory instead.
-                for (uint64_t idx = begin + tid; idx < end; idx += kThreads) {
-                    const uint32_t key = (uint32_t)keys[idx];
-                    if (key - kLdsBins < tail_range) LdsAdd(&sh.bins[key - kLdsBins], 1u);
-                }
+            for (uint64_t idx = begin + tid; idx < end; idx += kThreads) {
+                const uint32_t key = (uint32_t)keys[idx];
+                if (key - first < count) LdsAdd(&sh.bins[key - first], 1u);
             }
             __syncthreads();
-            SweepOut(sh, bins + kLdsBins, tail_range, rot);
+            for (uint32_t k = tid; k < kLdsBins; k += kThreads) {
+                const uint32_t i = (k + me * 2368u) % kLdsBins;   // another line for every group
+                const uint32_t c = sh.bins[i];
+                if (c != 0) GlobalAdd(bins + first + i, c);
+            }
+            __syncthreads();
         }
+    } else if (!kMerge) {
+        const uint32_t turn = me * 37u % (cold_words / kMergeWords) * kMergeWords;
+        auto sweep = [&](auto counters_per_word) {
+            constexpr uint32_t kCounters = decltype(counters_per_word)::value, kWidth = 32 / kCounters;
+#pragma unroll 4
+            for (uint32_t k = tid; k < cold_words; k += kThreads) {
+                const uint32_t i = k + turn < cold_words ? k + turn : k + turn - cold_words;
+                const uint32_t w = sh.bins[i];
+#pragma unroll
+                for (uint32_t c = 0; c < kCounters; ++c) {
+                    const uint32_t count = kCounters == 1 ? w : w >> (c * kWidth) & ((1u << (kWidth & 31)) - 1u);
+                    if (count != 0) GlobalAdd(bins + i + c * kColdWords, count);
+                }
+            }
+        };
+        if (!may_overflow) sweep(std::integral_constant<uint32_t, 1> {});
+        else if (width_log2 == 4) sweep(std::integral_constant<uint32_t, 2> {});
+        else sweep(std::integral_constant<uint32_t, 4> {});
+        if (tid % 4 == 0 && warm != 0) GlobalAdd(bins + tid / 4, warm);
     }
 
     if (kGuard) guard.Commit();
 }
 
+/// Few keys, many bins: a group of 256 threads has 1024 keys, four to a thread. Bins below 256 are
+/// counted in LDS and added to the result by the group's threads in order, one line-wide atomic
+/// per sixteen of them (these are the bins that every group has, and atomics on one line retire
+/// one after the other). Of the other counters (16 bits per bin: word k & 32767, half k >> 15;
+/// 1024 keys cannot overflow one) a group touches only the words of its own keys: each thread
+/// zeroes its four, then all count, then each takes what is in its four out again with one
+/// atomic that leaves zero behind, so of all threads that hold a key exactly one gets its count
+/// and adds it to the result. Nothing is cleared and nothing swept: with few keys to a group, the
+/// sweep over 65536 counters is 1024 wave-wide atomics with a lane or two in each (7 us).
+template <bool kGuard>
+__global__ __launch_bounds__(kFewThreads)
+void HistogramFewKeysKernel(const int32_t *__restrict__ keys, uint64_t n, uint32_t *__restrict__ bins,
+                            uint32_t n_bins, XGuardArgs g)
+{
+    __shared__ uint32_t halves[1u << 15];
+    __shared__ uint32_t warm[kWarmBins];
+    __shared__ uint32_t guard_word;
+    static_assert(kFewThreads == kWarmBins, "a thread per warm bin");
+
+    const uint32_t tid = threadIdx.x;
+    const uint64_t idx = (uint64_t)blockIdx.x * kFewKeys + (uint64_t)tid * 4;
+    i32x4 v = { -1, -1, -1, -1 };
+    if (idx + 3 < n) {
+        v = __builtin_nontemporal_load((const i32x4_any *)(keys + idx));
+    } else {
+        if (idx + 0 < n) v.x = keys[idx + 0];
+        if (idx + 1 < n) v.y = keys[idx + 1];
+        if (idx + 2 < n) v.z = keys[idx + 2];
+    }
+    warm[tid] = 0;
+    XGuardBlock guard(g, blockIdx.x, &guard_word);
+    if (kGuard && !guard.Enter()) return;
+
+    const uint32_t k[4] = { (uint32_t)v.x, (uint32_t)v.y, (uint32_t)v.z, (uint32_t)v.w };
+    const uint32_t cold_bins = n_bins > kWarmBins ? n_bins - kWarmBins : 0;   // k - kWarmBins < cold_bins: a cold key
+#pragma unroll
+    for (uint32_t j = 0; j < 4; ++j) if (k[j] - kWarmBins < cold_bins) halves[k[j] & 0x7FFFu] = 0;
+    __syncthreads();
+#pragma unroll
+    for (uint32_t j = 0; j < 4; ++j) {
+        if (k[j] - kWarmBins < cold_bins) LdsAdd(&halves[k[j] & 0x7FFFu], 1u << (k[j] >> 15) * 16);
+        else if (k[j] < n_bins) LdsAdd(&warm[k[j]], 1u);
+    }
+    __syncthreads();
+    uint32_t count[4];
+#pragma unroll
+    for (uint32_t j = 0; j < 4; ++j) {
+        count[j] = 0;
+        if (k[j] - kWarmBins >= cold_bins) continue;
+        const uint32_t shift = (k[j] >> 15) * 16;
+        const uint32_t old = __hip_atomic_fetch_and(&halves[k[j] & 0x7FFFu], ~(0xFFFFu << shift), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        count[j] = old >> shift & 0xFFFFu;
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < 4; ++j) if (count[j] != 0) GlobalAdd(bins + k[j], count[j]);
+    if (warm[tid] != 0) GlobalAdd(bins + tid, warm[tid]);
+    if (kGuard) guard.Commit();
+}
+
 /// Sums the partial histograms of the counting groups and adds the totals to bins. Group j
-/// owns column j of every partial: 64 words of byte counters (word w, byte b = bin
-/// w + b * 16384) and the count of bin j, which is kept outside the bytes. Thread (row, col)
-/// reads four byte words of its column from partials row, row + 16, ... (the sixteen threads
+/// owns column j of every partial: 64 cold words (counter i of word w = bin w + i * 16384; a
+/// byte, a half or the whole word each) if n_bins reaches that far, and the count of bin j,
+/// which is kept outside them. Thread (row, col)
+/// reads four cold words of its column from partials row, row + 16, ... (the sixteen threads
 /// of a row one partial's 256 bytes, the four rows of a wave four neighbouring partials: one
 /// KiB in a piece); the threads of col 0 also read the outside count. The group's progress
 /// byte is first_wg + j. Four waves per group: the kernel is one round trip to its partials,
@@ -612,7 +564,7 @@ void HistogramMergeKernel(const uint32_t *__restrict__ partials, uint32_t n_part
 {
     constexpr uint32_t kCols = kMergeWords / 4, kRows = kMergeThreads / kCols; // 16 x 16
     constexpr uint32_t kAhead = 16;                                      // rows requested before the guard's reads
-    __shared__ uint32_t red[kRows][16][kCols];   // per row: the 16 byte counters of each of the 16 word quads
+    __shared__ uint32_t red[kRows][16][kCols];   // per row: the 16 counters of each of the 16 word quads
     __shared__ uint32_t total[16][kCols];
     __shared__ uint32_t outside_total;
     __shared__ uint32_t guard_word;
@@ -620,19 +572,24 @@ void HistogramMergeKernel(const uint32_t *__restrict__ partials, uint32_t n_part
     const uint32_t tid = threadIdx.x;
     const uint32_t col = tid % kCols, row = tid / kCols;
     const uint32_t column = blockIdx.x;
+    const bool has_column = column * kMergeWords < ColdWordsOf(n_bins);
+    const bool bytes = n_bins > 2 * kColdWords, halves = n_bins > kColdWords;
+    const uint32_t even_mask = bytes ? 0x00FF00FFu : halves ? 0xFFFFu : 0xFFFFFFFFu;
+    const uint32_t odd_mask = halves ? even_mask : 0u, odd_shift = bytes ? 8u : 16u;
     auto load_words = [&](uint32_t p) {
-        return p < n_part ? *(const u32x4 *)(partials + ColumnAt(column, p, n_part) + col * 4) : u32x4 { 0, 0, 0, 0 };
+        return has_column && p < n_part ? *(const u32x4 *)(partials + ColumnAt(column, p, n_part) + col * 4) : u32x4 { 0, 0, 0, 0 };
     };
     auto load_outside = [&](uint32_t p) {
         return col == 0 && p < n_part ? partials[OutsideAt(p, n_part) + column] : 0u;
     };
-    // even[i] holds bytes 0 and 2 of word i in its halves, odd[i] bytes 1 and 3; a thread adds
-    // at most kMaxPartials / kRows = 64 values of 255 into a half.
+    // even[i] holds bytes 0 and 2 of word i in its halves, odd[i] bytes 1 and 3 (a thread adds
+    // at most kMaxPartials / kRows = 64 values of 255 into a half); or half 0 and half 1; or the
+    // whole word and nothing.
     uint32_t even[4] = { 0, 0, 0, 0 }, odd[4] = { 0, 0, 0, 0 }, outside = 0;
     auto add_words = [&](const u32x4 &w) {
         const uint32_t v[4] = { w.x, w.y, w.z, w.w };
 #pragma unroll
-        for (uint32_t i = 0; i < 4; ++i) { even[i] += v[i] & 0x00FF00FFu; odd[i] += (v[i] >> 8) & 0x00FF00FFu; }
+        for (uint32_t i = 0; i < 4; ++i) { even[i] += v[i] & even_mask; odd[i] += (v[i] >> odd_shift) & odd_mask; }
     };
     // The first rows are requested before the guard's reads: the kernel is short, and the
     // round trips overlap. Reading has no side effect (after a flushed counting launch the
@@ -668,13 +625,13 @@ void HistogramMergeKernel(const uint32_t *__restrict__ partials, uint32_t n_part
     for (uint32_t i = 0; i < kAhead; ++i) { add_words(first[i]); outside += first_outside[i]; }
 #pragma unroll 4
     for (uint32_t p = row + kAhead * kRows; p < n_part; p += kRows) { add_words(load_words(p)); outside += load_outside(p); }
-    // counter b * 4 + i of a thread: byte b of its word i
+    // counter b * 4 + i of a thread: counter b of its word i
 #pragma unroll
     for (uint32_t i = 0; i < 4; ++i) {
-        red[row][0 + i][col] = even[i] & 0xFFFFu;
-        red[row][4 + i][col] = odd[i] & 0xFFFFu;
-        red[row][8 + i][col] = even[i] >> 16;
-        red[row][12 + i][col] = odd[i] >> 16;
+        red[row][0 + i][col] = bytes ? even[i] & 0xFFFFu : even[i];
+        red[row][4 + i][col] = bytes ? odd[i] & 0xFFFFu : odd[i];
+        red[row][8 + i][col] = bytes ? even[i] >> 16 : 0u;
+        red[row][12 + i][col] = bytes ? odd[i] >> 16 : 0u;
     }
     if (outside != 0) LdsAdd(&outside_total, outside);
     __syncthreads();
@@ -698,7 +655,7 @@ void HistogramMergeKernel(const uint32_t *__restrict__ partials, uint32_t n_part
         if (count != 0 && bin < n_bins) GlobalAdd(bins + bin, count);
     }
     if (tid == 0) {
-        // bin <column>, counted outside the bytes (which hold nothing for bins below 256)
+        // bin <column>, counted outside the cold words (which hold nothing for bins below 256)
         if (outside_total != 0 && column < n_bins) GlobalAdd(bins + column, outside_total);
     }
     if (kGuard) {
@@ -710,13 +667,12 @@ void HistogramMergeKernel(const uint32_t *__restrict__ partials, uint32_t n_part
 class HipHistogramCommand final : public HipGuardedCommand
 {
 public:
-    /// n_count_wg counting groups; with `merge`, kMergeGroups merge groups follow them in
+    /// plan.groups counting groups; with two kernels, kMergeGroups merge groups follow them in
     /// the progress map.
-    HipHistogramCommand(const void *keys, size_t n, void *bins, uint32_t n_bins, uint32_t chunk,
-                        uint32_t n_count_wg, bool merge, int guard_mode)
-        : HipGuardedCommand(n_count_wg + (merge ? kMergeGroups : 0), guard_mode)
-        , keys_((const int32_t *)keys), n_(n), bins_((uint32_t *)bins), n_bins_(n_bins), chunk_(chunk)
-        , n_count_wg_(n_count_wg), merge_(merge) {}
+    HipHistogramCommand(const void *keys, size_t n, void *bins, uint32_t n_bins, const Plan &plan, int guard_mode)
+        : HipGuardedCommand((uint32_t)plan.groups + (plan.way == Way::kMerge ? kMergeGroups : 0), guard_mode)
+        , keys_((const int32_t *)keys), n_(n), bins_((uint32_t *)bins), n_bins_(n_bins), chunk_(plan.chunk)
+        , n_count_wg_((uint32_t)plan.groups), way_(plan.way) {}
     virtual ~HipHistogramCommand() { if (partials_ != nullptr) pool_->Release(partials_); }
 
 protected:
@@ -724,19 +680,19 @@ protected:
 
     virtual void ReserveOnSubmit(HipQueue &q) override
     {
-        if (merge_ && n_ != 0 && partials_ == nullptr) q.Scratch()->Reserve(ScratchBytes());
+        if (way_ == Way::kMerge && n_ != 0 && partials_ == nullptr) q.Scratch()->Reserve(ScratchBytes());
     }
 
     virtual hipError_t PrepareLaunch(HipQueue &q) override
     {
         // A replay must find the partials of the flushed launch: the buffer taken at the
         // first launch is kept until the command is destroyed.
-        if (!merge_ || n_ == 0 || partials_ != nullptr) return hipSuccess;
+        if (way_ != Way::kMerge || n_ == 0 || partials_ != nullptr) return hipSuccess;
         pool_ = q.Scratch();
         partials_ = (uint32_t *)pool_->Acquire(ScratchBytes());
-        // No scratch: the one-kernel layout works on the same chunks (decided before the
-        // first launch, so every replay takes the same path).
-        if (partials_ == nullptr) merge_ = false;
+        // No scratch: one kernel works on the same chunks (decided before the first launch,
+        // so every replay takes the same path).
+        if (partials_ == nullptr) way_ = Way::kSweep;
         return hipSuccess;
     }
 
@@ -744,21 +700,23 @@ protected:
     {
         if (n_ == 0) return hipSuccess;
         const dim3 grid(n_count_wg_), block(kThreads);
-        if (!merge_) {
-            const hipEvent_t stop = TakeStopEvent();
-            if (guarded) LaunchWithStop(stop, (HistogramKernel<true, false>), grid, block, stream, keys_, (uint64_t)n_, bins_, n_bins_, chunk_, (uint32_t *)nullptr, g);
-            else         LaunchWithStop(stop, (HistogramKernel<false, false>), grid, block, stream, keys_, (uint64_t)n_, bins_, n_bins_, chunk_, (uint32_t *)nullptr, g);
+        if (way_ == Way::kFew) {
+            LaunchWithStop(TakeStopEvent(), guarded ? HistogramFewKeysKernel<true> : HistogramFewKeysKernel<false>, grid, dim3(kFewThreads), stream,
+                           keys_, (uint64_t)n_, bins_, n_bins_, g);
             return hipGetLastError();
         }
-        hipEvent_t stop = nullptr;    // the merge kernel is the command's last
-        if (guarded) LaunchWithStop(stop, (HistogramKernel<true, true>), grid, block, stream, keys_, (uint64_t)n_, bins_, n_bins_, chunk_, partials_, g);
-        else         LaunchWithStop(stop, (HistogramKernel<false, true>), grid, block, stream, keys_, (uint64_t)n_, bins_, n_bins_, chunk_, partials_, g);
+        if (way_ == Way::kSweep) {
+            LaunchWithStop(TakeStopEvent(), guarded ? HistogramKernel<true, false> : HistogramKernel<false, false>, grid, block, stream,
+                           keys_, (uint64_t)n_, bins_, n_bins_, chunk_, (uint32_t *)nullptr, g);
+            return hipGetLastError();
+        }
+        // the merge kernel is the command's last
+        LaunchWithStop(nullptr, guarded ? HistogramKernel<true, true> : HistogramKernel<false, true>, grid, block, stream,
+                       keys_, (uint64_t)n_, bins_, n_bins_, chunk_, partials_, g);
         hipError_t err = hipGetLastError();
         if (err != hipSuccess) return err;
-        const dim3 merge_grid(kMergeGroups), merge_block(kMergeThreads);
-        stop = TakeStopEvent();
-        if (guarded) LaunchWithStop(stop, HistogramMergeKernel<true>, merge_grid, merge_block, stream, (const uint32_t *)partials_, n_count_wg_, bins_, n_bins_, n_count_wg_, g);
-        else         LaunchWithStop(stop, HistogramMergeKernel<false>, merge_grid, merge_block, stream, (const uint32_t *)partials_, n_count_wg_, bins_, n_bins_, n_count_wg_, g);
+        LaunchWithStop(TakeStopEvent(), guarded ? HistogramMergeKernel<true> : HistogramMergeKernel<false>, dim3(kMergeGroups), dim3(kMergeThreads), stream,
+                       (const uint32_t *)partials_, n_count_wg_, bins_, n_bins_, n_count_wg_, g);
         return hipGetLastError();
     }
 
@@ -769,18 +727,10 @@ private:
     const uint32_t n_bins_;
     const uint32_t chunk_;
     const uint32_t n_count_wg_;
-    bool merge_;
+    Way way_;
     std::shared_ptr<ScratchPool> pool_;
     uint32_t *partials_ = nullptr;
 };
-
-/// Keys from which the two-kernel layout is used (XSCHED_HIP_HIST_MERGE_MIN_KEYS).
-inline uint64_t MergeMinKeys()
-{
-    const char *env = getenv("XSCHED_HIP_HIST_MERGE_MIN_KEYS");
-    if (env == nullptr || *env == 0) return kMergeMinKeys;
-    return strtoull(env, nullptr, 0);
-}
 
 } // namespace hist
 
@@ -861,23 +811,29 @@ EXPORT_C_FUNC XResult HipHistogramLaunchNoAlloc(void *stream_ptr, const void *ke
     if (partials == nullptr) {
         res = kXSchedErrorHardware;
     } else {
-        // As few groups as the limit allows, each with a whole number of load units; every
-        // group stores its complete partial (all-zero after an overflow recount), so nothing
-        // of an earlier call's contents is read and nothing has to be cleared.
-        const uint32_t chunk = hist::ChunkFor(n, hist::kMergeMinChunk);   // grows with n: at most 256 groups up to 2^26 keys
-        const uint64_t n_wg = (n + chunk - 1) / chunk;
-        XASSERT(n_wg <= kNoAllocMaxGroups && chunk <= hist::kMaxChunk, "group count %llu / chunk %u out of range",
-                (unsigned long long)n_wg, chunk);
+        // Every group of the two-kernel way stores its complete partial (all-zero after an
+        // overflow recount), so nothing of an earlier call's contents is read and nothing has to
+        // be cleared.
+        const hist::Plan plan = hist::PlanFor(n, n_bins);   // its chunks grow with n: at most 256 groups up to 2^26 keys
+        XASSERT(plan.groups <= kNoAllocMaxGroups && plan.chunk <= hist::kMaxChunk, "group count %llu / chunk %u out of range",
+                (unsigned long long)plan.groups, plan.chunk);
         const XGuardArgs inert {};
-        const dim3 block(hist::kThreads);
-        hipLaunchKernelGGL((hist::HistogramKernel<false, true>), dim3((uint32_t)n_wg), block, 0, stream,
-                           (const int32_t *)keys, (uint64_t)n, (uint32_t *)bins, n_bins, chunk, partials, inert);
-        hipError_t err = hipGetLastError();
-        if (err == hipSuccess) {
-            hipLaunchKernelGGL(hist::HistogramMergeKernel<false>, dim3(hist::kMergeGroups), dim3(hist::kMergeThreads), 0, stream,
-                               (const uint32_t *)partials, (uint32_t)n_wg, (uint32_t *)bins, n_bins, (uint32_t)n_wg, inert);
-            err = hipGetLastError();
+        const dim3 grid((uint32_t)plan.groups), block(hist::kThreads);
+        const int32_t *const k = (const int32_t *)keys;
+        uint32_t *const out = (uint32_t *)bins;
+        if (plan.way == hist::Way::kFew) {
+            hipLaunchKernelGGL(hist::HistogramFewKeysKernel<false>, grid, dim3(hist::kFewThreads), 0, stream, k, (uint64_t)n, out, n_bins, inert);
+        } else if (plan.way == hist::Way::kSweep) {
+            hipLaunchKernelGGL((hist::HistogramKernel<false, false>), grid, block, 0, stream, k, (uint64_t)n, out, n_bins, plan.chunk,
+                               (uint32_t *)nullptr, inert);
+        } else {
+            hipLaunchKernelGGL((hist::HistogramKernel<false, true>), grid, block, 0, stream, k, (uint64_t)n, out, n_bins, plan.chunk, partials, inert);
+            if (hipGetLastError() == hipSuccess) {
+                hipLaunchKernelGGL(hist::HistogramMergeKernel<false>, dim3(hist::kMergeGroups), dim3(hist::kMergeThreads), 0, stream,
+                                   (const uint32_t *)partials, (uint32_t)plan.groups, out, n_bins, (uint32_t)plan.groups, inert);
+            }
         }
+        const hipError_t err = hipGetLastError();
         if (err != hipSuccess) {
             XWARN("HipHistogramLaunchNoAlloc: launch failed: %d (%s)", (int)err, hipGetErrorString(err));
             res = kXSchedErrorHardware;
@@ -894,19 +850,18 @@ EXPORT_C_FUNC XResult HipHistogramCommandCreate(HwCommandHandle *cmd, const void
         return kXSchedErrorInvalidValue;
     }
     if (n_bins == 0 || n_bins > 65536) return kXSchedErrorInvalidValue;
-    bool merge = n != 0 && n >= hist::MergeMinKeys();
-    const char *floor_env = getenv("XSCHED_HIP_HIST_MIN_CHUNK");
-    const uint64_t floor = floor_env && *floor_env ? strtoull(floor_env, nullptr, 0)
-                                                   : (merge ? hist::kMergeMinChunk : hist::kMinChunk);
-    uint32_t chunk = hist::ChunkFor(n, floor);
-    uint64_t n_wg = n == 0 ? 1 : (n + chunk - 1) / chunk;
-    if (merge && n_wg > hist::kMaxPartials) {
-        merge = false;
-        chunk = hist::ChunkFor(n);
-        n_wg = (n + chunk - 1) / chunk;
+    hist::Plan plan = hist::PlanFor(n == 0 ? 1 : n, n_bins);
+    // Two variables take the choice over: the number of keys from which two kernels are used
+    // (one kernel below it), and the least keys per work-group.
+    const char *min_keys = getenv("XSCHED_HIP_HIST_MERGE_MIN_KEYS"), *floor = getenv("XSCHED_HIP_HIST_MIN_CHUNK");
+    if (n != 0 && ((min_keys && *min_keys) || (floor && *floor))) {
+        if (plan.way == hist::Way::kFew) plan.way = hist::Way::kMerge;
+        plan.chunk = hist::ChunkFor(n, floor && *floor ? strtoull(floor, nullptr, 0) : hist::ChunkFloor(n));
+        plan.groups = (n + plan.chunk - 1) / plan.chunk;
+        if (min_keys && *min_keys) plan.way = n >= strtoull(min_keys, nullptr, 0) ? hist::Way::kMerge : hist::Way::kSweep;
+        if (plan.groups > hist::kMaxPartials) plan.way = hist::Way::kSweep;
     }
-    if (n_wg > GuardState::kMaxWorkGroups) return kXSchedErrorInvalidValue;
-    *cmd = HwCommandManager::Add(std::make_shared<hist::HipHistogramCommand>(
-        keys, n, bins, n_bins, chunk, (uint32_t)n_wg, merge, guard));
+    if (plan.groups > GuardState::kMaxWorkGroups) return kXSchedErrorInvalidValue;
+    *cmd = HwCommandManager::Add(std::make_shared<hist::HipHistogramCommand>(keys, n, bins, n_bins, plan, guard));
     return kXSchedSuccess;
 }
