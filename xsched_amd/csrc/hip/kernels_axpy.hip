@@ -12,7 +12,7 @@
 //   one single-wave work-group per chunk: plain launches of arrays below 2^23 elements.
 //       Every chunk is in flight at once, which is what a short array wants; on long
 //       arrays these short-lived waves stream at 6.2-6.3 TB/s on MI355X.
-//   two long-lived waves per CU, each walking chunks c, c + G, c + 2G, ... with the loads
+//   a few long-lived waves per CU (two, more for short arrays), each walking chunks c, c + G, c + 2G, ... with the loads
 //       of three steps in flight: guarded launches, and plain launches of long arrays.
 //       Same bandwidth (measured: 2 waves per CU 6.2 TB/s, 1 per CU 4.1, 4 or more per CU
 //       5.3-5.8 whatever the depth), and nearly all wave slots stay free: a short kernel of
@@ -40,7 +40,11 @@ namespace axpy
 constexpr uint32_t kLanes = 64;
 constexpr uint32_t kStepElems = 1024;                      // unit in which chunk sizes are counted
 
-typedef float float4 __attribute__((ext_vector_type(4))); // 128-bit access unit
+// 128-bit access unit. It is declared aligned to its elements only: a global access of 128 bits
+// takes any multiple of four bytes, so slices of larger arrays run on the same kernels. Aligned
+// arrays lose nothing by it (2^28 elements: 508 us, 511 with 16-byte alignment declared), arrays
+// four bytes off an aligned address take 3-6 % longer (2^24: 35.5 us against 34.3).
+typedef float float4 __attribute__((ext_vector_type(4), aligned(4)));
 
 __device__ __forceinline__ float4 ld_nt(const float4 *p) { return __builtin_nontemporal_load(p); }
 __device__ __forceinline__ void st_nt(float4 *p, float4 v) { __builtin_nontemporal_store(v, p); }
@@ -61,9 +65,11 @@ __device__ __forceinline__ float4 fma4(float a, float4 x, float4 y)
 // 4 -> steps of 1024 elements, 8 -> steps of 2048 elements.
 template <bool kGuard, uint32_t kVecPerStep>
 __global__ __launch_bounds__(64)
-void AxpyVec4Kernel(float alpha, const float4 *x, float4 *y,
+void AxpyVec4Kernel(float alpha, const float *x_first, float *y_first,
                     uint64_t n4, uint32_t tail, uint32_t steps, XGuardArgs g)
 {
+    const float4 *const x = (const float4 *)x_first;
+    float4 *const y = (float4 *)y_first;
     constexpr uint32_t kStepVecs = kLanes * kVecPerStep;
     const uint32_t wg = blockIdx.x;
     const uint32_t lane = threadIdx.x;
@@ -114,9 +120,11 @@ void AxpyVec4Kernel(float alpha, const float4 *x, float4 *y,
 // committed, so it is applied exactly once.
 template <uint32_t kDepth, bool kGuard>
 __global__ __launch_bounds__(64)
-void AxpyPersistentKernel(float alpha, const float4 *x, float4 *y, uint64_t n4, uint32_t tail,
+void AxpyPersistentKernel(float alpha, const float *x_first, float *y_first, uint64_t n4, uint32_t tail,
                           uint32_t steps, uint32_t n_chunks, XGuardArgs g)
 {
+    const float4 *const x = (const float4 *)x_first;
+    float4 *const y = (float4 *)y_first;
     constexpr uint32_t kVecPerStep = 4;
     constexpr uint32_t kStepVecs = kLanes * kVecPerStep;
     const uint32_t lane = threadIdx.x;
@@ -209,25 +217,6 @@ void AxpyPersistentKernel(float alpha, const float4 *x, float4 *y, uint64_t n4, 
     }
 }
 
-// Fallback for pointers that are not 16-byte aligned: same chunking, 32-bit accesses.
-template <bool kGuard>
-__global__ __launch_bounds__(64)
-void AxpyScalarKernel(float alpha, const float *__restrict__ x, float *__restrict__ y,
-                      uint64_t n, uint32_t steps, XGuardArgs g)
-{
-    const uint32_t wg = blockIdx.x;
-    XGuardWave guard(g, wg);
-    if (kGuard) {
-        if (!guard.Enter()) return;
-    }
-    const uint64_t begin = (uint64_t)wg * steps * kStepElems;
-    const uint64_t end = begin + (uint64_t)steps * kStepElems;
-    for (uint64_t i = begin + threadIdx.x; i < end && i < n; i += kLanes) {
-        y[i] = __builtin_fmaf(alpha, x[i], y[i]);
-    }
-    if (kGuard) guard.Commit();
-}
-
 class HipAxpyCommand final : public HipGuardedCommand
 {
 public:
@@ -242,59 +231,51 @@ protected:
     {
         if (n_ == 0) return hipSuccess;
         const hipEvent_t stop = TakeStopEvent();
-        const bool aligned = (((uintptr_t)x_ | (uintptr_t)y_) & 15) == 0;
         const dim3 grid(n_wg_), block(kLanes);
-        const uint32_t waves = PersistentWaves();
-        if (aligned && guarded && !chunk_grid_) {
+        const uint32_t waves = PersistentWaves(n_wg_);
+        const uint64_t n4 = n_ / 4;
+        const uint32_t tail = (uint32_t)(n_ % 4);
+        if (guarded && !chunk_grid_) {
             const dim3 pgrid(n_wg_ < waves ? n_wg_ : waves);
-            LaunchWithStop(stop, (AxpyPersistentKernel<3, true>), pgrid, block, stream, alpha_, (const float4 *)x_,
-                               (float4 *)y_, (uint64_t)(n_ / 4), (uint32_t)(n_ % 4), steps_, n_wg_, g);
-        } else if (aligned && !guarded && !chunk_grid_ && n_wg_ >= 16 * waves) {
+            LaunchWithStop(stop, (AxpyPersistentKernel<3, true>), pgrid, block, stream, alpha_, x_, y_, n4, tail, steps_, n_wg_, g);
+        } else if (!guarded && !chunk_grid_ && n_wg_ >= kLongChunks) {
             // A long array: the same few long-lived waves stream it as fast as one wave per
             // chunk does and leave nearly all wave slots to whatever else runs on the device.
-            LaunchWithStop(stop, (AxpyPersistentKernel<3, false>), dim3(waves), block, stream, alpha_, (const float4 *)x_,
-                               (float4 *)y_, (uint64_t)(n_ / 4), (uint32_t)(n_ % 4), steps_, n_wg_, g);
-        } else if (aligned) {
-            const uint64_t n4 = n_ / 4;
-            const uint32_t tail = (uint32_t)(n_ % 4);
+            LaunchWithStop(stop, (AxpyPersistentKernel<3, false>), dim3(waves), block, stream, alpha_, x_, y_, n4, tail, steps_, n_wg_, g);
+        } else {
             // An even chunk is walked in steps of 2048 elements (8 accesses in flight
             // per lane and stream), an odd one in steps of 1024.
             const bool wide = (steps_ % 2) == 0;
             const uint32_t steps = wide ? steps_ / 2 : steps_;
-            const float4 *xv = (const float4 *)x_;
-            float4 *yv = (float4 *)y_;
-            if (guarded && wide)       LaunchWithStop(stop, (AxpyVec4Kernel<true, 8>), grid, block, stream, alpha_, xv, yv, n4, tail, steps, g);
-            else if (guarded)          LaunchWithStop(stop, (AxpyVec4Kernel<true, 4>), grid, block, stream, alpha_, xv, yv, n4, tail, steps, g);
-            else if (wide)             LaunchWithStop(stop, (AxpyVec4Kernel<false, 8>), grid, block, stream, alpha_, xv, yv, n4, tail, steps, g);
-            else                       LaunchWithStop(stop, (AxpyVec4Kernel<false, 4>), grid, block, stream, alpha_, xv, yv, n4, tail, steps, g);
-        } else {
-            if (guarded) {
-                LaunchWithStop(stop, AxpyScalarKernel<true>, grid, block, stream, alpha_, x_, y_,
-                                   (uint64_t)n_, steps_, g);
-            } else {
-                LaunchWithStop(stop, AxpyScalarKernel<false>, grid, block, stream, alpha_, x_, y_,
-                                   (uint64_t)n_, steps_, g);
-            }
+            if (guarded && wide)       LaunchWithStop(stop, (AxpyVec4Kernel<true, 8>), grid, block, stream, alpha_, x_, y_, n4, tail, steps, g);
+            else if (guarded)          LaunchWithStop(stop, (AxpyVec4Kernel<true, 4>), grid, block, stream, alpha_, x_, y_, n4, tail, steps, g);
+            else if (wide)             LaunchWithStop(stop, (AxpyVec4Kernel<false, 8>), grid, block, stream, alpha_, x_, y_, n4, tail, steps, g);
+            else                       LaunchWithStop(stop, (AxpyVec4Kernel<false, 4>), grid, block, stream, alpha_, x_, y_, n4, tail, steps, g);
         }
         return hipGetLastError();
     }
 
 private:
-    /// Work-groups (= waves) of a guarded launch: a fixed number per compute unit.
-    static uint32_t PersistentWaves()
+    static constexpr uint32_t kLongChunks = 8192;   // from here on a plain launch uses long-lived waves
+
+    /// Long-lived waves of a launch over n_wg chunks: two per compute unit for long arrays, more
+    /// while each has only a few chunks, where what counts is how many requests are out at once
+    /// (us at 2, 4, 8 waves per CU: 2^21 elements 6.8, 6.4, 5.9; 2^22 11.2, 10.3, 9.7; 2^23
+    /// 18.9, 18.1, 18.2; 2^24 34.5, 33.5, 33.9; 2^25 65.2, 65.4, 66.0; 2^28 511, 549, 557).
+    static uint32_t PersistentWaves(uint32_t n_wg)
     {
-        static const uint32_t waves = []() {
-            int64_t per_cu = 2;
-            GetEnvInt64("XSCHED_HIP_AXPY_WAVES_PER_CU", per_cu);
-            if (per_cu < 1) per_cu = 1;
-            if (per_cu > 64) per_cu = 64;
-            int dev = 0, cus = 256;
-            if (hipGetDevice(&dev) == hipSuccess) {
-                (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-            }
-            return (uint32_t)(per_cu * (cus > 0 ? cus : 256));
+        static const uint32_t cus = []() {
+            int dev = 0, n = 256;
+            if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev);
+            return (uint32_t)(n > 0 ? n : 256);
         }();
-        return waves;
+        static const int64_t asked = []() {
+            int64_t per_cu = 0;
+            GetEnvInt64("XSCHED_HIP_AXPY_WAVES_PER_CU", per_cu);
+            return per_cu < 0 ? (int64_t)1 : per_cu > 64 ? (int64_t)64 : per_cu;
+        }();
+        if (asked > 0) return (uint32_t)asked * cus;
+        return (n_wg <= 16 * cus ? 8 : n_wg <= 64 * cus ? 4 : 2) * cus;
     }
 
     const float alpha_;
