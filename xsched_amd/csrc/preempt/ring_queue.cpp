@@ -600,14 +600,36 @@ CommandLog RingXQueue::InFlightLog()
 
 // Optional waits first, then the launcher stops handing over, then the device action of the
 // level, then the optional wait for the hardware queue (async_xqueue.cpp:91-113).
+//
+// Suspend() and Resume() may come from several threads at once: the application's own, and every
+// thread that runs a scheduling round (a round resumes each queue that its policy lets run,
+// whoever suspended it). What one of them does to the queue it does in one piece (op_mu_). Without
+// that, a Resume() that fell between the two halves of a Suspend() (the flag taken, the window
+// lock still with a launch under way) cleared the flag and was then overtaken: the queue was
+// paused and no later Resume() saw anything to undo.
 void RingXQueue::Suspend(int64_t flags)
 {
     if (closing_.load()) return;
-    if (suspended_.exchange(true)) return;
+    const bool waits = (flags & (kQueueSuspendFlagWaitIdle | kQueueSuspendFlagWaitAll)) != 0;
+    int64_t suspension;
+    {
+        Guard op(op_mu_);
+        if (suspended_.exchange(true)) return;
+        suspension = ++suspensions_;
+        if (!waits) PauseAndFlush();
+    }
+    if (waits) {
+        if (flags & kQueueSuspendFlagWaitIdle) WaitForIdle();
+        else WaitAll();
+        Guard op(op_mu_);
+        if (!suspended_.load() || suspensions_ != suspension) return;   // resumed meanwhile
+        PauseAndFlush();
+    }
+    if (flags & kQueueSuspendFlagSyncHwQueue) kHwQueue->Synchronize();
+}
 
-    if (flags & kQueueSuspendFlagWaitIdle) WaitForIdle();
-    else if (flags & kQueueSuspendFlagWaitAll) WaitAll();
-
+void RingXQueue::PauseAndFlush()
+{
     bool in_flight;
     {
         Guard g(win_mu_);
@@ -619,7 +641,6 @@ void RingXQueue::Suspend(int64_t flags)
     deactivated_.store(level_ >= kPreemptLevelDeactivate && (in_flight || !lazy_deactivation_), std::memory_order_release);
     if (deactivated_.load(std::memory_order_relaxed)) kHwQueue->Deactivate();
     if (level_ >= kPreemptLevelInterrupt) kHwQueue->Interrupt();
-    if (flags & kQueueSuspendFlagSyncHwQueue) kHwQueue->Synchronize();
 }
 
 // Level 1 just lets the launcher go on: what is in flight may still be running and stays in
@@ -629,6 +650,8 @@ void RingXQueue::Suspend(int64_t flags)
 // (async_xqueue.cpp:115-150).
 void RingXQueue::Resume(int64_t flags)
 {
+    if (!suspended_.load()) return;   // the usual case of a round: nothing to undo
+    Guard op(op_mu_);
     if (!suspended_.exchange(false)) return;
     const bool drop = (flags & kQueueResumeFlagDropCommands) != 0;
 

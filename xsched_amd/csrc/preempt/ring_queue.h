@@ -126,6 +126,7 @@ private:
     void PublishRetired(int64_t idx);
     void AwaitRetired(int64_t ticket);
     CommandLog InFlightLog();
+    void PauseAndFlush();                                          // op_mu_ held
 
     std::mutex win_mu_;
     std::condition_variable win_cv_;
@@ -148,7 +149,9 @@ private:
 
     XPreemptLevel level_;
     bool caller_may_launch_ = false;
-    std::atomic_bool suspended_ { false };
+    std::mutex op_mu_;                  // one Suspend() or Resume() at a time; taken before the locks above
+    int64_t suspensions_ = 0;           // op_mu_: number of the newest suspension
+    std::atomic_bool suspended_ { false };   // changed under op_mu_
     std::atomic_bool closing_ { false };
     std::thread launcher_;
 };
