@@ -35,3 +35,31 @@ def test_histogram_ways_by_size_and_bins(xs, gpu, n, offset, n_bins, level, guar
     want = oracle.histogram(keys_h[~outside], n_bins)
     assert np.array_equal(got[:n_bins], 2 * want)
     assert got[n_bins] == 0, "wrote beyond the bins array"
+
+
+@pytest.mark.parametrize("n_bins", [254, 4096, 4097, 65536])
+@pytest.mark.parametrize("n", [(1 << 16) + 1, (1 << 24) + 5, (1 << 25) + 5])
+def test_histogram_counters_of_the_hot_bins(xs, gpu, n, n_bins):
+    """Around the number of bins from which the hot ones have fewer counters, with the hottest bin
+    in every second key, and around the length from which work-groups share a compute unit: on
+    two queues at once, so that they do. Whole numbers: bit for bit the oracle's."""
+    torch = gpu
+    print(f"case hist-hot n={n} bins={n_bins}", flush=True)
+    rng = np.random.default_rng(n + n_bins)
+    keys_h = rng.integers(0, n_bins, n).astype(np.int32)
+    keys_h[::2] = rng.integers(0, 2) * 253
+    keys_h[1::64] = 254          # no bin where n_bins is 254
+    keys = torch.from_numpy(keys_h).cuda()
+    bins = [torch.zeros(n_bins + 1, dtype=torch.int32, device="cuda") for _ in range(2)]
+    queues = [Queue(xs, torch, 2) for _ in bins]
+    for q, b in zip(queues, bins):
+        q.submit(hist_cmd(xs, keys, n, b, n_bins, 1))
+    for q in queues:
+        q.wait()
+    got = [b.cpu().numpy().view(np.uint32) for b in bins]
+    for q in queues:
+        q.close()
+    want = oracle.histogram(keys_h[keys_h < n_bins], n_bins)
+    for g in got:
+        assert np.array_equal(g[:n_bins], want)
+        assert g[n_bins] == 0, "wrote beyond the bins array"

@@ -203,10 +203,15 @@ private:
 
 /// hipLaunchKernelGGL, with `stop` (may be null) bound to the dispatch as its stop event.
 template <typename... Args, typename F = void (*)(Args...)>
+inline void LaunchWithStopLds(uint32_t lds_bytes, hipEvent_t stop, F kernel, const dim3 &grid, const dim3 &block, hipStream_t stream, Args... args)
+{
+    if (stop != nullptr) hipExtLaunchKernelGGL(kernel, grid, block, lds_bytes, stream, nullptr, stop, 0, args...);
+    else hipLaunchKernelGGL(kernel, grid, block, lds_bytes, stream, args...);
+}
+template <typename... Args, typename F = void (*)(Args...)>
 inline void LaunchWithStop(hipEvent_t stop, F kernel, const dim3 &grid, const dim3 &block, hipStream_t stream, Args... args)
 {
-    if (stop != nullptr) hipExtLaunchKernelGGL(kernel, grid, block, 0, stream, nullptr, stop, 0, args...);
-    else hipLaunchKernelGGL(kernel, grid, block, 0, stream, args...);
+    LaunchWithStopLds(0, stop, kernel, grid, block, stream, args...);
 }
 
 /// Base of the guarded victim kernels.

@@ -10,18 +10,23 @@
 // ~90-110 G/s however they are arranged, and 256 groups times 65536 bins is a lot of
 // them; hence the second kernel below).
 //
-// One work-group of 1024 threads per compute unit owns a contiguous chunk of keys
+// One work-group of 1024 threads owns a contiguous chunk of keys
 // (sized so that a launch has about one work-group per CU) and keeps everything it
-// counts on chip until the end, in 128 KiB of LDS counters split in two. Bins below 256 (two
-// thirds of all Zipf(1.1) keys, a fifth of them in bins 0 and 1) have one 32-bit counter PER
-// LANE: 256 bins x 64 lanes, so the lanes of a wave never add to the same address for them, no
-// vote and no popcount is needed, and they cannot overflow. Every other bin shares one of 16384
+// counts on chip until the end, in 80 KiB of LDS counters split in two. Bins below 255 (two
+// thirds of all Zipf(1.1) keys, a fifth of them in bins 0 and 1) have sixteen 32-bit counters
+// each, one per lane modulo 16, so that at most four lanes of a wave add to the same address, no
+// vote and no popcount is needed, and they cannot overflow (64, one per lane, where n_bins leaves
+// the room: evenly spread keys over 1000 bins, a quarter of them in these bins, 54.7 us against
+// 56.8 with 16). Half of a compute unit's LDS and of its wave slots: two groups of different
+// queues share it, and one streams keys while the other clears, writes out or waits for its first
+// keys (four queues of 2^26 keys each 217 -> 207 us; with 64 counters for every one of these bins
+// and 128 KiB, a group had its unit to itself). Every other bin shares one of 16384
 // words with the bins 16384, 32768 and 49152 above it, as far as there are such bins: a BYTE
 // each when n_bins > 32768, a half word each when n_bins > 16384, the whole word otherwise; one
 // ds_add of 1 << (width * (key >> 14)) per key. One vote per iteration tells whether every key
 // of the wave is below n_bins, so the add needs no branch.
 //
-// A byte overflows only when one bin outside the first 256 takes 256 keys of a chunk (0.1 % of
+// A byte overflows only when one bin outside the first 255 takes 256 keys of a chunk (0.1 % of
 // it; the hottest such bin of a Zipf(1.1) chunk takes 80), a half when it takes 65536. Every
 // overflow lowers the sum of all counters by at least 255 and nothing raises it, so "sum of
 // counters == keys that must be in them" (all key slots of the chunk minus the invalid ones)
@@ -38,7 +43,7 @@
 //       partials would need more than 128 MiB of scratch, and when the scratch buffer cannot
 //       be allocated.
 //   two kernels (kMerge): the group stores a partial histogram of 65 KiB (less when n_bins is
-//       below 16384; the words as they are, the per-lane counters summed) into a scratch
+//       below 16384; the words as they are, the copies of the warm counters summed) into a scratch
 //       buffer, and a second kernel sums the partials column by column and adds the totals to
 //       the result with one atomic per bin.
 // The first version of this layout kept 16-bit halves for every bin and ballot counters for
@@ -71,7 +76,6 @@ namespace hist
 {
 
 constexpr uint32_t kThreads = 1024;
-constexpr uint32_t kLdsBins = 1u << 15;       // 128 KiB of counters
 #ifndef XSCHED_HIST_UNITS
 #define XSCHED_HIST_UNITS 1
 #endif
@@ -92,9 +96,14 @@ constexpr uint32_t kTargetGroups = 256;       // compute units of an MI355X
 constexpr uint32_t kFewThreads = 256;         // HistogramFewKeysKernel: threads
 constexpr uint32_t kFewKeys = kFewThreads * 4;        // keys per work-group
 constexpr uint64_t kFewMaxKeys = 1u << 16;            // and the most keys it is used for
+constexpr uint32_t kFewWarmBins = 256;                // its bins that are counted in order
 constexpr uint32_t kColdWords = 1u << 14;           // word w counts bins w + i * 16384
-constexpr uint32_t kWarmBins = 256;                 // bins below this have 32-bit counters of their own
-static_assert(kColdWords + kWarmBins * 64 <= kLdsBins, "the cold words, then a counter per warm bin and lane");
+constexpr uint32_t kWarmBins = 255;                 // bins below this have 32-bit counters of their own,
+constexpr uint32_t kCopies = 16;                    // one per lane modulo 16
+constexpr uint32_t kFewColdWords = 1u << 12;        // with at most this many cold words one per lane
+constexpr uint32_t kOutside = 256;                  // counts a partial keeps outside the cold words (the last is 0)
+constexpr uint32_t kLdsBins = kColdWords + kWarmBins * kCopies;   // the cold words, then the warm counters
+static_assert(kFewColdWords + kWarmBins * 64 <= kLdsBins, "a warm counter per lane beside few cold words");
 // The partial histograms of a launch in memory, n_part of them (one per counting group): the
 // cold words column by column, one column per merge group, and within a column partial by
 // partial: column c of partial p is the 64 words (256 bytes, two whole cache lines) at
@@ -107,7 +116,7 @@ static_assert(kColdWords + kWarmBins * 64 <= kLdsBins, "the cold words, then a c
 constexpr uint32_t kMergeGroups = 256;
 constexpr uint32_t kMergeThreads = 256;             // threads of a merge group
 constexpr uint32_t kMergeWords = kColdWords / kMergeGroups;          // cold words per column (64)
-constexpr uint32_t kPartialWords = kColdWords + kWarmBins;           // 65 KiB of scratch per counting group
+constexpr uint32_t kPartialWords = kColdWords + kOutside;           // 65 KiB of scratch per counting group
 
 /// Where column `column` of partial `p` lies, and where that partial's 256 outside counts do.
 __host__ __device__ inline size_t ColumnAt(uint32_t column, uint32_t p, uint32_t n_part)
@@ -116,10 +125,10 @@ __host__ __device__ inline size_t ColumnAt(uint32_t column, uint32_t p, uint32_t
 }
 __host__ __device__ inline size_t OutsideAt(uint32_t p, uint32_t n_part)
 {
-    return (size_t)n_part * kColdWords + (size_t)p * kWarmBins;
+    return (size_t)n_part * kColdWords + (size_t)p * kOutside;
 }
 constexpr uint32_t kMaxPartials = 1024;
-static_assert(kWarmBins == kMergeGroups, "column j carries the outside count of bin j");
+static_assert(kOutside == kMergeGroups && kWarmBins <= kOutside, "column j carries the outside count of bin j");
 typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef i32x4 i32x4_any __attribute__((aligned(4)));   // keys may start at any int32
@@ -157,6 +166,13 @@ enum class Way { kFew, kSweep, kMerge };
 /// How n keys are counted (see the head of this file), in work-groups of `chunk` keys.
 struct Plan { Way way; uint32_t chunk; uint64_t groups; };
 
+/// LDS asked for on top of a counting group's own, so that it has its compute unit to itself.
+/// Groups of long chunks may share one with another queue's (what one group does before its first
+/// and behind its last key hides behind the other's keys: four queues of 2^26 keys 217 -> 208 us).
+/// A launch of short ones is over before that pays, and two of its own groups on one unit while
+/// others are free cost it more (2^20 and 2^22 keys: 1.0 us).
+inline uint32_t ExtraLdsFor(uint32_t chunk) { return chunk < (1u << 17) ? 4096 : 0; }
+
 /// - Few keys and many bins: HistogramFewKeysKernel. 16384 Zipf keys over 65536 bins take 3.8 us
 ///   (two kernels: 10.4), 65536 take 7.2, evenly spread 5.4 (10.5); 131072 take 11.8 (10.7).
 /// - One kernel while the groups' sweeps are short, in wave-wide atomics of 64 neighbouring bins:
@@ -183,6 +199,7 @@ struct Shared
     uint32_t invalid;       // keys outside [0, n_bins), absent ones included
     uint32_t sum;           // sum of all counters
 };
+static_assert(sizeof(Shared) <= 80 * 1024, "two groups to a compute unit");
 
 __device__ __forceinline__ void LdsAdd(uint32_t *p, uint32_t v)
 {
@@ -199,11 +216,19 @@ __device__ __forceinline__ void ClearBins(Shared &sh, uint32_t first, uint32_t e
     for (uint32_t i = first + threadIdx.x * 4; i < end; i += kThreads * 4) *(u32x4 *)&sh.bins[i] = u32x4 { 0, 0, 0, 0 };
 }
 
-/// Where a valid key is counted, and by how much (see the head of this file).
-__device__ __forceinline__ void PackedSlot(uint32_t key, uint32_t lane, uint32_t width_log2, uint32_t &word, uint32_t &inc)
+/// Where the warm counters of a launch lie: counter `copy` of bin b is word first + (b << log2) + copy.
+struct WarmPlace { uint32_t first, log2; };
+__device__ __forceinline__ WarmPlace WarmPlaceOf(uint32_t cold_words)
 {
-    const bool warm = key < kWarmBins;
-    word = warm ? kColdWords + key * 64 + lane : key & (kColdWords - 1);
+    static_assert(kCopies == 16, "log2 of it below");
+    return cold_words <= kFewColdWords ? WarmPlace { kFewColdWords, 6 } : WarmPlace { kColdWords, 4 };
+}
+
+/// Where a valid key is counted, and by how much (see the head of this file); `copy` is the
+/// lane's copy of warm bin 0.
+__device__ __forceinline__ void PackedSlot(uint32_t key, uint32_t copy, uint32_t copies_log2, uint32_t width_log2, uint32_t &word, uint32_t &inc)
+{
+    word = key < kWarmBins ? copy + (key << copies_log2) : key & (kColdWords - 1);
     inc = 1u << ((key >> 14) << width_log2);
 }
 
@@ -229,7 +254,7 @@ __device__ __forceinline__ uint32_t WaveSum(uint32_t v)
 /// kMerge: the group stores its partial histogram (ColumnAt(), OutsideAt()) instead of adding its
 /// counts to bins itself; HistogramMergeKernel does.
 template <bool kGuard, bool kMerge>
-__global__ __launch_bounds__(kThreads)
+__global__ __launch_bounds__(kThreads, 8 /* waves per SIMD: two groups to a compute unit */)
 void HistogramKernel(const int32_t *__restrict__ keys, uint64_t n, uint32_t *__restrict__ bins,
                      uint32_t n_bins, uint32_t chunk, uint32_t *__restrict__ partials, XGuardArgs g)
 {
@@ -240,8 +265,10 @@ void HistogramKernel(const int32_t *__restrict__ keys, uint64_t n, uint32_t *__r
     const uint32_t cold_words = ColdWordsOf(n_bins), width_log2 = ColdWidthLog2(n_bins);
     XGuardBlock guard(g, blockIdx.x, &sh.guard_word);
 
+    const WarmPlace warm_at = WarmPlaceOf(cold_words);
+    const uint32_t copy = warm_at.first + (lane & ((1u << warm_at.log2) - 1u));
     ClearBins(sh, 0, cold_words);
-    ClearBins(sh, kColdWords, kColdWords + kWarmBins * 64);
+    ClearBins(sh, warm_at.first, warm_at.first + (kWarmBins << warm_at.log2));
     if (tid == 0) { sh.bailed = 0; sh.invalid = 0; sh.sum = 0; }
 
     const uint64_t begin = (uint64_t)blockIdx.x * chunk;
@@ -303,7 +330,7 @@ void HistogramKernel(const int32_t *__restrict__ keys, uint64_t n, uint32_t *__r
 #pragma unroll
             for (uint32_t j = 0; j < kN; ++j) {
                 uint32_t word, inc;
-                PackedSlot(k[j], lane, width_log2, word, inc);
+                PackedSlot(k[j], copy, warm_at.log2, width_log2, word, inc);
                 LdsAdd(&sh.bins[word], inc);
             }
         } else {
@@ -313,7 +340,7 @@ void HistogramKernel(const int32_t *__restrict__ keys, uint64_t n, uint32_t *__r
                     invalid += 1;
                 } else {
                     uint32_t word, inc;
-                    PackedSlot(k[j], lane, width_log2, word, inc);
+                    PackedSlot(k[j], copy, warm_at.log2, width_log2, word, inc);
                     LdsAdd(&sh.bins[word], inc);
                 }
             }
@@ -396,19 +423,17 @@ void HistogramKernel(const int32_t *__restrict__ keys, uint64_t n, uint32_t *__r
     uint32_t *const outside = kMerge ? partials + OutsideAt(me, n_part) : nullptr;
     const bool may_overflow = n_bins > kColdWords;
     uint32_t counted = 0;
-    // the 64 per-lane counters of warm bin tid / 4: four threads sum 16 each
+    // the copies of warm bin tid / 4: four threads sum a quarter each
     uint32_t warm = 0;
-    {
-        const uint32_t *mine = &sh.bins[kColdWords + (tid / 4) * 64 + (tid % 4) * 16];
-#pragma unroll
-        for (uint32_t q = 0; q < 4; ++q) {
-            const u32x4 w = *(const u32x4 *)&mine[q * 4];
+    if (tid / 4 < kWarmBins) {
+        for (uint32_t q = 0; q < 1u << (warm_at.log2 - 4); ++q) {
+            const u32x4 w = *(const u32x4 *)&sh.bins[warm_at.first + ((tid * 4) << (warm_at.log2 - 4)) + q * 4];
             warm += w.x + w.y + w.z + w.w;
         }
-        counted += warm;
-        warm += __shfl_xor(warm, 1);
-        warm += __shfl_xor(warm, 2);
     }
+    counted += warm;
+    warm += __shfl_xor(warm, 1);
+    warm += __shfl_xor(warm, 2);
     if (kMerge) {
         // Every group starts at a column of its own: column c of all partials is one run of
         // n_part * 256 bytes, and groups that all wrote column 0 first, then column 1, would
@@ -441,25 +466,44 @@ void HistogramKernel(const int32_t *__restrict__ keys, uint64_t n, uint32_t *__r
     }
     if (!exact) {
         // A counter overflowed: this group's partial counts nothing, and the chunk is counted
-        // again with 32-bit counters, one half of the bins at a time.
+        // again with 32-bit counters, one quarter of the bins at a time.
         __syncthreads();
         if (kMerge) {
             for (uint32_t i = tid * 4; i < cold_words; i += kThreads * 4) {
                 *(u32x4 *)&partials[ColumnAt(i / kMergeWords, me, n_part) + i % kMergeWords] = u32x4 { 0, 0, 0, 0 };
             }
-            if (tid < kWarmBins) outside[tid] = 0;
+            if (tid < kOutside) outside[tid] = 0;
         }
-        for (uint32_t first = 0; first < n_bins; first += kLdsBins) {
-            const uint32_t count = n_bins - first < kLdsBins ? n_bins - first : kLdsBins;
-            ClearBins(sh, 0, kLdsBins);
+        for (uint32_t first = 0; first < n_bins; first += kColdWords) {
+            const uint32_t count = n_bins - first < kColdWords ? n_bins - first : kColdWords;
+            ClearBins(sh, 0, kColdWords);
             __syncthreads();
-            for (uint64_t idx = begin + tid; idx < end; idx += kThreads) {
-                const uint32_t key = (uint32_t)keys[idx];
-                if (key - first < count) LdsAdd(&sh.bins[key - first], 1u);
+            for (uint64_t base = begin; base < end; base += 2 * kUnitKeys) {
+                i32x4 v[2];
+#pragma unroll
+                for (uint32_t u = 0; u < 2; ++u) {
+                    const uint64_t idx = base + u * kUnitKeys + (uint64_t)tid * 4;
+                    v[u] = i32x4 { -1, -1, -1, -1 };
+                    if (idx + 3 < end) {
+                        v[u] = *(const i32x4_any *)(keys + idx);
+                    } else {
+                        if (idx + 0 < end) v[u].x = keys[idx + 0];
+                        if (idx + 1 < end) v[u].y = keys[idx + 1];
+                        if (idx + 2 < end) v[u].z = keys[idx + 2];
+                    }
+                }
+#pragma unroll
+                for (uint32_t u = 0; u < 2; ++u) {
+#pragma unroll
+                    for (uint32_t j = 0; j < 4; ++j) {
+                        const uint32_t key = (uint32_t)v[u][j];
+                        if (key - first < count) LdsAdd(&sh.bins[key - first], 1u);
+                    }
+                }
             }
             __syncthreads();
-            for (uint32_t k = tid; k < kLdsBins; k += kThreads) {
-                const uint32_t i = (k + me * 2368u) % kLdsBins;   // another line for every group
+            for (uint32_t k = tid; k < kColdWords; k += kThreads) {
+                const uint32_t i = (k + me * 2368u) % kColdWords;   // another line for every group
                 const uint32_t c = sh.bins[i];
                 if (c != 0) GlobalAdd(bins + first + i, c);
             }
@@ -483,7 +527,7 @@ void HistogramKernel(const int32_t *__restrict__ keys, uint64_t n, uint32_t *__r
         if (!may_overflow) sweep(std::integral_constant<uint32_t, 1> {});
         else if (width_log2 == 4) sweep(std::integral_constant<uint32_t, 2> {});
         else sweep(std::integral_constant<uint32_t, 4> {});
-        if (tid % 4 == 0 && warm != 0) GlobalAdd(bins + tid / 4, warm);
+        if (tid % 4 == 0 && warm != 0) GlobalAdd(bins + tid / 4, warm);   // counts of bins that n_bins ends before are 0
     }
 
     if (kGuard) guard.Commit();
@@ -504,9 +548,9 @@ void HistogramFewKeysKernel(const int32_t *__restrict__ keys, uint64_t n, uint32
                             uint32_t n_bins, XGuardArgs g)
 {
     __shared__ uint32_t halves[1u << 15];
-    __shared__ uint32_t warm[kWarmBins];
+    __shared__ uint32_t warm[kFewWarmBins];
     __shared__ uint32_t guard_word;
-    static_assert(kFewThreads == kWarmBins, "a thread per warm bin");
+    static_assert(kFewThreads == kFewWarmBins, "a thread per warm bin");
 
     const uint32_t tid = threadIdx.x;
     const uint64_t idx = (uint64_t)blockIdx.x * kFewKeys + (uint64_t)tid * 4;
@@ -523,13 +567,13 @@ void HistogramFewKeysKernel(const int32_t *__restrict__ keys, uint64_t n, uint32
     if (kGuard && !guard.Enter()) return;
 
     const uint32_t k[4] = { (uint32_t)v.x, (uint32_t)v.y, (uint32_t)v.z, (uint32_t)v.w };
-    const uint32_t cold_bins = n_bins > kWarmBins ? n_bins - kWarmBins : 0;   // k - kWarmBins < cold_bins: a cold key
+    const uint32_t cold_bins = n_bins > kFewWarmBins ? n_bins - kFewWarmBins : 0;   // k - kFewWarmBins < cold_bins: a cold key
 #pragma unroll
-    for (uint32_t j = 0; j < 4; ++j) if (k[j] - kWarmBins < cold_bins) halves[k[j] & 0x7FFFu] = 0;
+    for (uint32_t j = 0; j < 4; ++j) if (k[j] - kFewWarmBins < cold_bins) halves[k[j] & 0x7FFFu] = 0;
     __syncthreads();
 #pragma unroll
     for (uint32_t j = 0; j < 4; ++j) {
-        if (k[j] - kWarmBins < cold_bins) LdsAdd(&halves[k[j] & 0x7FFFu], 1u << (k[j] >> 15) * 16);
+        if (k[j] - kFewWarmBins < cold_bins) LdsAdd(&halves[k[j] & 0x7FFFu], 1u << (k[j] >> 15) * 16);
         else if (k[j] < n_bins) LdsAdd(&warm[k[j]], 1u);
     }
     __syncthreads();
@@ -537,7 +581,7 @@ void HistogramFewKeysKernel(const int32_t *__restrict__ keys, uint64_t n, uint32
 #pragma unroll
     for (uint32_t j = 0; j < 4; ++j) {
         count[j] = 0;
-        if (k[j] - kWarmBins >= cold_bins) continue;
+        if (k[j] - kFewWarmBins >= cold_bins) continue;
         const uint32_t shift = (k[j] >> 15) * 16;
         const uint32_t old = __hip_atomic_fetch_and(&halves[k[j] & 0x7FFFu], ~(0xFFFFu << shift), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         count[j] = old >> shift & 0xFFFFu;
@@ -655,7 +699,8 @@ void HistogramMergeKernel(const uint32_t *__restrict__ partials, uint32_t n_part
         if (count != 0 && bin < n_bins) GlobalAdd(bins + bin, count);
     }
     if (tid == 0) {
-        // bin <column>, counted outside the cold words (which hold nothing for bins below 256)
+        // bin <column>, counted outside the cold words (which hold nothing for bins below 255; bin 255
+        // has its count there and 0 here)
         if (outside_total != 0 && column < n_bins) GlobalAdd(bins + column, outside_total);
     }
     if (kGuard) {
@@ -706,12 +751,12 @@ protected:
             return hipGetLastError();
         }
         if (way_ == Way::kSweep) {
-            LaunchWithStop(TakeStopEvent(), guarded ? HistogramKernel<true, false> : HistogramKernel<false, false>, grid, block, stream,
+            LaunchWithStopLds(ExtraLdsFor(chunk_), TakeStopEvent(), guarded ? HistogramKernel<true, false> : HistogramKernel<false, false>, grid, block, stream,
                            keys_, (uint64_t)n_, bins_, n_bins_, chunk_, (uint32_t *)nullptr, g);
             return hipGetLastError();
         }
         // the merge kernel is the command's last
-        LaunchWithStop(nullptr, guarded ? HistogramKernel<true, true> : HistogramKernel<false, true>, grid, block, stream,
+        LaunchWithStopLds(ExtraLdsFor(chunk_), nullptr, guarded ? HistogramKernel<true, true> : HistogramKernel<false, true>, grid, block, stream,
                        keys_, (uint64_t)n_, bins_, n_bins_, chunk_, partials_, g);
         hipError_t err = hipGetLastError();
         if (err != hipSuccess) return err;
@@ -824,10 +869,10 @@ EXPORT_C_FUNC XResult HipHistogramLaunchNoAlloc(void *stream_ptr, const void *ke
         if (plan.way == hist::Way::kFew) {
             hipLaunchKernelGGL(hist::HistogramFewKeysKernel<false>, grid, dim3(hist::kFewThreads), 0, stream, k, (uint64_t)n, out, n_bins, inert);
         } else if (plan.way == hist::Way::kSweep) {
-            hipLaunchKernelGGL((hist::HistogramKernel<false, false>), grid, block, 0, stream, k, (uint64_t)n, out, n_bins, plan.chunk,
+            hipLaunchKernelGGL((hist::HistogramKernel<false, false>), grid, block, hist::ExtraLdsFor(plan.chunk), stream, k, (uint64_t)n, out, n_bins, plan.chunk,
                                (uint32_t *)nullptr, inert);
         } else {
-            hipLaunchKernelGGL((hist::HistogramKernel<false, true>), grid, block, 0, stream, k, (uint64_t)n, out, n_bins, plan.chunk, partials, inert);
+            hipLaunchKernelGGL((hist::HistogramKernel<false, true>), grid, block, hist::ExtraLdsFor(plan.chunk), stream, k, (uint64_t)n, out, n_bins, plan.chunk, partials, inert);
             if (hipGetLastError() == hipSuccess) {
                 hipLaunchKernelGGL(hist::HistogramMergeKernel<false>, dim3(hist::kMergeGroups), dim3(hist::kMergeThreads), 0, stream,
                                    (const uint32_t *)partials, (uint32_t)plan.groups, out, n_bins, (uint32_t)plan.groups, inert);
