@@ -85,10 +85,10 @@ XResult HipAxpyCommandCreate(HwCommandHandle *cmd, float alpha, const void *x, v
 
 /* C[M,N] = A[M,K] * B[K,N]; A, B, C row-major bf16, fp32 accumulation in ascending
  * k, round-to-nearest-even on store. Any M, N, K >= 1 (at most 2^18 tiles), any alignment to
- * the element. The work is cut into tiles of C of 256x256 (M and N multiples of 256, K of 64,
- * enough of them to cover half of the compute units), 128x128 or 64x64, whichever keeps the
- * compute units busy (XSCHED_HIP_GEMM_TILE=64|128|256 overrides that where the shape allows).
- * Fastest where the rows of all three matrices start on 16-byte boundaries (N and K multiples
+ * the element. The work is cut into tiles of C of 256x256 (N and K multiples of 8, matrices
+ * aligned to 16 bytes), 128x128 or 64x64, whichever is estimated to be quickest, or into two
+ * launches, 256x256 for most rows and smaller ones for the rest
+ * (XSCHED_HIP_GEMM_TILE=64|128|256 overrides that where the shape allows). Fastest where the rows of all three matrices start on 16-byte boundaries (N and K multiples
  * of 8, matrices aligned to 16 bytes); up to twice as long where they do not. Every element is
  * summed in the same order on all paths. */
 XResult HipGemmBf16CommandCreate(HwCommandHandle *cmd, const void *A, const void *B, void *C,

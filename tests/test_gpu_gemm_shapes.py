@@ -24,8 +24,7 @@ def _shape(fit, tile, steps):
 
 @pytest.mark.parametrize("level,guard", [(1, 0), (2, 1)])
 @pytest.mark.parametrize("steps", [1, 2, 3, 4, 5, 6, 7, 9, 10, 13, 14, 18])
-@pytest.mark.parametrize("fit", ["exact", "edges", "unaligned"])
-@pytest.mark.parametrize("tile", [64, 128])
+@pytest.mark.parametrize("tile,fit", [(t, f) for t in (64, 128) for f in ("exact", "edges", "unaligned")] + [(256, "exact"), (256, "edges")])
 def test_gemm_pipeline_lengths_and_edges(xs, gpu, monkeypatch, tile, fit, steps, level, guard):
     """Integers in [-4, 4]: at most 18 x 64 x 16 < 2^24, so every sum is exact and the result is
     determined. The matrices lie between NaNs, which must not get into a sum, and C between
@@ -55,3 +54,32 @@ def test_gemm_pipeline_lengths_and_edges(xs, gpu, monkeypatch, tile, fit, steps,
     want = oracle.gemm_bf16(a_bits.ravel(), b_bits.ravel(), M, N, K)
     assert np.array_equal(got[pad:pad + M * N].reshape(M, N), want.reshape(M, N))
     assert np.all(got[:pad] == 0x1234) and np.all(got[pad + M * N:] == 0x1234)
+
+
+@pytest.mark.parametrize("M,N,K", [(4100, 4096, 512), (4096 + 257, 4096, 520), (8450, 2056, 448), (2100, 8192, 456)])
+@pytest.mark.parametrize("flush", [False, True])
+def test_gemm_in_two_launches(xs, gpu, M, N, K, flush):
+    """Rows that fill whole rounds of large tiles in one launch, the rest on smaller tiles in
+    another, one command: with the queue deactivated and reactivated in between, too. Integers
+    in [-4, 4] (K x 16 < 2^24): float32 sums are exact in any order."""
+    torch = gpu
+    print(f"case gemm-two-launches M={M} N={N} K={K} flush={flush}", flush=True)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(M + K)
+    a, b = (torch.randint(-4, 5, s, device="cuda", generator=gen).to(torch.bfloat16) for s in ((M, K), (K, N)))
+    cs = [torch.full((M + 2, N), 0.5, dtype=torch.bfloat16, device="cuda") for _ in range(6 if flush else 1)]
+    torch.cuda.synchronize()
+    q, p = Queue(xs, torch, 2), xs.preempt()
+    for c in cs:
+        cmd = c_uint64()
+        xs.check(xs.halhip().HipGemmBf16CommandCreate(byref(cmd), a.data_ptr(), b.data_ptr(), c.data_ptr(), M, N, K, 1))
+        q.submit(cmd.value)
+        if flush:
+            xs.check(p.XQueueSuspend(q.xq, xs.kQueueSuspendFlagSyncHwQueue))
+            xs.check(p.XQueueResume(q.xq, xs.kQueueResumeFlagNone))
+    q.wait()
+    q.close()
+    want = (a.float() @ b.float()).to(torch.bfloat16)
+    for c in cs:
+        assert torch.equal(c[:M], want)
+        assert bool((c[M:] == 0.5).all()), "wrote behind the last row"

@@ -35,6 +35,7 @@
 // transposing reads back), whole rows of 128 bytes per eight lanes.
 // Work-group ids are remapped so that the 32 CUs of one XCD (ids equal modulo 8 land on one
 // XCD) work on neighbouring tiles and share A/B panels in that XCD's L2.
+#include <cmath>
 #include <type_traits>
 #include <utility>
 
@@ -104,6 +105,55 @@ __device__ __forceinline__ void TileOf(uint32_t wg, uint32_t tiles_m, uint32_t t
 #define XS_PIN __builtin_amdgcn_sched_barrier(0)
 #define XS_WAIT_GLOBAL_LOADS __builtin_amdgcn_s_waitcnt(0x0F70) /* vmcnt(0), nothing else */
 
+// What the matrices have to be like is kFit:
+//   kExact      M, N multiples of the tile, K of kStepK, matrices aligned to 16 bytes
+//   kEdges      M any; N and K multiples of 8, matrices aligned to 16 bytes: every 16-byte piece
+//               lies inside the matrix or outside. Pieces outside are fetched from somewhere
+//               inside (their row or column of C is not stored); behind K the fragments are
+//               masked to zero, which adds nothing to a sum
+//   kUnaligned  any N >= 8, any alignment to the element: pieces start at any multiple of two
+//               bytes, which the loads into LDS do not take: they come through registers
+//               (a tile or two in flight) and are stored to the same places. Only
+//               the last K step can reach behind the end of a matrix: its pieces are checked
+//               one by one and fetched element by element where they do.
+enum class Fit { kExact, kEdges, kUnaligned };
+
+typedef u32x4 u32x4_any __attribute__((aligned(2)));
+typedef s16x8 s16x8_any __attribute__((aligned(2)));
+
+/// The 16 bytes of v moved down by d (0..15) bytes, zeroes behind them.
+__device__ __forceinline__ u32x4 ShiftDownBytes(u32x4 v, uint32_t d)
+{
+    const u32x4 zero = { 0, 0, 0, 0 };
+    v = d & 8 ? __builtin_shufflevector(v, zero, 2, 3, 4, 4) : v;
+    v = d & 4 ? __builtin_shufflevector(v, zero, 1, 2, 3, 4) : v;
+    return u32x4 { __builtin_amdgcn_alignbyte(v.y, v.x, d & 3), __builtin_amdgcn_alignbyte(v.z, v.y, d & 3),
+                   __builtin_amdgcn_alignbyte(v.w, v.z, d & 3), __builtin_amdgcn_alignbyte(0u, v.w, d & 3) };
+}
+
+/// Eight columns of a row of C, as far as they are inside.
+template <Fit kFit>
+__device__ __forceinline__ void StoreEight(uint16_t *C, size_t row, size_t col, int M, int N, s16x8 eight)
+{
+    uint16_t *const at = C + row * (size_t)N + col;
+    if constexpr (kFit == Fit::kExact) {
+        __builtin_nontemporal_store(eight, (s16x8 *)at);
+    } else if (row < (size_t)M) {
+        if constexpr (kFit == Fit::kEdges) {
+            if (col < (size_t)N) __builtin_nontemporal_store(eight, (s16x8 *)at);
+        } else if (col + 8 <= (size_t)N) {
+            *(s16x8_any *)at = eight;
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) if (col + e < (size_t)N) at[e] = (uint16_t)eight[e];
+        }
+    }
+}
+
+/// What a K step of the large-tile kernel requests: nothing, a tile that is not the last one, or the
+/// last one.
+enum TileRequest { kNoTile, kAnyButLast, kTheLast };
+
 // Two LDS buffers and ONE barrier per K step. While the MFMAs of step t read buffer t % 2,
 // tile t + 1 is landing in the other buffer (its loads were issued a whole step earlier);
 // after the barrier buffer t % 2 is free and the loads of tile t + 2 go out, one next to
@@ -111,17 +161,19 @@ __device__ __forceinline__ void TileOf(uint32_t wg, uint32_t tiles_m, uint32_t t
 // from LDS next to the MFMAs of the current slice, one read per MFMA.
 //
 // kTile x kTile is the tile of C, kWavesM x kWavesN the wave grid over it; a wave owns
-// kBlocksM x kBlocksN blocks of 32x32. Two shapes are built: 256 with 2x4 waves (4x2 blocks
-// per wave), and 128 with 2x2 waves (2x2 blocks) for outputs of too few large tiles to fill
-// the device. Every element is summed in the same order in both.
+// kBlocksM x kBlocksN blocks of 32x32. Built for 256 with 2x4 waves (4x2 blocks
+// per wave), for exact shapes and for ragged ones (kEdges): there the last tile's loads, the last
+// step and the stores look at the edges, and the steps before are the same code (4000^3 146 us on
+// 128 x 128 tiles, 114 on these).
 //
 // (The body is a device function: the host pass cannot parse the buffer-resource builtins
 // and would silently drop the launch stub of a kernel that uses them directly.)
-template <bool kGuard, int kTile, int kWavesM, int kWavesN>
+template <bool kGuard, Fit kFit, int kTile, int kWavesM, int kWavesN>
 __device__ __forceinline__
 void GemmBf16Body(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B,
                   uint16_t *__restrict__ C, int M, int N, int K, const XGuardArgs &g)
 {
+    static_assert(kFit != Fit::kUnaligned, "loads go straight into LDS");
     constexpr int kWaves = kWavesM * kWavesN;
     constexpr int kBlocksM = kTile / (32 * kWavesM);
     constexpr int kBlocksN = kTile / (32 * kWavesN);
@@ -130,7 +182,8 @@ void GemmBf16Body(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
     constexpr int kBBytes = kStepK * kTile * 2;          // one B tile
     constexpr int kALoads = kABytes / 1024 / kWaves;     // wave-wide 1 KiB loads per wave and tile
     constexpr int kBLoads = kBBytes / 1024 / kWaves;
-    constexpr int kLoadsPerMfma = (kALoads + kBLoads) / kMfmas;
+    constexpr int kLoads = kALoads + kBLoads;
+    constexpr int kLoadsPerMfma = kLoads / kMfmas;
     constexpr int kBRowBytes = kTile * 2;                // one k row of the B tile
     constexpr int kBSlotsPerRow = kBRowBytes / 16;
     constexpr int kBRowsPerLoad = 64 / kBSlotsPerRow;
@@ -152,8 +205,10 @@ void GemmBf16Body(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
     const uint32_t wn = wave % kWavesN;
 
     uint32_t tm, tn;
-    TileOf(blockIdx.x, (uint32_t)M / kTile, (uint32_t)N / kTile, tm, tn);
+    TileOf(blockIdx.x, ((uint32_t)M + kTile - 1) / kTile, ((uint32_t)N + kTile - 1) / kTile, tm, tn);
     const size_t m0 = (size_t)tm * kTile, n0 = (size_t)tn * kTile;
+    const int steps = kFit == Fit::kExact ? K / kStepK : (K + kStepK - 1) / kStepK;
+    const int rest = K - (steps - 1) * kStepK;           // K values of the last step
 
     // ---- global -> LDS: lane l of wave-wide load q fills LDS slot 64 q + l (16 bytes) ----
     // Byte offsets of what each lane fetches, relative to the first element of the tile.
@@ -163,7 +218,9 @@ void GemmBf16Body(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
         const uint32_t q = wave * kALoads + i;
         const uint32_t line = 4 * q + (lane >> 4);
         const uint32_t piece = (lane & 15) ^ (line & 15);   // which piece of the line belongs in this slot
-        const uint32_t row = 2 * line + (piece >> 3), kc = piece & 7;
+        uint32_t row = 2 * line + (piece >> 3);
+        const uint32_t kc = piece & 7;
+        if (kFit != Fit::kExact && m0 + row >= (size_t)M) row = (uint32_t)((size_t)M - 1 - m0);   // not stored
         a_off[i] = (row * (uint32_t)K + kc * 8) * 2;
     }
 #pragma unroll
@@ -172,25 +229,45 @@ void GemmBf16Body(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
         const uint32_t k = kBRowsPerLoad * q + lane / kBSlotsPerRow;
         const uint32_t slot = lane % kBSlotsPerRow;
         const uint32_t granule = (slot >> 2) ^ (((k & 3) | ((k >> 1) & 4)) & kBGranuleMask);
-        b_off[i] = (k * (uint32_t)N + granule * 32 + (slot & 3) * 8) * 2;
+        uint32_t col = granule * 32 + (slot & 3) * 8;
+        if (kFit != Fit::kExact && n0 + col >= (size_t)N) col = 0;                                // not stored
+        b_off[i] = (k * (uint32_t)N + col) * 2;
     }
     const uint16_t *const a_tile = A + m0 * (size_t)K;   // + 64 columns per step
     const uint16_t *const b_tile = B + n0;               // + 64 rows per step
 
-    // Load number idx (A first, then B) of the tile of K step `step` into buffer `buf`.
-    auto load_piece = [&](int buf, int step, int idx) {
+    // Byte offset of load number idx (A first, then B) within its matrix's part of a K step. In the
+    // last step pieces behind K come from k = 0 of the step instead.
+    auto piece_off = [&](int idx, bool last) -> uint32_t {
+        if (idx < kALoads) {
+            if (kFit == Fit::kExact || !last) return a_off[idx];
+            const uint32_t line = 4 * (wave * kALoads + idx) + (lane >> 4);
+            const uint32_t k = (((lane & 15) ^ (line & 15)) & 7) * 8;
+            return k < (uint32_t)rest ? a_off[idx] : a_off[idx] - k * 2;
+        }
+        if (kFit == Fit::kExact || !last) return b_off[idx - kALoads];
+        const uint32_t k = kBRowsPerLoad * (wave * kBLoads + idx - kALoads) + lane / kBSlotsPerRow;
+        return k < (uint32_t)rest ? b_off[idx - kALoads] : b_off[idx - kALoads] - k * (uint32_t)N * 2;
+    };
+    // Load number idx of the tile of K step `step` into buffer `buf`.
+    auto load_piece = [&](int buf, int step, int idx, bool last) {
         if (idx < kALoads) {
             const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void *)(a_tile + (size_t)step * kStepK), 0, 0x7fffffff, 0x00020000);
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (LdsVoid *)(As0 + buf * kABytes + (wave * kALoads + idx) * 1024), 16, a_off[idx], 0, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (LdsVoid *)(As0 + buf * kABytes + (wave * kALoads + idx) * 1024), 16, piece_off(idx, last), 0, 0, 0);
         } else {
             const int i = idx - kALoads;
             const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void *)(b_tile + (size_t)step * kStepK * N), 0, 0x7fffffff, 0x00020000);
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (LdsVoid *)(Bs0 + buf * kBBytes + (wave * kBLoads + i) * 1024), 16, b_off[i], 0, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (LdsVoid *)(Bs0 + buf * kBBytes + (wave * kBLoads + i) * 1024), 16, piece_off(idx, last), 0, 0, 0);
         }
     };
     auto load_tile = [&](int buf, int step) {
+        if (kFit != Fit::kExact && step == steps - 1) {
 #pragma unroll
-        for (int idx = 0; idx < kALoads + kBLoads; ++idx) load_piece(buf, step, idx);
+            for (int idx = 0; idx < kLoads; ++idx) load_piece(buf, step, idx, true);
+        } else {
+#pragma unroll
+            for (int idx = 0; idx < kLoads; ++idx) load_piece(buf, step, idx, false);
+        }
     };
 
     // ---- LDS -> fragments ----
@@ -231,7 +308,19 @@ void GemmBf16Body(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 
-    const int steps = K / kStepK;
+    // A lane's fragment of slice ks holds k = 16 ks + 8 (lane / 32) + 0..7 of the step, for A and
+    // for B alike: everything from `rest` on becomes zero.
+    auto mask_behind_k = [&](int ks, bf16x8 *a, bf16x8 *b) {
+        const int valid = rest - (16 * ks + 8 * (int)(lane >> 5));
+        u32x4 m;
+#pragma unroll
+        for (int d = 0; d < 4; ++d) m[d] = valid >= 2 * d + 2 ? 0xFFFFFFFFu : valid == 2 * d + 1 ? 0xFFFFu : 0u;
+#pragma unroll
+        for (int i = 0; i < kBlocksM; ++i) a[i] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, a[i]) & m);
+#pragma unroll
+        for (int j = 0; j < kBlocksN; ++j) b[j] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, b[j]) & m);
+    };
+
     load_tile(0, 0);
 
     if (kGuard) {
@@ -282,8 +371,9 @@ void GemmBf16Body(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
     // work-group has to leave.
     auto step = [&](int t, auto polling, auto loading, auto reading_ahead) -> bool {
         constexpr bool kPoll = decltype(polling)::value;
-        constexpr bool kLoad = decltype(loading)::value;
+        constexpr int kLoad = decltype(loading)::value;
         constexpr bool kReadAhead = decltype(reading_ahead)::value;
+        constexpr bool kMask = kFit != Fit::kExact && !kReadAhead;
         const int cur = t & 1;
         // Wave 0 asks for the preempt word here, with a vector load that is on its way during
         // the whole step, and looks at it just before the barrier: no wave ever waits for the
@@ -292,9 +382,13 @@ void GemmBf16Body(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
         uint32_t polled = 0;
         if (kPoll && wave == 0) polled = xguard_read_flag_begin(xguard_flag_copy(g, blockIdx.x));
 
+        if (kMask) mask_behind_k(0, fa[0], fb[0]);
         slice(0, cur, 1);
+        if (kMask) mask_behind_k(1, fa[1], fb[1]);
         slice(1, cur, 2);
+        if (kMask) mask_behind_k(2, fa[0], fb[0]);
         slice(0, cur, 3);
+        if (kMask) mask_behind_k(3, fa[1], fb[1]);
 
         if (kPoll && wave == 0) {
             const bool current = xguard_read_flag_end(polled) == g.epoch;
@@ -322,9 +416,10 @@ void GemmBf16Body(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
                     if (n < kBlocksM) fa[0][n] = read_a(cur ^ 1, 0, n);
                     else if (n < kBlocksM + kBlocksN) fb[0][n - kBlocksM] = read_b(cur ^ 1, 0, n - kBlocksM);
                 }
-                if (kLoad) {
 #pragma unroll
-                    for (int l = 0; l < kLoadsPerMfma; ++l) load_piece(cur, t + 2, n * kLoadsPerMfma + l);
+                for (int l = 0; l < kLoadsPerMfma; ++l) {
+                    if constexpr (kLoad == kAnyButLast) load_piece(cur, t + 2, n * kLoadsPerMfma + l, false);
+                    if constexpr (kLoad == kTheLast) load_piece(cur, t + 2, n * kLoadsPerMfma + l, true);
                 }
                 XS_PIN;
             }
@@ -332,19 +427,26 @@ void GemmBf16Body(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
     };
     constexpr std::true_type yes {};
     constexpr std::false_type no {};
+    constexpr std::integral_constant<int, kNoTile> no_tile {};
+    constexpr std::integral_constant<int, kAnyButLast> any_but_last {};
+    constexpr std::integral_constant<int, kTheLast> the_last {};
 
-    const int loading_steps = steps - 2; // steps whose tile t + 2 exists
+    // steps that request a tile (kExact: the last one is like the others)
+    const int main_steps = steps - 2 - (kFit == Fit::kExact ? 0 : 1);
     if constexpr (!kGuard) {
-        for (int t = 0; t < loading_steps; ++t) step(t, no, yes, yes);
+        for (int t = 0; t < main_steps; ++t) step(t, no, any_but_last, yes);
     } else {
-        for (int t0 = 0; t0 < loading_steps; t0 += kPollSteps) {
-            const int last = min(t0 + kPollSteps, loading_steps) - 1;
-            for (int t = t0; t < last; ++t) step(t, no, yes, yes);
-            if (!step(last, yes, yes, yes)) return;
+        for (int t0 = 0; t0 < main_steps; t0 += kPollSteps) {
+            const int last = min(t0 + kPollSteps, main_steps) - 1;
+            for (int t = t0; t < last; ++t) step(t, no, any_but_last, yes);
+            if (!step(last, yes, any_but_last, yes)) return;
         }
     }
-    if (steps >= 2) step(steps - 2, no, no, yes);
-    step(steps - 1, no, no, no);
+    if constexpr (kFit != Fit::kExact) {
+        if (steps > 2) step(steps - 3, no, the_last, yes);
+    }
+    if (steps >= 2) step(steps - 2, no, no_tile, yes);
+    step(steps - 1, no, no_tile, no);
 
     // Write-out. A lane holds one column of sixteen rows of each 32x32 block (four runs of four
     // consecutive rows), so storing from the accumulators would mean 2-byte stores to sixteen
@@ -385,7 +487,7 @@ void GemmBf16Body(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
             const s16x8 row = __builtin_shufflevector(left, right, 0, 1, 2, 3, 4, 5, 6, 7);
             // (non-temporal: C is written once and not read again; left in L2 it pushes out A and B panels
             // that the XCD's other tiles still need: 1 % of the kernel)
-            __builtin_nontemporal_store(row, (s16x8 *)(C + (row0 + 8 * q + get_row + (l16 & 3)) * (size_t)N + col0));
+            StoreEight<kFit>(C, row0 + 8 * q + get_row + (l16 & 3), col0, M, N, row);
         }
     }
 
@@ -395,12 +497,12 @@ void GemmBf16Body(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
     }
 }
 
-template <bool kGuard, int kTile, int kWavesM, int kWavesN>
+template <bool kGuard, Fit kFit, int kTile, int kWavesM, int kWavesN>
 __global__ __launch_bounds__(64 * kWavesM * kWavesN)
 void GemmBf16Kernel(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B,
                     uint16_t *__restrict__ C, int M, int N, int K, XGuardArgs g)
 {
-    GemmBf16Body<kGuard, kTile, kWavesM, kWavesN>(A, B, C, M, N, K, g);
+    GemmBf16Body<kGuard, kFit, kTile, kWavesM, kWavesN>(A, B, C, M, N, K, g);
 }
 
 
@@ -426,19 +528,6 @@ void GemmBf16Kernel(const uint16_t *__restrict__ A, const uint16_t *__restrict__
 //   2048^3            23.7 -> 17.8 us = 0.96 PFLOP/s
 //   2000^3            86.5 -> 21.8 us      2000 x 1999 x 2047   254 -> 31.0 us
 //   128 x 128 x 8192  76.0 -> 19.7 us      4097 x 4095 x 4097   2122 -> 243 us
-//
-// What the matrices have to be like is kFit:
-//   kExact      M, N multiples of the tile, K of kStepK, matrices aligned to 16 bytes
-//   kEdges      M any; N and K multiples of 8, matrices aligned to 16 bytes: every 16-byte piece
-//               lies inside the matrix or outside. Pieces outside are fetched from somewhere
-//               inside (their row or column of C is not stored); behind K the fragments are
-//               masked to zero, which adds nothing to a sum
-//   kUnaligned  any N >= 8, any alignment to the element: pieces start at any multiple of two
-//               bytes, which the loads into LDS do not take: they come through registers
-//               (kRegTiles tiles of them in flight) and are stored to the same places. Only
-//               the last K step can reach behind the end of a matrix: its pieces are checked
-//               one by one and fetched element by element where they do.
-enum class Fit { kExact, kEdges, kUnaligned };
 
 /// What a K step does besides its MFMAs (see GemmDeepBody).
 enum LoadKind { kNothing, kWholeTile, kLastTile };
@@ -451,25 +540,12 @@ struct Step
     static constexpr int kNewer = kNewer_;   // tiles in flight behind the one waited for
 };
 
-typedef u32x4 u32x4_any __attribute__((aligned(2)));
-typedef s16x8 s16x8_any __attribute__((aligned(2)));
-
 /// s_waitcnt vmcnt(n) lgkmcnt(0)
 template <int kVm>
 __device__ __forceinline__ void WaitLoadsAndLds()
 {
     static_assert(kVm >= 0 && kVm < 64, "vmcnt has six bits");
     __builtin_amdgcn_s_waitcnt((kVm & 15) | (7 << 4) | ((kVm >> 4) << 14));
-}
-
-/// The 16 bytes of v moved down by d (0..15) bytes, zeroes behind them.
-__device__ __forceinline__ u32x4 ShiftDownBytes(u32x4 v, uint32_t d)
-{
-    const u32x4 zero = { 0, 0, 0, 0 };
-    v = d & 8 ? __builtin_shufflevector(v, zero, 2, 3, 4, 4) : v;
-    v = d & 4 ? __builtin_shufflevector(v, zero, 1, 2, 3, 4) : v;
-    return u32x4 { __builtin_amdgcn_alignbyte(v.y, v.x, d & 3), __builtin_amdgcn_alignbyte(v.z, v.y, d & 3),
-                   __builtin_amdgcn_alignbyte(v.w, v.z, d & 3), __builtin_amdgcn_alignbyte(0u, v.w, d & 3) };
 }
 
 /// s_waitcnt as above with at most `newer` tiles of kLoads loads in flight (`newer` is uniform, at most kMost).
@@ -842,19 +918,7 @@ void GemmDeepBody(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
             const s16x4 right = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsS16x4 *)(p + 4 * kStripColumnBytes));
             const s16x8 eight = __builtin_shufflevector(left, right, 0, 1, 2, 3, 4, 5, 6, 7);
             const size_t row = row0 + kRowsPerStore * q + get_row + (l16 & 3);
-            uint16_t *const at = C + row * (size_t)N + col0;
-            if constexpr (kFit == Fit::kExact) {
-                __builtin_nontemporal_store(eight, (s16x8 *)at);
-            } else if (row < (size_t)M) {
-                if constexpr (kFit == Fit::kEdges) {
-                    if (col0 < (size_t)N) __builtin_nontemporal_store(eight, (s16x8 *)at);
-                } else if (col0 + 8 <= (size_t)N) {
-                    *(s16x8_any *)at = eight;
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) if (col0 + e < (size_t)N) at[e] = (uint16_t)eight[e];
-                }
-            }
+            StoreEight<kFit>(C, row, col0, M, N, eight);
         }
     }
 
@@ -956,64 +1020,80 @@ void GemmBf16AnyShapeKernel(const uint16_t *__restrict__ A, const uint16_t *__re
     if (kGuard) guard.Commit();
 }
 
-/// How a command computes its product: which kernel, on tiles of which size, and what it may
-/// assume about the matrices.
-struct Plan
+/// A run of rows of C and how they are computed: which kernel, on tiles of which size, and what it
+/// may assume about the matrices.
+struct Part
 {
+    int first_row, rows;
     int tile;       // edge of a tile of C
     Fit fit;        // of the kernels with 256, 128 and 64 tiles
     bool narrow;    // the kernel without requirements
     uint64_t tiles; // work-groups = bytes of the progress map
 };
 
+/// One launch, or two for rows that do not fill whole rounds of large tiles.
+struct Plan
+{
+    Part part[2];
+    int parts;
+    uint64_t Tiles() const { return part[0].tiles + (parts > 1 ? part[1].tiles : 0); }
+};
+
 class HipGemmCommand final : public HipGuardedCommand
 {
 public:
-    HipGemmCommand(const void *A, const void *B, void *C, int M, int N, int K, const Plan &plan, int guard_mode)
-        : HipGuardedCommand((uint32_t)plan.tiles, guard_mode)
-        , A_((const uint16_t *)A), B_((const uint16_t *)B), C_((uint16_t *)C), M_(M), N_(N), K_(K), plan_(plan) {}
+    HipGemmCommand(const void *A, const void *B, void *C, int N, int K, const Plan &plan, int guard_mode)
+        : HipGuardedCommand((uint32_t)plan.Tiles(), guard_mode)
+        , A_((const uint16_t *)A), B_((const uint16_t *)B), C_((uint16_t *)C), N_(N), K_(K), plan_(plan) {}
 
 protected:
     virtual hipError_t LaunchKernel(hipStream_t stream, bool guarded, const XGuardArgs &g) override
     {
-        if (plan_.narrow) {
-            const uint32_t tiles_n = (uint32_t)((N_ + kAnyTile - 1) / kAnyTile);
-            const dim3 grid((uint32_t)plan_.tiles), block(256);
-            const hipEvent_t stop = TakeStopEvent();
-            if (guarded) LaunchWithStop(stop, GemmBf16AnyShapeKernel<true>, grid, block, stream, A_, B_, C_, M_, N_, K_, tiles_n, g);
-            else         LaunchWithStop(stop, GemmBf16AnyShapeKernel<false>, grid, block, stream, A_, B_, C_, M_, N_, K_, tiles_n, g);
-        } else if (plan_.tile == kLargeTile) {
-            Launch(guarded ? GemmBf16Kernel<true, kLargeTile, 2, 4> : GemmBf16Kernel<false, kLargeTile, 2, 4>, 512, stream, g);
-        } else if (plan_.tile == kSmallTile) {
-            LaunchDeep<kSmallTile, 4>(stream, guarded, g);
-        } else {
-            LaunchDeep<kTinyTile, 4>(stream, guarded, g);
-        }
-        return hipGetLastError();
+        const hipEvent_t stop = TakeStopEvent();   // for the command's last kernel
+        if (plan_.parts == 1) return LaunchPart(plan_.part[0], stop, stream, guarded, g);
+        const hipError_t err = LaunchPart(plan_.part[0], nullptr, stream, guarded, g);
+        if (err != hipSuccess) return err;
+        // the second part's progress bytes follow the first part's
+        XGuardArgs behind = g;
+        if (behind.done != nullptr) behind.done += plan_.part[0].tiles;
+        return LaunchPart(plan_.part[1], stop, stream, guarded, behind);
     }
 
 private:
-    using Kernel = void (*)(const uint16_t *, const uint16_t *, uint16_t *, int, int, int, XGuardArgs);
-    void Launch(Kernel kernel, unsigned threads, hipStream_t stream, const XGuardArgs &g)
+    hipError_t LaunchPart(const Part &part, hipEvent_t stop, hipStream_t stream, bool guarded, const XGuardArgs &g)
     {
-        LaunchWithStop(TakeStopEvent(), kernel, dim3((uint32_t)plan_.tiles), dim3(threads), stream, A_, B_, C_, M_, N_, K_, g);
-    }
-    template <int kTile, int kStages>
-    void LaunchDeep(hipStream_t stream, bool guarded, const XGuardArgs &g)
-    {
-        switch (plan_.fit) {
-        case Fit::kExact:
-            return Launch(guarded ? GemmDeepKernel<true, Fit::kExact, kTile, kStages> : GemmDeepKernel<false, Fit::kExact, kTile, kStages>, 256, stream, g);
-        case Fit::kEdges:
-            return Launch(guarded ? GemmDeepKernel<true, Fit::kEdges, kTile, kStages> : GemmDeepKernel<false, Fit::kEdges, kTile, kStages>, 256, stream, g);
-        case Fit::kUnaligned:
-            return Launch(guarded ? GemmDeepKernel<true, Fit::kUnaligned, kTile, kStages> : GemmDeepKernel<false, Fit::kUnaligned, kTile, kStages>, 256, stream, g);
+        if (part.narrow) {
+            const uint32_t tiles_n = (uint32_t)((N_ + kAnyTile - 1) / kAnyTile);
+            const dim3 grid((uint32_t)part.tiles), block(256);
+            LaunchWithStop(stop, guarded ? GemmBf16AnyShapeKernel<true> : GemmBf16AnyShapeKernel<false>, grid, block, stream,
+                           A_ + (size_t)part.first_row * K_, B_, C_ + (size_t)part.first_row * N_, part.rows, N_, K_, tiles_n, g);
+            return hipGetLastError();
         }
+        Kernel kernel = nullptr;
+        switch (part.fit) {
+        case Fit::kExact:     kernel = KernelFor<Fit::kExact>(part.tile, guarded); break;
+        case Fit::kEdges:     kernel = KernelFor<Fit::kEdges>(part.tile, guarded); break;
+        case Fit::kUnaligned: kernel = KernelFor<Fit::kUnaligned>(part.tile, guarded); break;   // (never large)
+        }
+        LaunchWithStop(stop, kernel, dim3((uint32_t)part.tiles), dim3(part.tile == kLargeTile ? 512 : 256), stream,
+                       A_ + (size_t)part.first_row * K_, B_, C_ + (size_t)part.first_row * N_, part.rows, N_, K_, g);
+        return hipGetLastError();
+    }
+
+    using Kernel = void (*)(const uint16_t *, const uint16_t *, uint16_t *, int, int, int, XGuardArgs);
+    template <Fit kFit>
+    static Kernel KernelFor(int tile, bool guarded)
+    {
+        if constexpr (kFit != Fit::kUnaligned) {
+            if (tile == kLargeTile) return guarded ? GemmBf16Kernel<true, kFit, kLargeTile, 2, 4> : GemmBf16Kernel<false, kFit, kLargeTile, 2, 4>;
+        }
+        if (tile == kSmallTile) return guarded ? GemmDeepKernel<true, kFit, kSmallTile, 4> : GemmDeepKernel<false, kFit, kSmallTile, 4>;
+        return guarded ? GemmDeepKernel<true, kFit, kTinyTile, 4> : GemmDeepKernel<false, kFit, kTinyTile, 4>;
     }
 
     const uint16_t *A_, *B_;
     uint16_t *C_;
-    const int M_, N_, K_;
+    const int N_, K_;
     const Plan plan_;
 };
 
@@ -1032,28 +1112,93 @@ inline uint32_t ComputeUnits()
     return cus;
 }
 
-/// The plan for a shape. Large tiles do more arithmetic per byte read from LDS, but each keeps one
-/// compute unit busy, and so does a small one: large tiles when they cover more than half of the
-/// compute units (4096^3: 101 us against 119 on small tiles; 2048^3, a quarter covered: 41 against
-/// 17.8), small ones when they cover more than half (2048^3: 17.8 us against 27.7 on tiny tiles;
-/// 1024^3, a quarter covered: 9.4 against 5.8), else tiny ones. The large tiles take exact
-/// multiples only. XSCHED_HIP_GEMM_TILE=64|128|256 overrides the tile where the shape allows.
-inline Plan PlanFor(const void *A, const void *B, const void *C, int M, int N, int K)
+inline bool Aligned(const void *A, const void *B, const void *C, int N, int K)
 {
-    if (N < 8 || (int64_t)M * K < 8 || K > kMaxK || N > kMaxK) return Plan { kAnyTile, Fit::kUnaligned, true, TilesOf(M, N, kAnyTile) };
-    const bool aligned = (((uintptr_t)A | (uintptr_t)B | (uintptr_t)C) & 15) == 0 && N % 8 == 0 && K % 8 == 0;
-    auto exact = [&](int tile) { return aligned && M % tile == 0 && N % tile == 0 && K % kStepK == 0; };
-    int tile = kSmallTile;
+    return (((uintptr_t)A | (uintptr_t)B | (uintptr_t)C) & 15) == 0 && N % 8 == 0 && K % 8 == 0;
+}
+
+/// XSCHED_HIP_GEMM_TILE: 64, 128 or 256, else 0.
+inline int ForcedTile()
+{
     int64_t forced = 0;
-    if (GetEnvInt64("XSCHED_HIP_GEMM_TILE", forced) &&
-        (forced == kTinyTile || forced == kSmallTile || (forced == kLargeTile && exact(kLargeTile)))) {
-        tile = (int)forced;
-    } else if (exact(kLargeTile) && TilesOf(M, N, kLargeTile) * 2 > ComputeUnits()) {
-        tile = kLargeTile;
-    } else if (TilesOf(M, N, kSmallTile) * 2 <= ComputeUnits()) {
-        tile = kTinyTile;
+    GetEnvInt64("XSCHED_HIP_GEMM_TILE", forced);
+    return forced == kTinyTile || forced == kSmallTile || forced == kLargeTile ? (int)forced : 0;
+}
+
+inline Part PartOf(int first_row, int rows, int N, int K, bool aligned, int tile)
+{
+    const bool exact = aligned && rows % tile == 0 && N % tile == 0 && K % kStepK == 0;
+    return Part { first_row, rows, tile, exact ? Fit::kExact : aligned ? Fit::kEdges : Fit::kUnaligned, false, TilesOf(rows, N, tile) };
+}
+
+/// Roughly how long a part takes, in us: a launch, then rounds of one tile per compute unit, each
+/// with its first loads and its write-out, the last round quicker the fewer units it keeps busy.
+inline double MicrosOf(const Part &part, int K)
+{
+    // us of a round, and per K step of a full round and of one with a single tile: [exact, edges, unaligned]
+    struct Rates { double round, full, single; };
+    constexpr Rates large[3] = { { 2.5, 1.54, 0.95 }, { 2.5, 1.56, 0.97 }, {} };
+    constexpr Rates small[3] = { { 2.5, 0.45, 0.37 }, { 2.5, 0.53, 0.41 }, { 2.5, 0.80, 0.60 } };
+    constexpr Rates tiny[3] = { { 0.5, 0.195, 0.14 }, { 0.5, 0.25, 0.16 }, { 0.5, 0.35, 0.25 } };
+    const Rates &r = (part.tile == kLargeTile ? large : part.tile == kSmallTile ? small : tiny)[(int)part.fit];
+    const double rounds = (double)part.tiles / ComputeUnits(), whole = std::floor(rounds);
+    const double step = whole * r.full + (rounds > whole ? r.single + (r.full - r.single) * (rounds - whole) : 0.0);
+    return 3.0 + std::ceil(rounds) * r.round + step * ((K + kStepK - 1) / kStepK);
+}
+
+/// The plan for a shape: the quickest by the estimate above of one launch on large, small or tiny
+/// tiles and of two, large tiles for the rows that fill whole tiles, or whole rounds of them, and
+/// whatever is quickest for the rest. Large tiles do more arithmetic per byte read from LDS, but a
+/// round of few tiles leaves compute units idle (pass times in us, large and small tiles as they were
+/// chosen before by the share of the compute units covered and by exact multiples only, and now:
+/// 8197 x 8192 x 8192 1038 -> 836, 4100 x 4096 x 4096 156 -> 130, 6016 x 6016 x 8192 564 -> 485,
+/// 6000 x 6008 x 6000 539 -> 424, 4000^3 146 -> 114; 4096^3 106 per command on large tiles against
+/// 126 on small ones, 2048^3 20.9 on small against 30.1 on tiny ones, 1024^3 5.8 on tiny ones against
+/// 9.4 on small ones). Rows without 16-byte alignment do not go straight into LDS, which the large
+/// tiles need (a tile on its way through registers beside their accumulators does not fit).
+/// XSCHED_HIP_GEMM_TILE=64|128|256 overrides the tile where the shape allows.
+inline Plan PlanFor(const void *A, const void *B, const void *C, int M, int N, int K, int forced)
+{
+    if (N < 8 || (int64_t)M * K < 8 || K > kMaxK || N > kMaxK) {
+        return Plan { { Part { 0, M, kAnyTile, Fit::kUnaligned, true, TilesOf(M, N, kAnyTile) }, {} }, 1 };
     }
-    return Plan { tile, exact(tile) ? Fit::kExact : aligned ? Fit::kEdges : Fit::kUnaligned, false, TilesOf(M, N, tile) };
+    const bool aligned = Aligned(A, B, C, N, K);
+    if (forced != 0 && (forced != kLargeTile || aligned)) return Plan { { PartOf(0, M, N, K, aligned, forced), {} }, 1 };
+    auto best_part = [&](int first_row, int rows) {
+        Part best = PartOf(first_row, rows, N, K, aligned, kSmallTile);
+        for (const int tile : { kTinyTile, kLargeTile }) {
+            if (tile == kLargeTile && !aligned) continue;
+            const Part other = PartOf(first_row, rows, N, K, aligned, tile);
+            if (MicrosOf(other, K) < MicrosOf(best, K)) best = other;
+        }
+        return best;
+    };
+    Plan best { { best_part(0, M), {} }, 1 };
+    double least = MicrosOf(best.part[0], K);
+    auto consider = [&](int64_t large_rows) {
+        if (!aligned || large_rows <= 0 || large_rows >= M) return;
+        const Part first = PartOf(0, (int)large_rows, N, K, aligned, kLargeTile), rest = best_part((int)large_rows, M - (int)large_rows);
+        const double both = MicrosOf(first, K) + MicrosOf(rest, K);
+        if (both < least) { least = both; best = Plan { { first, rest }, 2 }; }
+    };
+    consider((int64_t)(M / kLargeTile) * kLargeTile);                       // all whole large tiles
+    const int64_t in_row = (N + kLargeTile - 1) / kLargeTile;                // all whole rounds of large tiles
+    const int64_t whole_rounds = (int64_t)TilesOf(M, N, kLargeTile) / ComputeUnits();
+    consider(whole_rounds * ComputeUnits() / in_row * kLargeTile);
+    return best;
+}
+
+/// Tiles by which a shape is accepted or refused. They are the tiles of the kernels that such shapes
+/// once ran on: 128 x 128 or 256 x 256 for the rows up to the last multiple of 128 where everything
+/// else is a multiple of the tiles, and 64 x 64.
+inline uint64_t CountedTiles(const void *A, const void *B, const void *C, int M, int N, int K, int forced)
+{
+    const int whole = M / kSmallTile * kSmallTile;
+    if (forced == kTinyTile || whole == 0 || !Aligned(A, B, C, N, K) || N % kSmallTile != 0 || K % kStepK != 0 || K > kMaxK || N > kMaxK) {
+        return TilesOf(M, N, kAnyTile);
+    }
+    const int tile = whole % kLargeTile == 0 && N % kLargeTile == 0 && forced != kSmallTile ? kLargeTile : kSmallTile;
+    return TilesOf(whole, N, tile) + TilesOf(M - whole, N, kAnyTile);
 }
 
 } // namespace gemm
@@ -1072,13 +1217,13 @@ EXPORT_C_FUNC XResult HipGemmBf16CommandCreate(HwCommandHandle *cmd, const void 
         XWARN("HipGemmBf16CommandCreate: M, N and K must be positive and the matrices aligned to their elements (got %d %d %d)", M, N, K);
         return kXSchedErrorInvalidValue;
     }
-    const gemm::Plan plan = gemm::PlanFor(A, B, C, M, N, K);
-    // one progress-map byte per tile; a shape without alignment is held to the limit in 64 x 64 tiles
-    const uint64_t tiles = plan.fit == gemm::Fit::kUnaligned ? gemm::TilesOf(M, N, gemm::kAnyTile) : plan.tiles;
-    if (tiles > GuardState::kMaxWorkGroups) {
+    const int forced = gemm::ForcedTile();
+    const gemm::Plan plan = gemm::PlanFor(A, B, C, M, N, K, forced);
+    // one progress-map byte per tile
+    if (plan.Tiles() > GuardState::kMaxWorkGroups || gemm::CountedTiles(A, B, C, M, N, K, forced) > GuardState::kMaxWorkGroups) {
         XWARN("HipGemmBf16CommandCreate: %d x %d needs more than 2^18 tiles", M, N);
         return kXSchedErrorInvalidValue;
     }
-    *cmd = HwCommandManager::Add(std::make_shared<gemm::HipGemmCommand>(A, B, C, M, N, K, plan, guard));
+    *cmd = HwCommandManager::Add(std::make_shared<gemm::HipGemmCommand>(A, B, C, N, K, plan, guard));
     return kXSchedSuccess;
 }
