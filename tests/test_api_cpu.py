@@ -82,6 +82,14 @@ def test_gemm_command_takes_any_shape_and_refuses_what_no_kernel_can_address(xs)
         assert ok(*bad) == xs.kXSchedErrorInvalidValue, bad
 
 
+def test_gemm_shapes_near_the_limit_of_tiles_are_taken(xs):
+    """262025 tiles by the count that decides about a shape, of at most 2^18 = 262144; the quickest
+    division into two launches would have 262295."""
+    from ctypes import byref, c_uint64
+    lib, cmd = xs.halhip(), c_uint64()
+    assert lib.HipGemmBf16CommandCreate(byref(cmd), 1 << 20, 2 << 20, 3 << 20, 13413745, 1280, 1024, 1) == xs.kXSchedSuccess
+
+
 def test_enum_values_are_the_wire_values():
     text = open(os.path.join(INC, "types.h")).read()
     want = {"kXSchedSuccess": 0, "kXSchedErrorNotFound": 3, "kXSchedErrorNotSupported": 5,

@@ -1157,6 +1157,8 @@ inline double MicrosOf(const Part &part, int K)
 /// 9.4 on small ones). Rows without 16-byte alignment do not go straight into LDS, which the large
 /// tiles need (a tile on its way through registers beside their accumulators does not fit).
 /// XSCHED_HIP_GEMM_TILE=64|128|256 overrides the tile where the shape allows.
+/// A plan of more tiles than the progress map holds is passed over for one that fits: 13413745 x
+/// 1280 x 1024, 262025 tiles by the count below, would be quickest as two launches of 262295.
 inline Plan PlanFor(const void *A, const void *B, const void *C, int M, int N, int K, int forced)
 {
     if (N < 8 || (int64_t)M * K < 8 || K > kMaxK || N > kMaxK) {
@@ -1169,7 +1171,8 @@ inline Plan PlanFor(const void *A, const void *B, const void *C, int M, int N, i
         for (const int tile : { kTinyTile, kLargeTile }) {
             if (tile == kLargeTile && !aligned) continue;
             const Part other = PartOf(first_row, rows, N, K, aligned, tile);
-            if (MicrosOf(other, K) < MicrosOf(best, K)) best = other;
+            const bool fits = other.tiles <= GuardState::kMaxWorkGroups, best_fits = best.tiles <= GuardState::kMaxWorkGroups;
+            if (fits && (!best_fits || MicrosOf(other, K) < MicrosOf(best, K))) best = other;
         }
         return best;
     };
@@ -1179,6 +1182,7 @@ inline Plan PlanFor(const void *A, const void *B, const void *C, int M, int N, i
         if (!aligned || large_rows <= 0 || large_rows >= M) return;
         const Part first = PartOf(0, (int)large_rows, N, K, aligned, kLargeTile), rest = best_part((int)large_rows, M - (int)large_rows);
         const double both = MicrosOf(first, K) + MicrosOf(rest, K);
+        if (first.tiles + rest.tiles > GuardState::kMaxWorkGroups) return;
         if (both < least) { least = both; best = Plan { { first, rest }, 2 }; }
     };
     consider((int64_t)(M / kLargeTile) * kLargeTile);                       // all whole large tiles
