@@ -26,9 +26,12 @@ constexpr int64_t kStandBySliceMicros = 25;  // how often it looks whether their
 constexpr int64_t kStandByPollMicros = 2;     // and how long it looks without a pause while another queue is paused
 constexpr unsigned long kLauncherTimerSlackNanos = 1000; // timed waits of the launcher end on time (the default slack is 50 us)
 
-/// Suspended XQueues of this process. What a running queue's Idle event is most likely to bring
-/// is the resume of one of them, and until then the device may stand idle.
-std::atomic<int> g_suspended_queues { 0 };
+/// XQueues of this process that were suspended with commands unfinished. What a running queue's
+/// Idle event is most likely to bring is the resume of one of them, and until then the device may
+/// stand idle. (Queues suspended with nothing to do don't count: an early Idle event would only
+/// resume them between two commands of the running queue, and its next Ready event suspend them
+/// again, 6 us per command.)
+std::atomic<int> g_interrupted_queues { 0 };
 
 size_t PowerOfTwoAtLeast(size_t n)
 {
@@ -213,8 +216,8 @@ RingXQueue::Step RingXQueue::NextStep(Pending *out)
                 const int64_t newest = handed_over_.load(std::memory_order_acquire);
                 if (newest != seen) { seen = newest; until = now + std::chrono::microseconds(kStandByMicros); }
                 if (now >= until) break;
-                if (g_suspended_queues.load(std::memory_order_relaxed) > 0 && !suspended_.load(std::memory_order_relaxed)) {
-                    // Another queue is paused, most likely for this one: from the end of this
+                if (g_interrupted_queues.load(std::memory_order_relaxed) > 0 && !suspended_.load(std::memory_order_relaxed)) {
+                    // Another queue was stopped in its work, most likely for this one: from the end of this
                     // queue's last command to its Idle event the device has nothing to do.
                     // Looking every 25 us left it idle for 20 us per preemption; here the
                     // launcher keeps looking (at its own counters, not at the runtime).
@@ -632,7 +635,8 @@ void RingXQueue::Suspend(int64_t flags)
     {
         Guard op(op_mu_);
         if (suspended_.exchange(true)) return;
-        g_suspended_queues.fetch_add(1, std::memory_order_relaxed);
+        interrupted_ = retired_.load(std::memory_order_acquire) < next_idx_.load(std::memory_order_acquire) - 1;
+        if (interrupted_) g_interrupted_queues.fetch_add(1, std::memory_order_relaxed);
         suspension = ++suspensions_;
         if (!waits) PauseAndFlush();
     }
@@ -671,7 +675,7 @@ void RingXQueue::Resume(int64_t flags)
     if (!suspended_.load()) return;   // the usual case of a round: nothing to undo
     Guard op(op_mu_);
     if (!suspended_.exchange(false)) return;
-    g_suspended_queues.fetch_sub(1, std::memory_order_relaxed);
+    if (interrupted_) g_interrupted_queues.fetch_sub(1, std::memory_order_relaxed);
     const bool drop = (flags & kQueueResumeFlagDropCommands) != 0;
 
     if (level_ > kPreemptLevelBlock) {

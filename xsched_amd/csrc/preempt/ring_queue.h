@@ -151,6 +151,7 @@ private:
     bool caller_may_launch_ = false;
     std::mutex op_mu_;                  // one Suspend() or Resume() at a time; taken before the locks above
     int64_t suspensions_ = 0;           // op_mu_: number of the newest suspension
+    bool interrupted_ = false;          // op_mu_: it found commands that were not finished
     std::atomic_bool suspended_ { false };   // changed under op_mu_
     std::atomic_bool closing_ { false };
     std::thread launcher_;
