@@ -1,0 +1,42 @@
+"""When a running queue's Idle event goes out, beside queues that it interrupts
+(tests/burst_driver.cpp). Figures of three kinds of builds on one machine: looking for the end of
+the foreground's commands every 25 us, without a pause whatever the foreground does, and without a
+pause only for isolated commands."""
+import os
+import re
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+LIB = os.path.join(ROOT, "xsched_amd", "lib")
+
+
+@pytest.fixture(scope="module")
+def driver(tmp_path_factory):
+    if not os.path.exists(os.path.join(LIB, "libhalhost.so")):
+        pytest.skip("libraries not built")
+    exe = str(tmp_path_factory.mktemp("burst") / "burst_driver")
+    subprocess.run(["g++", "-std=c++20", "-O2", "-I", os.path.join(ROOT, "include"),
+                    os.path.join(ROOT, "tests", "burst_driver.cpp"), "-o", exe,
+                    "-L", LIB, "-Wl,-rpath," + LIB, "-lhalhost", "-lpreempt", "-pthread"], check=True)
+
+    def figure(*args):
+        out = subprocess.run([exe, *map(str, args)], capture_output=True, text=True, timeout=60,
+                             env=dict(os.environ, XLOG_LEVEL="WARN"))
+        assert out.returncode == 0, out.stdout + out.stderr
+        return float(re.match(r"[\d.]+", out.stdout).group())
+    return figure
+
+
+def best(runs, figure):
+    """The least of up to `runs` figures (other work on the machine only ever adds)."""
+    return min(figure() for _ in range(runs))
+
+
+# 20 commands, each waited for, are one busy period while the caller is quick to send the next:
+# 2.1-3.4 and 4.2-6.1 replays of the background per burst with slices of 25 us, 26-29 and 22-31
+# with an Idle event after every command.
+@pytest.mark.parametrize("gap,most", [(0, 8), (5, 12)])
+def test_a_burst_of_waited_commands_does_not_resume_the_background_between_them(driver, gap, most):
+    assert best(3, lambda: driver("bursts", 40, gap)) <= most

@@ -23,7 +23,9 @@ constexpr int64_t kSpinMicros = 150; // a waiter polls this long before it sleep
 constexpr int64_t kDirectBurst = 8;           // submissions in a row without a wait that are still launched by the submitter
 constexpr int64_t kStandByMicros = 500;      // how long the launcher leaves the device to callers that launch themselves
 constexpr int64_t kStandBySliceMicros = 25;  // how often it looks whether their commands have retired
-constexpr int64_t kStandByPollMicros = 2;     // and how long it looks without a pause while another queue is paused
+constexpr int64_t kStandByPollMicros = 2;     // and how long it looks without a pause while another queue is interrupted
+constexpr int64_t kIsolatedMicros = 40;      // a busy period that begins this long after the last one is not its continuation
+constexpr int64_t kIsolatedRun = 4;          // so many of them in a row, and the next command is not waited for with the Idle event
 constexpr unsigned long kLauncherTimerSlackNanos = 1000; // timed waits of the launcher end on time (the default slack is 50 us)
 
 /// XQueues of this process that were suspended with commands unfinished. What a running queue's
@@ -47,7 +49,7 @@ RingXQueue::RingXQueue(std::shared_ptr<HwQueue> hwq, XPreemptLevel level, int64_
              kQueueFeatureSyncSuspend | kQueueFeatureResumeDropCommands |
              (hwq->SupportDynamicLevel() ? kQueueFeatureDynamicLevel : 0),
              hwq)
-    , ring_(kInitialRingSlots), threshold_(threshold), batch_(batch), level_(level)
+    , ring_(kInitialRingSlots), isolated_run_(kIsolatedRun), threshold_(threshold), batch_(batch), level_(level)
 {
     XASSERT(level_ > kPreemptLevelUnknown && level_ < kPreemptLevelMax, "invalid preempt level: %d", level_);
     // With fewer window slots than the marker period the window could fill up without a
@@ -111,7 +113,8 @@ void RingXQueue::Submit(std::shared_ptr<HwCommand> hw_cmd)
 {
     XASSERT(hw_cmd != nullptr, "hw_cmd should not be nullptr");
     hw_cmd->OnSubmit(shared_from_this());
-    hw_cmd->SetIdx(next_idx_.fetch_add(1, std::memory_order_acq_rel));
+    const int64_t idx = next_idx_.fetch_add(1, std::memory_order_acq_rel);
+    hw_cmd->SetIdx(idx);
     kHwQueue->OnHwCommandSubmit(hw_cmd);
     const bool wait_for_launch = hw_cmd->GetProps(kCommandPropertyBlockingSubmit) != 0;
     hw_cmd->SetState(kCommandStatePending);
@@ -129,6 +132,8 @@ void RingXQueue::Submit(std::shared_ptr<HwCommand> hw_cmd)
         Guard g(ring_mu_);
         if (reported_ == kQueueStateIdle) {
             reported_ = kQueueStateReady;
+            const auto since_idle = std::chrono::steady_clock::now() - idle_since_;
+            isolated_run_ = since_idle >= std::chrono::microseconds(kIsolatedMicros) ? isolated_run_ + 1 : 0;
             ready_event = std::make_shared<XQueueReadyEvent>(kHandle, std::chrono::system_clock::now());
             if (event_first) {
                 SchedAgent::SendEvent(ready_event);
@@ -138,6 +143,8 @@ void RingXQueue::Submit(std::shared_ptr<HwCommand> hw_cmd)
                 // the launcher reports no Idle while this Ready is still to be sent.
                 ready_unsent_ = true;
             }
+        } else if (retired_.load(std::memory_order_acquire) >= idx - 1) {
+            isolated_run_ = 0;   // everything before it had finished: it came between a command's end and the Idle event
         }
         const bool launcher_owed_nothing = owed_ == Owed::kNothing;
         owed_ = Owed::kBatchThenDrain;
@@ -209,6 +216,7 @@ RingXQueue::Step RingXQueue::NextStep(Pending *out)
             // The stand-by is counted from the callers' latest launch: while they keep
             // launching, the queue is busy and theirs.
             auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(kStandByMicros);
+            const auto poll_until = until;   // later launches do not prolong the looking without a pause
             int64_t seen = handed_over_.load(std::memory_order_acquire);
             parked_ = true;
             while (ring_count_ == 0 && retired_.load(std::memory_order_acquire) < handed_over_.load(std::memory_order_acquire)) {
@@ -216,11 +224,17 @@ RingXQueue::Step RingXQueue::NextStep(Pending *out)
                 const int64_t newest = handed_over_.load(std::memory_order_acquire);
                 if (newest != seen) { seen = newest; until = now + std::chrono::microseconds(kStandByMicros); }
                 if (now >= until) break;
-                if (g_interrupted_queues.load(std::memory_order_relaxed) > 0 && !suspended_.load(std::memory_order_relaxed)) {
+                if (isolated_run_ >= kIsolatedRun && now < poll_until && !suspended_.load(std::memory_order_relaxed) &&
+                    g_interrupted_queues.load(std::memory_order_relaxed) > 0) {
                     // Another queue was stopped in its work, most likely for this one: from the end of this
                     // queue's last command to its Idle event the device has nothing to do.
                     // Looking every 25 us left it idle for 20 us per preemption; here the
                     // launcher keeps looking (at its own counters, not at the runtime).
+                    // Only for a queue whose last busy periods lay apart: the commands of a caller that
+                    // waits for each and sends the next are bridged by the slices below. An
+                    // Idle event between two of them resumes the other queue, which the next
+                    // Ready event flushes again: 20 commands of 30 us in a row, each waited for,
+                    // cost it 21-28 replays instead of 2, and the caller half as much time again.
                     g.unlock();
                     const auto pause_end = now + std::chrono::microseconds(kStandByPollMicros);
                     while (retired_.load(std::memory_order_acquire) < handed_over_.load(std::memory_order_acquire) &&
@@ -246,6 +260,7 @@ RingXQueue::Step RingXQueue::NextStep(Pending *out)
                 idle_held_back_ = true;
             } else {
                 reported_ = kQueueStateIdle;
+                idle_since_ = std::chrono::steady_clock::now();
                 idle_round_++;
                 idle_cv_.notify_all();
                 SchedAgent::SendEvent(std::make_shared<XQueueIdleEvent>(kHandle));

@@ -28,6 +28,7 @@
 #pragma once
 
 #include <atomic>
+#include <chrono>
 #include <condition_variable>
 #include <memory>
 #include <mutex>
@@ -99,6 +100,8 @@ private:
     bool ready_unsent_ = false;         // reported_ turned Ready, the event is still with the submitter
     bool idle_held_back_ = false;       // the launcher found the queue idle meanwhile and waits for that event to be out
     uint64_t idle_round_ = 0;
+    std::chrono::steady_clock::time_point idle_since_ {};   // when reported_ last turned Idle
+    int64_t isolated_run_;              // busy periods in a row that did not follow closely on the one before
 
     // ---- in-flight window (win_mu_) ---------------------------------------------------
     struct Flight
