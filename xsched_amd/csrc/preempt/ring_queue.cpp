@@ -2,6 +2,7 @@
 // preempt/src/xqueue/{async_xqueue,command_buffer,launch_worker}.cpp (citations below name
 // the rule each block keeps).
 #include <chrono>
+#include <map>
 #include <typeinfo>
 
 #include <sys/prctl.h>
@@ -28,12 +29,18 @@ constexpr int64_t kIsolatedMicros = 40;      // a busy period that begins this l
 constexpr int64_t kIsolatedRun = 4;          // so many of them in a row, and the next command is not waited for with the Idle event
 constexpr unsigned long kLauncherTimerSlackNanos = 1000; // timed waits of the launcher end on time (the default slack is 50 us)
 
-/// XQueues of this process that were suspended with commands unfinished. What a running queue's
-/// Idle event is most likely to bring is the resume of one of them, and until then the device may
-/// stand idle. (Queues suspended with nothing to do don't count: an early Idle event would only
-/// resume them between two commands of the running queue, and its next Ready event suspend them
-/// again, 6 us per command.)
-std::atomic<int> g_interrupted_queues { 0 };
+/// How many XQueues of this process on `device` are paused with commands unfinished. What a
+/// running queue's Idle event is most likely to bring is the resume of one of them, and until then
+/// the device may stand idle. (Queues paused with nothing to do don't count: an early Idle event
+/// would only resume them between two commands of the running queue, and its next Ready event
+/// suspend them again, 6 us per command.) The counters live as long as the process.
+std::atomic<int> *InterruptedQueuesOf(XDevice device)
+{
+    static std::mutex mu;
+    static auto *counters = new std::map<XDevice, std::atomic<int>>();
+    std::lock_guard<std::mutex> g(mu);
+    return &(*counters)[device];
+}
 
 size_t PowerOfTwoAtLeast(size_t n)
 {
@@ -50,6 +57,7 @@ RingXQueue::RingXQueue(std::shared_ptr<HwQueue> hwq, XPreemptLevel level, int64_
              (hwq->SupportDynamicLevel() ? kQueueFeatureDynamicLevel : 0),
              hwq)
     , ring_(kInitialRingSlots), isolated_run_(kIsolatedRun), threshold_(threshold), batch_(batch), level_(level)
+    , interrupted_queues_(InterruptedQueuesOf(kDevice))
 {
     XASSERT(level_ > kPreemptLevelUnknown && level_ < kPreemptLevelMax, "invalid preempt level: %d", level_);
     // With fewer window slots than the marker period the window could fill up without a
@@ -225,7 +233,7 @@ RingXQueue::Step RingXQueue::NextStep(Pending *out)
                 if (newest != seen) { seen = newest; until = now + std::chrono::microseconds(kStandByMicros); }
                 if (now >= until) break;
                 if (isolated_run_ >= kIsolatedRun && now < poll_until && !suspended_.load(std::memory_order_relaxed) &&
-                    g_interrupted_queues.load(std::memory_order_relaxed) > 0) {
+                    interrupted_queues_->load(std::memory_order_relaxed) > 0) {
                     // Another queue was stopped in its work, most likely for this one: from the end of this
                     // queue's last command to its Idle event the device has nothing to do.
                     // Looking every 25 us left it idle for 20 us per preemption; here the
@@ -650,8 +658,6 @@ void RingXQueue::Suspend(int64_t flags)
     {
         Guard op(op_mu_);
         if (suspended_.exchange(true)) return;
-        interrupted_ = retired_.load(std::memory_order_acquire) < next_idx_.load(std::memory_order_acquire) - 1;
-        if (interrupted_) g_interrupted_queues.fetch_add(1, std::memory_order_relaxed);
         suspension = ++suspensions_;
         if (!waits) PauseAndFlush();
     }
@@ -667,6 +673,8 @@ void RingXQueue::Suspend(int64_t flags)
 
 void RingXQueue::PauseAndFlush()
 {
+    interrupted_ = retired_.load(std::memory_order_acquire) < next_idx_.load(std::memory_order_acquire) - 1;
+    if (interrupted_) interrupted_queues_->fetch_add(1, std::memory_order_relaxed);
     bool in_flight;
     {
         Guard g(win_mu_);
@@ -690,7 +698,8 @@ void RingXQueue::Resume(int64_t flags)
     if (!suspended_.load()) return;   // the usual case of a round: nothing to undo
     Guard op(op_mu_);
     if (!suspended_.exchange(false)) return;
-    if (interrupted_) g_interrupted_queues.fetch_sub(1, std::memory_order_relaxed);
+    if (interrupted_) interrupted_queues_->fetch_sub(1, std::memory_order_relaxed);
+    interrupted_ = false;   // (a suspension that is still waiting has paused nothing)
     const bool drop = (flags & kQueueResumeFlagDropCommands) != 0;
 
     if (level_ > kPreemptLevelBlock) {

@@ -154,7 +154,8 @@ private:
     bool caller_may_launch_ = false;
     std::mutex op_mu_;                  // one Suspend() or Resume() at a time; taken before the locks above
     int64_t suspensions_ = 0;           // op_mu_: number of the newest suspension
-    bool interrupted_ = false;          // op_mu_: it found commands that were not finished
+    bool interrupted_ = false;          // op_mu_: the queue is paused with commands unfinished
+    std::atomic<int> *const interrupted_queues_;   // how many queues of its device are
     std::atomic_bool suspended_ { false };   // changed under op_mu_
     std::atomic_bool closing_ { false };
     std::thread launcher_;
