@@ -94,6 +94,12 @@ XResult HipAxpyCommandCreate(HwCommandHandle *cmd, float alpha, const void *x, v
 XResult HipGemmBf16CommandCreate(HwCommandHandle *cmd, const void *A, const void *B, void *C,
                                  int M, int N, int K, int guard);
 
+/* For tests: how a GEMM of these matrices would be launched; nothing is launched or read. `out` receives
+ * 8 values, four for each of at most two launches (zeroes where there is no second one):
+ * rows of C, edge of a tile, kernel (0 two LDS buffers, 1 four stages, 2 any shape) and what it
+ * assumes of the matrices (0 whole tiles, 1 16-byte rows, 2 nothing). No counterpart in the reference. */
+XResult HipGemmBf16PlanOf(const void *A, const void *B, const void *C, int M, int N, int K, int32_t *out);
+
 /* bins[keys[i]] += 1 for i < n; keys are int32 in [0, n_bins), bins are uint32 and
  * are NOT cleared by the command. n_bins <= 65536. */
 XResult HipHistogramCommandCreate(HwCommandHandle *cmd, const void *keys, size_t n, void *bins,

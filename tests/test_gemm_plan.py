@@ -1,0 +1,60 @@
+"""Which kernel a GEMM runs on, and what the rule promises to it, on the CPU: the plan is made on
+the host and reads no matrix."""
+import random
+from ctypes import byref, c_int32, c_uint64
+
+import pytest
+
+TWO_BUFFERS, FOUR_STAGES, ANY_SHAPE = 0, 1, 2
+EXACT, EDGES, UNALIGNED = 0, 1, 2
+ADDRESS = 1 << 20
+
+
+def plan_of(xs, M, N, K, offset=0):
+    out = (c_int32 * 8)()
+    xs.check(xs.halhip().HipGemmBf16PlanOf(ADDRESS + offset, ADDRESS, ADDRESS, M, N, K, out))
+    return [tuple(out[i:i + 4]) for i in (0, 4) if out[i] != 0]
+
+
+@pytest.mark.parametrize("tile", [0, 64, 128, 256])
+def test_a_plan_covers_the_rows_and_assumes_only_what_holds(xs, monkeypatch, tile):
+    if tile != 0:
+        monkeypatch.setenv("XSCHED_HIP_GEMM_TILE", str(tile))
+    rng = random.Random(tile)
+    for _ in range(4000):
+        M, N, K = (int(2 ** rng.uniform(0, 14)) for _ in range(3))
+        unit = rng.choice([1, 8, 64, 128, 256])
+        M, N, K = (max(v // u * u, u) for v, u in ((M, rng.choice([1, unit])), (N, unit), (K, unit)))
+        offset = rng.choice([0, 0, 0, 2, 8])
+        plan = plan_of(xs, M, N, K, offset)
+        aligned = offset == 0 and N % 8 == 0 and K % 8 == 0
+        case = (M, N, K, offset, plan)
+        assert sum(rows for rows, *_ in plan) == M, case
+        tiles = 0
+        for rows, edge, kernel, fit in plan:
+            tiles += -(-rows // edge) * -(-N // edge)
+            if kernel == ANY_SHAPE:
+                assert edge == 64 and len(plan) == 1 and (N < 8 or M * K < 8), case
+                continue
+            assert N >= 8 and M * K >= 8, case
+            assert fit == UNALIGNED or aligned, case
+            assert (fit == EXACT) == (aligned and rows % edge == 0 and N % edge == 0 and K % 64 == 0), case
+            assert kernel == FOUR_STAGES if fit == UNALIGNED else True, case
+            assert (kernel, edge) in ((TWO_BUFFERS, 256), (TWO_BUFFERS, 128), (FOUR_STAGES, 128), (FOUR_STAGES, 64)), case
+            assert (kernel, edge) != (TWO_BUFFERS, 128) or fit == EXACT, case
+        cmd = c_uint64()
+        taken = xs.halhip().HipGemmBf16CommandCreate(byref(cmd), ADDRESS + offset, ADDRESS, ADDRESS, M, N, K, 1)
+        if taken == xs.kXSchedSuccess:
+            assert tiles <= 1 << 18, case
+            xs.check(xs.preempt().HwCommandDestroy(cmd.value))
+
+
+@pytest.mark.parametrize("M,N,K,want", [
+    # 257 to 512 tiles of 128 x 128 are two rounds for the kernel with four stages
+    (1920, 2944, 704, (128, TWO_BUFFERS)), (2560, 2560, 704, (128, TWO_BUFFERS)), (2048, 2944, 2048, (128, TWO_BUFFERS)),
+    # short K: a tile is little more than its first loads and its write-out
+    (2048, 2944, 128, (128, TWO_BUFFERS)), (3968, 4224, 64, (128, TWO_BUFFERS)), (2944, 1792, 192, (128, TWO_BUFFERS)),
+    (2048, 2048, 2048, (128, FOUR_STAGES)), (1024, 1024, 1024, (64, FOUR_STAGES)), (8192, 8192, 8192, (256, TWO_BUFFERS)),
+    (4096, 4096, 4096, (256, TWO_BUFFERS))])
+def test_the_kernel_that_measured_quickest_is_taken(xs, M, N, K, want):
+    assert [(edge, kernel) for _, edge, kernel, _ in plan_of(xs, M, N, K)] == [want]

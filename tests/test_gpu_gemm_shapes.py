@@ -1,17 +1,25 @@
 """GPU parity of the GEMM's tile kernels at the sizes where they change their ways: the number
 of K steps around the length of their pipelines and of their polls of the preempt word, the last
 step full and not, edges of tiles, and rows that start on 16-byte boundaries or do not."""
-from ctypes import byref, c_uint64
+from ctypes import byref, c_int32, c_uint64
 
 import numpy as np
 import pytest
 
 import oracle
-from test_gpu_kernels import Queue
+from test_gpu_kernels import Queue, gemm_cmd
 
 pytestmark = pytest.mark.gpu
 
 NAN = 0x7FC0
+TWO_BUFFERS, FOUR_STAGES, ANY_SHAPE = 0, 1, 2      # kernels of a plan
+
+
+def plan_of(xs, a, b, c, M, N, K):
+    """[(rows, tile, kernel, fit)] of the one or two launches of a GEMM."""
+    out = (c_int32 * 8)()
+    xs.check(xs.halhip().HipGemmBf16PlanOf(a.data_ptr(), b.data_ptr(), c.data_ptr(), M, N, K, out))
+    return [tuple(out[i:i + 4]) for i in (0, 4) if out[i] != 0]
 
 
 def _shape(fit, tile, steps):
@@ -83,3 +91,32 @@ def test_gemm_in_two_launches(xs, gpu, M, N, K, flush):
     for c in cs:
         assert torch.equal(c[:M], want)
         assert bool((c[M:] == 0.5).all()), "wrote behind the last row"
+
+
+# 257 to 512 tiles of 128 x 128, and short K: K of one step, two, and around the polls of the preempt word
+@pytest.mark.parametrize("M,N,K", [(2048, 2944, 64), (2048, 2944, 128), (1920, 2944, 192), (3968, 4224, 64), (1920, 2944, 320),
+                                   (1920, 2944, 384), (2560, 2560, 704)])
+@pytest.mark.parametrize("level,guard", [(1, 0), (2, 1)])
+def test_gemm_two_work_groups_to_a_compute_unit(xs, gpu, monkeypatch, M, N, K, level, guard):
+    """The kernel with two LDS buffers on 128 x 128 tiles. Its sums run in the order of the kernel
+    with four stages on the same tiles: the same bits for normally distributed inputs."""
+    torch = gpu
+    print(f"case gemm-two-per-unit M={M} N={N} K={K} level={level} guard={guard}", flush=True)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(M + K)
+    a, b = (torch.randn(s, device="cuda", generator=gen).to(torch.bfloat16) for s in ((M, K), (K, N)))
+    c = torch.full((M + 2, N), 0.5, dtype=torch.bfloat16, device="cuda")
+    want = torch.zeros(M, N, dtype=torch.bfloat16, device="cuda")
+    torch.cuda.synchronize()
+    assert plan_of(xs, a, b, c, M, N, K) == [(M, 128, TWO_BUFFERS, 0)]
+    q = Queue(xs, torch, level)
+    q.submit(gemm_cmd(xs, a, b, c, M, N, K, guard))
+    monkeypatch.setenv("XSCHED_HIP_GEMM_TILE", "128")
+    assert plan_of(xs, a, b, want, M, N, K) == [(M, 128, FOUR_STAGES, 0)]
+    q.submit(gemm_cmd(xs, a, b, want, M, N, K, guard))
+    q.wait()
+    q.close()
+    # 2^-8 for the result's rounding to bf16, the rest for sums in another order
+    torch.testing.assert_close(c[:M].float(), a.float() @ b.float(), rtol=2 ** -7, atol=2 ** -8 * K ** 0.5)
+    assert torch.equal(c[:M], want)
+    assert bool((c[M:] == 0.5).all()), "wrote behind the last row"

@@ -164,7 +164,13 @@ enum TileRequest { kNoTile, kAnyButLast, kTheLast };
 // kBlocksM x kBlocksN blocks of 32x32. Built for 256 with 2x4 waves (4x2 blocks
 // per wave), for exact shapes and for ragged ones (kEdges): there the last tile's loads, the last
 // step and the stores look at the edges, and the steps before are the same code (4000^3 146 us on
-// 128 x 128 tiles, 114 on these).
+// 128 x 128 tiles, 114 on these). And for 128 with 2x2 waves (2x2 blocks), exact shapes only: 64 KiB
+// of LDS and 4 waves, so two work-groups share a compute unit and one computes while the other
+// waits for its first loads or writes out. That is what outputs of 257 to 512 such tiles want,
+// which are two rounds for the four-stage kernel below (its 130 KiB let a unit have one group), and
+// what short K wants, where a tile is little more than its first loads and its write-out
+// (per command: 368 tiles at K = 192 10.1 -> 7.3 us, at 2048 33.5 -> 28.9; 276 at 4096 55.1 -> 50.1;
+// 1023 at 128 16.5 -> 10.7).
 //
 // (The body is a device function: the host pass cannot parse the buffer-resource builtins
 // and would silently drop the launch stub of a kernel that uses them directly.)
@@ -1020,14 +1026,17 @@ void GemmBf16AnyShapeKernel(const uint16_t *__restrict__ A, const uint16_t *__re
     if (kGuard) guard.Commit();
 }
 
+/// kTwoBuffers is GemmBf16Kernel, kFourStages GemmDeepKernel, kAnyShape GemmBf16AnyShapeKernel.
+enum class Body { kTwoBuffers, kFourStages, kAnyShape };
+
 /// A run of rows of C and how they are computed: which kernel, on tiles of which size, and what it
 /// may assume about the matrices.
 struct Part
 {
     int first_row, rows;
     int tile;       // edge of a tile of C
-    Fit fit;        // of the kernels with 256, 128 and 64 tiles
-    bool narrow;    // the kernel without requirements
+    Fit fit;        // of kTwoBuffers and kFourStages
+    Body body;
     uint64_t tiles; // work-groups = bytes of the progress map
 };
 
@@ -1062,7 +1071,7 @@ protected:
 private:
     hipError_t LaunchPart(const Part &part, hipEvent_t stop, hipStream_t stream, bool guarded, const XGuardArgs &g)
     {
-        if (part.narrow) {
+        if (part.body == Body::kAnyShape) {
             const uint32_t tiles_n = (uint32_t)((N_ + kAnyTile - 1) / kAnyTile);
             const dim3 grid((uint32_t)part.tiles), block(256);
             LaunchWithStop(stop, guarded ? GemmBf16AnyShapeKernel<true> : GemmBf16AnyShapeKernel<false>, grid, block, stream,
@@ -1071,9 +1080,9 @@ private:
         }
         Kernel kernel = nullptr;
         switch (part.fit) {
-        case Fit::kExact:     kernel = KernelFor<Fit::kExact>(part.tile, guarded); break;
-        case Fit::kEdges:     kernel = KernelFor<Fit::kEdges>(part.tile, guarded); break;
-        case Fit::kUnaligned: kernel = KernelFor<Fit::kUnaligned>(part.tile, guarded); break;   // (never large)
+        case Fit::kExact:     kernel = KernelFor<Fit::kExact>(part, guarded); break;
+        case Fit::kEdges:     kernel = KernelFor<Fit::kEdges>(part, guarded); break;
+        case Fit::kUnaligned: kernel = KernelFor<Fit::kUnaligned>(part, guarded); break;   // (never large)
         }
         LaunchWithStop(stop, kernel, dim3((uint32_t)part.tiles), dim3(part.tile == kLargeTile ? 512 : 256), stream,
                        A_ + (size_t)part.first_row * K_, B_, C_ + (size_t)part.first_row * N_, part.rows, N_, K_, g);
@@ -1082,12 +1091,15 @@ private:
 
     using Kernel = void (*)(const uint16_t *, const uint16_t *, uint16_t *, int, int, int, XGuardArgs);
     template <Fit kFit>
-    static Kernel KernelFor(int tile, bool guarded)
+    static Kernel KernelFor(const Part &part, bool guarded)
     {
-        if constexpr (kFit != Fit::kUnaligned) {
-            if (tile == kLargeTile) return guarded ? GemmBf16Kernel<true, kFit, kLargeTile, 2, 4> : GemmBf16Kernel<false, kFit, kLargeTile, 2, 4>;
+        if constexpr (kFit == Fit::kExact) {
+            if (part.body == Body::kTwoBuffers && part.tile == kSmallTile) return guarded ? GemmBf16Kernel<true, kFit, kSmallTile, 2, 2> : GemmBf16Kernel<false, kFit, kSmallTile, 2, 2>;
         }
-        if (tile == kSmallTile) return guarded ? GemmDeepKernel<true, kFit, kSmallTile, 4> : GemmDeepKernel<false, kFit, kSmallTile, 4>;
+        if constexpr (kFit != Fit::kUnaligned) {
+            if (part.tile == kLargeTile) return guarded ? GemmBf16Kernel<true, kFit, kLargeTile, 2, 4> : GemmBf16Kernel<false, kFit, kLargeTile, 2, 4>;
+        }
+        if (part.tile == kSmallTile) return guarded ? GemmDeepKernel<true, kFit, kSmallTile, 4> : GemmDeepKernel<false, kFit, kSmallTile, 4>;
         return guarded ? GemmDeepKernel<true, kFit, kTinyTile, 4> : GemmDeepKernel<false, kFit, kTinyTile, 4>;
     }
 
@@ -1128,20 +1140,26 @@ inline int ForcedTile()
 inline Part PartOf(int first_row, int rows, int N, int K, bool aligned, int tile)
 {
     const bool exact = aligned && rows % tile == 0 && N % tile == 0 && K % kStepK == 0;
-    return Part { first_row, rows, tile, exact ? Fit::kExact : aligned ? Fit::kEdges : Fit::kUnaligned, false, TilesOf(rows, N, tile) };
+    return Part { first_row, rows, tile, exact ? Fit::kExact : aligned ? Fit::kEdges : Fit::kUnaligned,
+                  tile == kLargeTile ? Body::kTwoBuffers : Body::kFourStages, TilesOf(rows, N, tile) };
 }
 
-/// Roughly how long a part takes, in us: a launch, then rounds of one tile per compute unit, each
-/// with its first loads and its write-out, the last round quicker the fewer units it keeps busy.
+/// Roughly how long a part takes, in us: a launch, then rounds of one tile per compute unit (two of
+/// 128 x 128 with two buffers), each with its first loads and its write-out, the last round quicker the fewer
+/// units it keeps busy. The rates are fitted to 23 outputs of 64 to 1600 tiles of 128 x 128 at eleven K from
+/// 64 to 8192: what it picks there takes 0.9 % longer on average than the quickest, 23 % at worst
+/// (1024 x 2048 x 8192 on tiny tiles), and at most 7 % longer than the quicker of the two kernels with two buffers.
 inline double MicrosOf(const Part &part, int K)
 {
     // us of a round, and per K step of a full round and of one with a single tile: [exact, edges, unaligned]
     struct Rates { double round, full, single; };
-    constexpr Rates large[3] = { { 2.5, 1.54, 0.95 }, { 2.5, 1.56, 0.97 }, {} };
+    constexpr Rates large[3] = { { 4.0, 1.54, 0.95 }, { 4.0, 1.56, 0.97 }, {} };
+    constexpr Rates pair = { 1.5, 0.95, 0.45 };
     constexpr Rates small[3] = { { 2.5, 0.45, 0.37 }, { 2.5, 0.53, 0.41 }, { 2.5, 0.80, 0.60 } };
     constexpr Rates tiny[3] = { { 0.5, 0.195, 0.14 }, { 0.5, 0.25, 0.16 }, { 0.5, 0.35, 0.25 } };
-    const Rates &r = (part.tile == kLargeTile ? large : part.tile == kSmallTile ? small : tiny)[(int)part.fit];
-    const double rounds = (double)part.tiles / ComputeUnits(), whole = std::floor(rounds);
+    const bool two_per_unit = part.tile == kSmallTile && part.body == Body::kTwoBuffers;
+    const Rates &r = two_per_unit ? pair : (part.tile == kLargeTile ? large : part.tile == kSmallTile ? small : tiny)[(int)part.fit];
+    const double rounds = (double)part.tiles / ((two_per_unit ? 2 : 1) * ComputeUnits()), whole = std::floor(rounds);
     const double step = whole * r.full + (rounds > whole ? r.single + (r.full - r.single) * (rounds - whole) : 0.0);
     return 3.0 + std::ceil(rounds) * r.round + step * ((K + kStepK - 1) / kStepK);
 }
@@ -1156,18 +1174,23 @@ inline double MicrosOf(const Part &part, int K)
 /// 126 on small ones, 2048^3 20.9 on small against 30.1 on tiny ones, 1024^3 5.8 on tiny ones against
 /// 9.4 on small ones). Rows without 16-byte alignment do not go straight into LDS, which the large
 /// tiles need (a tile on its way through registers beside their accumulators does not fit).
-/// XSCHED_HIP_GEMM_TILE=64|128|256 overrides the tile where the shape allows.
+/// XSCHED_HIP_GEMM_TILE=64|128|256 overrides the tile where the shape allows (128: four stages).
 /// A plan of more tiles than the progress map holds is passed over for one that fits: 13413745 x
 /// 1280 x 1024, 262025 tiles by the count below, would be quickest as two launches of 262295.
 inline Plan PlanFor(const void *A, const void *B, const void *C, int M, int N, int K, int forced)
 {
     if (N < 8 || (int64_t)M * K < 8 || K > kMaxK || N > kMaxK) {
-        return Plan { { Part { 0, M, kAnyTile, Fit::kUnaligned, true, TilesOf(M, N, kAnyTile) }, {} }, 1 };
+        return Plan { { Part { 0, M, kAnyTile, Fit::kUnaligned, Body::kAnyShape, TilesOf(M, N, kAnyTile) }, {} }, 1 };
     }
     const bool aligned = Aligned(A, B, C, N, K);
     if (forced != 0 && (forced != kLargeTile || aligned)) return Plan { { PartOf(0, M, N, K, aligned, forced), {} }, 1 };
     auto best_part = [&](int first_row, int rows) {
         Part best = PartOf(first_row, rows, N, K, aligned, kSmallTile);
+        if (best.fit == Fit::kExact) {
+            Part two_per_unit = best;
+            two_per_unit.body = Body::kTwoBuffers;
+            if (MicrosOf(two_per_unit, K) < MicrosOf(best, K)) best = two_per_unit;
+        }
         for (const int tile : { kTinyTile, kLargeTile }) {
             if (tile == kLargeTile && !aligned) continue;
             const Part other = PartOf(first_row, rows, N, K, aligned, tile);
@@ -1210,6 +1233,21 @@ inline uint64_t CountedTiles(const void *A, const void *B, const void *C, int M,
 } // namespace xsched::hip
 
 using namespace xsched::hip;
+
+EXPORT_C_FUNC XResult HipGemmBf16PlanOf(const void *A, const void *B, const void *C, int M, int N, int K, int32_t *out)
+{
+    if (out == nullptr || M <= 0 || N <= 0 || K <= 0) return kXSchedErrorInvalidValue;
+    const gemm::Plan plan = gemm::PlanFor(A, B, C, M, N, K, gemm::ForcedTile());
+    for (int i = 0; i < 8; ++i) out[i] = 0;
+    for (int i = 0; i < plan.parts; ++i) {
+        const gemm::Part &part = plan.part[i];
+        out[4 * i + 0] = part.rows;
+        out[4 * i + 1] = part.tile;
+        out[4 * i + 2] = (int32_t)part.body;
+        out[4 * i + 3] = (int32_t)part.fit;
+    }
+    return kXSchedSuccess;
+}
 
 EXPORT_C_FUNC XResult HipGemmBf16CommandCreate(HwCommandHandle *cmd, const void *A, const void *B,
                                                void *C, int M, int N, int K, int guard)
