@@ -34,9 +34,10 @@ def test_a_plan_covers_the_rows_and_assumes_only_what_holds(xs, monkeypatch, til
         for rows, edge, kernel, fit in plan:
             tiles += -(-rows // edge) * -(-N // edge)
             if kernel == ANY_SHAPE:
-                assert edge == 64 and len(plan) == 1 and (N < 8 or M * K < 8), case
+                assert edge == 64 and len(plan) == 1, case
+                assert N < 8 or M * K < 8 or (tile == 0 and K <= 128), case
                 continue
-            assert N >= 8 and M * K >= 8, case
+            assert N >= 8 and M * K >= 8 and (tile != 0 or K > 32), case
             assert fit == UNALIGNED or aligned, case
             assert (fit == EXACT) == (aligned and rows % edge == 0 and N % edge == 0 and K % 64 == 0), case
             assert kernel == FOUR_STAGES if fit == UNALIGNED else True, case
@@ -55,6 +56,12 @@ def test_a_plan_covers_the_rows_and_assumes_only_what_holds(xs, monkeypatch, til
     # short K: a tile is little more than its first loads and its write-out
     (2048, 2944, 128, (128, TWO_BUFFERS)), (3968, 4224, 64, (128, TWO_BUFFERS)), (2944, 1792, 192, (128, TWO_BUFFERS)),
     (2048, 2048, 2048, (128, FOUR_STAGES)), (1024, 1024, 1024, (64, FOUR_STAGES)), (8192, 8192, 8192, (256, TWO_BUFFERS)),
-    (4096, 4096, 4096, (256, TWO_BUFFERS))])
+    (4096, 4096, 4096, (256, TWO_BUFFERS)),
+    # short K of ragged shapes, and where it ends
+    (2000, 1999, 32, (64, ANY_SHAPE)), (4000, 4008, 32, (64, ANY_SHAPE)), (4000, 4008, 40, (256, TWO_BUFFERS)),
+    (7000, 7000, 64, (64, ANY_SHAPE)), (7040, 7040, 64, (128, TWO_BUFFERS)), (7001, 7003, 128, (64, ANY_SHAPE)),
+    (7001, 7003, 136, (128, FOUR_STAGES)), (4001, 4003, 48, (64, ANY_SHAPE)), (4001, 4003, 49, (128, FOUR_STAGES)),
+    (300, 301, 33, (64, FOUR_STAGES)), (8191, 515, 96, (64, ANY_SHAPE)), (2000, 1999, 64, (64, ANY_SHAPE)),
+    (1000, 1001, 64, (64, FOUR_STAGES))])
 def test_the_kernel_that_measured_quickest_is_taken(xs, M, N, K, want):
     assert [(edge, kernel) for _, edge, kernel, _ in plan_of(xs, M, N, K)] == [want]

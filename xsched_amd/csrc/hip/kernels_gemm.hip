@@ -944,13 +944,18 @@ void GemmDeepKernel(const uint16_t *__restrict__ A, const uint16_t *__restrict__
 }
 
 
-// What the kernels above do not take: fewer than eight columns or fewer than eight elements of A
+// Short K (ShortK() below), and what the kernels above do not take: fewer than eight columns or
+// fewer than eight elements of A
 // (less than one 16-byte piece to fetch), K or N above kMaxK (their 32-bit offsets). Any M, N, K >= 1,
 // any alignment of the three matrices to two bytes. 64 x 64 tiles of C, four waves of one 32x32
 // block each, K in steps of 32 (two slices of 16 through the same MFMA as above and in the same
 // order; what lies beyond K is zero). Every load and store is checked against the matrix; a
 // thread's eight neighbouring elements come as one 16-byte load where they lie inside the matrix
 // and are aligned, one by one otherwise. The guard is at entry only: a tile is short.
+// 10 KiB of LDS and few registers: many work-groups share a compute unit, and with short K, where
+// a product is mostly the writing of C, one computes while the others write (us per command, the
+// kernels above and this one: 7001 x 7003 x 32 89.3 -> 32.0, 2000 x 1999 x 16 9.4 -> 6.7,
+// 4000 x 4008 x 32 13.7 -> 11.9, 300 x 301 x 8 5.2 -> 4.6).
 constexpr int kAnyTile = 64;
 constexpr int kAnyK = 32;
 
@@ -1164,6 +1169,30 @@ inline double MicrosOf(const Part &part, int K)
     return 3.0 + std::ceil(rounds) * r.round + step * ((K + kStepK - 1) / kStepK);
 }
 
+/// Whether K is so short that the any-shape kernel is the quickest: up to 32, one step of it, always;
+/// further for outputs of many tiles, whose write-out it overlaps best, and the further the fewer of
+/// its loads come one by one. Measured on either side, any-shape kernel against the quickest of the others, us:
+/// with 16-byte rows in all three matrices, 7000^2 at K = 64 35.9 against 41.6, at 72 47.5 against
+/// 47.6, 4000 x 4008 at 64 14.8 against 13.7; with 16-byte rows in A, 7001 x 7003 at 128 84 against 102, at 160 103 against
+/// 96, 8191 x 515 at 96 12.1 against 13.9, at 128 14.4 against 13.9, 2000 x 1999 at 64 9.0 against
+/// 9.4, at 72 10.5 against 10.3, 1000 x 1001 at 40 5.5 against 5.3; without, 2000 x 1999 at 31 8.3 against 9.4, at 33
+/// 9.5 against 9.9, at 63 13.3 against 9.5, 4001 x 4003 at 31 18.6 against 31.2, at 63 36.8 against 31.4.
+inline bool ShortK(const void *A, const void *B, const void *C, int M, int N, int K)
+{
+    const uint64_t tiles = TilesOf(M, N, kAnyTile), units = ComputeUnits();
+    if (tiles > GuardState::kMaxWorkGroups) return false;
+    int limit = 32;
+    if (Aligned(A, B, C, N, K)) {
+        const bool whole_tiles = M % kSmallTile == 0 && N % kSmallTile == 0 && K % kStepK == 0;   // two work-groups to a unit do the same for them
+        if (tiles >= 32 * units && !whole_tiles) limit = 64;
+    } else if (((uintptr_t)A & 15) == 0 && K % 8 == 0) {
+        limit = tiles >= 12 * units ? 128 : 2 * tiles >= 9 * units ? 96 : tiles >= 4 * units ? 64 : 32;
+    } else if (tiles > 4 * units) {
+        limit = 48;
+    }
+    return K <= limit;
+}
+
 /// The plan for a shape: the quickest by the estimate above of one launch on large, small or tiny
 /// tiles and of two, large tiles for the rows that fill whole tiles, or whole rounds of them, and
 /// whatever is quickest for the rest. Large tiles do more arithmetic per byte read from LDS, but a
@@ -1179,10 +1208,10 @@ inline double MicrosOf(const Part &part, int K)
 /// 1280 x 1024, 262025 tiles by the count below, would be quickest as two launches of 262295.
 inline Plan PlanFor(const void *A, const void *B, const void *C, int M, int N, int K, int forced)
 {
-    if (N < 8 || (int64_t)M * K < 8 || K > kMaxK || N > kMaxK) {
-        return Plan { { Part { 0, M, kAnyTile, Fit::kUnaligned, Body::kAnyShape, TilesOf(M, N, kAnyTile) }, {} }, 1 };
-    }
+    const Plan any_shape { { Part { 0, M, kAnyTile, Fit::kUnaligned, Body::kAnyShape, TilesOf(M, N, kAnyTile) }, {} }, 1 };
+    if (N < 8 || (int64_t)M * K < 8 || K > kMaxK || N > kMaxK) return any_shape;
     const bool aligned = Aligned(A, B, C, N, K);
+    if (forced == 0 && ShortK(A, B, C, M, N, K)) return any_shape;
     if (forced != 0 && (forced != kLargeTile || aligned)) return Plan { { PartOf(0, M, N, K, aligned, forced), {} }, 1 };
     auto best_part = [&](int first_row, int rows) {
         Part best = PartOf(first_row, rows, N, K, aligned, kSmallTile);
