@@ -377,8 +377,9 @@ def test_gemm_shapes_that_only_small_tiles_fit(xs, gpu, M, N, K, level, guard):
                                    (256, 128, 100), (200, 256, 64), (128, 128, 8), (1, 300, 129), (300, 1, 250)])
 @pytest.mark.parametrize("level,guard", [(1, 0), (2, 1)])
 def test_gemm_any_shape(xs, gpu, M, N, K, level, guard):
-    """Shapes the fast kernels do not take (M or N no multiple of 128, K no multiple of 64) go
-    to the any-shape kernel: integers as above, so the result is determined; the matrices lie
+    """Shapes that are no whole tiles, from one element on, at odd multiples of two bytes: the
+    any-shape kernel up to K of 32 and below eight columns, 64 x 64 tiles through registers otherwise.
+    Integers as above, so the result is determined; the matrices lie
     in larger buffers whose other elements must come back untouched."""
     torch = gpu
     print(f"case gemm-any M={M} N={N} K={K} level={level} guard={guard}", flush=True)
@@ -405,10 +406,9 @@ def test_gemm_any_shape(xs, gpu, M, N, K, level, guard):
 
 @pytest.mark.parametrize("M,N,K", [(129, 128, 64), (200, 256, 64), (1000, 384, 128), (2049, 256, 192), (127, 256, 64)])
 @pytest.mark.parametrize("level,guard", [(1, 0), (2, 1)])
-def test_gemm_ragged_rows_are_split_between_the_kernels(xs, gpu, M, N, K, level, guard):
-    """N and K as the fast kernel wants them, M not (the usual ragged dimension): the rows up to
-    the last multiple of 128 go to the fast kernel, the rest to the any-shape kernel, in one
-    command (M below 128: all of it to the any-shape kernel). Integers, so the result is
+def test_gemm_ragged_rows(xs, gpu, M, N, K, level, guard):
+    """N and K whole tiles, M not (the usual ragged dimension): a tile's last rows are fetched from
+    inside the matrix and not stored. Integers, so the result is
     determined; the rows behind the matrix in C's buffer stay untouched."""
     torch = gpu
     print(f"case gemm-split M={M} N={N} K={K} level={level} guard={guard}", flush=True)
@@ -429,9 +429,10 @@ def test_gemm_ragged_rows_are_split_between_the_kernels(xs, gpu, M, N, K, level,
     assert np.all(got[M:] == 0x1234)
 
 
-def test_gemm_any_shape_kernel_sums_as_the_fast_kernels_do(xs, gpu, monkeypatch):
-    """Seeded normal inputs on a shape every kernel takes: the any-shape kernel (forced)
-    feeds the matrix cores the same slices of 16 along K in the same order, so the bits agree."""
+def test_gemm_tiny_and_small_tiles_give_the_same_bits(xs, gpu, monkeypatch):
+    """Seeded normal inputs on a shape that 64 and 128 tiles take: both
+    feed the matrix cores the same slices of 16 along K in the same order, so the bits agree.
+    (The any-shape kernel: test_gemm_any_shape_kernel_adds_in_the_order_of_the_others.)"""
     M, N, K = 256, 384, 512
     print(f"case gemm-any-vs-fast M={M} N={N} K={K}", flush=True)
     a_bits = oracle.fill_normal_bf16(19, 1, 0, M * K)
