@@ -37,7 +37,7 @@ def test_histogram_ways_by_size_and_bins(xs, gpu, n, offset, n_bins, level, guar
     assert got[n_bins] == 0, "wrote beyond the bins array"
 
 
-@pytest.mark.parametrize("n_bins", [254, 4096, 4097, 65536])
+@pytest.mark.parametrize("n_bins", [254, 255, 256, 257, 4032, 4033, 4096, 4097, 65536])
 @pytest.mark.parametrize("n", [(1 << 16) + 1, (1 << 24) + 5, (1 << 25) + 5])
 def test_histogram_counters_of_the_hot_bins(xs, gpu, n, n_bins):
     """Around the number of bins from which the hot ones have fewer counters, with the hottest bin
@@ -63,3 +63,29 @@ def test_histogram_counters_of_the_hot_bins(xs, gpu, n, n_bins):
     for g in got:
         assert np.array_equal(g[:n_bins], want)
         assert g[n_bins] == 0, "wrote beyond the bins array"
+
+
+def _command_us(xs, torch, keys, n_bins):
+    """Least time of a histogram command of several, in us."""
+    bins = torch.zeros(n_bins, dtype=torch.int32, device="cuda")
+    stream = torch.cuda.current_stream()
+    best = float("inf")
+    for _ in range(7):
+        start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        start.record()
+        for _ in range(4):
+            xs.check(xs.halhip().HipHistogramLaunchNoAlloc(stream.cuda_stream, keys.data_ptr(), keys.numel(), bins.data_ptr(), n_bins))
+        end.record()
+        torch.cuda.synchronize()
+        best = min(best, start.elapsed_time(end) * 250)
+    return best
+
+
+def test_histogram_of_256_bins_counts_the_last_bin_like_the_others(xs, gpu):
+    """Bytes that are all 255 (an image's white) took 5 times as long as bytes that are all 0: one
+    counter for all lanes of a work-group."""
+    torch = gpu
+    print("case hist-256", flush=True)
+    first, last = (_command_us(xs, torch, torch.full((1 << 25,), key, dtype=torch.int32, device="cuda"), 256) for key in (0, 255))
+    print("us", first, last, flush=True)
+    assert last < 2 * first

@@ -16,7 +16,7 @@
 // thirds of all Zipf(1.1) keys, a fifth of them in bins 0 and 1) have sixteen 32-bit counters
 // each, one per lane modulo 16, so that at most four lanes of a wave add to the same address, no
 // vote and no popcount is needed, and they cannot overflow (64, one per lane, where n_bins leaves
-// the room: evenly spread keys over 1000 bins, a quarter of them in these bins, 54.7 us against
+// the room, and then for bin 255 too, which is all that 256 bins have: evenly spread keys over 1000 bins, a quarter of them in these bins, 54.7 us against
 // 56.8 with 16). Half of a compute unit's LDS and of its wave slots: two groups of different
 // queues share it, and one streams keys while the other clears, writes out or waits for its first
 // keys (four queues of 2^26 keys each 217 -> 207 us; with 64 counters for every one of these bins
@@ -100,10 +100,11 @@ constexpr uint32_t kFewWarmBins = 256;                // its bins that are count
 constexpr uint32_t kColdWords = 1u << 14;           // word w counts bins w + i * 16384
 constexpr uint32_t kWarmBins = 255;                 // bins below this have 32-bit counters of their own,
 constexpr uint32_t kCopies = 16;                    // one per lane modulo 16
-constexpr uint32_t kFewColdWords = 1u << 12;        // with at most this many cold words one per lane
+constexpr uint32_t kFewColdWords = 63u * 64;        // with at most this many cold words one per lane,
+constexpr uint32_t kFewColdWarmBins = 256;          // and one bin more
 constexpr uint32_t kOutside = 256;                  // counts a partial keeps outside the cold words (the last is 0)
 constexpr uint32_t kLdsBins = kColdWords + kWarmBins * kCopies;   // the cold words, then the warm counters
-static_assert(kFewColdWords + kWarmBins * 64 <= kLdsBins, "a warm counter per lane beside few cold words");
+static_assert(kFewColdWords + kFewColdWarmBins * 64 <= kLdsBins && kFewColdWarmBins <= kOutside, "a warm counter per lane beside few cold words");
 // The partial histograms of a launch in memory, n_part of them (one per counting group): the
 // cold words column by column, one column per merge group, and within a column partial by
 // partial: column c of partial p is the 64 words (256 bytes, two whole cache lines) at
@@ -216,19 +217,19 @@ __device__ __forceinline__ void ClearBins(Shared &sh, uint32_t first, uint32_t e
     for (uint32_t i = first + threadIdx.x * 4; i < end; i += kThreads * 4) *(u32x4 *)&sh.bins[i] = u32x4 { 0, 0, 0, 0 };
 }
 
-/// Where the warm counters of a launch lie: counter `copy` of bin b is word first + (b << log2) + copy.
-struct WarmPlace { uint32_t first, log2; };
+/// Where the warm counters of a launch lie: counter `copy` of bin b < bins is word first + (b << log2) + copy.
+struct WarmPlace { uint32_t first, log2, bins; };
 __device__ __forceinline__ WarmPlace WarmPlaceOf(uint32_t cold_words)
 {
     static_assert(kCopies == 16, "log2 of it below");
-    return cold_words <= kFewColdWords ? WarmPlace { kFewColdWords, 6 } : WarmPlace { kColdWords, 4 };
+    return cold_words <= kFewColdWords ? WarmPlace { kFewColdWords, 6, kFewColdWarmBins } : WarmPlace { kColdWords, 4, kWarmBins };
 }
 
 /// Where a valid key is counted, and by how much (see the head of this file); `copy` is the
 /// lane's copy of warm bin 0.
-__device__ __forceinline__ void PackedSlot(uint32_t key, uint32_t copy, uint32_t copies_log2, uint32_t width_log2, uint32_t &word, uint32_t &inc)
+__device__ __forceinline__ void PackedSlot(uint32_t key, uint32_t copy, const WarmPlace &warm_at, uint32_t width_log2, uint32_t &word, uint32_t &inc)
 {
-    word = key < kWarmBins ? copy + (key << copies_log2) : key & (kColdWords - 1);
+    word = key < warm_at.bins ? copy + (key << warm_at.log2) : key & (kColdWords - 1);
     inc = 1u << ((key >> 14) << width_log2);
 }
 
@@ -268,7 +269,7 @@ void HistogramKernel(const int32_t *__restrict__ keys, uint64_t n, uint32_t *__r
     const WarmPlace warm_at = WarmPlaceOf(cold_words);
     const uint32_t copy = warm_at.first + (lane & ((1u << warm_at.log2) - 1u));
     ClearBins(sh, 0, cold_words);
-    ClearBins(sh, warm_at.first, warm_at.first + (kWarmBins << warm_at.log2));
+    ClearBins(sh, warm_at.first, warm_at.first + (warm_at.bins << warm_at.log2));
     if (tid == 0) { sh.bailed = 0; sh.invalid = 0; sh.sum = 0; }
 
     const uint64_t begin = (uint64_t)blockIdx.x * chunk;
@@ -330,7 +331,7 @@ void HistogramKernel(const int32_t *__restrict__ keys, uint64_t n, uint32_t *__r
 #pragma unroll
             for (uint32_t j = 0; j < kN; ++j) {
                 uint32_t word, inc;
-                PackedSlot(k[j], copy, warm_at.log2, width_log2, word, inc);
+                PackedSlot(k[j], copy, warm_at, width_log2, word, inc);
                 LdsAdd(&sh.bins[word], inc);
             }
         } else {
@@ -340,7 +341,7 @@ void HistogramKernel(const int32_t *__restrict__ keys, uint64_t n, uint32_t *__r
                     invalid += 1;
                 } else {
                     uint32_t word, inc;
-                    PackedSlot(k[j], copy, warm_at.log2, width_log2, word, inc);
+                    PackedSlot(k[j], copy, warm_at, width_log2, word, inc);
                     LdsAdd(&sh.bins[word], inc);
                 }
             }
@@ -425,7 +426,7 @@ void HistogramKernel(const int32_t *__restrict__ keys, uint64_t n, uint32_t *__r
     uint32_t counted = 0;
     // the copies of warm bin tid / 4: four threads sum a quarter each
     uint32_t warm = 0;
-    if (tid / 4 < kWarmBins) {
+    if (tid / 4 < warm_at.bins) {
         for (uint32_t q = 0; q < 1u << (warm_at.log2 - 4); ++q) {
             const u32x4 w = *(const u32x4 *)&sh.bins[warm_at.first + ((tid * 4) << (warm_at.log2 - 4)) + q * 4];
             warm += w.x + w.y + w.z + w.w;
