@@ -89,3 +89,45 @@ def test_histogram_of_256_bins_counts_the_last_bin_like_the_others(xs, gpu):
     first, last = (_command_us(xs, torch, torch.full((1 << 25,), key, dtype=torch.int32, device="cuda"), 256) for key in (0, 255))
     print("us", first, last, flush=True)
     assert last < 2 * first
+
+
+def test_histogram_of_one_key_outside_the_warm_bins(xs, gpu):
+    """Equal keys outside the first 255 of 65536 bins overflow their counters: counted, and counted again,
+    within 4 times what equal keys of bin 0 take (6.5 times before runs of one key were added together)."""
+    torch = gpu
+    print("case hist-one-key", flush=True)
+    first, cold = (_command_us(xs, torch, torch.full((1 << 24,), key, dtype=torch.int32, device="cuda"), 65536) for key in (0, 300))
+    print("us", first, cold, flush=True)
+    assert cold < 4 * first
+
+
+@pytest.mark.parametrize("n,offset", [(4096, 0), (8192, 1), ((1 << 16) + 1, 0), ((1 << 18) + 4095, 3), ((1 << 22) + 5, 0)])
+@pytest.mark.parametrize("n_bins", [1000, 20000, 40000, 65536])
+@pytest.mark.parametrize("shape", ["constant", "sorted", "descending", "runs", "ends"])
+def test_histogram_of_runs(xs, gpu, n, offset, n_bins, shape):
+    """Runs of one key of every kind, with keys outside the bins among them: bit for bit the oracle's."""
+    torch = gpu
+    print(f"case hist-runs n={n} offset={offset} bins={n_bins} {shape}", flush=True)
+    rng = np.random.default_rng(n + n_bins)
+    if shape == "constant":
+        keys_h = np.full(n, n_bins - 300, np.int32)
+    elif shape == "sorted":
+        keys_h = np.sort(rng.integers(-3, n_bins + 3, n)).astype(np.int32)
+    elif shape == "descending":
+        keys_h = np.sort(rng.integers(0, n_bins, n))[::-1].astype(np.int32)
+    elif shape == "runs":
+        keys_h = np.repeat(rng.integers(-1, n_bins + 1, n // 7 + 1), rng.integers(1, 600, n // 7 + 1))[:n].astype(np.int32)
+        keys_h = np.resize(keys_h, n)
+    else:   # two keys far apart: the quarters of the bins between them are empty
+        keys_h = np.where(np.arange(n) // 512 % 2 == 0, 300, n_bins - 1).astype(np.int32)
+    keys = torch.from_numpy(np.concatenate([np.zeros(offset, np.int32), keys_h])).cuda()[offset:]
+    bins = torch.zeros(n_bins + 1, dtype=torch.int32, device="cuda")
+    q = Queue(xs, torch, 2)
+    for _ in range(2):
+        q.submit(hist_cmd(xs, keys, n, bins, n_bins, 1))
+    q.wait()
+    got = bins.cpu().numpy().view(np.uint32)
+    q.close()
+    want = oracle.histogram(np.ascontiguousarray(keys_h[(keys_h >= 0) & (keys_h < n_bins)]), n_bins)
+    assert np.array_equal(got[:n_bins], 2 * want)
+    assert got[n_bins] == 0, "wrote beyond the bins array"
