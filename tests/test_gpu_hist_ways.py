@@ -1,10 +1,13 @@
 """GPU parity of the histogram where it changes its ways by itself: few keys, one kernel or two,
 whole-word, half-word and byte counters, and key arrays at any multiple of four bytes."""
+import threading
+
 import numpy as np
 import pytest
 
 import oracle
 from test_gpu_kernels import Queue, hist_cmd
+from test_gpu_preempt import churn, hip_stats
 
 pytestmark = pytest.mark.gpu
 
@@ -131,3 +134,65 @@ def test_histogram_of_runs(xs, gpu, n, offset, n_bins, shape):
     want = oracle.histogram(np.ascontiguousarray(keys_h[(keys_h >= 0) & (keys_h < n_bins)]), n_bins)
     assert np.array_equal(got[:n_bins], 2 * want)
     assert got[n_bins] == 0, "wrote beyond the bins array"
+
+
+@pytest.mark.parametrize("n_bins,hot", [(20000, [300]), (20000, [300, 300 + 16384]), (32768, [32767]), (32768, [16383, 32767]),
+                                        (65536, [300, 300 + 16384, 300 + 49152]), (16384, [300]), (16384, [255, 16383]), (5000, [4999])])
+@pytest.mark.parametrize("way", ["sweep", "merge"])
+@pytest.mark.parametrize("n", [1 << 18, (1 << 19) + 70001])
+def test_histogram_counters_that_take_more_than_16_bits(xs, gpu, monkeypatch, n_bins, hot, way, n):
+    """Work-groups of 2^18 keys with one, two or three bins outside the warm ones, in one word where a word holds
+    several, that take more than 2^16 keys of a group each: half words (and bytes) overflow and are recounted, whole
+    words hold them, through both ways of merging. Whole numbers: bit for bit the oracle's."""
+    torch = gpu
+    print(f"case hist-16bit n={n} bins={n_bins} hot={hot} {way}", flush=True)
+    monkeypatch.setenv("XSCHED_HIP_HIST_MIN_CHUNK", str(1 << 18))
+    monkeypatch.setenv("XSCHED_HIP_HIST_MERGE_MIN_KEYS", "1" if way == "merge" else str(1 << 40))
+    rng = np.random.default_rng(n_bins + len(hot))
+    keys_h = rng.integers(0, n_bins, n).astype(np.int32)
+    hot_at = rng.random(n) < 0.9
+    keys_h[hot_at] = rng.choice(np.array(hot, np.int32), int(hot_at.sum()))
+    keys = torch.from_numpy(keys_h).cuda()
+    bins = torch.zeros(n_bins + 1, dtype=torch.int32, device="cuda")
+    q = Queue(xs, torch, 2)
+    q.submit(hist_cmd(xs, keys, n, bins, n_bins, 1))
+    q.wait()
+    got = bins.cpu().numpy().view(np.uint32)
+    q.close()
+    want = oracle.histogram(keys_h, n_bins)
+    assert min(int(np.sum(keys_h[:1 << 18] == h)) for h in hot) > 1 << 16
+    assert np.array_equal(got[:n_bins], want)
+    assert got[n_bins] == 0, "wrote beyond the bins array"
+
+
+@pytest.mark.parametrize("n,n_bins", [((1 << 16) - 3, 65536), (1 << 16, 20000)])
+def test_few_keys_flushed_and_replayed(xs, gpu, n, n_bins):
+    """The kernel for few keys over many bins, suspended and resumed until launches of it have been
+    replayed a few times: every command counts once. A command takes some 5 us, so they come in rounds."""
+    torch = gpu
+    print(f"case few-keys-flush n={n} bins={n_bins}", flush=True)
+    rng = np.random.default_rng(n)
+    keys_h = rng.integers(0, n_bins, n).astype(np.int32)
+    keys = torch.from_numpy(keys_h).cuda()
+    bins = torch.zeros(n_bins, dtype=torch.int32, device="cuda")
+    q = Queue(xs, torch, level=2, threshold=4, batch=2)
+    stop = threading.Event()
+    t = threading.Thread(target=churn, args=(xs, q, stop, 5))
+    t.start()
+    times = 0
+    while times < 20000:
+        for _ in range(100):
+            q.submit(hist_cmd(xs, keys, n, bins, n_bins, 1))
+        times += 100
+        st = hip_stats(xs, q.hwq)
+        if st[1] >= 5 and st[2] >= 5:
+            break
+    stop.set()
+    t.join()
+    q.wait()
+    st = hip_stats(xs, q.hwq)
+    got = bins.cpu().numpy().view(np.uint32)
+    q.close()
+    print("stats", st, "commands", times, flush=True)
+    assert st[1] >= 5 and st[2] >= 5, "too few launches were replayed"
+    assert np.array_equal(got.astype(np.uint64), (oracle.histogram(keys_h, n_bins).astype(np.uint64) * times) & 0xFFFFFFFF)
