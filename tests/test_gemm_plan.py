@@ -37,7 +37,7 @@ def test_a_plan_covers_the_rows_and_assumes_only_what_holds(xs, monkeypatch, til
                 assert edge == 64 and len(plan) == 1, case
                 assert N < 8 or M * K < 8 or (tile == 0 and K <= 128), case
                 continue
-            assert N >= 8 and M * K >= 8 and (tile != 0 or K > 32), case
+            assert N >= 8 and M * K >= 8 and (tile != 0 or K > 32 or (aligned and N % 32 == 0)), case
             assert fit == UNALIGNED or aligned, case
             assert (fit == EXACT) == (aligned and rows % edge == 0 and N % edge == 0 and K % 64 == 0), case
             assert kernel == FOUR_STAGES if fit == UNALIGNED else True, case
@@ -61,6 +61,10 @@ def test_a_plan_covers_the_rows_and_assumes_only_what_holds(xs, monkeypatch, til
     (2000, 1999, 32, (64, ANY_SHAPE)), (4000, 4008, 32, (64, ANY_SHAPE)), (4000, 4008, 40, (256, TWO_BUFFERS)),
     (7000, 7000, 64, (64, ANY_SHAPE)), (7040, 7040, 64, (128, TWO_BUFFERS)), (7001, 7003, 128, (64, ANY_SHAPE)),
     (7001, 7003, 136, (128, FOUR_STAGES)), (4001, 4003, 48, (64, ANY_SHAPE)), (4001, 4003, 49, (128, FOUR_STAGES)),
+    # rows of C of whole 64-byte pieces: only where a last round of large tiles is at most half full
+    (4096, 4096, 32, (256, TWO_BUFFERS)), (8192, 8192, 24, (256, TWO_BUFFERS)), (6353, 7168, 40, (256, TWO_BUFFERS)),
+    (6353, 7200, 64, (256, TWO_BUFFERS)), (1024, 1024, 32, (64, FOUR_STAGES)), (7912, 4800, 32, (64, ANY_SHAPE)),
+    (7912, 4800, 40, (256, TWO_BUFFERS)), (6353, 7176, 64, (64, ANY_SHAPE)),
     (300, 301, 33, (64, FOUR_STAGES)), (8191, 515, 96, (64, ANY_SHAPE)), (2000, 1999, 64, (64, ANY_SHAPE)),
     (1000, 1001, 64, (64, FOUR_STAGES))])
 def test_the_kernel_that_measured_quickest_is_taken(xs, M, N, K, want):

@@ -1169,7 +1169,7 @@ inline double MicrosOf(const Part &part, int K)
     return 3.0 + std::ceil(rounds) * r.round + step * ((K + kStepK - 1) / kStepK);
 }
 
-/// Whether K is so short that the any-shape kernel is the quickest: up to 32, one step of it, always;
+/// Whether K is so short that the any-shape kernel is the quickest: up to 32, one step of it;
 /// further for outputs of many tiles, whose write-out it overlaps best, and the further the fewer of
 /// its loads come one by one. Measured on either side, any-shape kernel against the quickest of the others, us:
 /// with 16-byte rows in all three matrices, 7000^2 at K = 64 35.9 against 41.6, at 72 47.5 against
@@ -1177,14 +1177,24 @@ inline double MicrosOf(const Part &part, int K)
 /// 96, 8191 x 515 at 96 12.1 against 13.9, at 128 14.4 against 13.9, 2000 x 1999 at 64 9.0 against
 /// 9.4, at 72 10.5 against 10.3, 1000 x 1001 at 40 5.5 against 5.3; without, 2000 x 1999 at 31 8.3 against 9.4, at 33
 /// 9.5 against 9.9, at 63 13.3 against 9.5, 4001 x 4003 at 31 18.6 against 31.2, at 63 36.8 against 31.4.
+/// Where rows of C are whole 64-byte pieces the other kernels write them as fast as memory takes them, and
+/// what the any-shape kernel can win is a last round of large tiles that is at most half full. Passes, us:
+/// 4096^2 at 32 (one whole round) 25.6 against 20.0, 8192^2 at 32 (four) 56.5 against 49.3, 6353 x 7168 at 32 (2.7)
+/// 43.7 against 38.1, at 64 47.0 against 41.1; 4400 x 4096 at 32 (1.1) 26.2 against 27.9, 6400 x 8192 (3.1) 42.6
+/// against 45.7, 7912 x 4800 (2.3) 35.3 against 38.4, but at 64 41.3 against 39.0. (With rows of other lengths,
+/// 6353 x 7176 at 64: 49.4 against 57.5.)
 inline bool ShortK(const void *A, const void *B, const void *C, int M, int N, int K)
 {
     const uint64_t tiles = TilesOf(M, N, kAnyTile), units = ComputeUnits();
     if (tiles > GuardState::kMaxWorkGroups) return false;
     int limit = 32;
     if (Aligned(A, B, C, N, K)) {
-        const bool whole_tiles = M % kSmallTile == 0 && N % kSmallTile == 0 && K % kStepK == 0;   // two work-groups to a unit do the same for them
-        if (tiles >= 32 * units && !whole_tiles) limit = 64;
+        if (N % 32 == 0) {
+            const uint64_t large = TilesOf(M, N, kLargeTile), over = large % units;
+            if (large < units || over == 0 || 2 * over > units) limit = 0;
+        } else if (tiles >= 32 * units) {
+            limit = 64;
+        }
     } else if (((uintptr_t)A & 15) == 0 && K % 8 == 0) {
         limit = tiles >= 12 * units ? 128 : 2 * tiles >= 9 * units ? 96 : tiles >= 4 * units ? 64 : 32;
     } else if (tiles > 4 * units) {
