@@ -114,8 +114,8 @@ __device__ __forceinline__ void TileOf(uint32_t wg, uint32_t tiles_m, uint32_t t
 //   kUnaligned  any N >= 8, any alignment to the element: pieces start at any multiple of two
 //               bytes, which the loads into LDS do not take: they come through registers
 //               (a tile or two in flight) and are stored to the same places. Only
-//               the last K step can reach behind the end of a matrix: its pieces are checked
-//               one by one and fetched element by element where they do.
+//               the last K step can reach behind the end of a matrix: a piece that does is fetched
+//               from the matrix's last 16 bytes instead and shifted into place.
 enum class Fit { kExact, kEdges, kUnaligned };
 
 typedef u32x4 u32x4_any __attribute__((aligned(2)));

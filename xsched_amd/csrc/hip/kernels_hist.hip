@@ -16,8 +16,8 @@
 // thirds of all Zipf(1.1) keys, a fifth of them in bins 0 and 1) have sixteen 32-bit counters
 // each, one per lane modulo 16, so that at most four lanes of a wave add to the same address, no
 // vote and no popcount is needed, and they cannot overflow (64, one per lane, where n_bins leaves
-// the room, and then for bin 255 too, which is all that 256 bins have: evenly spread keys over 1000 bins, a quarter of them in these bins, 54.7 us against
-// 56.8 with 16). Half of a compute unit's LDS and of its wave slots: two groups of different
+// the room, and then for bin 255 too, which is all that 256 bins have: 2^26 evenly spread keys over 1000 bins,
+// a quarter of them in these bins, 54.7 us a pass through a queue against 56.8 with 16). Half of a compute unit's LDS and of its wave slots: two groups of different
 // queues share it, and one streams keys while the other clears, writes out or waits for its first
 // keys (four queues of 2^26 keys each 217 -> 207 us; with 64 counters for every one of these bins
 // and 128 KiB, a group had its unit to itself). Every other bin shares one of 16384
@@ -36,7 +36,7 @@
 // a group that saw some passes over the quarters of the bins that have no keys: 2^26 equal keys outside the
 // first 255 of 65536 bins 559 -> 130 us, 2^22 78 -> 27, sorted 2^22 over 20000 bins 34.5 -> 18.3. Whole words need no test:
 // with bytes for any n_bins, 2^26 evenly spread keys over 1000 bins overflowed in every group
-// (262 keys of a chunk to a bin) and took 182 us instead of 49.
+// (262 keys of a chunk to a bin): 186 us a launch, 42 with whole words (a pass through a queue 199 and 55).
 //
 // What becomes of a group's counts (PlanFor() chooses, with the figures):
 //   few keys over many bins: another kernel, HistogramFewKeysKernel below.
@@ -55,8 +55,8 @@
 // bins.
 //
 // Guard: entry check, and because a group has no side effects before its write-out,
-// every wave re-reads the preempt word every 32768 keys of the group and the group abandons
-// itself (its progress byte stays untagged, a replay redoes the chunk). The write-out
+// every wave re-reads the preempt word every kLoopKeys keys of the group (16384; a shorter chunk is checked
+// at entry only) and the group abandons itself (its progress byte stays untagged, a replay redoes the chunk). The write-out
 // runs to completion and commits. The groups of the merge kernel have progress bytes
 // of their own behind those of the counting groups, and run only when every counting
 // group has committed; the scratch buffer is the command's own from its first launch
@@ -106,7 +106,7 @@ constexpr uint32_t kWarmBins = 255;                 // bins below this have 32-b
 constexpr uint32_t kCopies = 16;                    // one per lane modulo 16
 constexpr uint32_t kFewColdWords = 63u * 64;        // with at most this many cold words one per lane,
 constexpr uint32_t kFewColdWarmBins = 256;          // and one bin more
-constexpr uint32_t kOutside = 256;                  // counts a partial keeps outside the cold words (the last is 0)
+constexpr uint32_t kOutside = 256;                  // counts a partial keeps outside the cold words (the last is 0 with more than kFewColdWords of them)
 constexpr uint32_t kLdsBins = kColdWords + kWarmBins * kCopies;   // the cold words, then the warm counters
 static_assert(kFewColdWords + kFewColdWarmBins * 64 <= kLdsBins && kFewColdWarmBins <= kOutside, "a warm counter per lane beside few cold words");
 // The partial histograms of a launch in memory, n_part of them (one per counting group): the
@@ -771,7 +771,7 @@ void HistogramMergeKernel(const uint32_t *__restrict__ partials, uint32_t n_part
     }
     if (tid == 0) {
         // bin <column>, counted outside the cold words (which hold nothing for bins below 255; bin 255
-        // has its count there and 0 here)
+        // has its count in one of the two and 0 in the other)
         if (outside_total != 0 && column < n_bins) GlobalAdd(bins + column, outside_total);
     }
     if (kGuard) {
