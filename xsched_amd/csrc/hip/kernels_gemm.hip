@@ -11,20 +11,27 @@
 //                       bits of its row, chosen so that every fragment read below touches
 //                       each LDS bank once.
 //                       A tile: [256 rows][64 k], two rows to a 256-byte line of sixteen
-//                       slots, slot = ((row & 1) * 8 + k / 8) ^ (line & 15).
-//                       B tile: as it sits in memory, [64 k][256 cols], eight 64-byte granules
-//                       to a row, granule = (col / 32) ^ ((k & 3) | ((k >> 1) & 4)).
-//   LDS -> MFMA         v_mfma_f32_32x32x16_bf16; wave (wm, wn) of the 2x4 wave grid
-//                       accumulates a 128x64 sub-tile = 4x2 blocks of 32x32
+//                       slots, slot = (row & 1) * 8 + ((k / 8) ^ (line & 7)).
+//                       B tile: as it sits in memory, [64 k][256 cols], sixteen 32-byte granules
+//                       to a row, granule = (col / 16) ^ ((k & 3) * 2 + ((k >> 3) & 1)).
+//   LDS -> MFMA         v_mfma_f32_16x16x32_bf16; wave (wm, wn) of the 2x4 wave grid
+//                       accumulates a 128x64 sub-tile = 8x4 blocks of 16x16
 // An MFMA operand wants eight consecutive k per lane. A has them contiguous in memory; for B
 // (k is the strided dimension) the transposing LDS read of gfx950, ds_read_b64_tr_b16, turns
-// four rows of four columns into four k of one column per lane, two of them per fragment.
+// four rows of sixteen columns into four k of one column per lane, two of them per fragment.
 // There is no split-K: every element of C is summed by one wave in one fixed order, which
 // makes a replayed tile bit-identical.
 //
-// Under this load the device runs against its power limit (the clock settles near 1.85 GHz),
-// so bytes moved cost time even when nothing waits for them: the loop issues one LDS read or
-// one global load next to each MFMA and nothing else.
+// Under this load the device runs against its power limit (all operands zero, when next to nothing
+// switches, 8192^3 takes 567 us, normally distributed ones 782 on the same box and code), so
+// energy is time:
+//   - blocks of 16x16 rather than 32x32: MFMAs alone, operands in registers, reach 2.0 PFLOP/s on
+//     normally distributed operands with the one and 1.78 with the other (2.4 both on zeroes; an MFMA
+//     of 32x32 reads and writes twice the accumulators per flop). The sums are bit for bit the same.
+//   - neighbouring MFMAs share an operand (the columns of every other row of blocks run backwards): 1 %.
+//   - the loads of a step are spread evenly over half of it: next to every fourth MFMA 727 us, next to
+//     every second 733, every one 750.
+// 8192^3 782 -> 725 us per launch, 4096^3 102.0 -> 94.8 (1.52 and 1.45 PFLOP/s).
 //
 // Guard: the tile is computed in registers and written once at the end, so a
 // work-group may give up at any K step without side effects. The preempt word is
@@ -52,6 +59,7 @@ namespace gemm
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
@@ -99,9 +107,6 @@ __device__ __forceinline__ void TileOf(uint32_t wg, uint32_t tiles_m, uint32_t t
     tn = in_band / rows;
 }
 
-// The compiler keeps the instructions of one group in the order the groups are listed:
-// mask 0x008 = MFMA, 0x100 = LDS read.
-#define XS_GROUP(mask, n) __builtin_amdgcn_sched_group_barrier(mask, n, 0)
 #define XS_PIN __builtin_amdgcn_sched_barrier(0)
 #define XS_WAIT_GLOBAL_LOADS __builtin_amdgcn_s_waitcnt(0x0F70) /* vmcnt(0), nothing else */
 
@@ -154,23 +159,26 @@ __device__ __forceinline__ void StoreEight(uint16_t *C, size_t row, size_t col, 
 /// last one.
 enum TileRequest { kNoTile, kAnyButLast, kTheLast };
 
-// Two LDS buffers and ONE barrier per K step. While the MFMAs of step t read buffer t % 2,
-// tile t + 1 is landing in the other buffer (its loads were issued a whole step earlier);
-// after the barrier buffer t % 2 is free and the loads of tile t + 2 go out, one next to
-// each MFMA of the step's last k slice. The fragments of the next 16-wide k slice are read
-// from LDS next to the MFMAs of the current slice, one read per MFMA.
+// Two LDS buffers and ONE barrier per K step. A step is two k slices of 32. While the MFMAs of the
+// first one run, the fragments of the second are read from buffer t % 2, and tile t + 1 lands in the
+// other buffer (its loads were issued over the slice before); after the barrier buffer t % 2 is free:
+// next to the MFMAs of the second slice the first fragments of tile t + 1 are read and the loads of
+// tile t + 2 go out.
 //
 // kTile x kTile is the tile of C, kWavesM x kWavesN the wave grid over it; a wave owns
-// kBlocksM x kBlocksN blocks of 32x32. Built for 256 with 2x4 waves (4x2 blocks
+// kBlocksM x kBlocksN blocks of 16x16. Built for 256 with 2x4 waves (8x4 blocks
 // per wave), for exact shapes and for ragged ones (kEdges): there the last tile's loads, the last
 // step and the stores look at the edges, and the steps before are the same code (4000^3 146 us on
-// 128 x 128 tiles, 114 on these). And for 128 with 2x2 waves (2x2 blocks), exact shapes only: 64 KiB
+// 128 x 128 tiles, 106 on these). And for 128 with 2x2 waves (4x4 blocks), exact shapes only: 64 KiB
 // of LDS and 4 waves, so two work-groups share a compute unit and one computes while the other
 // waits for its first loads or writes out. That is what outputs of 257 to 512 such tiles want,
 // which are two rounds for the four-stage kernel below (its 130 KiB let a unit have one group), and
 // what short K wants, where a tile is little more than its first loads and its write-out
 // (per command: 368 tiles at K = 192 10.1 -> 7.3 us, at 2048 33.5 -> 28.9; 276 at 4096 55.1 -> 50.1;
 // 1023 at 128 16.5 -> 10.7).
+// Four waves of 128x128 on the large tile (a third fewer LDS reads, one wave per SIMD, accumulators
+// in AGPRs) take 732 us for 8192^3 where eight take 725, and 595 against 567 on zeroes: nothing runs
+// beside their barrier.
 //
 // (The body is a device function: the host pass cannot parse the buffer-resource builtins
 // and would silently drop the launch stub of a kernel that uses them directly.)
@@ -181,21 +189,22 @@ void GemmBf16Body(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
 {
     static_assert(kFit != Fit::kUnaligned, "loads go straight into LDS");
     constexpr int kWaves = kWavesM * kWavesN;
-    constexpr int kBlocksM = kTile / (32 * kWavesM);
-    constexpr int kBlocksN = kTile / (32 * kWavesN);
-    constexpr int kMfmas = kBlocksM * kBlocksN;          // per wave and 16-wide k slice
+    constexpr int kBlocksM = kTile / (16 * kWavesM);
+    constexpr int kBlocksN = kTile / (16 * kWavesN);
+    constexpr int kMfmas = kBlocksM * kBlocksN;          // per wave and 32-wide k slice
+    constexpr int kReads = kBlocksM + kBlocksN;          // fragments of a slice
     constexpr int kABytes = kTile * kStepK * 2;          // one A tile in LDS
     constexpr int kBBytes = kStepK * kTile * 2;          // one B tile
     constexpr int kALoads = kABytes / 1024 / kWaves;     // wave-wide 1 KiB loads per wave and tile
     constexpr int kBLoads = kBBytes / 1024 / kWaves;
     constexpr int kLoads = kALoads + kBLoads;
-    constexpr int kLoadsPerMfma = kLoads / kMfmas;
+    constexpr int kLoadEvery = kMfmas / kLoads;          // one load next to so many MFMAs
     constexpr int kBRowBytes = kTile * 2;                // one k row of the B tile
     constexpr int kBSlotsPerRow = kBRowBytes / 16;
     constexpr int kBRowsPerLoad = 64 / kBSlotsPerRow;
-    constexpr uint32_t kBGranuleMask = kBRowBytes / 64 - 1;
-    static_assert(kBlocksN == 2, "the block index is XORed into the granule number as one bit");
-    static_assert(kMfmas * kLoadsPerMfma == kALoads + kBLoads && kBlocksM + kBlocksN <= kMfmas, "loads and reads pair up with the MFMAs of a slice");
+    static_assert(kBlocksN == 4, "the block index is XORed into the granule number as two bits");
+    static_assert(kBRowBytes >= 256, "a granule number has the three bits that are XORed");
+    static_assert(kLoadEvery * kLoads == kMfmas && 2 * kReads <= kMfmas, "loads and reads pair up with the MFMAs of a slice");
     // One LDS object for everything, the word the waves agree on a poll through included:
     // with a second object the compiler attaches alias scopes to the LDS accesses and then
     // makes every fragment read wait for all global loads that are on their way into LDS.
@@ -219,23 +228,18 @@ void GemmBf16Body(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
     // ---- global -> LDS: lane l of wave-wide load q fills LDS slot 64 q + l (16 bytes) ----
     // Byte offsets of what each lane fetches, relative to the first element of the tile.
     uint32_t a_off[kALoads], b_off[kBLoads];
+    auto a_k = [&](int i) -> uint32_t { return ((lane & 7) ^ ((4 * (wave * kALoads + i) + (lane >> 4)) & 7)) * 8; };   // first k of its piece
+    auto b_k = [&](int i) -> uint32_t { return kBRowsPerLoad * (wave * kBLoads + i) + lane / kBSlotsPerRow; };
 #pragma unroll
     for (int i = 0; i < kALoads; ++i) {
-        const uint32_t q = wave * kALoads + i;
-        const uint32_t line = 4 * q + (lane >> 4);
-        const uint32_t piece = (lane & 15) ^ (line & 15);   // which piece of the line belongs in this slot
-        uint32_t row = 2 * line + (piece >> 3);
-        const uint32_t kc = piece & 7;
+        uint32_t row = 2 * (4 * (wave * kALoads + i) + (lane >> 4)) + ((lane >> 3) & 1);
         if (kFit != Fit::kExact && m0 + row >= (size_t)M) row = (uint32_t)((size_t)M - 1 - m0);   // not stored
-        a_off[i] = (row * (uint32_t)K + kc * 8) * 2;
+        a_off[i] = (row * (uint32_t)K + a_k(i)) * 2;
     }
 #pragma unroll
     for (int i = 0; i < kBLoads; ++i) {
-        const uint32_t q = wave * kBLoads + i;
-        const uint32_t k = kBRowsPerLoad * q + lane / kBSlotsPerRow;
-        const uint32_t slot = lane % kBSlotsPerRow;
-        const uint32_t granule = (slot >> 2) ^ (((k & 3) | ((k >> 1) & 4)) & kBGranuleMask);
-        uint32_t col = granule * 32 + (slot & 3) * 8;
+        const uint32_t k = b_k(i), slot = lane % kBSlotsPerRow;
+        uint32_t col = ((slot >> 1) ^ ((k & 3) << 1 | ((k >> 3) & 1))) * 16 + (slot & 1) * 8;
         if (kFit != Fit::kExact && n0 + col >= (size_t)N) col = 0;                                // not stored
         b_off[i] = (k * (uint32_t)N + col) * 2;
     }
@@ -247,12 +251,11 @@ void GemmBf16Body(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
     auto piece_off = [&](int idx, bool last) -> uint32_t {
         if (idx < kALoads) {
             if (kFit == Fit::kExact || !last) return a_off[idx];
-            const uint32_t line = 4 * (wave * kALoads + idx) + (lane >> 4);
-            const uint32_t k = (((lane & 15) ^ (line & 15)) & 7) * 8;
+            const uint32_t k = a_k(idx);
             return k < (uint32_t)rest ? a_off[idx] : a_off[idx] - k * 2;
         }
         if (kFit == Fit::kExact || !last) return b_off[idx - kALoads];
-        const uint32_t k = kBRowsPerLoad * (wave * kBLoads + idx - kALoads) + lane / kBSlotsPerRow;
+        const uint32_t k = b_k(idx - kALoads);
         return k < (uint32_t)rest ? b_off[idx - kALoads] : b_off[idx - kALoads] - k * (uint32_t)N * 2;
     };
     // Load number idx of the tile of K step `step` into buffer `buf`.
@@ -277,54 +280,56 @@ void GemmBf16Body(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
     };
 
     // ---- LDS -> fragments ----
-    // A: lane reads row a_row0 + 32 i, pieces 2 ks + (lane >> 5). 32 rows further is 16 lines
+    // A: lane reads row a_row0 + 16 i, piece 4 ks + (lane >> 4). 16 rows further is 8 lines
     // further: the same swizzle bits, so one base address serves all blocks of the wave.
-    const uint32_t a_row0 = 32 * kBlocksM * wm + (lane & 31);
+    const uint32_t a_row0 = 16 * kBlocksM * wm + (lane & 15);
     const uint32_t a_line = a_row0 >> 1;
-    const uint32_t a_base = a_line * 256 + (((((lane & 1) << 3) | (lane >> 5)) ^ (a_line & 15)) << 4);
+    const uint32_t a_base = a_line * 256 + ((((lane & 1) << 3) | ((lane >> 4) ^ (a_line & 7))) << 4);
     auto read_a = [&](int buf, int ks, int i) {
-        return *(const bf16x8 *)(As0 + buf * kABytes + (a_base ^ (ks << 5)) + i * 4096);
+        return *(const bf16x8 *)(As0 + buf * kABytes + (a_base ^ (ks << 6)) + i * 2048);
     };
     // B sits in LDS as it sits in memory, [k][n]. The transposing read hands lane l of every 16
     // lanes the element (l & 3) of what lanes 4 * j + (l >> 2), j = 0..3, of the same 16 point
     // at: with lane r pointing at row (r >> 2), columns 4 * (r & 3) .. + 3, lane l receives
     // column l of rows 0..3. Two reads give the eight consecutive k of one fragment. The rows
     // a lane points at all have the same swizzle bits (k & 3 and bit 3 of k are fixed per lane).
-    const uint32_t b_row = 8 * (lane >> 5) + ((lane & 15) >> 2);
-    const uint32_t b_swz = (((lane & 15) >> 2) | ((lane >> 5) << 2)) & kBGranuleMask;
-    const uint32_t b_base = b_row * kBRowBytes + (((kBlocksN * wn) ^ b_swz) << 6) + (16 * ((lane >> 4) & 1) + 4 * (lane & 3)) * 2;
+    const uint32_t b_row = 8 * (lane >> 4) + ((lane & 15) >> 2);
+    const uint32_t b_swz = ((lane & 15) >> 2) << 1 | ((lane >> 4) & 1);
+    const uint32_t b_base = b_row * kBRowBytes + (((kBlocksN * wn) ^ b_swz) << 5) + 4 * (lane & 3) * 2;
     auto read_b = [&](int buf, int ks, int j) {
-        const uint8_t *p = Bs0 + buf * kBBytes + ks * 16 * kBRowBytes + (b_base ^ (j << 6));
+        const uint8_t *p = Bs0 + buf * kBBytes + ks * 32 * kBRowBytes + (b_base ^ (j << 5));
         const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsS16x4 *)p);
         const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsS16x4 *)(p + 4 * kBRowBytes));
         return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
     };
-    auto read_frags = [&](int buf, int ks, bf16x8 *fa, bf16x8 *fb) {
-#pragma unroll
-        for (int i = 0; i < kBlocksM; ++i) fa[i] = read_a(buf, ks, i);
-#pragma unroll
-        for (int j = 0; j < kBlocksN; ++j) fb[j] = read_b(buf, ks, j);
+    bf16x8 fa[2][kBlocksM], fb[2][kBlocksN];
+    // Fragment number n of slice ks into set ks, in the order in which the MFMAs want them.
+    auto read_frag = [&](int buf, int ks, int n) {
+        if (n < kBlocksN) fb[ks][n] = read_b(buf, ks, n);
+        else fa[ks][n - kBlocksN] = read_a(buf, ks, n - kBlocksN);
     };
 
-    f32x16 acc[kBlocksM][kBlocksN];
+    f32x4 acc[kBlocksM][kBlocksN];
 #pragma unroll
     for (int i = 0; i < kBlocksM; ++i)
 #pragma unroll
-        for (int j = 0; j < kBlocksN; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+        for (int j = 0; j < kBlocksN; ++j) acc[i][j] = f32x4 { 0.f, 0.f, 0.f, 0.f };
+    auto mfma = [&](int ks, int n) {
+        const int i = n / kBlocksN, j = i & 1 ? kBlocksN - 1 - n % kBlocksN : n % kBlocksN;
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[ks][i], fb[ks][j], acc[i][j], 0, 0, 0);
+    };
 
-    // A lane's fragment of slice ks holds k = 16 ks + 8 (lane / 32) + 0..7 of the step, for A and
+    // A lane's fragment of slice ks holds k = 32 ks + 8 (lane / 16) + 0..7 of the step, for A and
     // for B alike: everything from `rest` on becomes zero.
-    auto mask_behind_k = [&](int ks, bf16x8 *a, bf16x8 *b) {
-        const int valid = rest - (16 * ks + 8 * (int)(lane >> 5));
+    auto mask_behind_k = [&](int ks) {
+        const int valid = rest - (32 * ks + 8 * (int)(lane >> 4));
         u32x4 m;
 #pragma unroll
         for (int d = 0; d < 4; ++d) m[d] = valid >= 2 * d + 2 ? 0xFFFFFFFFu : valid == 2 * d + 1 ? 0xFFFFu : 0u;
 #pragma unroll
-        for (int i = 0; i < kBlocksM; ++i) a[i] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, a[i]) & m);
+        for (int i = 0; i < kBlocksM; ++i) fa[ks][i] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, fa[ks][i]) & m);
 #pragma unroll
-        for (int j = 0; j < kBlocksN; ++j) b[j] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, b[j]) & m);
+        for (int j = 0; j < kBlocksN; ++j) fb[ks][j] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, fb[ks][j]) & m);
     };
 
     load_tile(0, 0);
@@ -340,39 +345,14 @@ void GemmBf16Body(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
     XS_WAIT_GLOBAL_LOADS;
     __syncthreads();
     load_tile(1, steps > 1 ? 1 : 0);
-
-    bf16x8 fa[2][kBlocksM], fb[2][kBlocksN];
-    read_frags(0, 0, fa[0], fb[0]);
-
-    // One k slice: the MFMAs on fragment set `set`, the reads of the next slice into the other
-    // set, one read after each of the first MFMAs (the small tile has fewer MFMAs than reads:
-    // there a B fragment's two reads follow one MFMA).
-    auto slice = [&](int set, int next_buf, int next_ks) {
-        XS_PIN;
-        read_frags(next_buf, next_ks, fa[set ^ 1], fb[set ^ 1]);
 #pragma unroll
-        for (int i = 0; i < kBlocksM; ++i)
-#pragma unroll
-            for (int j = 0; j < kBlocksN; ++j)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[set][i], fb[set][j], acc[i][j], 0, 0, 0);
-        constexpr int kReads = kBlocksM + 2 * kBlocksN;
-        if constexpr (kMfmas >= kReads) {
-#pragma unroll
-            for (int n = 0; n < kReads; ++n) { XS_GROUP(0x008, 1); XS_GROUP(0x100, 1); }
-        } else {
-#pragma unroll
-            for (int n = 0; n < kBlocksM; ++n) { XS_GROUP(0x008, 1); XS_GROUP(0x100, 1); }
-#pragma unroll
-            for (int n = 0; n < kBlocksN; ++n) { XS_GROUP(0x008, 1); XS_GROUP(0x100, 2); }
-        }
-        XS_PIN;
-    };
+    for (int n = 0; n < kReads; ++n) read_frag(0, 0, n);
 
     // One K step. The polling form (every kPollSteps-th step of a guarded launch) is a body of
     // its own: its branches split the step into several scheduling regions and put the address
     // arithmetic of the loads behind the barrier, which costs the step about 3 % - paid on one
     // step in kPollSteps instead of on all of them. The last two steps have nothing left to
-    // load (`loading` false), the last one nothing to read ahead either (`reading_ahead`
+    // load (`loading` kNoTile), the last one nothing to read ahead either (`reading_ahead`
     // false): after its barrier no wave touches the tile buffers any more. False: the
     // work-group has to leave.
     auto step = [&](int t, auto polling, auto loading, auto reading_ahead) -> bool {
@@ -382,19 +362,22 @@ void GemmBf16Body(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
         constexpr bool kMask = kFit != Fit::kExact && !kReadAhead;
         const int cur = t & 1;
         // Wave 0 asks for the preempt word here, with a vector load that is on its way during
-        // the whole step, and looks at it just before the barrier: no wave ever waits for the
+        // the first slice, and looks at it just before the barrier: no wave ever waits for the
         // word alone (a scalar load at the barrier made wave 0 wait for the uncached round trip
         // and for all of its LDS reads while the other seven waves stood at the barrier).
         uint32_t polled = 0;
         if (kPoll && wave == 0) polled = xguard_read_flag_begin(xguard_flag_copy(g, blockIdx.x));
 
-        if (kMask) mask_behind_k(0, fa[0], fb[0]);
-        slice(0, cur, 1);
-        if (kMask) mask_behind_k(1, fa[1], fb[1]);
-        slice(1, cur, 2);
-        if (kMask) mask_behind_k(2, fa[0], fb[0]);
-        slice(0, cur, 3);
-        if (kMask) mask_behind_k(3, fa[1], fb[1]);
+        // First slice: one read next to each of the first MFMAs, so that all have arrived by its end.
+        if (kMask) mask_behind_k(0);
+        XS_PIN;
+#pragma unroll
+        for (int n = 0; n < kMfmas; ++n) {
+            mfma(0, n);
+            if (n < kReads) read_frag(cur, 1, n);
+            XS_PIN;
+        }
+        if (kMask) mask_behind_k(1);
 
         if (kPoll && wave == 0) {
             const bool current = xguard_read_flag_end(polled) == g.epoch;
@@ -409,26 +392,19 @@ void GemmBf16Body(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
             if (*(LdsVolatileWord *)&guard_word == 0) return false; // the whole group leaves together; nothing was written, no load is in flight
         }
 
-        // Last slice of the step: its MFMAs, next to them the first fragments of tile t + 1
+        // Second slice: next to its MFMAs the first fragments of tile t + 1, one to every second MFMA,
         // and the loads of tile t + 2 into the buffer that has just become free.
         XS_PIN;
 #pragma unroll
-        for (int i = 0; i < kBlocksM; ++i)
-#pragma unroll
-            for (int j = 0; j < kBlocksN; ++j) {
-                const int n = i * kBlocksN + j;
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[1][i], fb[1][j], acc[i][j], 0, 0, 0);
-                if (kReadAhead) {
-                    if (n < kBlocksM) fa[0][n] = read_a(cur ^ 1, 0, n);
-                    else if (n < kBlocksM + kBlocksN) fb[0][n - kBlocksM] = read_b(cur ^ 1, 0, n - kBlocksM);
-                }
-#pragma unroll
-                for (int l = 0; l < kLoadsPerMfma; ++l) {
-                    if constexpr (kLoad == kAnyButLast) load_piece(cur, t + 2, n * kLoadsPerMfma + l, false);
-                    if constexpr (kLoad == kTheLast) load_piece(cur, t + 2, n * kLoadsPerMfma + l, true);
-                }
-                XS_PIN;
+        for (int n = 0; n < kMfmas; ++n) {
+            mfma(1, n);
+            if (kReadAhead && n % 2 == 0 && n / 2 < kReads) read_frag(cur ^ 1, 0, n / 2);
+            if (n % kLoadEvery == kLoadEvery - 1) {
+                if constexpr (kLoad == kAnyButLast) load_piece(cur, t + 2, n / kLoadEvery, false);
+                if constexpr (kLoad == kTheLast) load_piece(cur, t + 2, n / kLoadEvery, true);
             }
+            XS_PIN;
+        }
         return true;
     };
     constexpr std::true_type yes {};
@@ -454,36 +430,36 @@ void GemmBf16Body(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
     if (steps >= 2) step(steps - 2, no, no_tile, yes);
     step(steps - 1, no, no_tile, no);
 
-    // Write-out. A lane holds one column of sixteen rows of each 32x32 block (four runs of four
-    // consecutive rows), so storing from the accumulators would mean 2-byte stores to sixteen
-    // different rows. Instead every wave turns its strips of 32 rows x 64 columns over in LDS,
-    // in an area of its own inside the tile buffers (nobody reads those any more, and nothing
-    // is on its way into them): a run of four rows of one column goes in as ONE 64-bit store
-    // (the strip is kept column-major, a column padded from 64 to 72 bytes so that the 32
-    // columns of a store fall into 32 different 8-byte bank groups), and the transposing read
+    // Write-out. A lane holds four consecutive rows of one column of each 16x16 block, so storing
+    // from the accumulators would mean 2-byte stores to four different rows. Instead every wave
+    // turns its strips of 32 rows x 64 columns over in LDS, in an area of its own inside the
+    // tile buffers (nobody reads those any more, and nothing is on its way into them): a block's
+    // four rows of one column go in as ONE 64-bit store (the strip is kept column-major, a column
+    // padded from 64 to 80 bytes so that the sixteen columns of a store fall into different
+    // banks), and the transposing read
     // brings it back out row-major: pointed at four rows of columns 8 q + j (lane 4 j + q of
     // every 16), it hands lane l row (l & 3) of columns 8 (l >> 2) + 0..3; a second read four
     // columns further completes 16 bytes per lane, and 8 rows x 128 bytes leave per store.
-    constexpr int kStripColumnBytes = 64 + 8;
+    constexpr int kStripColumnBytes = 64 + 16;
     constexpr int kStripBytes = 64 * kStripColumnBytes;
     static_assert(2 * kABytes >= kWaves * kStripBytes, "the A buffers hold one strip per wave");
     uint8_t *const strip = As0 + wave * kStripBytes;
-    const uint32_t put_at = (lane & 31) * kStripColumnBytes + 4 * (lane >> 5) * 2;
     const uint32_t l16 = lane & 15, patch = lane >> 4;   // a patch: 4 rows x 32 columns per 16 lanes
+    const uint32_t put_at = l16 * kStripColumnBytes + 4 * patch * 2;
     const uint32_t get_row = 4 * (patch >> 1), get_col = 32 * (patch & 1);
     const uint32_t get_at = (get_col + 8 * (l16 & 3) + (l16 >> 2)) * kStripColumnBytes + get_row * 2;
 #pragma unroll
-    for (int i = 0; i < kBlocksM; ++i) {
+    for (int s = 0; s < kBlocksM / 2; ++s) {
 #pragma unroll
-        for (int j = 0; j < kBlocksN; ++j) {
+        for (int half = 0; half < 2; ++half) {
 #pragma unroll
-            for (int run = 0; run < 4; ++run) {
-                const uint32_t lo = f32x2_to_bf16x2_rne(acc[i][j][4 * run], acc[i][j][4 * run + 1]);
-                const uint32_t hi = f32x2_to_bf16x2_rne(acc[i][j][4 * run + 2], acc[i][j][4 * run + 3]);
-                *(u32x2 *)(strip + 32 * j * kStripColumnBytes + put_at + 8 * run * 2) = u32x2 { lo, hi };
+            for (int j = 0; j < kBlocksN; ++j) {
+                const f32x4 v = acc[2 * s + half][j];
+                *(u32x2 *)(strip + 16 * j * kStripColumnBytes + put_at + 16 * half * 2) =
+                    u32x2 { f32x2_to_bf16x2_rne(v.x, v.y), f32x2_to_bf16x2_rne(v.z, v.w) };
             }
         }
-        const size_t row0 = m0 + 32 * kBlocksM * wm + 32 * i;
+        const size_t row0 = m0 + 16 * kBlocksM * wm + 32 * s;
         const size_t col0 = n0 + 64 * wn + get_col + 8 * (l16 >> 2);
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
@@ -504,7 +480,7 @@ void GemmBf16Body(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
 }
 
 template <bool kGuard, Fit kFit, int kTile, int kWavesM, int kWavesN>
-__global__ __launch_bounds__(64 * kWavesM * kWavesN)
+__global__ __launch_bounds__(64 * kWavesM * kWavesN, 2 /* waves per SIMD: no accumulators move between AGPRs and VGPRs */)
 void GemmBf16Kernel(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B,
                     uint16_t *__restrict__ C, int M, int N, int K, XGuardArgs g)
 {
