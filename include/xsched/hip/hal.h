@@ -89,7 +89,9 @@ XResult HipAxpyCommandCreate(HwCommandHandle *cmd, float alpha, const void *x, v
  * aligned to 16 bytes), 128x128 or 64x64, whichever is estimated to be quickest, or into two
  * launches, 256x256 for most rows and smaller ones for the rest
  * (XSCHED_HIP_GEMM_TILE=64|128|256 overrides that where the shape allows). Fastest where the rows of all three matrices start on 16-byte boundaries (N and K multiples
- * of 8, matrices aligned to 16 bytes); up to twice as long where they do not. Every element is
+ * of 8, matrices aligned to 16 bytes). Where rows of A or B do not, large products copy that matrix first, to
+ * memory of the queue (up to 1 GiB, kept for the next command, given back with the queue; without
+ * it, or on a stream under capture, the product takes up to twice as long). Every element is
  * summed in the same order on all paths. */
 XResult HipGemmBf16CommandCreate(HwCommandHandle *cmd, const void *A, const void *B, void *C,
                                  int M, int N, int K, int guard);
@@ -99,6 +101,12 @@ XResult HipGemmBf16CommandCreate(HwCommandHandle *cmd, const void *A, const void
  * rows of C, edge of a tile, kernel (0 two LDS buffers, 1 four stages, 2 any shape) and what it
  * assumes of the matrices (0 whole tiles, 1 16-byte rows, 2 nothing). No counterpart in the reference. */
 XResult HipGemmBf16PlanOf(const void *A, const void *B, const void *C, int M, int N, int K, int32_t *out);
+
+/* For tests: the same for the launches on copies of A and B whose rows start on 16-byte boundaries. `out`
+ * receives 10 values: the eight above (all zero where the matrices are multiplied as they lie), then the work-groups
+ * that copy A and B (0: not copied). Without memory for the copies, or on a stream under
+ * capture, HipGemmBf16PlanOf() holds. No counterpart in the reference. */
+XResult HipGemmBf16CopyPlanOf(const void *A, const void *B, const void *C, int M, int N, int K, int32_t *out);
 
 /* bins[keys[i]] += 1 for i < n; keys are int32 in [0, n_bins), bins are uint32 and
  * are NOT cleared by the command. n_bins <= 65536. */

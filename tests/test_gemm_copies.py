@@ -1,0 +1,222 @@
+"""Products whose rows lie off 16-byte boundaries and are copied to rows on them first: when that is
+planned (on the CPU: the plan reads no matrix), and on the GPU the edges of the copies, the queue's one
+buffer shared by several commands under flushes, and a stream under capture, which gets no copies."""
+import random
+import time
+from ctypes import byref, c_int32, c_uint64
+
+import numpy as np
+import pytest
+
+TWO_BUFFERS, FOUR_STAGES, ANY_SHAPE = 0, 1, 2
+EXACT, EDGES = 0, 1
+COPIED_PER_GROUP = 256 * 4 * 8      # elements that a work-group copies
+
+
+def plans_of(xs, a, b, c, M, N, K):
+    """(launches as they lie, launches on copies, work-groups that copy A, and B)"""
+    out = (c_int32 * 10)()
+    parts = lambda: [tuple(out[i:i + 4]) for i in (0, 4) if out[i] != 0]
+    xs.check(xs.halhip().HipGemmBf16PlanOf(a, b, c, M, N, K, out))
+    in_place = parts()
+    xs.check(xs.halhip().HipGemmBf16CopyPlanOf(a, b, c, M, N, K, out))
+    return in_place, parts(), out[8], out[9]
+
+
+def test_what_is_copied(xs):
+    rng = random.Random(5)
+    copied = 0
+    for _ in range(4000):
+        M, N, K = (int(2 ** rng.uniform(0, 14)) for _ in range(3))
+        if rng.random() < 0.3:
+            N = max(8, N // 8 * 8)
+        if rng.random() < 0.3:
+            K = max(8, K // 8 * 8)
+        a, b, c = ((1 << 20) + rng.choice([0, 0, 0, 2]) for _ in range(3))
+        in_place, parts, groups_a, groups_b = plans_of(xs, a, b, c, M, N, K)
+        case = (M, N, K, a, b, c, in_place, parts, groups_a, groups_b)
+        off_a, off_b = a % 16 != 0 or K % 8 != 0, b % 16 != 0 or N % 8 != 0
+        if not parts:
+            assert groups_a == groups_b == 0, case
+            continue
+        copied += 1
+        assert in_place[0][2] != ANY_SHAPE, case
+        assert (groups_a > 0, groups_b > 0) == (off_a, off_b) and (off_a or off_b), case
+        for groups, rows, cols in ((groups_a, M, K), (groups_b, K, N)):
+            if groups:
+                assert groups == -(-rows * (-(-cols // 64) * 64) // COPIED_PER_GROUP), case
+        assert sum(rows for rows, *_ in parts) == M, case
+        tiles = groups_a + groups_b
+        for rows, edge, kernel, fit in parts:
+            tiles += -(-rows // edge) * -(-N // edge)
+            whole = c % 16 == 0 and N % edge == 0 and rows % edge == 0 and K % 64 == 0
+            assert fit == (EXACT if whole else EDGES), case
+        assert tiles <= 1 << 18, case
+    assert copied > 300
+
+
+def test_what_is_not_copied(xs, monkeypatch):
+    at = 1 << 20
+    assert plans_of(xs, at, at, at, 4001, 4003, 2048)[1] != []
+    assert plans_of(xs, at, at, at + 2, 4096, 4096, 2048)[1] == []          # only C is off: nothing to copy
+    assert plans_of(xs, at, at, at + 2, 4096, 4096, 2048)[0] == [(4096, 256, TWO_BUFFERS, EDGES)]
+    assert plans_of(xs, at, at, at, 20001, 20003, 20001)[1] == []           # copies of 1.6 GB
+    assert plans_of(xs, at, at, at, 300, 301, 303)[1] == []                 # copying takes longer than it saves
+    monkeypatch.setenv("XSCHED_HIP_GEMM_TILE", "128")
+    assert plans_of(xs, at, at, at, 4001, 4003, 2048)[1] == []
+
+
+def _ints(torch, gen, shape, offset):
+    """Integers in [-2, 2] between NaNs, `offset` elements behind an aligned address."""
+    rows, cols = shape
+    flat = torch.full((rows * cols + offset + 64,), float("nan"), dtype=torch.bfloat16, device="cuda")
+    flat[offset:offset + rows * cols] = torch.randint(-2, 3, (rows * cols,), device="cuda", generator=gen).to(torch.bfloat16)
+    return flat[offset:offset + rows * cols].view(rows, cols)
+
+
+# both, A alone, B alone; rows of one piece more or less than whole lines, the last piece of one and of
+# seven elements, K of the last step 1 and 63; matrices off by an element; C alone off
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,offsets,copied", [
+    (3000, 2999, 301, (0, 0, 0), "ab"), (2500, 2503, 1025, (0, 0, 0), "ab"), (3001, 3009, 1087, (1, 3, 5), "ab"),
+    (3000, 3008, 1001, (0, 0, 0), "a"), (3000, 3001, 1000, (0, 0, 0), "b"), (4096, 4096, 1024, (1, 0, 0), "a"),
+    (4096, 4096, 1024, (0, 7, 1), "b"), (4100, 4104, 1024, (0, 0, 1), "")])
+@pytest.mark.parametrize("level,guard", [(1, 0), (2, 1)])
+def test_gemm_on_copies(xs, gpu, M, N, K, offsets, copied, level, guard):
+    """(K x 4 < 2^24: float32 sums are exact in any order.)"""
+    from test_gpu_kernels import Queue, gemm_cmd
+    torch = gpu
+    print(f"case gemm-copies M={M} N={N} K={K} offsets={offsets} level={level} guard={guard}", flush=True)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(M + K)
+    a, b = _ints(torch, gen, (M, K), offsets[0]), _ints(torch, gen, (K, N), offsets[1])
+    c_flat = torch.full((M * N + offsets[2] + 64,), 0.5, dtype=torch.bfloat16, device="cuda")
+    c = c_flat[offsets[2]:offsets[2] + M * N].view(M, N)
+    torch.cuda.synchronize()
+    _, parts, groups_a, groups_b = plans_of(xs, a.data_ptr(), b.data_ptr(), c.data_ptr(), M, N, K)
+    assert ("a" if groups_a else "") + ("b" if groups_b else "") == copied and bool(parts) == bool(copied)
+    q = Queue(xs, torch, level)
+    q.submit(gemm_cmd(xs, a, b, c, M, N, K, guard))
+    q.wait()
+    q.close()
+    assert torch.equal(c, (a.float() @ b.float()).to(torch.bfloat16))
+    assert bool((c_flat[:offsets[2]] == 0.5).all()) and bool((c_flat[offsets[2] + M * N:] == 0.5).all())
+
+
+@pytest.mark.gpu
+def test_copied_matrices_are_summed_in_the_same_order(xs, gpu, monkeypatch):
+    """Normally distributed inputs: the same bits as through registers."""
+    from test_gpu_kernels import Queue, gemm_cmd
+    torch = gpu
+    M, N, K = 3001, 2999, 1001
+    print(f"case gemm-copies-order M={M} N={N} K={K}", flush=True)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(1)
+    a, b = (torch.randn(s, device="cuda", generator=gen).to(torch.bfloat16) for s in ((M, K), (K, N)))
+    got, want = (torch.zeros(M, N, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    torch.cuda.synchronize()
+    assert plans_of(xs, a.data_ptr(), b.data_ptr(), got.data_ptr(), M, N, K)[1] != []
+    q = Queue(xs, torch, 2)
+    q.submit(gemm_cmd(xs, a, b, got, M, N, K, 1))
+    monkeypatch.setenv("XSCHED_HIP_GEMM_TILE", "128")
+    q.submit(gemm_cmd(xs, a, b, want, M, N, K, 1))
+    q.wait()
+    q.close()
+    assert torch.equal(got, want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("forced", ["", "128"])
+def test_commands_that_share_the_buffer_flushed_and_replayed(xs, gpu, monkeypatch, forced):
+    """Three products in flight, of different matrices and sizes, whose copies go to the same buffer one
+    after the other: suspended at a random moment and resumed, until one has been flushed in
+    the middle three times. (Forced to 128 x 128 tiles: the same through registers, without copies.)"""
+    from test_gpu_kernels import Queue, gemm_cmd
+    from test_gpu_preempt import hip_stats
+    torch = gpu
+    if forced:
+        monkeypatch.setenv("XSCHED_HIP_GEMM_TILE", forced)
+    print(f"case gemm-copies-flush forced={forced}", flush=True)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(3)
+    products = []
+    for M, N, K in ((3001, 3003, 1001), (4001, 4003, 2047), (2999, 3500, 1500)):
+        a, b = _ints(torch, gen, (M, K), 0), _ints(torch, gen, (K, N), 1)
+        c = torch.zeros(M, N, dtype=torch.bfloat16, device="cuda")
+        assert (plans_of(xs, a.data_ptr(), b.data_ptr(), c.data_ptr(), M, N, K)[1] == []) == bool(forced)
+        products.append((a, b, c, (a.float() @ b.float()).to(torch.bfloat16)))
+    q, p, rnd = Queue(xs, torch, 2), xs.preempt(), random.Random(3)
+
+    def submit():
+        for a, b, c, _ in products:
+            q.submit(gemm_cmd(xs, a, b, c, a.shape[0], b.shape[1], a.shape[1], 1))
+    torch.cuda.synchronize()
+    submit()
+    q.wait()
+    began = time.perf_counter()
+    submit()
+    q.wait()
+    span = time.perf_counter() - began
+    flushed = rounds = 0
+    while flushed < 3 and rounds < 600:
+        rounds += 1
+        for _, _, c, _ in products:
+            c.fill_(float("nan"))
+        torch.cuda.synchronize()
+        submit()
+        until = time.perf_counter() + rnd.uniform(0.0, 1.2 * span)
+        while time.perf_counter() < until:
+            pass
+        xs.check(p.XQueueSuspend(q.xq, xs.kQueueSuspendFlagSyncHwQueue))
+        missing = [torch.isnan(c) for _, _, c, _ in products]
+        some = any(bool(m.any()) and not bool(m.all()) for m in missing)
+        xs.check(p.XQueueResume(q.xq, xs.kQueueResumeFlagNone))
+        q.wait()
+        for i, (_, _, c, want) in enumerate(products):
+            assert torch.equal(c, want), f"product {i}, round {rounds}, flushed in the middle: {some}"
+        flushed += some
+    st = hip_stats(xs, q.hwq)
+    q.close()
+    print("stats", st, "rounds", rounds, "flushed in the middle", flushed, flush=True)
+    assert flushed == 3 and st[1] >= 3
+
+
+@pytest.mark.gpu
+def test_a_captured_product_uses_no_buffer_of_the_queue(xs, gpu):
+    """A graph outlives the command and its queue: under capture the matrices are read where they lie.
+    Replayed three times after the queue is gone, with other work in between."""
+    torch = gpu
+    M, N, K = 3001, 2999, 1001
+    print(f"case gemm-copies-capture M={M} N={N} K={K}", flush=True)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(2)
+    a, b = _ints(torch, gen, (M, K), 0), _ints(torch, gen, (K, N), 0)
+    c = torch.zeros(M, N, dtype=torch.bfloat16, device="cuda")
+    want = (a.float() @ b.float()).to(torch.bfloat16)
+    p, h, stream = xs.preempt(), xs.halhip(), torch.cuda.Stream()
+    hwq = xs.hip_queue_create(stream.cuda_stream)
+
+    def launch():
+        cmd = c_uint64()
+        xs.check(h.HipGemmBf16CommandCreate(byref(cmd), a.data_ptr(), b.data_ptr(), c.data_ptr(), M, N, K, 0))
+        xs.check(p.HwQueueLaunch(hwq, cmd.value))
+    assert plans_of(xs, a.data_ptr(), b.data_ptr(), c.data_ptr(), M, N, K)[1] != []
+    torch.cuda.synchronize()
+    launch()                            # eagerly first: on copies
+    stream.synchronize()
+    assert torch.equal(c, want)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        launch()
+    torch.cuda.synchronize()
+    xs.check(p.HwQueueDestroy(hwq))
+    other = torch.zeros(1 << 26, device="cuda")   # may lie where the queue's buffer was
+    for replay in range(3):
+        c.fill_(float("nan"))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(c, want), f"replay {replay}"
+        other.add_(1.0)
+        torch.cuda.synchronize()
+    assert bool((other == 3.0).all())

@@ -147,6 +147,32 @@ private:
     std::vector<Buffer> buffers_;
 };
 
+/// One device buffer that the commands of a queue use in turn, for data that a command writes and reads
+/// within its own launches. Later commands may write over it: the launches of a queue run one after
+/// the other, and after a work-group has been flushed no later launch of that epoch runs (the
+/// `flushed` word), so what a flushed command has in the buffer is still there for its replay,
+/// which comes before every later command's. A command keeps the buffer of its first launch for its
+/// replays. When a larger one is wanted the old one stays until the queue goes (sizes double, so all
+/// together they are at most twice the largest).
+class SharedScratch
+{
+public:
+    explicit SharedScratch(int device): device_(device) {}
+    ~SharedScratch();
+    /// A buffer of at least `bytes`, or nullptr when the device has no memory for one. Allocates when the
+    /// newest one is smaller; called at submission, so that the call at launch finds one.
+    void *Get(size_t bytes);
+
+private:
+    void *Newest(size_t bytes);
+    static constexpr size_t kLeastBytes = (size_t)16 << 20;
+    const int device_;
+    std::mutex grow_mtx_;            // one allocation at a time
+    std::mutex mtx_;                 // never held across an allocation
+    std::vector<void *> buffers_;
+    size_t newest_bytes_ = 0;
+};
+
 class HipQueue;
 
 class HipCommand : public preempt::HwCommand, public preempt::HwCommandExtension
@@ -291,6 +317,7 @@ public:
     void SetMarkerOnKernel(bool on) { marker_on_kernel_.store(on, std::memory_order_relaxed); }
     const std::shared_ptr<GuardState> &Guard() const { return guard_; }
     const std::shared_ptr<ScratchPool> &Scratch() const { return scratch_; }
+    const std::shared_ptr<class SharedScratch> &SharedScratch() const { return shared_scratch_; }
 
     // statistics (see HipQueueGetStats)
     std::atomic<uint64_t> n_launch { 0 }, n_replay { 0 }, n_deactivate { 0 }, n_reactivate { 0 };
@@ -305,6 +332,7 @@ private:
     std::shared_ptr<GuardState> guard_;
     hipStream_t op_stream_ = nullptr; // flag writes when the word lives in device memory
     std::shared_ptr<ScratchPool> scratch_;
+    std::shared_ptr<class SharedScratch> shared_scratch_;
 
     // The newest command handed to the stream, while it carries a marker that was recorded
     // right behind it: Synchronize() then waits for that marker instead of putting another

@@ -495,6 +495,7 @@ HipQueue::HipQueue(hipStream_t stream): stream_(stream)
     xdevice_ = MakeDevice(kDeviceTypeGPU, MakePciId(prop.pciDomainID, prop.pciBusID, prop.pciDeviceID, 0));
     guard_ = std::make_shared<GuardState>(device_);
     scratch_ = std::make_shared<ScratchPool>(device_);
+    shared_scratch_ = std::make_shared<class SharedScratch>(device_);
     marker_on_kernel_.store(GetEnvOption("XSCHED_HIP_MARKER_ON_KERNEL", true));
     HIP_ASSERT(hipStreamCreateWithFlags(&op_stream_, hipStreamNonBlocking)); // default priority
     // The entry point that allocates nothing needs the address of its static array on this
@@ -603,6 +604,34 @@ size_t ScratchPool::Bytes()
     size_t bytes = 0;
     for (auto &buf : buffers_) bytes += buf.bytes;
     return bytes;
+}
+
+SharedScratch::~SharedScratch()
+{
+    for (void *buf : buffers_) (void)hipFree(buf);
+}
+
+void *SharedScratch::Newest(size_t bytes)
+{
+    std::lock_guard<std::mutex> lock(mtx_);
+    return newest_bytes_ >= bytes ? buffers_.back() : nullptr;
+}
+
+void *SharedScratch::Get(size_t bytes)
+{
+    if (void *ptr = Newest(bytes)) return ptr;
+    std::lock_guard<std::mutex> one_at_a_time(grow_mtx_);
+    if (void *ptr = Newest(bytes)) return ptr;
+    size_t size = kLeastBytes;
+    while (size < bytes) size *= 2;
+    DeviceScope scope(device_);
+    RelaxedCaptureScope relaxed;
+    void *ptr = nullptr;
+    if (hipMalloc(&ptr, size) != hipSuccess) { (void)hipGetLastError(); return nullptr; }
+    std::lock_guard<std::mutex> lock(mtx_);
+    buffers_.push_back(ptr);
+    newest_bytes_ = size;
+    return ptr;
 }
 
 // On the submitting thread, before the XQueue takes any of its locks: a guarded command takes

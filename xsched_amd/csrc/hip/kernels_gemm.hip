@@ -42,6 +42,7 @@
 // transposing reads back), whole rows of 128 bytes per eight lanes.
 // Work-group ids are remapped so that the 32 CUs of one XCD (ids equal modulo 8 land on one
 // XCD) work on neighbouring tiles and share A/B panels in that XCD's L2.
+#include <algorithm>
 #include <cmath>
 #include <type_traits>
 #include <utility>
@@ -112,8 +113,9 @@ __device__ __forceinline__ void TileOf(uint32_t wg, uint32_t tiles_m, uint32_t t
 
 // What the matrices have to be like is kFit:
 //   kExact      M, N multiples of the tile, K of kStepK, matrices aligned to 16 bytes
-//   kEdges      M any; N and K multiples of 8, matrices aligned to 16 bytes: every 16-byte piece
-//               lies inside the matrix or outside. Pieces outside are fetched from somewhere
+//   kEdges      rows of A and B that start on 16-byte boundaries (their lengths in memory, lda and ldb,
+//               are multiples of 8; M, N, K and C are any): a 16-byte piece begins inside the matrix
+//               or lies outside. Pieces outside are fetched from somewhere
 //               inside (their row or column of C is not stored); behind K the fragments are
 //               masked to zero, which adds nothing to a sum
 //   kUnaligned  any N >= 8, any alignment to the element: pieces start at any multiple of two
@@ -136,15 +138,18 @@ __device__ __forceinline__ u32x4 ShiftDownBytes(u32x4 v, uint32_t d)
                    __builtin_amdgcn_alignbyte(v.w, v.z, d & 3), __builtin_amdgcn_alignbyte(0u, v.w, d & 3) };
 }
 
-/// Eight columns of a row of C, as far as they are inside.
+/// Whether rows of C start on 16-byte boundaries (uniform).
+__device__ __forceinline__ bool WholeRowPieces(const uint16_t *C, int N) { return (((uintptr_t)C | (uint32_t)N * 2u) & 15) == 0; }
+
+/// Eight columns of a row of C, as far as they are inside. `whole`: WholeRowPieces().
 template <Fit kFit>
-__device__ __forceinline__ void StoreEight(uint16_t *C, size_t row, size_t col, int M, int N, s16x8 eight)
+__device__ __forceinline__ void StoreEight(uint16_t *C, size_t row, size_t col, int M, int N, bool whole, s16x8 eight)
 {
     uint16_t *const at = C + row * (size_t)N + col;
     if constexpr (kFit == Fit::kExact) {
         __builtin_nontemporal_store(eight, (s16x8 *)at);
     } else if (row < (size_t)M) {
-        if constexpr (kFit == Fit::kEdges) {
+        if (kFit == Fit::kEdges && whole) {
             if (col < (size_t)N) __builtin_nontemporal_store(eight, (s16x8 *)at);
         } else if (col + 8 <= (size_t)N) {
             *(s16x8_any *)at = eight;
@@ -185,7 +190,7 @@ enum TileRequest { kNoTile, kAnyButLast, kTheLast };
 template <bool kGuard, Fit kFit, int kTile, int kWavesM, int kWavesN>
 __device__ __forceinline__
 void GemmBf16Body(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B,
-                  uint16_t *__restrict__ C, int M, int N, int K, const XGuardArgs &g)
+                  uint16_t *__restrict__ C, int M, int N, int K, int lda, int ldb, const XGuardArgs &g)
 {
     static_assert(kFit != Fit::kUnaligned, "loads go straight into LDS");
     constexpr int kWaves = kWavesM * kWavesN;
@@ -234,16 +239,16 @@ void GemmBf16Body(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
     for (int i = 0; i < kALoads; ++i) {
         uint32_t row = 2 * (4 * (wave * kALoads + i) + (lane >> 4)) + ((lane >> 3) & 1);
         if (kFit != Fit::kExact && m0 + row >= (size_t)M) row = (uint32_t)((size_t)M - 1 - m0);   // not stored
-        a_off[i] = (row * (uint32_t)K + a_k(i)) * 2;
+        a_off[i] = (row * (uint32_t)lda + a_k(i)) * 2;
     }
 #pragma unroll
     for (int i = 0; i < kBLoads; ++i) {
         const uint32_t k = b_k(i), slot = lane % kBSlotsPerRow;
         uint32_t col = ((slot >> 1) ^ ((k & 3) << 1 | ((k >> 3) & 1))) * 16 + (slot & 1) * 8;
         if (kFit != Fit::kExact && n0 + col >= (size_t)N) col = 0;                                // not stored
-        b_off[i] = (k * (uint32_t)N + col) * 2;
+        b_off[i] = (k * (uint32_t)ldb + col) * 2;
     }
-    const uint16_t *const a_tile = A + m0 * (size_t)K;   // + 64 columns per step
+    const uint16_t *const a_tile = A + m0 * (size_t)lda;   // + 64 columns per step
     const uint16_t *const b_tile = B + n0;               // + 64 rows per step
 
     // Byte offset of load number idx (A first, then B) within its matrix's part of a K step. In the
@@ -256,7 +261,7 @@ void GemmBf16Body(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
         }
         if (kFit == Fit::kExact || !last) return b_off[idx - kALoads];
         const uint32_t k = b_k(idx - kALoads);
-        return k < (uint32_t)rest ? b_off[idx - kALoads] : b_off[idx - kALoads] - k * (uint32_t)N * 2;
+        return k < (uint32_t)rest ? b_off[idx - kALoads] : b_off[idx - kALoads] - k * (uint32_t)ldb * 2;
     };
     // Load number idx of the tile of K step `step` into buffer `buf`.
     auto load_piece = [&](int buf, int step, int idx, bool last) {
@@ -265,7 +270,7 @@ void GemmBf16Body(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
             __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (LdsVoid *)(As0 + buf * kABytes + (wave * kALoads + idx) * 1024), 16, piece_off(idx, last), 0, 0, 0);
         } else {
             const int i = idx - kALoads;
-            const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void *)(b_tile + (size_t)step * kStepK * N), 0, 0x7fffffff, 0x00020000);
+            const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void *)(b_tile + (size_t)step * kStepK * ldb), 0, 0x7fffffff, 0x00020000);
             __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (LdsVoid *)(Bs0 + buf * kBBytes + (wave * kBLoads + i) * 1024), 16, piece_off(idx, last), 0, 0, 0);
         }
     };
@@ -446,6 +451,7 @@ void GemmBf16Body(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
     uint8_t *const strip = As0 + wave * kStripBytes;
     const uint32_t l16 = lane & 15, patch = lane >> 4;   // a patch: 4 rows x 32 columns per 16 lanes
     const uint32_t put_at = l16 * kStripColumnBytes + 4 * patch * 2;
+    const bool whole = WholeRowPieces(C, N);
     const uint32_t get_row = 4 * (patch >> 1), get_col = 32 * (patch & 1);
     const uint32_t get_at = (get_col + 8 * (l16 & 3) + (l16 >> 2)) * kStripColumnBytes + get_row * 2;
 #pragma unroll
@@ -469,7 +475,7 @@ void GemmBf16Body(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
             const s16x8 row = __builtin_shufflevector(left, right, 0, 1, 2, 3, 4, 5, 6, 7);
             // (non-temporal: C is written once and not read again; left in L2 it pushes out A and B panels
             // that the XCD's other tiles still need: 1 % of the kernel)
-            StoreEight<kFit>(C, row0 + 8 * q + get_row + (l16 & 3), col0, M, N, row);
+            StoreEight<kFit>(C, row0 + 8 * q + get_row + (l16 & 3), col0, M, N, whole, row);
         }
     }
 
@@ -482,9 +488,9 @@ void GemmBf16Body(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
 template <bool kGuard, Fit kFit, int kTile, int kWavesM, int kWavesN>
 __global__ __launch_bounds__(64 * kWavesM * kWavesN, 2 /* waves per SIMD: no accumulators move between AGPRs and VGPRs */)
 void GemmBf16Kernel(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B,
-                    uint16_t *__restrict__ C, int M, int N, int K, XGuardArgs g)
+                    uint16_t *__restrict__ C, int M, int N, int K, int lda, int ldb, XGuardArgs g)
 {
-    GemmBf16Body<kGuard, kFit, kTile, kWavesM, kWavesN>(A, B, C, M, N, K, g);
+    GemmBf16Body<kGuard, kFit, kTile, kWavesM, kWavesN>(A, B, C, M, N, K, lda, ldb, g);
 }
 
 
@@ -542,7 +548,7 @@ __device__ __forceinline__ void WaitNewer(int newer)
 template <bool kGuard, Fit kFit, int kTile, int kStages>
 __device__ __forceinline__
 void GemmDeepBody(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B,
-                  uint16_t *__restrict__ C, int M, int N, int K, const XGuardArgs &g)
+                  uint16_t *__restrict__ C, int M, int N, int K, int lda, int ldb, const XGuardArgs &g)
 {
     constexpr bool kDirect = kFit != Fit::kUnaligned;      // loads go straight into LDS
     constexpr int kWaves = 4;
@@ -589,7 +595,7 @@ void GemmDeepBody(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
         uint32_t row = 2 * line + (piece >> 3);
         const uint32_t kc = piece & 7;
         if (kFit != Fit::kExact && m0 + row >= (size_t)M) row = (uint32_t)((size_t)M - 1 - m0);
-        off[i] = (row * (uint32_t)K + kc * 8) * 2;
+        off[i] = (row * (uint32_t)lda + kc * 8) * 2;
         k_of[i] = kc * 8;
     }
 #pragma unroll
@@ -600,16 +606,16 @@ void GemmDeepBody(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
         const uint32_t swz = kTile == 64 ? (k >> 1) & 1 : k & 3;
         uint32_t col = ((slot >> 2) ^ swz) * 32 + (slot & 3) * 8;
         if (kFit != Fit::kExact && n0 + col >= (size_t)N) col = 0;
-        off[kHalfLoads + i] = (k * (uint32_t)N + col) * 2;
+        off[kHalfLoads + i] = (k * (uint32_t)ldb + col) * 2;
         k_of[kHalfLoads + i] = k;
     }
-    const uint16_t *const a_tile = A + m0 * (size_t)K;     // + kStepK columns per step
+    const uint16_t *const a_tile = A + m0 * (size_t)lda;     // + kStepK columns per step
     const uint16_t *const b_tile = B + n0;                 // + kStepK rows per step
 
     // Offset of piece idx in the last step: pieces behind K come from k = 0 of the step instead.
     auto last_off = [&](int idx) -> uint32_t {
         if (kFit == Fit::kExact || k_of[idx] < (uint32_t)rest) return off[idx];
-        return idx < kHalfLoads ? off[idx] - k_of[idx] * 2 : off[idx] - k_of[idx] * (uint32_t)N * 2;
+        return idx < kHalfLoads ? off[idx] - k_of[idx] * 2 : off[idx] - k_of[idx] * (uint32_t)ldb * 2;
     };
     auto load_direct = [&](int step, int idx, uint32_t at) {
         const int buf = step & (kBuffers - 1);
@@ -617,7 +623,7 @@ void GemmDeepBody(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
             const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void *)(a_tile + (size_t)step * kStepK), 0, 0x7fffffff, 0x00020000);
             __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (LdsVoid *)(As0 + buf * kTileBytes + (wave * kHalfLoads + idx) * 1024), 16, at, 0, 0, 0);
         } else {
-            const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void *)(b_tile + (size_t)step * kStepK * N), 0, 0x7fffffff, 0x00020000);
+            const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void *)(b_tile + (size_t)step * kStepK * ldb), 0, 0x7fffffff, 0x00020000);
             __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (LdsVoid *)(Bs0 + buf * kTileBytes + (wave * kHalfLoads + idx - kHalfLoads) * 1024), 16, at, 0, 0, 0);
         }
     };
@@ -625,12 +631,12 @@ void GemmDeepBody(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
     u32x4 held[kDirect ? 1 : kRegTiles][kDirect ? 1 : kLoads];
     auto load_held = [&](int set, int step, int idx) {
         const uint8_t *base = idx < kHalfLoads ? (const uint8_t *)(a_tile + (size_t)step * kStepK)
-                                               : (const uint8_t *)(b_tile + (size_t)step * kStepK * N);
+                                               : (const uint8_t *)(b_tile + (size_t)step * kStepK * ldb);
         held[set][idx] = *(const u32x4_any *)(base + off[idx]);
     };
     auto load_held_last = [&](int set, int step, int idx) {
         const uint8_t *base = idx < kHalfLoads ? (const uint8_t *)(a_tile + (size_t)step * kStepK)
-                                               : (const uint8_t *)(b_tile + (size_t)step * kStepK * N);
+                                               : (const uint8_t *)(b_tile + (size_t)step * kStepK * ldb);
         const uint8_t *const end = idx < kHalfLoads ? (const uint8_t *)(A + (size_t)M * K) : (const uint8_t *)(B + (size_t)K * N);
         // A piece that would reach behind the matrix is fetched from its last 16 bytes instead and
         // shifted into place; what is then missing lies behind K or in columns behind N.
@@ -878,6 +884,7 @@ void GemmDeepBody(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
     const uint32_t put_at = (lane & 31) * kStripColumnBytes + 4 * (lane >> 5) * 2;
     const uint32_t l16 = lane & 15, patch = lane >> 4;     // a patch: 4 rows x 32 columns per 16 lanes
     constexpr int kRowsPerStore = 16 / kBlocks;
+    const bool whole = WholeRowPieces(C, N);
     const uint32_t get_row = 4 * (patch / kBlocks), get_col = 32 * (patch % kBlocks);
     const uint32_t get_at = (get_col + 8 * (l16 & 3) + (l16 >> 2)) * kStripColumnBytes + get_row * 2;
 #pragma unroll
@@ -900,7 +907,7 @@ void GemmDeepBody(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
             const s16x4 right = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsS16x4 *)(p + 4 * kStripColumnBytes));
             const s16x8 eight = __builtin_shufflevector(left, right, 0, 1, 2, 3, 4, 5, 6, 7);
             const size_t row = row0 + kRowsPerStore * q + get_row + (l16 & 3);
-            StoreEight<kFit>(C, row, col0, M, N, eight);
+            StoreEight<kFit>(C, row, col0, M, N, whole, eight);
         }
     }
 
@@ -914,9 +921,9 @@ void GemmDeepBody(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
 template <bool kGuard, Fit kFit, int kTile, int kStages>
 __global__ __launch_bounds__(256)
 void GemmDeepKernel(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B,
-                    uint16_t *__restrict__ C, int M, int N, int K, XGuardArgs g)
+                    uint16_t *__restrict__ C, int M, int N, int K, int lda, int ldb, XGuardArgs g)
 {
-    GemmDeepBody<kGuard, kFit, kTile, kStages>(A, B, C, M, N, K, g);
+    GemmDeepBody<kGuard, kFit, kTile, kStages>(A, B, C, M, N, K, lda, ldb, g);
 }
 
 
@@ -1007,6 +1014,56 @@ void GemmBf16AnyShapeKernel(const uint16_t *__restrict__ A, const uint16_t *__re
     if (kGuard) guard.Commit();
 }
 
+/// A matrix that is copied to rows on 16-byte boundaries: `rows` rows of `cols` elements, one after
+/// the other from `from` on, to rows of `ld` (a multiple of 8) from `to` on. The elements of `to`
+/// between cols and ld take whatever follows in memory: nothing depends on them (kEdges).
+struct RowCopy
+{
+    const uint16_t *from;
+    uint16_t *to;
+    uint32_t rows, cols, ld;
+    uint32_t groups;   // work-groups that copy it, 0: it stays where it is
+};
+constexpr uint32_t kCopyThreads = 256;
+constexpr uint32_t kCopyPieces = 4;    // 16-byte pieces per thread, all on their way at once
+inline uint32_t CopyGroups(uint64_t rows, uint64_t ld) { return (uint32_t)((rows * (ld / 8) + kCopyThreads * kCopyPieces - 1) / (kCopyThreads * kCopyPieces)); }
+
+/// Copies A, B or both in one launch, for kernels whose loads go straight into LDS. Bound by memory: each
+/// element is read and written once (the pieces are read at any multiple of two bytes, which memory
+/// does not mind). The guard is at entry only: a group copies 16 KiB.
+template <bool kGuard>
+__global__ __launch_bounds__(kCopyThreads)
+void CopyRowsKernel(RowCopy a, RowCopy b, XGuardArgs g)
+{
+    __shared__ uint32_t guard_word;
+    const bool second = blockIdx.x >= a.groups;
+    const RowCopy &m = second ? b : a;
+    const uint32_t pieces_per_row = m.ld / 8, pieces = m.rows * pieces_per_row;   // (at most 2^26: PlanFor)
+    const uint32_t first = (blockIdx.x - (second ? a.groups : 0)) * (kCopyThreads * kCopyPieces) + threadIdx.x;
+    const size_t last = (size_t)m.rows * m.cols - 8;   // first element of the matrix's last 16 bytes
+    u32x4 v[kCopyPieces];
+    uint32_t d[kCopyPieces];
+    // (requested before the guard's reads, so that the round trips overlap)
+#pragma unroll
+    for (uint32_t u = 0; u < kCopyPieces; ++u) {
+        const uint32_t p = min(first + u * kCopyThreads, pieces - 1);
+        const uint32_t row = p / pieces_per_row;
+        const size_t at = (size_t)row * m.cols + (p - row * pieces_per_row) * 8;
+        // a piece that would reach behind the matrix: its last 16 bytes, shifted into place
+        const size_t inside = at < last ? at : last;
+        v[u] = *(const u32x4_any *)(m.from + inside);
+        d[u] = (uint32_t)(at - inside) * 2;
+    }
+    XGuardBlock guard(g, blockIdx.x, &guard_word);
+    if (kGuard && !guard.Enter()) return;
+#pragma unroll
+    for (uint32_t u = 0; u < kCopyPieces; ++u) {
+        const uint32_t p = first + u * kCopyThreads;
+        if (p < pieces) *(u32x4 *)(m.to + (size_t)p * 8) = ShiftDownBytes(v[u], d[u]);   // rows of ld elements follow each other: piece p is p * 16 bytes on
+    }
+    if (kGuard) guard.Commit();
+}
+
 /// kTwoBuffers is GemmBf16Kernel, kFourStages GemmDeepKernel, kAnyShape GemmBf16AnyShapeKernel.
 enum class Body { kTwoBuffers, kFourStages, kAnyShape };
 
@@ -1029,34 +1086,82 @@ struct Plan
     uint64_t Tiles() const { return part[0].tiles + (parts > 1 ? part[1].tiles : 0); }
 };
 
+/// A plan for copies of A, B or both with rows on 16-byte boundaries, if that is quicker (else no parts).
+struct CopyPlan
+{
+    Plan plan {};
+    int lda = 0, ldb = 0;                  // of what the plan's kernels read
+    uint32_t a_groups = 0, b_groups = 0;   // work-groups that copy (0: the matrix stays where it is)
+    size_t a_bytes = 0, b_bytes = 0;
+    uint64_t Groups() const { return (uint64_t)a_groups + b_groups + plan.Tiles(); }
+};
+
 class HipGemmCommand final : public HipGuardedCommand
 {
 public:
-    HipGemmCommand(const void *A, const void *B, void *C, int N, int K, const Plan &plan, int guard_mode)
-        : HipGuardedCommand((uint32_t)plan.Tiles(), guard_mode)
-        , A_((const uint16_t *)A), B_((const uint16_t *)B), C_((uint16_t *)C), N_(N), K_(K), plan_(plan) {}
+    HipGemmCommand(const void *A, const void *B, void *C, int M, int N, int K, const Plan &plan, const CopyPlan &copies, int guard_mode)
+        : HipGuardedCommand((uint32_t)std::max(plan.Tiles(), copies.Groups()), guard_mode)
+        , A_((const uint16_t *)A), B_((const uint16_t *)B), C_((uint16_t *)C), M_(M), N_(N), K_(K), plan_(plan), copies_(copies) {}
 
 protected:
+    virtual void ReserveOnSubmit(HipQueue &q) override
+    {
+        if (copies_.plan.parts != 0 && !decided_) (void)q.SharedScratch()->Get(copies_.a_bytes + copies_.b_bytes);
+    }
+
+    /// Where the copies go is decided at the first launch: every replay takes the same way.
+    virtual hipError_t PrepareLaunch(HipQueue &q) override
+    {
+        if (copies_.plan.parts == 0 || decided_) return hipSuccess;
+        decided_ = true;
+        // A graph outlives the command and its queue: what is captured reads A and B themselves.
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(q.Stream(), &capture) != hipSuccess) (void)hipGetLastError();
+        if (capture != hipStreamCaptureStatusNone) return hipSuccess;
+        scratch_ = q.SharedScratch();
+        at_ = (uint8_t *)scratch_->Get(copies_.a_bytes + copies_.b_bytes);   // nullptr: no memory, in place
+        return hipSuccess;
+    }
+
     virtual hipError_t LaunchKernel(hipStream_t stream, bool guarded, const XGuardArgs &g) override
     {
         const hipEvent_t stop = TakeStopEvent();   // for the command's last kernel
-        if (plan_.parts == 1) return LaunchPart(plan_.part[0], stop, stream, guarded, g);
-        const hipError_t err = LaunchPart(plan_.part[0], nullptr, stream, guarded, g);
+        if (at_ == nullptr) return LaunchPlan(plan_, A_, B_, K_, N_, stop, stream, guarded, g);
+        const CopyPlan &c = copies_;
+        const RowCopy a { A_, (uint16_t *)at_, (uint32_t)M_, (uint32_t)K_, (uint32_t)c.lda, c.a_groups };
+        const RowCopy b { B_, (uint16_t *)(at_ + c.a_bytes), (uint32_t)K_, (uint32_t)N_, (uint32_t)c.ldb, c.b_groups };
+        LaunchWithStop(nullptr, guarded ? CopyRowsKernel<true> : CopyRowsKernel<false>, dim3(c.a_groups + c.b_groups), dim3(kCopyThreads), stream, a, b, g);
+        const hipError_t err = hipGetLastError();
         if (err != hipSuccess) return err;
-        // the second part's progress bytes follow the first part's
-        XGuardArgs behind = g;
-        if (behind.done != nullptr) behind.done += plan_.part[0].tiles;
-        return LaunchPart(plan_.part[1], stop, stream, guarded, behind);
+        return LaunchPlan(c.plan, c.a_groups != 0 ? a.to : A_, c.b_groups != 0 ? b.to : B_, c.lda, c.ldb, stop, stream, guarded, Behind(g, c.a_groups + c.b_groups));
     }
 
 private:
-    hipError_t LaunchPart(const Part &part, hipEvent_t stop, hipStream_t stream, bool guarded, const XGuardArgs &g)
+    /// The guard of a launch whose progress bytes follow those of `groups` work-groups.
+    static XGuardArgs Behind(const XGuardArgs &g, uint64_t groups)
     {
+        XGuardArgs behind = g;
+        if (behind.done != nullptr) behind.done += groups;
+        return behind;
+    }
+
+    hipError_t LaunchPlan(const Plan &plan, const uint16_t *A, const uint16_t *B, int lda, int ldb, hipEvent_t stop, hipStream_t stream, bool guarded, const XGuardArgs &g)
+    {
+        if (plan.parts == 1) return LaunchPart(plan.part[0], A, B, lda, ldb, stop, stream, guarded, g);
+        const hipError_t err = LaunchPart(plan.part[0], A, B, lda, ldb, nullptr, stream, guarded, g);
+        if (err != hipSuccess) return err;
+        return LaunchPart(plan.part[1], A, B, lda, ldb, stop, stream, guarded, Behind(g, plan.part[0].tiles));
+    }
+
+    hipError_t LaunchPart(const Part &part, const uint16_t *A, const uint16_t *B, int lda, int ldb, hipEvent_t stop, hipStream_t stream, bool guarded, const XGuardArgs &g)
+    {
+        const uint16_t *const a = A + (size_t)part.first_row * lda;
+        uint16_t *const c = C_ + (size_t)part.first_row * N_;
         if (part.body == Body::kAnyShape) {
             const uint32_t tiles_n = (uint32_t)((N_ + kAnyTile - 1) / kAnyTile);
             const dim3 grid((uint32_t)part.tiles), block(256);
             LaunchWithStop(stop, guarded ? GemmBf16AnyShapeKernel<true> : GemmBf16AnyShapeKernel<false>, grid, block, stream,
-                           A_ + (size_t)part.first_row * K_, B_, C_ + (size_t)part.first_row * N_, part.rows, N_, K_, tiles_n, g);
+                           a, B, c, part.rows, N_, K_, tiles_n, g);
             return hipGetLastError();
         }
         Kernel kernel = nullptr;
@@ -1066,11 +1171,11 @@ private:
         case Fit::kUnaligned: kernel = KernelFor<Fit::kUnaligned>(part, guarded); break;   // (never large)
         }
         LaunchWithStop(stop, kernel, dim3((uint32_t)part.tiles), dim3(part.tile == kLargeTile ? 512 : 256), stream,
-                       A_ + (size_t)part.first_row * K_, B_, C_ + (size_t)part.first_row * N_, part.rows, N_, K_, g);
+                       a, B, c, part.rows, N_, K_, lda, ldb, g);
         return hipGetLastError();
     }
 
-    using Kernel = void (*)(const uint16_t *, const uint16_t *, uint16_t *, int, int, int, XGuardArgs);
+    using Kernel = void (*)(const uint16_t *, const uint16_t *, uint16_t *, int, int, int, int, int, XGuardArgs);
     template <Fit kFit>
     static Kernel KernelFor(const Part &part, bool guarded)
     {
@@ -1086,8 +1191,12 @@ private:
 
     const uint16_t *A_, *B_;
     uint16_t *C_;
-    const int N_, K_;
-    const Plan plan_;
+    const int M_, N_, K_;
+    const Plan plan_;         // for A and B as they lie
+    const CopyPlan copies_;   // for their copies
+    std::shared_ptr<class SharedScratch> scratch_;
+    uint8_t *at_ = nullptr;   // the copies, A's first; nullptr: plan_
+    bool decided_ = false;
 };
 
 inline uint64_t TilesOf(int M, int N, int tile)
@@ -1105,10 +1214,9 @@ inline uint32_t ComputeUnits()
     return cus;
 }
 
-inline bool Aligned(const void *A, const void *B, const void *C, int N, int K)
-{
-    return (((uintptr_t)A | (uintptr_t)B | (uintptr_t)C) & 15) == 0 && N % 8 == 0 && K % 8 == 0;
-}
+/// Whether the rows of a matrix of `cols` columns start on 16-byte boundaries.
+inline bool Aligned(const void *matrix, int cols) { return ((uintptr_t)matrix & 15) == 0 && cols % 8 == 0; }
+inline bool Aligned(const void *A, const void *B, const void *C, int N, int K) { return Aligned(A, K) && Aligned(B, N) && Aligned(C, N); }
 
 /// XSCHED_HIP_GEMM_TILE: 64, 128 or 256, else 0.
 inline int ForcedTile()
@@ -1118,24 +1226,27 @@ inline int ForcedTile()
     return forced == kTinyTile || forced == kSmallTile || forced == kLargeTile ? (int)forced : 0;
 }
 
-inline Part PartOf(int first_row, int rows, int N, int K, bool aligned, int tile)
+/// What a plan may assume: rows of A and B (or of their copies), and rows of C, start on 16-byte boundaries.
+struct Rows { bool inputs, output; };
+
+inline Part PartOf(int first_row, int rows, int N, int K, Rows aligned, int tile)
 {
-    const bool exact = aligned && rows % tile == 0 && N % tile == 0 && K % kStepK == 0;
-    return Part { first_row, rows, tile, exact ? Fit::kExact : aligned ? Fit::kEdges : Fit::kUnaligned,
+    const bool exact = aligned.inputs && aligned.output && rows % tile == 0 && N % tile == 0 && K % kStepK == 0;
+    return Part { first_row, rows, tile, exact ? Fit::kExact : aligned.inputs ? Fit::kEdges : Fit::kUnaligned,
                   tile == kLargeTile ? Body::kTwoBuffers : Body::kFourStages, TilesOf(rows, N, tile) };
 }
 
 /// Roughly how long a part takes, in us: a launch, then rounds of one tile per compute unit (two of
 /// 128 x 128 with two buffers), each with its first loads and its write-out, the last round quicker the fewer
-/// units it keeps busy. The rates are fitted to 23 outputs of 64 to 1600 tiles of 128 x 128 at eleven K from
-/// 64 to 8192: what it picks there takes 0.9 % longer on average than the quickest, 23 % at worst
-/// (1024 x 2048 x 8192 on tiny tiles), and at most 7 % longer than the quicker of the two kernels with two buffers.
+/// units it keeps busy. The rates are fitted to outputs of 4 to 4096 tiles of 128 x 128 at K from 128 to 8192:
+/// of 35 such products the plan is within 3 % of the quickest of the three tile sizes but for
+/// 2048 x 2048 x 8192 (66.3 us, 63.9 with the tile given) and 4096 x 4096 x 128 (11.4, 10.5).
 inline double MicrosOf(const Part &part, int K)
 {
     // us of a round, and per K step of a full round and of one with a single tile: [exact, edges, unaligned]
     struct Rates { double round, full, single; };
-    constexpr Rates large[3] = { { 4.0, 1.54, 0.95 }, { 4.0, 1.56, 0.97 }, {} };
-    constexpr Rates pair = { 1.5, 0.95, 0.45 };
+    constexpr Rates large[3] = { { 5.0, 1.36, 1.00 }, { 5.0, 1.43, 1.05 }, {} };
+    constexpr Rates pair = { 1.7, 0.90, 0.45 };
     constexpr Rates small[3] = { { 2.5, 0.45, 0.37 }, { 2.5, 0.53, 0.41 }, { 2.5, 0.80, 0.60 } };
     constexpr Rates tiny[3] = { { 0.5, 0.195, 0.14 }, { 0.5, 0.25, 0.16 }, { 0.5, 0.35, 0.25 } };
     const bool two_per_unit = part.tile == kSmallTile && part.body == Body::kTwoBuffers;
@@ -1143,6 +1254,13 @@ inline double MicrosOf(const Part &part, int K)
     const double rounds = (double)part.tiles / ((two_per_unit ? 2 : 1) * ComputeUnits()), whole = std::floor(rounds);
     const double step = whole * r.full + (rounds > whole ? r.single + (r.full - r.single) * (rounds - whole) : 0.0);
     return 3.0 + std::ceil(rounds) * r.round + step * ((K + kStepK - 1) / kStepK);
+}
+
+inline double MicrosOf(const Plan &plan, int K)
+{
+    double us = 0.0;
+    for (int i = 0; i < plan.parts; ++i) us += MicrosOf(plan.part[i], K);
+    return us;
 }
 
 /// Whether K is so short that the any-shape kernel is the quickest: up to 32, one step of it;
@@ -1192,13 +1310,8 @@ inline bool ShortK(const void *A, const void *B, const void *C, int M, int N, in
 /// XSCHED_HIP_GEMM_TILE=64|128|256 overrides the tile where the shape allows (128: four stages).
 /// A plan of more tiles than the progress map holds is passed over for one that fits: 13413745 x
 /// 1280 x 1024, 262025 tiles by the count below, would be quickest as two launches of 262295.
-inline Plan PlanFor(const void *A, const void *B, const void *C, int M, int N, int K, int forced)
+inline Plan QuickestPlan(int M, int N, int K, Rows aligned)
 {
-    const Plan any_shape { { Part { 0, M, kAnyTile, Fit::kUnaligned, Body::kAnyShape, TilesOf(M, N, kAnyTile) }, {} }, 1 };
-    if (N < 8 || (int64_t)M * K < 8 || K > kMaxK || N > kMaxK) return any_shape;
-    const bool aligned = Aligned(A, B, C, N, K);
-    if (forced == 0 && ShortK(A, B, C, M, N, K)) return any_shape;
-    if (forced != 0 && (forced != kLargeTile || aligned)) return Plan { { PartOf(0, M, N, K, aligned, forced), {} }, 1 };
     auto best_part = [&](int first_row, int rows) {
         Part best = PartOf(first_row, rows, N, K, aligned, kSmallTile);
         if (best.fit == Fit::kExact) {
@@ -1207,7 +1320,7 @@ inline Plan PlanFor(const void *A, const void *B, const void *C, int M, int N, i
             if (MicrosOf(two_per_unit, K) < MicrosOf(best, K)) best = two_per_unit;
         }
         for (const int tile : { kTinyTile, kLargeTile }) {
-            if (tile == kLargeTile && !aligned) continue;
+            if (tile == kLargeTile && !aligned.inputs) continue;
             const Part other = PartOf(first_row, rows, N, K, aligned, tile);
             const bool fits = other.tiles <= GuardState::kMaxWorkGroups, best_fits = best.tiles <= GuardState::kMaxWorkGroups;
             if (fits && (!best_fits || MicrosOf(other, K) < MicrosOf(best, K))) best = other;
@@ -1217,7 +1330,7 @@ inline Plan PlanFor(const void *A, const void *B, const void *C, int M, int N, i
     Plan best { { best_part(0, M), {} }, 1 };
     double least = MicrosOf(best.part[0], K);
     auto consider = [&](int64_t large_rows) {
-        if (!aligned || large_rows <= 0 || large_rows >= M) return;
+        if (!aligned.inputs || large_rows <= 0 || large_rows >= M) return;
         const Part first = PartOf(0, (int)large_rows, N, K, aligned, kLargeTile), rest = best_part((int)large_rows, M - (int)large_rows);
         const double both = MicrosOf(first, K) + MicrosOf(rest, K);
         if (first.tiles + rest.tiles > GuardState::kMaxWorkGroups) return;
@@ -1228,6 +1341,48 @@ inline Plan PlanFor(const void *A, const void *B, const void *C, int M, int N, i
     const int64_t whole_rounds = (int64_t)TilesOf(M, N, kLargeTile) / ComputeUnits();
     consider(whole_rounds * ComputeUnits() / in_row * kLargeTile);
     return best;
+}
+
+/// The plan for the matrices as they lie.
+inline Plan PlanFor(const void *A, const void *B, const void *C, int M, int N, int K, int forced)
+{
+    const Plan any_shape { { Part { 0, M, kAnyTile, Fit::kUnaligned, Body::kAnyShape, TilesOf(M, N, kAnyTile) }, {} }, 1 };
+    if (N < 8 || (int64_t)M * K < 8 || K > kMaxK || N > kMaxK) return any_shape;
+    if (forced == 0 && ShortK(A, B, C, M, N, K)) return any_shape;
+    const Rows aligned { Aligned(A, K) && Aligned(B, N), Aligned(C, N) };
+    if (forced != 0 && (forced != kLargeTile || aligned.inputs)) return Plan { { PartOf(0, M, N, K, aligned, forced), {} }, 1 };
+    return QuickestPlan(M, N, K, aligned);
+}
+
+constexpr size_t kMaxCopyBytes = (size_t)1 << 30;   // of A and B together
+constexpr double kCopyMicros = 4.5;                 // launch of the copying kernel, and its bytes per us, read and written
+constexpr double kCopyRate = 5.9e6;
+
+/// The plan for copies of whichever of A and B has rows off 16-byte boundaries; no parts where `in_place` is
+/// as quick, or where the copies are too large. Through registers a step waits for loads at any multiple of two
+/// bytes (0.7 us against 0.45 for 128 x 128 tiles of 64 k), and large tiles do not fit; the copies cost
+/// their launch and two passes over the matrices (8191^2 elements 87 us = 6.2 TB/s with what is
+/// written, 2000 x 2047 and 2047 x 1999 together 9.5). Rows of the copies are whole 128-byte lines (rows of 2000 and
+/// 2048 elements rather than of 2048: 27 us for the 2000 x 1999 x 2047 that takes 23.5). us per command,
+/// in place / on copies: 500 x 499 x 4095 26.5 / 24.7, x 2047 13.7 / 15.8; 1500 x 1499 x 4095 49.5 / 40.0, x 1001
+/// 18.1 / 21.2; 2000 x 1999 x 2047 31.3 / 31.7, x 4095 53.6 / 46.5; 3000 x 2999 x 301 31.6 / 26.9, x 101 25.3 / 21.6;
+/// 4000 x 3999 x 2047 118.5 / 70.4; 128 x 8191 x 8191 50.7 / 76.2. A pass of 8191^3 1791 / 918.
+inline CopyPlan CopyPlanFor(const void *A, const void *B, const void *C, int M, int N, int K, int forced, const Plan &in_place)
+{
+    CopyPlan p;
+    const bool copy_a = !Aligned(A, K), copy_b = !Aligned(B, N);
+    if (forced != 0 || in_place.part[0].body == Body::kAnyShape || !(copy_a || copy_b)) return p;
+    p.lda = copy_a ? (K + 63) / 64 * 64 : K;
+    p.ldb = copy_b ? (N + 63) / 64 * 64 : N;
+    p.a_bytes = copy_a ? (size_t)M * p.lda * 2 : 0;
+    p.b_bytes = copy_b ? (size_t)K * p.ldb * 2 : 0;
+    if (p.a_bytes + p.b_bytes > kMaxCopyBytes || K > kMaxK - 64 || N > kMaxK - 64) return CopyPlan {};
+    p.a_groups = copy_a ? CopyGroups(M, p.lda) : 0;
+    p.b_groups = copy_b ? CopyGroups(K, p.ldb) : 0;
+    p.plan = QuickestPlan(M, N, K, Rows { true, Aligned(C, N) });
+    if (p.Groups() > GuardState::kMaxWorkGroups) return CopyPlan {};
+    const double copying = kCopyMicros + 2.0 * (double)(p.a_bytes + p.b_bytes) / kCopyRate;
+    return copying + MicrosOf(p.plan, K) < MicrosOf(in_place, K) ? p : CopyPlan {};
 }
 
 /// Tiles by which a shape is accepted or refused. They are the tiles of the kernels that such shapes
@@ -1249,10 +1404,8 @@ inline uint64_t CountedTiles(const void *A, const void *B, const void *C, int M,
 
 using namespace xsched::hip;
 
-EXPORT_C_FUNC XResult HipGemmBf16PlanOf(const void *A, const void *B, const void *C, int M, int N, int K, int32_t *out)
+static void PutParts(const gemm::Plan &plan, int32_t *out)
 {
-    if (out == nullptr || M <= 0 || N <= 0 || K <= 0) return kXSchedErrorInvalidValue;
-    const gemm::Plan plan = gemm::PlanFor(A, B, C, M, N, K, gemm::ForcedTile());
     for (int i = 0; i < 8; ++i) out[i] = 0;
     for (int i = 0; i < plan.parts; ++i) {
         const gemm::Part &part = plan.part[i];
@@ -1261,6 +1414,23 @@ EXPORT_C_FUNC XResult HipGemmBf16PlanOf(const void *A, const void *B, const void
         out[4 * i + 2] = (int32_t)part.body;
         out[4 * i + 3] = (int32_t)part.fit;
     }
+}
+
+EXPORT_C_FUNC XResult HipGemmBf16PlanOf(const void *A, const void *B, const void *C, int M, int N, int K, int32_t *out)
+{
+    if (out == nullptr || M <= 0 || N <= 0 || K <= 0) return kXSchedErrorInvalidValue;
+    PutParts(gemm::PlanFor(A, B, C, M, N, K, gemm::ForcedTile()), out);
+    return kXSchedSuccess;
+}
+
+EXPORT_C_FUNC XResult HipGemmBf16CopyPlanOf(const void *A, const void *B, const void *C, int M, int N, int K, int32_t *out)
+{
+    if (out == nullptr || M <= 0 || N <= 0 || K <= 0) return kXSchedErrorInvalidValue;
+    const int forced = gemm::ForcedTile();
+    const gemm::CopyPlan copies = gemm::CopyPlanFor(A, B, C, M, N, K, forced, gemm::PlanFor(A, B, C, M, N, K, forced));
+    PutParts(copies.plan, out);
+    out[8] = (int32_t)copies.a_groups;
+    out[9] = (int32_t)copies.b_groups;
     return kXSchedSuccess;
 }
 
@@ -1281,6 +1451,6 @@ EXPORT_C_FUNC XResult HipGemmBf16CommandCreate(HwCommandHandle *cmd, const void 
         XWARN("HipGemmBf16CommandCreate: %d x %d needs more than 2^18 tiles", M, N);
         return kXSchedErrorInvalidValue;
     }
-    *cmd = HwCommandManager::Add(std::make_shared<gemm::HipGemmCommand>(A, B, C, N, K, plan, guard));
+    *cmd = HwCommandManager::Add(std::make_shared<gemm::HipGemmCommand>(A, B, C, M, N, K, plan, gemm::CopyPlanFor(A, B, C, M, N, K, forced, plan), guard));
     return kXSchedSuccess;
 }
