@@ -95,7 +95,6 @@ constexpr uint32_t kPollTurns = XSCHED_HIST_POLL_TURNS; // turns of the ring per
 constexpr uint32_t kUnitKeys = kThreads * 4;
 constexpr uint32_t kIterKeys = kUnitKeys * kUnits;
 constexpr uint32_t kMinChunk = kUnitKeys;
-constexpr uint32_t kShortDepth = 4;             // the same for short chunks, one 128-bit load per thread each
 constexpr uint32_t kMaxChunk = 1u << 18;
 constexpr uint32_t kTargetGroups = 256;       // compute units of an MI355X
 constexpr uint32_t kFewThreads = 256;         // HistogramFewKeysKernel: threads
@@ -265,11 +264,7 @@ __device__ __forceinline__ uint32_t WaveSum(uint32_t v)
 /// bins 9.3 -> 8.0 us, 2^24 16.3 -> 14.0, 2^26 43.2 -> 40.5).
 /// kMerge: the group stores its partial histogram (ColumnAt(), OutsideAt()) instead of adding its
 /// counts to bins itself; HistogramMergeKernel does.
-/// kShort: chunks of a few iterations (ShortChunk()), in launches of which few work-groups read at once or
-/// none for long. What they take is round trips to memory: kShortDepth iterations are in
-/// flight instead of kDepth, and what a chunk has beyond whole trips of the loop is among them, the ragged
-/// end included. (Long chunks in all compute units keep memory busy with kDepth; more in flight is 2-5 % slower there.)
-template <bool kGuard, bool kMerge, bool kPacked, bool kShort>
+template <bool kGuard, bool kMerge, bool kPacked>
 __global__ __launch_bounds__(kThreads, 8 /* waves per SIMD: two groups to a compute unit */)
 void HistogramKernel(const int32_t *__restrict__ keys, uint64_t n, uint32_t *__restrict__ bins,
                      uint32_t n_bins, uint32_t chunk, uint32_t *__restrict__ partials, XGuardArgs g)
@@ -307,39 +302,7 @@ void HistogramKernel(const int32_t *__restrict__ keys, uint64_t n, uint32_t *__r
     constexpr uint64_t kLoopKeys = kTurnKeys * kPollTurns; // one trip of the main loop
     const uint64_t turns_end = begin + (full_end - begin) / kLoopKeys * kLoopKeys;
     i32x4 ring[kDepth][kUnits];
-
-    // Short chunks: iteration i of the chunk's `iters`, the last of which may be ragged. Every load lies inside
-    // the array: one that would reach behind it is made from its last 16 bytes (SetRight()).
-    const uint32_t full_iters = (uint32_t)(end - begin) / kUnitKeys;
-    const uint32_t iters = ((uint32_t)(end - begin) + kUnitKeys - 1) / kUnitKeys;
-    constexpr uint32_t kTrip = kShortDepth;                // iterations of a trip of their loop
-    const uint32_t trips = full_iters / kTrip;
-    i32x4 held[kShortDepth];
-    auto load_short = [&](uint32_t i) {
-        const uint64_t idx = begin + (uint64_t)i * kUnitKeys + (uint64_t)tid * 4;
-        return __builtin_nontemporal_load((const i32x4_any *)(keys + (idx + 4 <= n ? idx : n - 4)));
-    };
-    if (kShort) {
-        if (n < 4) {
-            held[0] = i32x4 { -1, -1, -1, -1 };
-            if (tid == 0) {
-                held[0].x = keys[0];
-                if (n > 1) held[0].y = keys[1];
-                if (n > 2) held[0].z = keys[2];
-            }
-        } else if (trips != 0) {
-            // (no branch around a load here and in the loop: the compiler counts them)
-#pragma unroll
-            for (uint32_t d = 0; d < kShortDepth; ++d) {
-                held[d] = load_short(d);
-                asm volatile("" ::: "memory");
-            }
-        } else {
-#pragma unroll
-            for (uint32_t d = 0; d < kShortDepth; ++d) if (d < iters) held[d] = load_short(d);
-        }
-    }
-    if (!kShort && begin < turns_end) {
+    if (begin < turns_end) {
         // Every set is loaded, no branch per set, and in the order in which the loop
         // refills them (the empty statements keep the scheduler from permuting the loads:
         // the loop's waits count on that order). A chunk shorter than one trip of the loop
@@ -420,41 +383,6 @@ void HistogramKernel(const int32_t *__restrict__ keys, uint64_t n, uint32_t *__r
     // a trip of the loop (kPollTurns turns) and looked at at its end: by then the refills
     // issued behind it are the only loads it does not wait for.
     auto count_chunk = [&]() -> bool {
-        if constexpr (kShort) {
-            // The keys of the ragged iteration as they were asked for, absent ones as the sentinel.
-            auto set_right = [&](uint32_t i, i32x4 v) -> i32x4 {
-                const uint64_t idx = begin + (uint64_t)i * kUnitKeys + (uint64_t)tid * 4;
-                const uint32_t behind = n < 4 || idx + 4 <= n ? 0 : (uint32_t)(idx + 4 - n < 4 ? idx + 4 - n : 4);
-                if (behind & 1) v = i32x4 { v.y, v.z, v.w, -1 };
-                if (behind & 2) v = i32x4 { v.z, v.w, -1, -1 };
-                if (behind & 4) v = i32x4 { -1, -1, -1, -1 };
-                return v;
-            };
-            uint32_t i = 0;
-            if (trips != 0) {
-                look_for_runs(held[0]);
-                do {
-                    const uint32_t polled = kGuard ? guard.WavePollBegin() : 0u;
-#pragma unroll
-                    for (uint32_t d = 0; d < kShortDepth; ++d) {
-                        process(&held[d], OneUnit {});
-                        const uint32_t next = i + kShortDepth + d;
-                        held[d] = load_short(next < iters ? next : iters - 1);
-                    }
-                    i += kTrip;
-                    if (kGuard && !guard.WavePollEnd(polled)) return false;
-                } while (i + kTrip <= full_iters);
-            }
-            // up to kShortDepth iterations, on their way already
-#pragma unroll
-            for (uint32_t d = 0; d < kShortDepth; ++d) {
-                if (i + d < iters) {
-                    const i32x4 v = i + d < full_iters ? held[d] : set_right(i + d, held[d]);
-                    process(&v, OneUnit {});
-                }
-            }
-            return true;
-        }
         uint64_t base = begin;
         if (base < turns_end) {
             look_for_runs(ring[0][0]);
@@ -673,22 +601,12 @@ void HistogramKernel(const int32_t *__restrict__ keys, uint64_t n, uint32_t *__r
     if (kGuard) guard.Commit();
 }
 
-/// Chunks of up to 16 iterations, which is up to 2^24 keys: with four iterations in flight a pass of 2^23 keys over
-/// 65536 bins takes 31.0 us (32.9 with two), 2^24 37.9 (38.7) or 36.7 (38.0), 2^20 25.5 to 26.3 (26.0 to 26.5),
-/// over 1000 bins 2^23 21.8 (22.7), 2^24 27.4 (27.9); 2^24.7 keys over 65536 bins 44.4 (43.5).
-inline bool ShortChunk(uint32_t chunk) { return chunk <= (1u << 16); }
-
 using CountKernelFn = void (*)(const int32_t *, uint64_t, uint32_t *, uint32_t, uint32_t, uint32_t *, XGuardArgs);
-template <bool kMerge, bool kShort>
+template <bool kMerge>
 inline CountKernelFn CountKernel(bool guarded, uint32_t n_bins)
 {
-    if (n_bins > kColdWords) return guarded ? HistogramKernel<true, kMerge, true, kShort> : HistogramKernel<false, kMerge, true, kShort>;
-    return guarded ? HistogramKernel<true, kMerge, false, kShort> : HistogramKernel<false, kMerge, false, kShort>;
-}
-template <bool kMerge>
-inline CountKernelFn CountKernel(bool guarded, uint32_t n_bins, uint32_t chunk)
-{
-    return ShortChunk(chunk) ? CountKernel<kMerge, true>(guarded, n_bins) : CountKernel<kMerge, false>(guarded, n_bins);
+    if (n_bins > kColdWords) return guarded ? HistogramKernel<true, kMerge, true> : HistogramKernel<false, kMerge, true>;
+    return guarded ? HistogramKernel<true, kMerge, false> : HistogramKernel<false, kMerge, false>;
 }
 
 /// Few keys, many bins: a group of 256 threads has 1024 keys, four to a thread. Bins below 256 are
@@ -909,12 +827,12 @@ protected:
             return hipGetLastError();
         }
         if (way_ == Way::kSweep) {
-            LaunchWithStopLds(ExtraLdsFor(chunk_), TakeStopEvent(), CountKernel<false>(guarded, n_bins_, chunk_), grid, block, stream,
+            LaunchWithStopLds(ExtraLdsFor(chunk_), TakeStopEvent(), CountKernel<false>(guarded, n_bins_), grid, block, stream,
                            keys_, (uint64_t)n_, bins_, n_bins_, chunk_, (uint32_t *)nullptr, g);
             return hipGetLastError();
         }
         // the merge kernel is the command's last
-        LaunchWithStopLds(ExtraLdsFor(chunk_), nullptr, CountKernel<true>(guarded, n_bins_, chunk_), grid, block, stream,
+        LaunchWithStopLds(ExtraLdsFor(chunk_), nullptr, CountKernel<true>(guarded, n_bins_), grid, block, stream,
                        keys_, (uint64_t)n_, bins_, n_bins_, chunk_, partials_, g);
         hipError_t err = hipGetLastError();
         if (err != hipSuccess) return err;
@@ -1027,10 +945,10 @@ EXPORT_C_FUNC XResult HipHistogramLaunchNoAlloc(void *stream_ptr, const void *ke
         if (plan.way == hist::Way::kFew) {
             hipLaunchKernelGGL(hist::HistogramFewKeysKernel<false>, grid, dim3(hist::kFewThreads), 0, stream, k, (uint64_t)n, out, n_bins, inert);
         } else if (plan.way == hist::Way::kSweep) {
-            hipLaunchKernelGGL(hist::CountKernel<false>(false, n_bins, plan.chunk), grid, block, hist::ExtraLdsFor(plan.chunk), stream, k, (uint64_t)n, out, n_bins, plan.chunk,
+            hipLaunchKernelGGL(hist::CountKernel<false>(false, n_bins), grid, block, hist::ExtraLdsFor(plan.chunk), stream, k, (uint64_t)n, out, n_bins, plan.chunk,
                                (uint32_t *)nullptr, inert);
         } else {
-            hipLaunchKernelGGL(hist::CountKernel<true>(false, n_bins, plan.chunk), grid, block, hist::ExtraLdsFor(plan.chunk), stream, k, (uint64_t)n, out, n_bins, plan.chunk, partials, inert);
+            hipLaunchKernelGGL(hist::CountKernel<true>(false, n_bins), grid, block, hist::ExtraLdsFor(plan.chunk), stream, k, (uint64_t)n, out, n_bins, plan.chunk, partials, inert);
             if (hipGetLastError() == hipSuccess) {
                 hipLaunchKernelGGL(hist::HistogramMergeKernel<false>, dim3(hist::kMergeGroups), dim3(hist::kMergeThreads), 0, stream,
                                    (const uint32_t *)partials, (uint32_t)plan.groups, out, n_bins, (uint32_t)plan.groups, inert);
