@@ -31,8 +31,9 @@
 // counter, so nothing has to be cleared or read back on resume; one byte per
 // work-group instead of two words.
 //
-// Cost: one uncached and one cached scalar load per work-group (hidden by the other
-// resident waves), two compares, and one byte store per work-group.
+// Cost: one uncached and one cached load per work-group, both on their way at once (hidden by the other
+// resident waves, or behind what lies between EnterBegin() and EnterEnd()), two compares, and one byte
+// store per work-group.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -149,6 +150,26 @@ __device__ __forceinline__ bool xguard_epoch_flushed(const XGuardArgs &g)
 /// queue behind the launch (`kernel<<<grid, block, 0, stream>>>(..., XGuardArgs{})`).
 __device__ __forceinline__ bool xguard_inert(const XGuardArgs &g) { return g.flag == nullptr; }
 
+/// The words that decide at entry, on their way: vector loads (see xguard_read_flag_begin()), one behind
+/// the other and neither waiting for the other's round trip to memory.
+struct XGuardEntry { uint32_t copy, flushed_word; };
+
+__device__ __forceinline__ XGuardEntry xguard_enter_begin(const XGuardArgs &g, uint32_t wg)
+{
+    XGuardEntry e;
+    e.copy = xguard_read_flag_begin(xguard_flag_copy(g, wg));
+    e.flushed_word = g.flushed != nullptr ? __hip_atomic_load(g.flushed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : ~g.epoch;
+    return e;
+}
+
+__device__ __forceinline__ XGuardVerdict xguard_enter_end(const XGuardArgs &g, uint32_t wg, const XGuardEntry &e)
+{
+    const uint32_t copy = xguard_read_flag_end(e.copy), flushed_word = xguard_read_flag_end(e.flushed_word);
+    const bool replay_with_map = g.resume && g.done;
+    const uint32_t tag = replay_with_map && copy == g.epoch ? xguard_read_tag(g, wg) : 0u;
+    return xguard_entry_verdict(copy, flushed_word, g.epoch, g.resume, g.done != nullptr, tag, g.gen);
+}
+
 /// Guard of a work-group that is ONE wavefront (blockDim == 64): the decision is
 /// wave-uniform by construction, no LDS or barrier is needed.
 class XGuardWave
@@ -160,11 +181,7 @@ public:
     __device__ __forceinline__ bool Enter() const
     {
         if (xguard_inert(g_)) return true;
-        const uint32_t flushed_word = xguard_read_flushed(g_);
-        const uint32_t copy = xguard_read_flag(xguard_flag_copy(g_, wg_));
-        const bool replay_with_map = g_.resume && g_.done;
-        const uint32_t tag = replay_with_map && copy == g_.epoch ? xguard_read_tag(g_, wg_) : 0u;
-        const XGuardVerdict v = xguard_entry_verdict(copy, flushed_word, g_.epoch, g_.resume, g_.done != nullptr, tag, g_.gen);
+        const XGuardVerdict v = xguard_enter_end(g_, wg_, xguard_enter_begin(g_, wg_));
         if (v.note_flush && (threadIdx.x & 63) == 0) xguard_note_flush(g_);
         return v.run != 0;
     }
@@ -188,15 +205,22 @@ public:
     __device__ __forceinline__ XGuardBlock(const XGuardArgs &g, uint32_t wg, uint32_t *lds_word)
         : g_(g), wg_(wg), lds_(lds_word) {}
 
-    __device__ __forceinline__ bool Enter() const
+    __device__ __forceinline__ bool Enter() const { return EnterEnd(EnterBegin()); }
+
+    /// Enter() in two halves: EnterBegin() requests the words it decides by, EnterEnd() decides. What
+    /// lies between runs while they are on their way, and must have no side effect. Loads
+    /// requested there are not waited for by EnterEnd().
+    __device__ __forceinline__ XGuardEntry EnterBegin() const
+    {
+        if (xguard_inert(g_) || threadIdx.x >= 64) return XGuardEntry { 0, 0 };
+        return xguard_enter_begin(g_, wg_);
+    }
+
+    __device__ __forceinline__ bool EnterEnd(const XGuardEntry &entry) const
     {
         if (xguard_inert(g_)) return true;
         if (threadIdx.x < 64) {
-            const uint32_t flushed_word = xguard_read_flushed(g_);
-            const uint32_t copy = xguard_read_flag(xguard_flag_copy(g_, wg_));
-            const bool replay_with_map = g_.resume && g_.done;
-            const uint32_t tag = replay_with_map && copy == g_.epoch ? xguard_read_tag(g_, wg_) : 0u;
-            const XGuardVerdict v = xguard_entry_verdict(copy, flushed_word, g_.epoch, g_.resume, g_.done != nullptr, tag, g_.gen);
+            const XGuardVerdict v = xguard_enter_end(g_, wg_, entry);
             if (threadIdx.x == 0) {
                 if (v.note_flush) xguard_note_flush(g_);
                 *lds_ = v.run;

@@ -130,8 +130,6 @@ void AxpyPersistentKernel(float alpha, const float *x_first, float *y_first, uin
     const uint32_t lane = threadIdx.x;
     const uint32_t stride = gridDim.x;
     const uint32_t *flag = kGuard ? xguard_flag_copy(g, blockIdx.x) : nullptr;
-    // an earlier launch of this epoch was flushed: this one must not run ahead of its replay
-    if (kGuard && xguard_epoch_flushed(g)) return;
 
     // Ring slot d holds step ring_s[d] of chunk ring_c[d]; the slots follow each other in
     // the wave's sequence of steps.
@@ -158,6 +156,10 @@ void AxpyPersistentKernel(float alpha, const float *x_first, float *y_first, uin
             }
         }
     }
+
+    // An earlier launch of this epoch was flushed: this one must not run ahead of its replay. (Looked at behind
+    // the first loads, which have no side effect: a scalar load, so nobody waits for them.)
+    if (kGuard && xguard_epoch_flushed(g)) return;
 
     bool skip = false;   // the chunk whose steps are passing by was committed before the flush
     while (true) {

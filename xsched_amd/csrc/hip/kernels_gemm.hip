@@ -337,11 +337,14 @@ void GemmBf16Body(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
         for (int j = 0; j < kBlocksN; ++j) fb[ks][j] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, fb[ks][j]) & m);
     };
 
+    // (the guard's words are requested first: waiting for them waits for nothing else)
+    const XGuardBlock guard(g, blockIdx.x, &guard_word);
+    const XGuardEntry entry = kGuard ? guard.EnterBegin() : XGuardEntry {};
+    XS_PIN;
     load_tile(0, 0);
 
     if (kGuard) {
-        XGuardBlock guard(g, blockIdx.x, &guard_word);
-        if (!guard.Enter()) {
+        if (!guard.EnterEnd(entry)) {
             XS_WAIT_GLOBAL_LOADS; // nothing may still be on its way into LDS when the group is gone
             return;
         }
@@ -479,10 +482,7 @@ void GemmBf16Body(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
         }
     }
 
-    if (kGuard) {
-        XGuardBlock guard(g, blockIdx.x, &guard_word);
-        guard.Commit();
-    }
+    if (kGuard) guard.Commit();
 }
 
 template <bool kGuard, Fit kFit, int kTile, int kWavesM, int kWavesN>
@@ -566,10 +566,12 @@ void GemmDeepBody(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
     constexpr int kBRowsPerLoad = 64 / kBSlotsPerRow;
     static_assert(2 * kFrags % kMfmas == 0 || 2 * kFrags <= kMfmas, "reads pair up with the MFMAs of a step");
     static_assert((kStages & (kStages - 1)) == 0 && kStages >= 4, "stages are numbered modulo a power of two");
-    // one LDS object (see above): the tiles, then two slots for the preempt word and the guard's own word
+    // one LDS object (see above): the tiles, then two slots for the preempt word, one for the `flushed` word and the
+    // guard's own word
     constexpr int kFlagAt = 2 * kBuffers * kTileBytes;
-    __shared__ __attribute__((aligned(1024))) uint8_t lds[kFlagAt + 2 * 256 + 16];
-    uint32_t &guard_word = *(uint32_t *)(lds + kFlagAt + 2 * 256);
+    constexpr int kFlushedSlot = 2;
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[kFlagAt + 3 * 256 + 16];
+    uint32_t &guard_word = *(uint32_t *)(lds + kFlagAt + 3 * 256);
     uint8_t *const As0 = lds;
     uint8_t *const Bs0 = lds + kBuffers * kTileBytes;
 
@@ -703,7 +705,33 @@ void GemmDeepBody(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
     };
 #define XS_BARRIER do { asm volatile("" ::: "memory"); XS_PIN; __builtin_amdgcn_s_barrier(); XS_PIN; asm volatile("" ::: "memory"); } while (0)
 
-    // ---- prologue: the first tiles on their way, the guard's reads beside them ----
+    // ---- prologue: the first tiles on their way, the guard's words in front of them ----
+    // The words travel like a tile: wave 0 has them loaded into LDS (one wave-wide load each, in order with
+    // the tiles'), and every wave reads them there once tile 0 has been waited for in front of a
+    // barrier. (A load into a register would have to be waited for with all tiles requested behind it
+    // as far as the compiler can tell; scalar loads are two more round trips, and the decision a barrier of its own.)
+    // A replay also looks at its byte of the progress map, the ordinary way.
+    const XGuardBlock guard(g, blockIdx.x, &guard_word);
+    auto request_word = [&](const uint32_t *word, int slot) {
+        if (wave == 0) {
+            const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void *)word, 0, 4, 0x00020000);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (LdsVoid *)(lds + kFlagAt + slot * 256), 4, 0, 0, 0, 0x11 /* sc0 sc1: system scope */);
+        }
+    };
+    auto word_of = [&](int slot) -> uint32_t {
+        return (uint32_t)__builtin_amdgcn_readfirstlane((int)*(LdsVolatileWord *)(lds + kFlagAt + slot * 256));
+    };
+    auto request_flag = [&](int slot) { request_word(xguard_flag_copy(g, blockIdx.x), slot); };
+    auto flag_is_current = [&](int slot) -> bool { return word_of(slot) == g.epoch; };
+    const bool by_words = kGuard && !xguard_inert(g) && !g.resume && g.flushed != nullptr;
+    if (kGuard) {
+        if (by_words) {
+            request_flag(1);
+            request_word(g.flushed, kFlushedSlot);
+        } else if (!guard.Enter()) {
+            return;
+        }
+    }
     constexpr int kAhead = kDirect ? kStages : kRegTiles;
 #pragma unroll
     for (int t = 0; t < kAhead; ++t) {
@@ -713,13 +741,6 @@ void GemmDeepBody(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
             if constexpr (kDirect) load_direct(t, idx, t == steps - 1 ? last_off(idx) : off[idx]);
             else if (t == steps - 1) load_held_last(t, t, idx);
             else load_held(t, t, idx);
-        }
-    }
-    if (kGuard) {
-        XGuardBlock guard(g, blockIdx.x, &guard_word);
-        if (!guard.Enter()) {
-            XS_WAIT_GLOBAL_LOADS; // nothing may still be on its way into LDS when the group is gone
-            return;
         }
     }
     // Waits until tile t has landed, i.e. all but the `newer` tiles requested behind it.
@@ -744,25 +765,23 @@ void GemmDeepBody(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
             }
         }
         static_assert(kDirect || kRegTiles == kBuffers, "tiles 0 .. kRegTiles - 1 each have a buffer");
-        __builtin_amdgcn_s_waitcnt(0xC07F); // lgkmcnt(0): the stores to LDS are done
+        __builtin_amdgcn_s_waitcnt(0xC07F); // lgkmcnt(0): the stores to LDS are done (tile 0 has come through registers, and the guard's words before it)
     }
     XS_BARRIER;
-
-    // The preempt word travels like a tile: wave 0 has it loaded into LDS (one more wave-wide
-    // load, in order with the tiles'), and kPollSteps steps later, when that load has landed
-    // because loads requested behind it have been waited for in front of a barrier, every wave
-    // reads it there. (A load into a register would have to be waited for with all tiles
-    // requested before it; a scalar load with all LDS reads.) Two slots in turn: between two
-    // writes of one slot lie the barriers of eight steps and one look at it.
-    auto request_flag = [&](int slot) {
-        if (wave == 0) {
-            const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void *)xguard_flag_copy(g, blockIdx.x), 0, 4, 0x00020000);
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (LdsVoid *)(lds + kFlagAt + slot * 256), 4, 0, 0, 0, 0x11 /* sc0 sc1: system scope */);
+    if (kGuard && by_words) {
+        const XGuardVerdict v = xguard_entry_verdict(word_of(1), word_of(kFlushedSlot), g.epoch, 0, 0, 0, g.gen);
+        if (!v.run) {
+            XS_WAIT_GLOBAL_LOADS; // nothing may still be on its way into LDS when the group is gone
+            if (v.note_flush && tid == 0) xguard_note_flush(g);
+            return;
         }
-    };
-    auto flag_is_current = [&](int slot) -> bool {
-        return (uint32_t)__builtin_amdgcn_readfirstlane((int)*(LdsVolatileWord *)(lds + kFlagAt + slot * 256)) == g.epoch;
-    };
+    }
+
+    // Later looks at the preempt word are the same: requested into LDS, and kPollSteps steps later, when
+    // that load has landed because loads requested behind it have been waited for in front of a barrier,
+    // read there by every wave. (A scalar load would have to be waited for with all LDS reads.) Two slots
+    // in turn (the one of the entry is the second): between two writes of one slot lie the barriers of
+    // eight steps and one look at it.
 
     // One step. Tile t + 1 is waited for (kNewer tiles requested behind it stay in flight), then
     // come the MFMAs on the fragments of tile t, next to them the fragment reads of tile t + 1 and
@@ -911,10 +930,7 @@ void GemmDeepBody(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
         }
     }
 
-    if (kGuard) {
-        XGuardBlock guard(g, blockIdx.x, &guard_word);
-        guard.Commit();
-    }
+    if (kGuard) guard.Commit();
 }
 #undef XS_BARRIER
 
@@ -952,8 +968,8 @@ void GemmBf16AnyShapeKernel(const uint16_t *__restrict__ A, const uint16_t *__re
     __shared__ __attribute__((aligned(16))) uint16_t b_cols[kAnyTile][kAnyK + 8];   // B transposed: [column][k]
     __shared__ uint32_t guard_word;
 
-    XGuardBlock guard(g, blockIdx.x, &guard_word);
-    if (kGuard && !guard.Enter()) return;
+    const XGuardBlock guard(g, blockIdx.x, &guard_word);
+    const XGuardEntry entry = kGuard ? guard.EnterBegin() : XGuardEntry {};
 
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const uint32_t wm = wave >> 1, wn = wave & 1;
@@ -986,6 +1002,7 @@ void GemmBf16AnyShapeKernel(const uint16_t *__restrict__ A, const uint16_t *__re
     for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
 
     Eight a = load_a(0), b = load_b(0);
+    if (kGuard && !guard.EnterEnd(entry)) return;
     for (size_t k0 = 0; k0 < Ks; k0 += kAnyK) {
         __syncthreads();   // the fragments of the previous step have been read
         *(u32x4 *)&a_rows[a_row][a_k] = a.v;
@@ -1036,6 +1053,8 @@ __global__ __launch_bounds__(kCopyThreads)
 void CopyRowsKernel(RowCopy a, RowCopy b, XGuardArgs g)
 {
     __shared__ uint32_t guard_word;
+    const XGuardBlock guard(g, blockIdx.x, &guard_word);
+    const XGuardEntry entry = kGuard ? guard.EnterBegin() : XGuardEntry {};
     const bool second = blockIdx.x >= a.groups;
     const RowCopy &m = second ? b : a;
     const uint32_t pieces_per_row = m.ld / 8, pieces = m.rows * pieces_per_row;   // (at most 2^26: PlanFor)
@@ -1043,7 +1062,6 @@ void CopyRowsKernel(RowCopy a, RowCopy b, XGuardArgs g)
     const size_t last = (size_t)m.rows * m.cols - 8;   // first element of the matrix's last 16 bytes
     u32x4 v[kCopyPieces];
     uint32_t d[kCopyPieces];
-    // (requested before the guard's reads, so that the round trips overlap)
 #pragma unroll
     for (uint32_t u = 0; u < kCopyPieces; ++u) {
         const uint32_t p = min(first + u * kCopyThreads, pieces - 1);
@@ -1054,8 +1072,7 @@ void CopyRowsKernel(RowCopy a, RowCopy b, XGuardArgs g)
         v[u] = *(const u32x4_any *)(m.from + inside);
         d[u] = (uint32_t)(at - inside) * 2;
     }
-    XGuardBlock guard(g, blockIdx.x, &guard_word);
-    if (kGuard && !guard.Enter()) return;
+    if (kGuard && !guard.EnterEnd(entry)) return;
 #pragma unroll
     for (uint32_t u = 0; u < kCopyPieces; ++u) {
         const uint32_t p = first + u * kCopyThreads;

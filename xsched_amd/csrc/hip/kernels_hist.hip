@@ -274,7 +274,8 @@ void HistogramKernel(const int32_t *__restrict__ keys, uint64_t n, uint32_t *__r
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = tid & 63;
     const uint32_t cold_words = ColdWordsOf(n_bins), width_log2 = ColdWidthLog2(n_bins);
-    XGuardBlock guard(g, blockIdx.x, &sh.guard_word);
+    const XGuardBlock guard(g, blockIdx.x, &sh.guard_word);
+    const XGuardEntry entry = kGuard ? guard.EnterBegin() : XGuardEntry {};   // on its way while the counters are cleared
 
     const WarmPlace warm_at = WarmPlaceOf(cold_words);
     const uint32_t copy = warm_at.first + (lane & ((1u << warm_at.log2) - 1u));
@@ -295,9 +296,8 @@ void HistogramKernel(const int32_t *__restrict__ keys, uint64_t n, uint32_t *__r
         }
     };
     // A ring of kDepth register sets: the set just counted is refilled with the keys of
-    // kDepth iterations ahead. The first sets are requested before the guard's uncached
-    // read of the preempt word, so that the memory round trips overlap (reading keys has
-    // no side effect).
+    // kDepth iterations ahead. The first sets are requested before the guard's decision
+    // (reading keys has no side effect).
     constexpr uint64_t kTurnKeys = (uint64_t)kDepth * kIterKeys;
     constexpr uint64_t kLoopKeys = kTurnKeys * kPollTurns; // one trip of the main loop
     const uint64_t turns_end = begin + (full_end - begin) / kLoopKeys * kLoopKeys;
@@ -315,7 +315,7 @@ void HistogramKernel(const int32_t *__restrict__ keys, uint64_t n, uint32_t *__r
     }
 
     if (kGuard) {
-        if (!guard.Enter()) return; // Enter() contains the barrier that also publishes the cleared counters
+        if (!guard.EnterEnd(entry)) return; // contains the barrier that also publishes the cleared counters
     } else {
         __syncthreads();
     }
@@ -628,6 +628,8 @@ void HistogramFewKeysKernel(const int32_t *__restrict__ keys, uint64_t n, uint32
     __shared__ uint32_t guard_word;
     static_assert(kFewThreads == kFewWarmBins, "a thread per warm bin");
 
+    const XGuardBlock guard(g, blockIdx.x, &guard_word);
+    const XGuardEntry entry = kGuard ? guard.EnterBegin() : XGuardEntry {};
     const uint32_t tid = threadIdx.x;
     const uint64_t idx = (uint64_t)blockIdx.x * kFewKeys + (uint64_t)tid * 4;
     i32x4 v = { -1, -1, -1, -1 };
@@ -639,8 +641,7 @@ void HistogramFewKeysKernel(const int32_t *__restrict__ keys, uint64_t n, uint32
         if (idx + 2 < n) v.z = keys[idx + 2];
     }
     warm[tid] = 0;
-    XGuardBlock guard(g, blockIdx.x, &guard_word);
-    if (kGuard && !guard.Enter()) return;
+    if (kGuard && !guard.EnterEnd(entry)) return;
 
     const uint32_t k[4] = { (uint32_t)v.x, (uint32_t)v.y, (uint32_t)v.z, (uint32_t)v.w };
     const uint32_t cold_bins = n_bins > kFewWarmBins ? n_bins - kFewWarmBins : 0;   // k - kFewWarmBins < cold_bins: a cold key
