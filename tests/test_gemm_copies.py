@@ -78,7 +78,7 @@ def _ints(torch, gen, shape, offset):
 # seven elements, K of the last step 1 and 63; matrices off by an element; C alone off
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K,offsets,copied", [
-    (3000, 2999, 301, (0, 0, 0), "ab"), (2500, 2503, 1025, (0, 0, 0), "ab"), (3001, 3009, 1087, (1, 3, 5), "ab"),
+    (4000, 3999, 301, (0, 0, 0), "ab"), (3500, 3503, 1025, (0, 0, 0), "ab"), (3001, 3009, 1087, (1, 3, 5), "ab"),
     (3000, 3008, 1001, (0, 0, 0), "a"), (3000, 3001, 1000, (0, 0, 0), "b"), (4096, 4096, 1024, (1, 0, 0), "a"),
     (4096, 4096, 1024, (0, 7, 1), "b"), (4100, 4104, 1024, (0, 0, 1), "")])
 @pytest.mark.parametrize("level,guard", [(1, 0), (2, 1)])

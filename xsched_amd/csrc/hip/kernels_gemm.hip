@@ -514,16 +514,16 @@ void GemmBf16Kernel(const uint16_t *__restrict__ A, const uint16_t *__restrict__
 // lead, or a bounds-checked kernel of 64 x 64 tiles for what is not a multiple of the tiles):
 //   1024^3            10.8 -> 5.8 us (64 x 64: 256 work-groups instead of 64)
 //   2048^3            23.7 -> 17.8 us = 0.96 PFLOP/s
-//   2000^3            86.5 -> 21.8 us      2000 x 1999 x 2047   254 -> 31.0 us
+//   2000^3            86.5 -> 21.8 us      2000 x 1999 x 2047   254 -> 28.5 us
 //   128 x 128 x 8192  76.0 -> 19.7 us      4097 x 4095 x 4097   2122 -> 243 us
 
 /// What a K step does besides its MFMAs (see GemmDeepBody).
 enum LoadKind { kNothing, kWholeTile, kLastTile };
-template <int kLoad_, bool kPut_, bool kRead_, int kNewer_>
+template <int kLoad_, int kPut_, bool kRead_, int kNewer_>
 struct Step
 {
     static constexpr int kLoad = kLoad_;     // request a tile
-    static constexpr bool kPut = kPut_;      // kUnaligned: store a tile that has arrived to LDS
+    static constexpr int kPut = kPut_;       // kUnaligned: store a tile that has arrived to LDS
     static constexpr bool kRead = kRead_;    // read the next tile's fragments
     static constexpr int kNewer = kNewer_;   // tiles in flight behind the one waited for
 };
@@ -636,21 +636,29 @@ void GemmDeepBody(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
                                                : (const uint8_t *)(b_tile + (size_t)step * kStepK * ldb);
         held[set][idx] = *(const u32x4_any *)(base + off[idx]);
     };
-    auto load_held_last = [&](int set, int step, int idx) {
+    // The last step's pieces: one that would reach behind the matrix is fetched from its last 16 bytes
+    // instead, and shifted into place when it is put into LDS (not here: the shift would wait for the
+    // load); what is then missing lies behind K or in columns behind N.
+    auto last_piece = [&](int step, int idx, uint32_t &shift) -> const uint8_t * {
         const uint8_t *base = idx < kHalfLoads ? (const uint8_t *)(a_tile + (size_t)step * kStepK)
                                                : (const uint8_t *)(b_tile + (size_t)step * kStepK * ldb);
         const uint8_t *const end = idx < kHalfLoads ? (const uint8_t *)(A + (size_t)M * K) : (const uint8_t *)(B + (size_t)K * N);
-        // A piece that would reach behind the matrix is fetched from its last 16 bytes instead and
-        // shifted into place; what is then missing lies behind K or in columns behind N.
         const uint8_t *const p = base + last_off(idx);
         const uint8_t *const inside = p + 16 <= end ? p : end - 16;
-        held[set][idx] = ShiftDownBytes(*(const u32x4_any *)inside, (uint32_t)(p - inside));
+        shift = (uint32_t)(p - inside);
+        return inside;
     };
-    auto put_held = [&](int set, int step, int idx) {
+    auto load_held_last = [&](int set, int step, int idx) {
+        uint32_t shift;
+        held[set][idx] = *(const u32x4_any *)last_piece(step, idx, shift);
+    };
+    auto put_held = [&](int set, int step, int idx, bool last) {
         const int buf = step & (kBuffers - 1);
         uint8_t *const at = idx < kHalfLoads ? As0 + buf * kTileBytes + (wave * kHalfLoads + idx) * 1024
                                              : Bs0 + buf * kTileBytes + (wave * kHalfLoads + idx - kHalfLoads) * 1024;
-        *(u32x4 *)(at + lane * 16) = held[set][idx];
+        uint32_t shift = 0;
+        if (last) (void)last_piece(step, idx, shift);
+        *(u32x4 *)(at + lane * 16) = last ? ShiftDownBytes(held[set][idx], shift) : held[set][idx];
     };
 
     // ---- LDS -> fragments, as above ----
@@ -732,50 +740,66 @@ void GemmDeepBody(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
             return;
         }
     }
-    constexpr int kAhead = kDirect ? kStages : kRegTiles;
-#pragma unroll
-    for (int t = 0; t < kAhead; ++t) {
-        if (t >= steps) break;
-#pragma unroll
-        for (int idx = 0; idx < kLoads; ++idx) {
-            if constexpr (kDirect) load_direct(t, idx, t == steps - 1 ? last_off(idx) : off[idx]);
-            else if (t == steps - 1) load_held_last(t, t, idx);
-            else load_held(t, t, idx);
-        }
-    }
     // Waits until tile t has landed, i.e. all but the `newer` tiles requested behind it.
     auto wait_tile = [&](int newer) { WaitNewer<kStages - 1, kLoads>(newer); };
-    if constexpr (kDirect) {
-        wait_tile(min(kStages, steps) - 1);
-    } else {
-        // tile 0, then tile 1, into their LDS buffers; the next ones into the registers they leave
+    // Tiles 0, 1, .. on their way, tile 0 (kUnaligned: and 1) waited for. `many`: at least kTail steps, none of
+    // these tiles is the last, and there is no branch between loads. (With branches the compiler loses
+    // count of the loads in flight behind them: at the head of the main loop it then waited for all of them but one,
+    // and through registers a step in four took the round trip to memory.)
+    auto request_first = [&](auto many) {
+        constexpr bool kMany = decltype(many)::value;
+        constexpr int kAhead = kDirect ? kStages : kRegTiles;
 #pragma unroll
-        for (int t = 0; t < kRegTiles; ++t) {
-            if (t < steps) {
+        for (int t = 0; t < kAhead; ++t) {
+            if (!kMany && t >= steps) break;
 #pragma unroll
-                for (int idx = 0; idx < kLoads; ++idx) put_held(t, t, idx);
-            }
-            const int next = t + kRegTiles;
-            if (next < steps - 1) {
-#pragma unroll
-                for (int idx = 0; idx < kLoads; ++idx) load_held(t, next, idx);
-            } else if (next == steps - 1) {
-#pragma unroll
-                for (int idx = 0; idx < kLoads; ++idx) load_held_last(t, next, idx);
+            for (int idx = 0; idx < kLoads; ++idx) {
+                if constexpr (kDirect) load_direct(t, idx, !kMany && t == steps - 1 ? last_off(idx) : off[idx]);
+                else if (!kMany && t == steps - 1) load_held_last(t, t, idx);
+                else load_held(t, t, idx);
+                if constexpr (kMany && !kDirect) XS_PIN;   // (in this order, which the waits count on)
             }
         }
-        static_assert(kDirect || kRegTiles == kBuffers, "tiles 0 .. kRegTiles - 1 each have a buffer");
-        __builtin_amdgcn_s_waitcnt(0xC07F); // lgkmcnt(0): the stores to LDS are done (tile 0 has come through registers, and the guard's words before it)
-    }
-    XS_BARRIER;
-    if (kGuard && by_words) {
-        const XGuardVerdict v = xguard_entry_verdict(word_of(1), word_of(kFlushedSlot), g.epoch, 0, 0, 0, g.gen);
-        if (!v.run) {
-            XS_WAIT_GLOBAL_LOADS; // nothing may still be on its way into LDS when the group is gone
-            if (v.note_flush && tid == 0) xguard_note_flush(g);
-            return;
+        if constexpr (kDirect) {
+            if constexpr (kMany) WaitLoadsAndLds<(kStages - 1) * kLoads>();
+            else wait_tile(min(kStages, steps) - 1);
+        } else {
+            // tile 0, then tile 1, into their LDS buffers; the next ones into the registers they leave
+#pragma unroll
+            for (int t = 0; t < kRegTiles; ++t) {
+                if (kMany || t < steps) {
+#pragma unroll
+                    for (int idx = 0; idx < kLoads; ++idx) put_held(t, t, idx, !kMany && t == steps - 1);
+                }
+                const int next = t + kRegTiles;
+                if (kMany || next < steps - 1) {
+#pragma unroll
+                    for (int idx = 0; idx < kLoads; ++idx) {
+                        load_held(t, next, idx);
+                        if constexpr (kMany) XS_PIN;
+                    }
+                } else if (next == steps - 1) {
+#pragma unroll
+                    for (int idx = 0; idx < kLoads; ++idx) load_held_last(t, next, idx);
+                }
+            }
+            static_assert(kDirect || kRegTiles == kBuffers, "tiles 0 .. kRegTiles - 1 each have a buffer");
+            __builtin_amdgcn_s_waitcnt(0xC07F); // lgkmcnt(0): the stores to LDS are done (tile 0 has come through registers, and the guard's words before it)
         }
-    }
+    };
+    // The barrier that tile 0 is complete behind, and the guard's decision; false: the group has to leave.
+    auto enter = [&]() -> bool {
+        XS_BARRIER;
+        if (kGuard && by_words) {
+            const XGuardVerdict v = xguard_entry_verdict(word_of(1), word_of(kFlushedSlot), g.epoch, 0, 0, 0, g.gen);
+            if (!v.run) {
+                XS_WAIT_GLOBAL_LOADS; // nothing may still be on its way into LDS when the group is gone
+                if (v.note_flush && tid == 0) xguard_note_flush(g);
+                return false;
+            }
+        }
+        return true;
+    };
 
     // Later looks at the preempt word are the same: requested into LDS, and kPollSteps steps later, when
     // that load has landed because loads requested behind it have been waited for in front of a barrier,
@@ -810,7 +834,7 @@ void GemmDeepBody(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
                     if constexpr (Do::kLoad == kWholeTile) load_direct(t + kStages, idx, off[idx]);
                     if constexpr (Do::kLoad == kLastTile) load_direct(t + kStages, idx, last_off(idx));
                 } else {
-                    if constexpr (Do::kPut) put_held(p, t + 2, idx);
+                    if constexpr (Do::kPut != kNothing) put_held(p, t + 2, idx, Do::kPut == kLastTile);
                     if constexpr (Do::kLoad == kWholeTile) load_held(p, t + 2 + kRegTiles, idx);
                     if constexpr (Do::kLoad == kLastTile) load_held_last(p, t + 2 + kRegTiles, idx);
                 }
@@ -820,12 +844,15 @@ void GemmDeepBody(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
     };
     constexpr std::integral_constant<int, 0> even {};
     constexpr std::integral_constant<int, 1> odd {};
-    using Main = Step<kWholeTile, true, true, kStages - 2>;
+    using Main = Step<kWholeTile, kWholeTile, true, kStages - 2>;
 
     // The main steps load whole tiles; the kTail steps behind them load the last tile (kExact: it
     // is like the others) or nothing, and the last reads no fragments.
     constexpr int kTail = kDirect ? (kFit == Fit::kExact ? kStages : kStages + 1) : 3 + kRegTiles;
     if (steps >= kTail) {
+        static_assert(kTail > (kDirect ? kStages : 2 * kRegTiles) || kFit == Fit::kExact, "request_first() meets no last tile");
+        request_first(std::true_type {});
+        if (!enter()) return;
         const int main_steps = steps - kTail;
         int t = 0;
 #pragma unroll
@@ -853,7 +880,7 @@ void GemmDeepBody(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
                 constexpr int left = kTail - 1 - j;                              // steps behind this one
                 constexpr bool loads_last = kFit != Fit::kExact && j == 0;
                 constexpr int newer = left - 1 < 0 ? 0 : left - 1 < kStages - 2 ? left - 1 : kStages - 2;
-                using Do = Step<loads_last ? kLastTile : kNothing, (left >= 2), (left >= 1), newer>;
+                using Do = Step<loads_last ? kLastTile : kNothing, (left > 2 ? kWholeTile : left == 2 ? kLastTile : kNothing), (left >= 1), newer>;
                 step(main_steps + j, std::integral_constant<int, (p + j) & 1> {}, Do {});
             };
             [&]<int... j>(std::integer_sequence<int, j...>) { (at(std::integral_constant<int, j> {}), ...); }(std::make_integer_sequence<int, kTail> {});
@@ -867,6 +894,8 @@ void GemmDeepBody(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
     } else {
         // K of a few steps: everything is on its way (or here) already, and the fragments are
         // read in front of their MFMAs.
+        request_first(std::false_type {});
+        if (!enter()) return;
         if constexpr (kDirect) WaitLoadsAndLds<0>();
         XS_BARRIER;
         for (int t = 0; t < steps; ++t) {
@@ -881,7 +910,7 @@ void GemmDeepBody(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
                 XS_BARRIER;
 #pragma unroll
                 for (int idx = 0; idx < kLoads; ++idx) {
-                    if (t + 2 < steps) { if (t & 1) put_held(1, t + 2, idx); else put_held(0, t + 2, idx); }
+                    if (t + 2 < steps) { if (t & 1) put_held(1, t + 2, idx, t + 2 == steps - 1); else put_held(0, t + 2, idx, t + 2 == steps - 1); }
                 }
                 WaitLoadsAndLds<0>();
                 XS_BARRIER;
@@ -1258,25 +1287,25 @@ inline Part PartOf(int first_row, int rows, int N, int K, Rows aligned, int tile
 /// units it keeps busy. The rates are fitted to outputs of 4 to 4096 tiles of 128 x 128 at K from 128 to 8192:
 /// of 35 such products the plan is within 3 % of the quickest of the three tile sizes but for
 /// 2048 x 2048 x 8192 (66.3 us, 63.9 with the tile given) and 4096 x 4096 x 128 (11.4, 10.5).
-inline double MicrosOf(const Part &part, int K)
+inline double MicrosOf(const Part &part, int K, double pace = 1.0 /* of the steps */)
 {
     // us of a round, and per K step of a full round and of one with a single tile: [exact, edges, unaligned]
     struct Rates { double round, full, single; };
     constexpr Rates large[3] = { { 5.0, 1.36, 1.00 }, { 5.0, 1.43, 1.05 }, {} };
     constexpr Rates pair = { 1.7, 0.90, 0.45 };
-    constexpr Rates small[3] = { { 2.5, 0.45, 0.37 }, { 2.5, 0.53, 0.41 }, { 2.5, 0.80, 0.60 } };
-    constexpr Rates tiny[3] = { { 0.5, 0.195, 0.14 }, { 0.5, 0.25, 0.16 }, { 0.5, 0.35, 0.25 } };
+    constexpr Rates small[3] = { { 2.5, 0.45, 0.37 }, { 2.5, 0.53, 0.41 }, { 2.5, 0.69, 0.48 } };
+    constexpr Rates tiny[3] = { { 0.5, 0.195, 0.14 }, { 0.5, 0.25, 0.16 }, { 0.5, 0.32, 0.29 } };
     const bool two_per_unit = part.tile == kSmallTile && part.body == Body::kTwoBuffers;
     const Rates &r = two_per_unit ? pair : (part.tile == kLargeTile ? large : part.tile == kSmallTile ? small : tiny)[(int)part.fit];
     const double rounds = (double)part.tiles / ((two_per_unit ? 2 : 1) * ComputeUnits()), whole = std::floor(rounds);
     const double step = whole * r.full + (rounds > whole ? r.single + (r.full - r.single) * (rounds - whole) : 0.0);
-    return 3.0 + std::ceil(rounds) * r.round + step * ((K + kStepK - 1) / kStepK);
+    return 3.0 + std::ceil(rounds) * r.round + pace * step * ((K + kStepK - 1) / kStepK);
 }
 
-inline double MicrosOf(const Plan &plan, int K)
+inline double MicrosOf(const Plan &plan, int K, double pace = 1.0)
 {
     double us = 0.0;
-    for (int i = 0; i < plan.parts; ++i) us += MicrosOf(plan.part[i], K);
+    for (int i = 0; i < plan.parts; ++i) us += MicrosOf(plan.part[i], K, pace);
     return us;
 }
 
@@ -1372,18 +1401,22 @@ inline Plan PlanFor(const void *A, const void *B, const void *C, int M, int N, i
 }
 
 constexpr size_t kMaxCopyBytes = (size_t)1 << 30;   // of A and B together
-constexpr double kCopyMicros = 4.5;                 // launch of the copying kernel, and its bytes per us, read and written
-constexpr double kCopyRate = 5.9e6;
+// What copies cost by the estimate, fitted to 21 products of 300 x 301 x 6001 to 4000 x 3999 x 301, each timed in place and on
+// copies: the quicker way is taken for all of them.
+constexpr double kCopyMicros = 8.0;                 // launch of the copying kernel and the one behind it,
+constexpr double kCopyRate = 12e6;                  // bytes per us, read and written (the copies are then read from the caches),
+constexpr double kCopyPace = 0.85;                  // time of a step on rows of whole cache lines against any rows on 16-byte boundaries
 
 /// The plan for copies of whichever of A and B has rows off 16-byte boundaries; no parts where `in_place` is
 /// as quick, or where the copies are too large. Through registers a step waits for loads at any multiple of two
-/// bytes (0.7 us against 0.45 for 128 x 128 tiles of 64 k), and large tiles do not fit; the copies cost
+/// bytes, each 128-byte piece of a row in two cache lines (0.7 us against 0.45 for 128 x 128 tiles of 64 k), and large tiles do not fit; the copies cost
 /// their launch and two passes over the matrices (8191^2 elements 87 us = 6.2 TB/s with what is
 /// written, 2000 x 2047 and 2047 x 1999 together 9.5). Rows of the copies are whole 128-byte lines (rows of 2000 and
 /// 2048 elements rather than of 2048: 27 us for the 2000 x 1999 x 2047 that takes 23.5). us per command,
-/// in place / on copies: 500 x 499 x 4095 26.5 / 24.7, x 2047 13.7 / 15.8; 1500 x 1499 x 4095 49.5 / 40.0, x 1001
-/// 18.1 / 21.2; 2000 x 1999 x 2047 31.3 / 31.7, x 4095 53.6 / 46.5; 3000 x 2999 x 301 31.6 / 26.9, x 101 25.3 / 21.6;
-/// 4000 x 3999 x 2047 118.5 / 70.4; 128 x 8191 x 8191 50.7 / 76.2. A pass of 8191^3 1791 / 918.
+/// in place / on copies: 500 x 499 x 4095 23.6 / 26.5; 1500 x 1499 x 4095 44.4 / 41.0, x 2047 25.8 / 29.8; 2000 x 1999
+/// x 2047 28.4 / 31.7, x 3001 38.9 / 38.8, x 4095 51.2 / 47.2; 2500 x 2501 x 1001 32.1 / 36.3; 3000 x 2999 x 301
+/// 28.0 / 28.5, x 101 25.5 / 23.7; 4000 x 3999 x 301 38.3 / 31.4; 1000 x 999 x 8001 44.3 / 43.5; 128 x 8191 x 8191
+/// 66.8 / 76.6. A pass of 8191^3 1791 / 918.
 inline CopyPlan CopyPlanFor(const void *A, const void *B, const void *C, int M, int N, int K, int forced, const Plan &in_place)
 {
     CopyPlan p;
@@ -1399,7 +1432,7 @@ inline CopyPlan CopyPlanFor(const void *A, const void *B, const void *C, int M, 
     p.plan = QuickestPlan(M, N, K, Rows { true, Aligned(C, N) });
     if (p.Groups() > GuardState::kMaxWorkGroups) return CopyPlan {};
     const double copying = kCopyMicros + 2.0 * (double)(p.a_bytes + p.b_bytes) / kCopyRate;
-    return copying + MicrosOf(p.plan, K) < MicrosOf(in_place, K) ? p : CopyPlan {};
+    return copying + MicrosOf(p.plan, K, kCopyPace) < MicrosOf(in_place, K) ? p : CopyPlan {};
 }
 
 /// Tiles by which a shape is accepted or refused. They are the tiles of the kernels that such shapes
