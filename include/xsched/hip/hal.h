@@ -108,6 +108,10 @@ XResult HipGemmBf16PlanOf(const void *A, const void *B, const void *C, int M, in
  * capture, HipGemmBf16PlanOf() holds. No counterpart in the reference. */
 XResult HipGemmBf16CopyPlanOf(const void *A, const void *B, const void *C, int M, int N, int K, int32_t *out);
 
+/* For tests: among how many work-groups the K of a tile is divided, out[0] where A and B are read as they lie, out[1] on their
+ * copies (0: there are none). 1 on a stream under capture, or without memory. No counterpart in the reference. */
+XResult HipGemmBf16SplitsOf(const void *A, const void *B, const void *C, int M, int N, int K, int32_t *out);
+
 /* bins[keys[i]] += 1 for i < n; keys are int32 in [0, n_bins), bins are uint32 and
  * are NOT cleared by the command. n_bins <= 65536. */
 XResult HipHistogramCommandCreate(HwCommandHandle *cmd, const void *keys, size_t n, void *bins,

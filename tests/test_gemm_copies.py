@@ -26,7 +26,7 @@ def plans_of(xs, a, b, c, M, N, K):
 def test_what_is_copied(xs):
     rng = random.Random(5)
     copied = 0
-    for _ in range(4000):
+    for _ in range(8000):
         M, N, K = (int(2 ** rng.uniform(0, 14)) for _ in range(3))
         if rng.random() < 0.3:
             N = max(8, N // 8 * 8)

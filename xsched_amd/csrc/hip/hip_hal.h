@@ -163,8 +163,19 @@ public:
     /// newest one is smaller; called at submission, so that the call at launch finds one.
     void *Get(size_t bytes);
 
+    /// kTicketWords 64-bit words for commands whose work-groups have to find out which of them is the last, or
+    /// nullptr without memory; allocated at the first call. Whoever is told that they are new clears
+    /// them, on the queue's stream. Each such command takes a number, from 1 on.
+    static constexpr uint32_t kTicketWords = 256;
+    uint64_t *Tickets();
+    bool TicketsAreNew() { return tickets_new_.exchange(false); }
+    uint64_t NextCommand() { return commands_.fetch_add(1) + 1; }
+
 private:
     void *Newest(size_t bytes);
+    uint64_t *tickets_ = nullptr;
+    std::atomic<bool> tickets_new_ { true };
+    std::atomic<uint64_t> commands_ { 0 };
     static constexpr size_t kLeastBytes = (size_t)16 << 20;
     const int device_;
     std::mutex grow_mtx_;            // one allocation at a time

@@ -609,6 +609,18 @@ size_t ScratchPool::Bytes()
 SharedScratch::~SharedScratch()
 {
     for (void *buf : buffers_) (void)hipFree(buf);
+    if (tickets_ != nullptr) (void)hipFree(tickets_);
+}
+
+uint64_t *SharedScratch::Tickets()
+{
+    std::lock_guard<std::mutex> one_at_a_time(grow_mtx_);
+    if (tickets_ != nullptr) return tickets_;
+    DeviceScope scope(device_);
+    RelaxedCaptureScope relaxed;
+    void *ptr = nullptr;
+    if (hipMalloc(&ptr, kTicketWords * sizeof(uint64_t)) != hipSuccess) { (void)hipGetLastError(); return nullptr; }
+    return tickets_ = (uint64_t *)ptr;
 }
 
 void *SharedScratch::Newest(size_t bytes)

@@ -19,8 +19,8 @@
 // An MFMA operand wants eight consecutive k per lane. A has them contiguous in memory; for B
 // (k is the strided dimension) the transposing LDS read of gfx950, ds_read_b64_tr_b16, turns
 // four rows of sixteen columns into four k of one column per lane, two of them per fragment.
-// There is no split-K: every element of C is summed by one wave in one fixed order, which
-// makes a replayed tile bit-identical.
+// Every element of C is summed by one wave in one fixed order, or, where K is split (SplitK), by
+// one wave per part whose sums are added in one fixed order: a replayed tile is bit-identical.
 //
 // Under this load the device runs against its power limit (all operands zero, when next to nothing
 // switches, 8192^3 takes 567 us, normally distributed ones 782 on the same box and code), so
@@ -91,14 +91,18 @@ __device__ __forceinline__ uint32_t f32x2_to_bf16x2_rne(float lo, float hi)
     return __builtin_bit_cast(uint32_t, pair);
 }
 
-// Work-group id -> tile coordinates. Ids with equal (id % 8) run on one XCD; each
-// XCD gets a contiguous run of tiles, ordered in bands of kGroupRows tile rows.
-__device__ __forceinline__ void TileOf(uint32_t wg, uint32_t tiles_m, uint32_t tiles_n,
+// Work-group id -> number of its work. Ids with equal (id % 8) run on one XCD; each XCD gets a
+// contiguous run of the n numbers.
+__device__ __forceinline__ uint32_t WorkOf(uint32_t wg, uint32_t n)
+{
+    const uint32_t xcd = wg % kXcds, whole = n / kXcds, more = n % kXcds;   // `more` XCDs get one more
+    return xcd * whole + min(xcd, more) + wg / kXcds;
+}
+
+// Tile number t -> tile coordinates, in bands of kGroupRows tile rows.
+__device__ __forceinline__ void TileAt(uint32_t t, uint32_t tiles_m, uint32_t tiles_n,
                                        uint32_t &tm, uint32_t &tn)
 {
-    const uint32_t n_tiles = tiles_m * tiles_n;
-    const uint32_t xcd = wg % kXcds, whole = n_tiles / kXcds, more = n_tiles % kXcds;   // `more` XCDs get one tile more
-    const uint32_t t = xcd * whole + min(xcd, more) + wg / kXcds;
     const uint32_t band = kGroupRows * tiles_n;
     const uint32_t band_id = t / band;
     const uint32_t first_row = band_id * kGroupRows;
@@ -225,7 +229,8 @@ void GemmBf16Body(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
     const uint32_t wn = wave % kWavesN;
 
     uint32_t tm, tn;
-    TileOf(blockIdx.x, ((uint32_t)M + kTile - 1) / kTile, ((uint32_t)N + kTile - 1) / kTile, tm, tn);
+    const uint32_t tiles_m = ((uint32_t)M + kTile - 1) / kTile, tiles_n = ((uint32_t)N + kTile - 1) / kTile;
+    TileAt(WorkOf(blockIdx.x, tiles_m * tiles_n), tiles_m, tiles_n, tm, tn);
     const size_t m0 = (size_t)tm * kTile, n0 = (size_t)tn * kTile;
     const int steps = kFit == Fit::kExact ? K / kStepK : (K + kStepK - 1) / kStepK;
     const int rest = K - (steps - 1) * kStepK;           // K values of the last step
@@ -545,10 +550,30 @@ __device__ __forceinline__ void WaitNewer(int newer)
     else WaitNewer<kMost - 1, kLoads>(newer);
 }
 
-template <bool kGuard, Fit kFit, int kTile, int kStages>
+/// K of every tile divided among `parts` work-groups, `steps` K steps each (the last of them what is left).
+/// Outputs of few tiles leave most of the device idle, and a step is bound by what one compute unit loads and
+/// multiplies. A group stores its sums to partials (a tile of floats per group, as they lie in the
+/// registers) and draws a ticket of its tile; who draws the last one adds up the parts in their order,
+/// whichever group it is, so that the result does not depend on who came when, and writes C. A
+/// ticket word holds the number of the command that last used it (they ascend) above the tickets drawn.
+/// A group that has drawn a ticket has passed its last look at the preempt word: it commits, and no replay
+/// draws for it again.
+/// Plain launches and split ones, us per command: see QuickestPlan().
+struct SplitK
+{
+    float *partials;
+    unsigned long long *tickets;   // one per tile
+    unsigned long long command;
+    uint32_t parts, steps;
+};
+constexpr int kTicketBits = 24;    // below the command's number
+constexpr uint32_t kMaxSplitTiles = 256;
+static_assert(kMaxSplitTiles <= SharedScratch::kTicketWords, "a ticket per tile");
+
+template <bool kGuard, Fit kFit, int kTile, int kStages, bool kSplit>
 __device__ __forceinline__
 void GemmDeepBody(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B,
-                  uint16_t *__restrict__ C, int M, int N, int K, int lda, int ldb, const XGuardArgs &g)
+                  uint16_t *__restrict__ C, int M, int N, int K, int lda, int ldb, const XGuardArgs &g, const SplitK &split)
 {
     constexpr bool kDirect = kFit != Fit::kUnaligned;      // loads go straight into LDS
     constexpr int kWaves = 4;
@@ -581,10 +606,16 @@ void GemmDeepBody(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
     const uint32_t wm = wave >> 1, wn = wave & 1;
 
     uint32_t tm, tn;
-    TileOf(blockIdx.x, ((uint32_t)M + kTile - 1) / kTile, ((uint32_t)N + kTile - 1) / kTile, tm, tn);
+    const uint32_t tiles_m = ((uint32_t)M + kTile - 1) / kTile, tiles_n = ((uint32_t)N + kTile - 1) / kTile;
+    const uint32_t tiles = tiles_m * tiles_n, work = WorkOf(blockIdx.x, kSplit ? tiles * split.parts : tiles);
+    const uint32_t part = kSplit ? work / tiles : 0, tile = kSplit ? work - part * tiles : work;   // (neighbours share A and B, parts share nothing)
+    TileAt(tile, tiles_m, tiles_n, tm, tn);
     const size_t m0 = (size_t)tm * kTile, n0 = (size_t)tn * kTile;
-    const int steps = kFit == Fit::kExact ? K / kStepK : (K + kStepK - 1) / kStepK;
-    const int rest = K - (steps - 1) * kStepK;             // K values of the last step
+    const int all_steps = kFit == Fit::kExact ? K / kStepK : (K + kStepK - 1) / kStepK;
+    const int first_step = kSplit ? (int)(part * split.steps) : 0;
+    const int steps = kSplit ? min((int)split.steps, all_steps - first_step) : all_steps;
+    // K values of the last step
+    const int rest = kFit == Fit::kExact || (kSplit && first_step + steps < all_steps) ? kStepK : K - (all_steps - 1) * kStepK;
 
     // ---- what each lane fetches: byte offsets from the tile's first element, as above ----
     uint32_t off[kLoads];
@@ -611,8 +642,8 @@ void GemmDeepBody(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
         off[kHalfLoads + i] = (k * (uint32_t)ldb + col) * 2;
         k_of[kHalfLoads + i] = k;
     }
-    const uint16_t *const a_tile = A + m0 * (size_t)lda;     // + kStepK columns per step
-    const uint16_t *const b_tile = B + n0;                 // + kStepK rows per step
+    const uint16_t *const a_tile = A + m0 * (size_t)lda + (size_t)first_step * kStepK;     // + kStepK columns per step
+    const uint16_t *const b_tile = B + n0 + (size_t)first_step * kStepK * (size_t)ldb;     // + kStepK rows per step
 
     // Offset of piece idx in the last step: pieces behind K come from k = 0 of the step instead.
     auto last_off = [&](int idx) -> uint32_t {
@@ -922,6 +953,53 @@ void GemmDeepBody(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
     }
     if (kGuard) XS_WAIT_GLOBAL_LOADS;                      // the last look at the preempt word that nobody took
 
+    if constexpr (kSplit) {
+        // Partial sums go past the L2 of the group's XCD (system-coherent accesses of device scope, sc1) and are read the same
+        // way: they have arrived when the wave's stores have, and no L2 is written back or
+        // invalidated (with release fences, 256 groups took 20 us longer).
+        constexpr int kThreads = 64 * kWaves, kDeviceScope = 0x10;
+        constexpr int kPieces = kBlocks * kBlocks * 4;
+        constexpr int kPartBytes = kTile * kTile * 4;
+        constexpr int kUnroll = kTile == kTinyTile ? 4 : 1;   // parts read at a time: as many as fit into the registers
+        const __amdgpu_buffer_rsrc_t parts = __builtin_amdgcn_make_buffer_rsrc((void *)(split.partials + (size_t)tile * split.parts * (kTile * kTile)), 0,
+                                                                               (int)(split.parts * kPartBytes), 0x00020000);
+#pragma unroll
+        for (int n = 0; n < kPieces; ++n) {
+            const f32x16 &v = acc[n / 4 / kBlocks][n / 4 % kBlocks];
+            const f32x4 four = { v[n % 4 * 4], v[n % 4 * 4 + 1], v[n % 4 * 4 + 2], v[n % 4 * 4 + 3] };
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, four), parts, (n * kThreads + tid) * 16, part * kPartBytes, kDeviceScope);
+        }
+        XS_WAIT_GLOBAL_LOADS;   // (stores count as loads do)
+        XS_BARRIER;
+        if (tid == 0) {
+            unsigned long long *const word = split.tickets + tile;
+            (void)__hip_atomic_fetch_max(word, split.command << kTicketBits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const unsigned long long drawn = __hip_atomic_fetch_add(word, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            guard_word = ((uint32_t)drawn & ((1u << kTicketBits) - 1)) % split.parts == split.parts - 1 ? 1u : 0u;
+        }
+        __syncthreads();
+        if (*(LdsVolatileWord *)&guard_word == 0) {
+            if (kGuard) guard.Commit();
+            return;
+        }
+        XS_PIN;
+        f32x4 sum[kPieces];
+        auto piece = [&](uint32_t p, int n) -> f32x4 {
+            return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(parts, (n * kThreads + tid) * 16, p * kPartBytes, kDeviceScope));
+        };
+#pragma unroll
+        for (int n = 0; n < kPieces; ++n) sum[n] = piece(0, n);
+#pragma unroll kUnroll
+        for (uint32_t p = 1; p < split.parts; ++p) {
+#pragma unroll
+            for (int n = 0; n < kPieces; ++n) sum[n] += piece(p, n);
+        }
+#pragma unroll
+        for (int n = 0; n < kPieces; ++n)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[n / 4 / kBlocks][n / 4 % kBlocks][n % 4 * 4 + e] = sum[n][e];
+    }
+
     // ---- write-out, as above: strips of 32 rows x 32 kBlocks columns turned over in LDS ----
     // (behind the last step's barrier nobody reads the tile buffers any more, and nothing is on
     // its way into them)
@@ -968,8 +1046,20 @@ __global__ __launch_bounds__(256)
 void GemmDeepKernel(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B,
                     uint16_t *__restrict__ C, int M, int N, int K, int lda, int ldb, XGuardArgs g)
 {
-    GemmDeepBody<kGuard, kFit, kTile, kStages>(A, B, C, M, N, K, lda, ldb, g);
+    GemmDeepBody<kGuard, kFit, kTile, kStages, false>(A, B, C, M, N, K, lda, ldb, g, SplitK {});
 }
+
+template <bool kGuard, Fit kFit, int kTile, int kStages>
+__global__ __launch_bounds__(256)
+void GemmSplitKernel(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B,
+                     uint16_t *__restrict__ C, int M, int N, int K, int lda, int ldb, XGuardArgs g, SplitK split)
+{
+    GemmDeepBody<kGuard, kFit, kTile, kStages, true>(A, B, C, M, N, K, lda, ldb, g, split);
+}
+
+/// A queue's ticket words, before the first command that uses them.
+__global__ __launch_bounds__(kMaxSplitTiles)
+void ClearTicketsKernel(unsigned long long *tickets) { tickets[threadIdx.x] = 0; }
 
 
 // Short K (ShortK() below), and what the kernels above do not take: fewer than eight columns or
@@ -1122,6 +1212,11 @@ struct Part
     Fit fit;        // of kTwoBuffers and kFourStages
     Body body;
     uint64_t tiles; // work-groups = bytes of the progress map
+    int split_parts = 1, split_steps = 0;   // kFourStages: into how many parts of how many steps K is divided (SplitK)
+
+    bool Split() const { return split_parts > 1; }
+    size_t PartialBytes() const { return Split() ? (size_t)tiles * tile * tile * 4 : 0; }
+    Part Whole() const { Part p = *this; p.tiles /= (uint64_t)split_parts; p.split_parts = 1; return p; }
 };
 
 /// One launch, or two for rows that do not fill whole rounds of large tiles.
@@ -1130,6 +1225,7 @@ struct Plan
     Part part[2];
     int parts;
     uint64_t Tiles() const { return part[0].tiles + (parts > 1 ? part[1].tiles : 0); }
+    size_t PartialBytes() const { return parts == 1 ? part[0].PartialBytes() : 0; }   // (one launch: see QuickestPlan())
 };
 
 /// A plan for copies of A, B or both with rows on 16-byte boundaries, if that is quicker (else no parts).
@@ -1140,6 +1236,7 @@ struct CopyPlan
     uint32_t a_groups = 0, b_groups = 0;   // work-groups that copy (0: the matrix stays where it is)
     size_t a_bytes = 0, b_bytes = 0;
     uint64_t Groups() const { return (uint64_t)a_groups + b_groups + plan.Tiles(); }
+    size_t CopyBytes() const { return a_bytes + b_bytes; }   // (rows of whole 128-byte lines: what follows is aligned)
 };
 
 class HipGemmCommand final : public HipGuardedCommand
@@ -1152,27 +1249,45 @@ public:
 protected:
     virtual void ReserveOnSubmit(HipQueue &q) override
     {
-        if (copies_.plan.parts != 0 && !decided_) (void)q.SharedScratch()->Get(copies_.a_bytes + copies_.b_bytes);
+        if (decided_ || ScratchBytes() == 0) return;
+        (void)q.SharedScratch()->Get(ScratchBytes());
+        if (PlanWithScratch().PartialBytes() != 0) (void)q.SharedScratch()->Tickets();
     }
 
-    /// Where the copies go is decided at the first launch: every replay takes the same way.
+    /// Where copies and partial sums go is decided at the first launch: every replay takes the same way.
     virtual hipError_t PrepareLaunch(HipQueue &q) override
     {
-        if (copies_.plan.parts == 0 || decided_) return hipSuccess;
+        if (decided_ || ScratchBytes() == 0) return hipSuccess;
         decided_ = true;
-        // A graph outlives the command and its queue: what is captured reads A and B themselves.
+        // A graph outlives the command and its queue: what is captured reads A and B themselves, and adds up in one go.
         hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
         if (hipStreamIsCapturing(q.Stream(), &capture) != hipSuccess) (void)hipGetLastError();
         if (capture != hipStreamCaptureStatusNone) return hipSuccess;
         scratch_ = q.SharedScratch();
-        at_ = (uint8_t *)scratch_->Get(copies_.a_bytes + copies_.b_bytes);   // nullptr: no memory, in place
+        if (PlanWithScratch().PartialBytes() != 0) {
+            split_.tickets = (unsigned long long *)scratch_->Tickets();
+            if (split_.tickets == nullptr) return hipSuccess;
+            split_.command = scratch_->NextCommand();
+            if (scratch_->TicketsAreNew()) {
+                ClearTicketsKernel<<<dim3(1), dim3(kMaxSplitTiles), 0, q.Stream()>>>(split_.tickets);
+                const hipError_t err = hipGetLastError();
+                if (err != hipSuccess) return err;
+            }
+        }
+        at_ = (uint8_t *)scratch_->Get(ScratchBytes());   // nullptr: no memory, in place and in one go
+        split_.partials = (float *)(at_ + copies_.CopyBytes());
         return hipSuccess;
     }
 
     virtual hipError_t LaunchKernel(hipStream_t stream, bool guarded, const XGuardArgs &g) override
     {
         const hipEvent_t stop = TakeStopEvent();   // for the command's last kernel
-        if (at_ == nullptr) return LaunchPlan(plan_, A_, B_, K_, N_, stop, stream, guarded, g);
+        if (at_ == nullptr) {
+            Plan plan = plan_;
+            plan.part[0] = plan.part[0].Whole();
+            return LaunchPlan(plan, A_, B_, K_, N_, stop, stream, guarded, g);
+        }
+        if (copies_.plan.parts == 0) return LaunchPlan(plan_, A_, B_, K_, N_, stop, stream, guarded, g);
         const CopyPlan &c = copies_;
         const RowCopy a { A_, (uint16_t *)at_, (uint32_t)M_, (uint32_t)K_, (uint32_t)c.lda, c.a_groups };
         const RowCopy b { B_, (uint16_t *)(at_ + c.a_bytes), (uint32_t)K_, (uint32_t)N_, (uint32_t)c.ldb, c.b_groups };
@@ -1210,6 +1325,19 @@ private:
                            a, B, c, part.rows, N_, K_, tiles_n, g);
             return hipGetLastError();
         }
+        if (part.Split()) {
+            SplitK split = split_;
+            split.parts = (uint32_t)part.split_parts;
+            split.steps = (uint32_t)part.split_steps;
+            SplitKernel kernel = nullptr;
+            switch (part.fit) {
+            case Fit::kExact:     kernel = SplitKernelFor<Fit::kExact>(part, guarded); break;
+            case Fit::kEdges:     kernel = SplitKernelFor<Fit::kEdges>(part, guarded); break;
+            case Fit::kUnaligned: kernel = SplitKernelFor<Fit::kUnaligned>(part, guarded); break;
+            }
+            LaunchWithStop(stop, kernel, dim3((uint32_t)part.tiles), dim3(256), stream, a, B, c, part.rows, N_, K_, lda, ldb, g, split);
+            return hipGetLastError();
+        }
         Kernel kernel = nullptr;
         switch (part.fit) {
         case Fit::kExact:     kernel = KernelFor<Fit::kExact>(part, guarded); break;
@@ -1235,13 +1363,26 @@ private:
         return guarded ? GemmDeepKernel<true, kFit, kTinyTile, 4> : GemmDeepKernel<false, kFit, kTinyTile, 4>;
     }
 
+    using SplitKernel = void (*)(const uint16_t *, const uint16_t *, uint16_t *, int, int, int, int, int, XGuardArgs, SplitK);
+    template <Fit kFit>
+    static SplitKernel SplitKernelFor(const Part &part, bool guarded)
+    {
+        if (part.tile == kSmallTile) return guarded ? GemmSplitKernel<true, kFit, kSmallTile, 4> : GemmSplitKernel<false, kFit, kSmallTile, 4>;
+        return guarded ? GemmSplitKernel<true, kFit, kTinyTile, 4> : GemmSplitKernel<false, kFit, kTinyTile, 4>;
+    }
+
+    /// The plan where there is memory for copies and partial sums, and how much that takes.
+    const Plan &PlanWithScratch() const { return copies_.plan.parts != 0 ? copies_.plan : plan_; }
+    size_t ScratchBytes() const { return copies_.CopyBytes() + PlanWithScratch().PartialBytes(); }
+
     const uint16_t *A_, *B_;
     uint16_t *C_;
     const int M_, N_, K_;
     const Plan plan_;         // for A and B as they lie
     const CopyPlan copies_;   // for their copies
     std::shared_ptr<class SharedScratch> scratch_;
-    uint8_t *at_ = nullptr;   // the copies, A's first; nullptr: plan_
+    uint8_t *at_ = nullptr;   // the copies, A's first, then partial sums; nullptr: plan_, not split
+    SplitK split_ {};
     bool decided_ = false;
 };
 
@@ -1343,6 +1484,23 @@ inline bool ShortK(const void *A, const void *B, const void *C, int M, int N, in
     return K <= limit;
 }
 
+constexpr int kLeastSplitSteps = 17;   // below, less than a us can be won
+constexpr int kLeastPartSteps = 8;
+/// What a split adds: the partial sums on their way past the L2, the ticket, and the last group's way
+/// through all parts. Fitted to the products of QuickestPlan()'s comment, and a us more: what is won in a stream
+/// of commands is partly lost again where a command is waited for alone.
+inline double SplitMicros(const Part &part)
+{
+    const double parts = part.split_parts, groups = (double)part.tiles;
+    return part.tile == kSmallTile ? 1.0 + 0.3 * parts + 0.015 * groups : 0.5 + 0.25 * parts + 0.012 * groups;
+}
+
+inline double MicrosOfPlan(const Plan &plan, int K, double pace = 1.0)
+{
+    const Part &first = plan.part[0];
+    return first.Split() ? MicrosOf(first, first.split_steps * kStepK, pace) + SplitMicros(first) : MicrosOf(plan, K, pace);
+}
+
 /// The plan for a shape: the quickest by the estimate above of one launch on large, small or tiny
 /// tiles and of two, large tiles for the rows that fill whole tiles, or whole rounds of them, and
 /// whatever is quickest for the rest. Large tiles do more arithmetic per byte read from LDS, but a
@@ -1353,6 +1511,11 @@ inline bool ShortK(const void *A, const void *B, const void *C, int M, int N, in
 /// 126 on small ones, 2048^3 20.9 on small against 30.1 on tiny ones, 1024^3 5.8 on tiny ones against
 /// 9.4 on small ones). Rows without 16-byte alignment do not go straight into LDS, which the large
 /// tiles need (a tile on its way through registers beside their accumulators does not fit).
+/// Where tiny or small tiles leave compute units idle and K is long, K is divided (SplitK). us per command, whole / in 2 / 3 / 4 /
+/// 8 / 16 parts on tiles of 64: 128 x 128 x 8192 22.7 / 14.1 / 11.3 / 10.3 / 9.8 / 10.5, 256 x 256 x 4096 13.6 / 9.3 / 9.1 /
+/// 9.5 / 10.0 / 12.5, x 2048 8.5 / 8.1 / 8.2 / 8.7 / 9.5, 512 x 512 x 2048 9.0 / 8.5 / 9.1 / 10.1, 500 x 499 x 4095
+/// 23.4 / 15.4 / 13.2 / 13.5; whole on tiles of 64 / in 2 / 3 / 4 parts on tiles of 128: 1024 x 1024 x 8192 31.5 / 28.9 /
+/// 26.0 / 27.7, 1000 x 999 x 8001 44.3 / 46.6 / 36.9 / 34.4, but 1024 x 1024 x 4096 17.5 / 18.5 / 18.6 / 20.5.
 /// XSCHED_HIP_GEMM_TILE=64|128|256 overrides the tile where the shape allows (128: four stages).
 /// A plan of more tiles than the progress map holds is passed over for one that fits: 13413745 x
 /// 1280 x 1024, 262025 tiles by the count below, would be quickest as two launches of 262295.
@@ -1383,6 +1546,21 @@ inline Plan QuickestPlan(int M, int N, int K, Rows aligned)
         if (both < least) { least = both; best = Plan { { first, rest }, 2 }; }
     };
     consider((int64_t)(M / kLargeTile) * kLargeTile);                       // all whole large tiles
+    // K divided among the work-groups of a tile, as far as the tiles leave compute units idle
+    const int steps = (K + kStepK - 1) / kStepK;
+    for (const int tile : { kTinyTile, kSmallTile }) {
+        const Part whole = PartOf(0, M, N, K, aligned, tile);
+        if (whole.tiles > kMaxSplitTiles || steps < kLeastSplitSteps) continue;
+        for (int parts = 2; whole.tiles * (uint64_t)parts <= ComputeUnits(); ++parts) {
+            Part split = whole;
+            split.split_steps = (steps + parts - 1) / parts;
+            split.split_parts = (steps + split.split_steps - 1) / split.split_steps;
+            if (split.split_steps < kLeastPartSteps) break;
+            split.tiles *= (uint64_t)split.split_parts;
+            const double us = MicrosOf(split, split.split_steps * kStepK) + SplitMicros(split);
+            if (us < least) { least = us; best = Plan { { split, {} }, 1 }; }
+        }
+    }
     const int64_t in_row = (N + kLargeTile - 1) / kLargeTile;                // all whole rounds of large tiles
     const int64_t whole_rounds = (int64_t)TilesOf(M, N, kLargeTile) / ComputeUnits();
     consider(whole_rounds * ComputeUnits() / in_row * kLargeTile);
@@ -1432,7 +1610,7 @@ inline CopyPlan CopyPlanFor(const void *A, const void *B, const void *C, int M, 
     p.plan = QuickestPlan(M, N, K, Rows { true, Aligned(C, N) });
     if (p.Groups() > GuardState::kMaxWorkGroups) return CopyPlan {};
     const double copying = kCopyMicros + 2.0 * (double)(p.a_bytes + p.b_bytes) / kCopyRate;
-    return copying + MicrosOf(p.plan, K, kCopyPace) < MicrosOf(in_place, K) ? p : CopyPlan {};
+    return copying + MicrosOfPlan(p.plan, K, kCopyPace) < MicrosOfPlan(in_place, K) ? p : CopyPlan {};
 }
 
 /// Tiles by which a shape is accepted or refused. They are the tiles of the kernels that such shapes
@@ -1481,6 +1659,17 @@ EXPORT_C_FUNC XResult HipGemmBf16CopyPlanOf(const void *A, const void *B, const 
     PutParts(copies.plan, out);
     out[8] = (int32_t)copies.a_groups;
     out[9] = (int32_t)copies.b_groups;
+    return kXSchedSuccess;
+}
+
+EXPORT_C_FUNC XResult HipGemmBf16SplitsOf(const void *A, const void *B, const void *C, int M, int N, int K, int32_t *out)
+{
+    if (out == nullptr || M <= 0 || N <= 0 || K <= 0) return kXSchedErrorInvalidValue;
+    const int forced = gemm::ForcedTile();
+    const gemm::Plan plan = gemm::PlanFor(A, B, C, M, N, K, forced);
+    const gemm::CopyPlan copies = gemm::CopyPlanFor(A, B, C, M, N, K, forced, plan);
+    out[0] = plan.part[0].split_parts;
+    out[1] = copies.plan.parts != 0 ? copies.plan.part[0].split_parts : 0;
     return kXSchedSuccess;
 }
 
