@@ -454,21 +454,21 @@ private:
 
     void Fold(const Event &e)
     {
-        using Folder = void (Rounds::*)(const Event &);
-        static const std::map<EventType, Folder> folders = {
-            { kEventHint, &Rounds::FoldHint },
-            { kEventProcessCreate, &Rounds::FoldProcessCreate },
-            { kEventProcessDestroy, &Rounds::FoldProcessDestroy },
-            { kEventXQueueCreate, &Rounds::FoldQueueConfig },
-            { kEventXQueueConfigUpdate, &Rounds::FoldQueueConfig },
-            { kEventXQueueDestroy, &Rounds::FoldQueueDestroy },
-            { kEventXQueueReady, &Rounds::FoldQueueReady },
-            { kEventXQueueIdle, &Rounds::FoldQueueIdle },
-            { kEventXQueueQuery, &Rounds::FoldQueryOne },
-            { kEventXQueueQueryAll, &Rounds::FoldQueryAll },
-        };
-        auto it = folders.find(e.Type());
-        if (it != folders.end()) (this->*(it->second))(e);
+        // No static table: the exit hook that stops this thread was registered before such an object would be
+        // made, so the object would go first, and the rounds until then would look into freed memory.
+        switch (e.Type()) {
+        case kEventHint:               return FoldHint(e);
+        case kEventProcessCreate:      return FoldProcessCreate(e);
+        case kEventProcessDestroy:     return FoldProcessDestroy(e);
+        case kEventXQueueCreate:
+        case kEventXQueueConfigUpdate: return FoldQueueConfig(e);
+        case kEventXQueueDestroy:      return FoldQueueDestroy(e);
+        case kEventXQueueReady:        return FoldQueueReady(e);
+        case kEventXQueueIdle:         return FoldQueueIdle(e);
+        case kEventXQueueQuery:        return FoldQueryOne(e);
+        case kEventXQueueQueryAll:     return FoldQueryAll(e);
+        default:                       return;
+        }
     }
 
     LocalScheduler *const owner_;
