@@ -92,7 +92,8 @@ XResult HipAxpyCommandCreate(HwCommandHandle *cmd, float alpha, const void *x, v
  * of 8, matrices aligned to 16 bytes). Where rows of A or B do not, large products copy that matrix first, to
  * memory of the queue (up to 1 GiB, kept for the next command, given back with the queue; without
  * it, or on a stream under capture, the product takes up to twice as long). Every element is
- * summed in the same order on all paths. */
+ * summed in the same order on all paths but one: where the tiles do not fill the device and K is above 1024, K may be
+ * divided among work-groups, whose sums are added in an order that the sizes alone decide. */
 XResult HipGemmBf16CommandCreate(HwCommandHandle *cmd, const void *A, const void *B, void *C,
                                  int M, int N, int K, int guard);
 
