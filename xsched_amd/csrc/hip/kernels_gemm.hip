@@ -963,11 +963,16 @@ void GemmDeepBody(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
         constexpr int kUnroll = kTile == kTinyTile ? 4 : 1;   // parts read at a time: as many as fit into the registers
         const __amdgpu_buffer_rsrc_t parts = __builtin_amdgcn_make_buffer_rsrc((void *)(split.partials + (size_t)tile * split.parts * (kTile * kTile)), 0,
                                                                                (int)(split.parts * kPartBytes), 0x00020000);
+        // (The part is in the resource and not in a scalar offset: with one the compiler lets the next instruction write
+        // over the registers of a 16-byte store, as documented. Where it did so, in a form of eight waves,
+        // lanes 12-15 of sixteen now and then stored the address that came next in place of their first value.)
+        const __amdgpu_buffer_rsrc_t mine = __builtin_amdgcn_make_buffer_rsrc((void *)(split.partials + ((size_t)tile * split.parts + part) * (kTile * kTile)), 0,
+                                                                              kPartBytes, 0x00020000);
 #pragma unroll
         for (int n = 0; n < kPieces; ++n) {
             const f32x16 &v = acc[n / 4 / kBlocks][n / 4 % kBlocks];
             const f32x4 four = { v[n % 4 * 4], v[n % 4 * 4 + 1], v[n % 4 * 4 + 2], v[n % 4 * 4 + 3] };
-            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, four), parts, (n * kThreads + tid) * 16, part * kPartBytes, kDeviceScope);
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, four), mine, (n * kThreads + tid) * 16, 0, kDeviceScope);
         }
         XS_WAIT_GLOBAL_LOADS;   // (stores count as loads do)
         XS_BARRIER;
