@@ -102,8 +102,8 @@ XResult HipGemmBf16CommandCreate(HwCommandHandle *cmd, const void *A, const void
 
 /* For tests: how a GEMM of these matrices would be launched; nothing is launched or read. `out` receives
  * 8 values, four for each of at most two launches (zeroes where there is no second one):
- * rows of C, edge of a tile, kernel (0 two LDS buffers, 1 four stages, 2 any shape) and what it
- * assumes of the matrices (0 whole tiles, 1 16-byte rows, 2 nothing). No counterpart in the reference. */
+ * rows of C, columns of a tile, kernel (0 two LDS buffers, 1 four stages, 2 any shape) and what the
+ * matrices are to square tiles of that edge (0 whole tiles, 1 16-byte rows, 2 anything). No counterpart in the reference. */
 XResult HipGemmBf16PlanOf(const void *A, const void *B, const void *C, int M, int N, int K, int32_t *out);
 
 /* For tests: the same for the launches on copies of A and B whose rows start on 16-byte boundaries. `out`
@@ -111,6 +111,10 @@ XResult HipGemmBf16PlanOf(const void *A, const void *B, const void *C, int M, in
  * that copy A and B (0: not copied). Without memory for the copies, or on a stream under
  * capture, HipGemmBf16PlanOf() holds, with divided K in turn. No counterpart in the reference. */
 XResult HipGemmBf16CopyPlanOf(const void *A, const void *B, const void *C, int M, int N, int K, int32_t *out);
+
+/* For tests: rows of a tile in each of these launches (four values, 0: no such launch): the two of
+ * HipGemmBf16PlanOf(), then the two of HipGemmBf16CopyPlanOf(). No counterpart in the reference. */
+XResult HipGemmBf16TileRowsOf(const void *A, const void *B, const void *C, int M, int N, int K, int32_t *out);
 
 /* For tests: into how many parts the K of a tile is divided, out[0] where A and B are read as they lie, out[1] on their
  * copies (0: there are none). One work-group does them in turn on a stream under capture, or without memory. No counterpart in

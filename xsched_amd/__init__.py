@@ -127,6 +127,7 @@ HALHIP_API = {
     "HipGemmBf16SplitsOf": (XResult, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, POINTER(c_int32)]),
     "HipGemmBf16TicketsOf": (XResult, [c_uint64, POINTER(c_uint64)]),
     "HipGemmBf16CopyPlanOf": (XResult, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, POINTER(c_int32)]),
+    "HipGemmBf16TileRowsOf": (XResult, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, POINTER(c_int32)]),
     "HipHistogramCommandCreate": (XResult, [POINTER(c_uint64), c_void_p, c_size_t, c_void_p,
                                             c_uint32, c_int]),
     "HipHistogramLaunchNoAlloc": (XResult, [c_void_p, c_void_p, c_size_t, c_void_p, c_uint32]),

@@ -74,6 +74,7 @@ typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kLargeTile = 256;     // edge of the large tile of C (M and N)
+constexpr int kThreeQuarterRows = 192, kHalfRows = 128;   // rows of the large tile where fewer than 256 of them divide M better
 constexpr int kSmallTile = 128;     // edge of the small one
 constexpr int kTinyTile = 64;       // and of the smallest
 constexpr int kStepK = 64;          // K per step
@@ -176,11 +177,14 @@ enum TileRequest { kNoTile, kAnyButLast, kTheLast };
 // next to the MFMAs of the second slice the first fragments of tile t + 1 are read and the loads of
 // tile t + 2 go out.
 //
-// kTile x kTile is the tile of C, kWavesM x kWavesN the wave grid over it; a wave owns
-// kBlocksM x kBlocksN blocks of 16x16. Built for 256 with 2x4 waves (8x4 blocks
+// kTileM x kTileN is the tile of C, kWavesM x kWavesN the wave grid over it; a wave owns
+// kBlocksM x kBlocksN blocks of 16x16. Built for 256 x 256 with 2x4 waves (8x4 blocks
 // per wave), for exact shapes and for ragged ones (kEdges): there the last tile's loads, the last
 // step and the stores look at the edges, and the steps before are the same code (4000^3 146 us on
-// 128 x 128 tiles, 106 on these). And for 128 with 2x2 waves (4x4 blocks), exact shapes only: 64 KiB
+// 128 x 128 tiles, 106 on these). For 192 x 256 and 128 x 256, with the same waves of 6x4 and 4x4 blocks: a step
+// takes 1.08 and 0.82 us of a full round where 256 rows take 1.36, so a round that 256 rows leave half empty is shorter by up to
+// a quarter (who takes which: QuickestPlan()). More bytes go through LDS per flop (11 % and 33 %), which is why they are not taken
+// where whole rounds of 256 rows fit. And for 128 x 128 with 2x2 waves (4x4 blocks), exact shapes only: 64 KiB
 // of LDS and 4 waves, so two work-groups share a compute unit and one computes while the other
 // waits for its first loads or writes out. That is what outputs of 257 to 512 such tiles want,
 // which are two rounds for the four-stage kernel below (its 130 KiB let a unit have one group), and
@@ -193,29 +197,29 @@ enum TileRequest { kNoTile, kAnyButLast, kTheLast };
 //
 // (The body is a device function: the host pass cannot parse the buffer-resource builtins
 // and would silently drop the launch stub of a kernel that uses them directly.)
-template <bool kGuard, Fit kFit, int kTile, int kWavesM, int kWavesN>
+template <bool kGuard, Fit kFit, int kTileM, int kTileN, int kWavesM, int kWavesN>
 __device__ __forceinline__
 void GemmBf16Body(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B,
                   uint16_t *__restrict__ C, int M, int N, int K, int lda, int ldb, const XGuardArgs &g)
 {
     static_assert(kFit != Fit::kUnaligned, "loads go straight into LDS");
     constexpr int kWaves = kWavesM * kWavesN;
-    constexpr int kBlocksM = kTile / (16 * kWavesM);
-    constexpr int kBlocksN = kTile / (16 * kWavesN);
+    constexpr int kBlocksM = kTileM / (16 * kWavesM);
+    constexpr int kBlocksN = kTileN / (16 * kWavesN);
     constexpr int kMfmas = kBlocksM * kBlocksN;          // per wave and 32-wide k slice
     constexpr int kReads = kBlocksM + kBlocksN;          // fragments of a slice
-    constexpr int kABytes = kTile * kStepK * 2;          // one A tile in LDS
-    constexpr int kBBytes = kStepK * kTile * 2;          // one B tile
+    constexpr int kABytes = kTileM * kStepK * 2;          // one A tile in LDS
+    constexpr int kBBytes = kStepK * kTileN * 2;          // one B tile
     constexpr int kALoads = kABytes / 1024 / kWaves;     // wave-wide 1 KiB loads per wave and tile
     constexpr int kBLoads = kBBytes / 1024 / kWaves;
     constexpr int kLoads = kALoads + kBLoads;
     constexpr int kLoadEvery = kMfmas / kLoads;          // one load next to so many MFMAs
-    constexpr int kBRowBytes = kTile * 2;                // one k row of the B tile
+    constexpr int kBRowBytes = kTileN * 2;                // one k row of the B tile
     constexpr int kBSlotsPerRow = kBRowBytes / 16;
     constexpr int kBRowsPerLoad = 64 / kBSlotsPerRow;
     static_assert(kBlocksN == 4, "the block index is XORed into the granule number as two bits");
     static_assert(kBRowBytes >= 256, "a granule number has the three bits that are XORed");
-    static_assert(kLoadEvery * kLoads == kMfmas && 2 * kReads <= kMfmas, "loads and reads pair up with the MFMAs of a slice");
+    static_assert(kLoadEvery * kLoads <= kMfmas && 2 * kReads <= kMfmas, "loads and reads pair up with the MFMAs of a slice");
     // One LDS object for everything, the word the waves agree on a poll through included:
     // with a second object the compiler attaches alias scopes to the LDS accesses and then
     // makes every fragment read wait for all global loads that are on their way into LDS.
@@ -231,9 +235,9 @@ void GemmBf16Body(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
     const uint32_t wn = wave % kWavesN;
 
     uint32_t tm, tn;
-    const uint32_t tiles_m = ((uint32_t)M + kTile - 1) / kTile, tiles_n = ((uint32_t)N + kTile - 1) / kTile;
+    const uint32_t tiles_m = ((uint32_t)M + kTileM - 1) / kTileM, tiles_n = ((uint32_t)N + kTileN - 1) / kTileN;
     TileAt(WorkOf(blockIdx.x, tiles_m * tiles_n), tiles_m, tiles_n, tm, tn);
-    const size_t m0 = (size_t)tm * kTile, n0 = (size_t)tn * kTile;
+    const size_t m0 = (size_t)tm * kTileM, n0 = (size_t)tn * kTileN;
     const int steps = kFit == Fit::kExact ? K / kStepK : (K + kStepK - 1) / kStepK;
     const int rest = K - (steps - 1) * kStepK;           // K values of the last step
 
@@ -414,7 +418,7 @@ void GemmBf16Body(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
         for (int n = 0; n < kMfmas; ++n) {
             mfma(1, n);
             if (kReadAhead && n % 2 == 0 && n / 2 < kReads) read_frag(cur ^ 1, 0, n / 2);
-            if (n % kLoadEvery == kLoadEvery - 1) {
+            if (n % kLoadEvery == kLoadEvery - 1 && n / kLoadEvery < kLoads) {
                 if constexpr (kLoad == kAnyButLast) load_piece(cur, t + 2, n / kLoadEvery, false);
                 if constexpr (kLoad == kTheLast) load_piece(cur, t + 2, n / kLoadEvery, true);
             }
@@ -457,7 +461,7 @@ void GemmBf16Body(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
     // columns further completes 16 bytes per lane, and 8 rows x 128 bytes leave per store.
     constexpr int kStripColumnBytes = 64 + 16;
     constexpr int kStripBytes = 64 * kStripColumnBytes;
-    static_assert(2 * kABytes >= kWaves * kStripBytes, "the A buffers hold one strip per wave");
+    static_assert(2 * (kABytes + kBBytes) >= kWaves * kStripBytes, "the tile buffers hold one strip per wave");
     uint8_t *const strip = As0 + wave * kStripBytes;
     const uint32_t l16 = lane & 15, patch = lane >> 4;   // a patch: 4 rows x 32 columns per 16 lanes
     const uint32_t put_at = l16 * kStripColumnBytes + 4 * patch * 2;
@@ -492,12 +496,12 @@ void GemmBf16Body(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B
     if (kGuard) guard.Commit();
 }
 
-template <bool kGuard, Fit kFit, int kTile, int kWavesM, int kWavesN>
+template <bool kGuard, Fit kFit, int kTileM, int kTileN, int kWavesM, int kWavesN>
 __global__ __launch_bounds__(64 * kWavesM * kWavesN, 2 /* waves per SIMD: no accumulators move between AGPRs and VGPRs */)
 void GemmBf16Kernel(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B,
                     uint16_t *__restrict__ C, int M, int N, int K, int lda, int ldb, XGuardArgs g)
 {
-    GemmBf16Body<kGuard, kFit, kTile, kWavesM, kWavesN>(A, B, C, M, N, K, lda, ldb, g);
+    GemmBf16Body<kGuard, kFit, kTileM, kTileN, kWavesM, kWavesN>(A, B, C, M, N, K, lda, ldb, g);
 }
 
 
@@ -1279,6 +1283,7 @@ struct Part
     Fit fit;        // of kTwoBuffers and kFourStages
     Body body;
     uint64_t tiles; // work-groups, at least as many as bytes of the progress map (a byte for a tile)
+    int tile_rows;  // rows of a tile: as many as `tile`, or with 256 columns and two buffers fewer
     Sum sum = Sum::kOneGo;                  // the others: kFourStages, one launch for all of C
     int split_parts = 1, split_steps = 0;   // into how many parts of how many steps K is divided (SplitK)
 
@@ -1430,14 +1435,18 @@ private:
     }
 
     using Kernel = void (*)(const uint16_t *, const uint16_t *, uint16_t *, int, int, int, int, int, XGuardArgs);
+    template <Fit kFit, int kTileM, int kTileN, int kWavesM, int kWavesN>
+    static Kernel LargeKernelFor(bool guarded) { return guarded ? GemmBf16Kernel<true, kFit, kTileM, kTileN, kWavesM, kWavesN> : GemmBf16Kernel<false, kFit, kTileM, kTileN, kWavesM, kWavesN>; }
     template <Fit kFit>
     static Kernel KernelFor(const Part &part, bool guarded)
     {
         if constexpr (kFit == Fit::kExact) {
-            if (part.body == Body::kTwoBuffers && part.tile == kSmallTile) return guarded ? GemmBf16Kernel<true, kFit, kSmallTile, 2, 2> : GemmBf16Kernel<false, kFit, kSmallTile, 2, 2>;
+            if (part.body == Body::kTwoBuffers && part.tile == kSmallTile) return LargeKernelFor<kFit, kSmallTile, kSmallTile, 2, 2>(guarded);
         }
         if constexpr (kFit != Fit::kUnaligned) {
-            if (part.tile == kLargeTile) return guarded ? GemmBf16Kernel<true, kFit, kLargeTile, 2, 4> : GemmBf16Kernel<false, kFit, kLargeTile, 2, 4>;
+            if (part.tile == kLargeTile && part.tile_rows == kThreeQuarterRows) return LargeKernelFor<kFit, kThreeQuarterRows, kLargeTile, 2, 4>(guarded);
+            if (part.tile == kLargeTile && part.tile_rows == kHalfRows) return LargeKernelFor<kFit, kHalfRows, kLargeTile, 2, 4>(guarded);
+            if (part.tile == kLargeTile) return LargeKernelFor<kFit, kLargeTile, kLargeTile, 2, 4>(guarded);
         }
         if (part.tile == kSmallTile) return guarded ? GemmDeepKernel<true, kFit, kSmallTile, 4> : GemmDeepKernel<false, kFit, kSmallTile, 4>;
         return guarded ? GemmDeepKernel<true, kFit, kTinyTile, 4> : GemmDeepKernel<false, kFit, kTinyTile, 4>;
@@ -1470,10 +1479,11 @@ private:
     bool decided_ = false, no_memory_ = false;
 };
 
-inline uint64_t TilesOf(int M, int N, int tile)
+inline uint64_t TilesOf(int M, int N, int tile_rows, int tile)
 {
-    return ((uint64_t)M + (unsigned)tile - 1) / (unsigned)tile * (((uint64_t)N + (unsigned)tile - 1) / (unsigned)tile);
+    return ((uint64_t)M + (unsigned)tile_rows - 1) / (unsigned)tile_rows * (((uint64_t)N + (unsigned)tile - 1) / (unsigned)tile);
 }
+inline uint64_t TilesOf(int M, int N, int tile) { return TilesOf(M, N, tile, tile); }
 
 inline uint32_t ComputeUnits()
 {
@@ -1497,33 +1507,49 @@ inline int ForcedTile()
     return forced == kTinyTile || forced == kSmallTile || forced == kLargeTile ? (int)forced : 0;
 }
 
+/// XSCHED_HIP_GEMM_TILE_ROWS beside XSCHED_HIP_GEMM_TILE=256: 128, 192 or 256 (the default).
+inline int ForcedTileRows()
+{
+    int64_t rows = 0;
+    GetEnvInt64("XSCHED_HIP_GEMM_TILE_ROWS", rows);
+    return rows == kHalfRows || rows == kThreeQuarterRows ? (int)rows : kLargeTile;
+}
+
 /// What a plan may assume: rows of A and B (or of their copies), and rows of C, start on 16-byte boundaries.
 struct Rows { bool inputs, output; };
 
-inline Part PartOf(int first_row, int rows, int N, int K, Rows aligned, int tile)
+inline Part PartOf(int first_row, int rows, int N, int K, Rows aligned, int tile, int tile_rows)
 {
-    const bool exact = aligned.inputs && aligned.output && rows % tile == 0 && N % tile == 0 && K % kStepK == 0;
+    const bool exact = aligned.inputs && aligned.output && rows % tile_rows == 0 && N % tile == 0 && K % kStepK == 0;
     return Part { first_row, rows, tile, exact ? Fit::kExact : aligned.inputs ? Fit::kEdges : Fit::kUnaligned,
-                  tile == kLargeTile ? Body::kTwoBuffers : Body::kFourStages, TilesOf(rows, N, tile) };
+                  tile == kLargeTile ? Body::kTwoBuffers : Body::kFourStages, TilesOf(rows, N, tile_rows, tile), tile_rows };
 }
+inline Part PartOf(int first_row, int rows, int N, int K, Rows aligned, int tile) { return PartOf(first_row, rows, N, K, aligned, tile, tile); }
 
 /// Roughly how long a part takes, in us: a launch, then rounds of one tile per compute unit (two of
 /// 128 x 128 with two buffers), each with its first loads and its write-out, the last round quicker the fewer
-/// units it keeps busy. The rates are fitted to outputs of 4 to 4096 tiles of 128 x 128 at K from 128 to 8192:
-/// of 35 such products the plan is within 3 % of the quickest of the three tile sizes but for
-/// 2048 x 2048 x 8192 (66.3 us, 63.9 with the tile given) and 4096 x 4096 x 128 (11.4, 10.5).
+/// units it keeps busy: in proportion, or, on tiles of 192 x 256, only where few units idle (the cube: a full round runs
+/// against the power limit, and units that idle leave the others a higher clock; the rates of 256 x 256 are fitted without
+/// it, for their choice between one launch and two: with it 4992^3 is slower by 3 %). The rates are fitted to outputs of 4 to 4096 tiles of 128 x 128 at
+/// K from 128 to 8192: of 181 products, half of them ragged, each timed on every tile, what the plan takes is 0.7 % behind the
+/// quickest on average, and at most 7 % (K up to 320).
 inline double MicrosOf(const Part &part, int K, double pace = 1.0 /* of the steps */)
 {
     // us of a round, and per K step of a full round and of one with a single tile: [exact, edges, unaligned]
     struct Rates { double round, full, single; };
     constexpr Rates large[3] = { { 5.0, 1.36, 1.00 }, { 5.0, 1.43, 1.05 }, {} };
+    constexpr Rates three_quarters[3] = { { 4.5, 1.08, 0.80 }, { 5.0, 1.17, 0.86 }, {} };
+    constexpr Rates half[3] = { { 3.5, 0.82, 0.66 }, { 3.5, 0.86, 0.66 }, {} };
     constexpr Rates pair = { 1.7, 0.90, 0.45 };
     constexpr Rates small[3] = { { 2.5, 0.45, 0.37 }, { 2.5, 0.53, 0.41 }, { 2.5, 0.69, 0.48 } };
     constexpr Rates tiny[3] = { { 0.5, 0.195, 0.14 }, { 0.5, 0.25, 0.16 }, { 0.5, 0.32, 0.29 } };
     const bool two_per_unit = part.tile == kSmallTile && part.body == Body::kTwoBuffers;
-    const Rates &r = two_per_unit ? pair : (part.tile == kLargeTile ? large : part.tile == kSmallTile ? small : tiny)[(int)part.fit];
+    const bool power_bound = part.tile == kLargeTile && part.tile_rows == kThreeQuarterRows;
+    const Rates *const of_large = part.tile_rows == kLargeTile ? large : part.tile_rows == kThreeQuarterRows ? three_quarters : half;
+    const Rates &r = two_per_unit ? pair : (part.tile == kLargeTile ? of_large : part.tile == kSmallTile ? small : tiny)[(int)part.fit];
     const double rounds = (double)part.tiles / ((two_per_unit ? 2 : 1) * ComputeUnits()), whole = std::floor(rounds);
-    const double step = whole * r.full + (rounds > whole ? r.single + (r.full - r.single) * (rounds - whole) : 0.0);
+    const double busy = power_bound ? (rounds - whole) * (rounds - whole) * (rounds - whole) : rounds - whole;
+    const double step = whole * r.full + (rounds > whole ? r.single + (r.full - r.single) * busy : 0.0);
     return 3.0 + std::ceil(rounds) * r.round + pace * step * ((K + kStepK - 1) / kStepK);
 }
 
@@ -1601,7 +1627,9 @@ inline bool CanSplit(const Part &part) { return part.MapBytes() <= kMaxSplitTile
 
 /// The plan for a shape: the quickest by the estimate above of one launch on large, small or tiny
 /// tiles and of two, large tiles for the rows that fill whole tiles, or whole rounds of them, and
-/// whatever is quickest for the rest. Large tiles do more arithmetic per byte read from LDS, but a
+/// whatever is quickest for the rest. Large tiles have 256 columns and 256, 192 or 128 rows: outputs of 150 to 250 tiles of 256 x 256 leave
+/// compute units idle that 192 rows keep busy, ragged ones of 257 to 512 tiles of 128 x 128 are one round of 128 x 256 (us per command, without
+/// these and with them: 3072^3 57.4 -> 49.8, 3456 x 3456 x 512 18.0 -> 15.2, 7451 x 2632 x 1232 69.2 -> 56.8, 5801 x 760 x 3344 59.4 -> 51.3, 805 x 7704 x 104 12.1 -> 9.6). Large tiles do more arithmetic per byte read from LDS, but a
 /// round of few tiles leaves compute units idle (pass times in us, large and small tiles as they were
 /// chosen before by the share of the compute units covered and by exact multiples only, and now:
 /// 8197 x 8192 x 8192 1038 -> 836, 4100 x 4096 x 4096 156 -> 130, 6016 x 6016 x 8192 564 -> 485,
@@ -1656,6 +1684,17 @@ inline Plan QuickestPlan(int M, int N, int K, Rows aligned, int split_steps)
     const int64_t in_row = (N + kLargeTile - 1) / kLargeTile;                // all whole rounds of large tiles
     const int64_t whole_rounds = (int64_t)TilesOf(M, N, kLargeTile) / ComputeUnits();
     consider(whole_rounds * ComputeUnits() / in_row * kLargeTile);
+    // All of C on large tiles of fewer rows. Behind a whole round the estimates of these and of two launches are 5 % to 10 %
+    // off, each in its own direction: there they have to be quicker by more than that (4608^3 161 us in two launches and 155 on 192 rows, by the
+    // estimate 160 and 155; 4994 x 6840 x 456 58.8 and 53.9, by the estimate 45 and 44).
+    if (aligned.inputs) {
+        for (const int tile_rows : { kThreeQuarterRows, kHalfRows }) {
+            const Part part = PartOf(0, M, N, K, aligned, kLargeTile, tile_rows);
+            if (part.tiles > GuardState::kMaxWorkGroups) continue;
+            const double us = MicrosOf(part, K);
+            if ((part.tiles <= ComputeUnits() || best.parts == 1 ? us : us / 0.9) < least) { least = us; best = Plan { { part, {} }, 1 }; }
+        }
+    }
     return best;
 }
 
@@ -1665,7 +1704,7 @@ constexpr size_t kMaxScratchBytes = SharedScratch::kMaxBytes;   // copies of A a
 constexpr double kCopyMicros = 8.0;                 // launch of the copying kernel and the one behind it,
 constexpr double kCopyRate = 12e6;                  // bytes per us, read and written, as long as matrices and copies stay in the last-level
 constexpr double kCachedCopyBytes = 100e6;          // cache (256 MB): up to so many bytes of copies,
-constexpr double kFarCopyRate = 4.3e6;              // and for those beyond, with reading them again from memory,
+constexpr double kFarCopyRate = 3.5e6;              // and for those beyond, with reading them again from memory,
 constexpr double kCopyPace = 0.85;                  // time of a step on rows of whole cache lines against any rows on 16-byte boundaries
 
 inline double CopyMicros(const CopyPlan &p)
@@ -1733,20 +1772,20 @@ inline int SplitStepsFor(int M, int N, int K)
 /// in place / on copies: 500 x 499 x 4095 23.6 / 26.5; 1500 x 1499 x 4095 44.4 / 41.0, x 2047 25.8 / 29.8; 2000 x 1999
 /// x 2047 28.4 / 31.7, x 3001 38.9 / 38.8, x 4095 51.2 / 47.2; 2500 x 2501 x 1001 32.1 / 36.3; 3000 x 2999 x 301
 /// 28.0 / 28.5, x 101 25.5 / 23.7; 4000 x 3999 x 301 38.3 / 31.4; 1000 x 999 x 8001 44.3 / 43.5; 128 x 8191 x 8191
-/// 66.8 / 76.6. Above the size of the last-level cache: 8191 x 512 x 8191 80.7 / 110.9, 500 x 12287 x 8191 167 / 218, 16383 x 300 x
-/// 8191 166 / 242, 512 x 16383 x 8191 217 / 265, but 700 x 8191 x 8191 179 / 158, 8191 x 1023 x 8191 187 / 174, 8191 x 2047 x 8191
-/// 364 / 249. A pass of 8191^3 1791 / 918.
+/// 66.8 / 76.6. Above the size of the last-level cache (copies on large tiles of any rows): 8191 x 511 x 8191 89.5 / 113, 500 x 12287 x 8191 166 / 211, 16383 x 300 x
+/// 8191 162 / 239, 512 x 16383 x 8191 216 / 247, but 8191 x 767 x 8191 165 / 151, 700 x 8191 x 8191 176 / 151, 8191 x 1023 x 8191 180 / 164, 600 x 16383 x 4095
+/// 138 / 126, 900 x 16383 x 4095 204 / 148, 8191 x 2047 x 8191 359 / 254. A pass of 8191^3 1791 / 918.
 inline Plans PlansFor(const void *A, const void *B, const void *C, int M, int N, int K, int forced)
 {
     Plans plans {};
-    plans.in_place = Plan { { Part { 0, M, kAnyTile, Fit::kUnaligned, Body::kAnyShape, TilesOf(M, N, kAnyTile) }, {} }, 1 };
+    plans.in_place = Plan { { Part { 0, M, kAnyTile, Fit::kUnaligned, Body::kAnyShape, TilesOf(M, N, kAnyTile), kAnyTile }, {} }, 1 };
     plans.without_memory = plans.in_place;
     if (N < 8 || (int64_t)M * K < 8 || K > kMaxK || N > kMaxK) return plans;
     if (forced == 0 && ShortK(A, B, C, M, N, K)) return plans;
     const bool a_aligned = Aligned(A, K), b_aligned = Aligned(B, N);
     const Rows aligned { a_aligned && b_aligned, Aligned(C, N) };
     if (forced != 0 && (forced != kLargeTile || aligned.inputs)) {
-        plans.in_place = Plan { { PartOf(0, M, N, K, aligned, forced), {} }, 1 };
+        plans.in_place = Plan { { PartOf(0, M, N, K, aligned, forced, forced == kLargeTile ? ForcedTileRows() : forced), {} }, 1 };
         plans.without_memory = plans.in_place;
         return plans;
     }
@@ -1790,22 +1829,27 @@ inline uint64_t CountedTiles(const void *A, const void *B, const void *C, int M,
 
 using namespace xsched::hip;
 
-static void PutParts(const gemm::Plan &plan, int32_t *out)
+static void PutParts(const gemm::Plan &plan, const void *C, int N, int K, int32_t *out)
 {
     for (int i = 0; i < 8; ++i) out[i] = 0;
     for (int i = 0; i < plan.parts; ++i) {
         const gemm::Part &part = plan.part[i];
+        gemm::Fit fit = part.fit;
+        if (part.tile_rows != part.tile) {   // said of square tiles, whatever rows the launch's tiles have
+            const bool whole = part.rows % part.tile == 0 && N % part.tile == 0 && K % gemm::kStepK == 0 && gemm::Aligned(C, N);
+            fit = whole ? gemm::Fit::kExact : gemm::Fit::kEdges;
+        }
         out[4 * i + 0] = part.rows;
         out[4 * i + 1] = part.tile;
         out[4 * i + 2] = (int32_t)part.body;
-        out[4 * i + 3] = (int32_t)part.fit;
+        out[4 * i + 3] = (int32_t)fit;
     }
 }
 
 EXPORT_C_FUNC XResult HipGemmBf16PlanOf(const void *A, const void *B, const void *C, int M, int N, int K, int32_t *out)
 {
     if (out == nullptr || M <= 0 || N <= 0 || K <= 0) return kXSchedErrorInvalidValue;
-    PutParts(gemm::PlansFor(A, B, C, M, N, K, gemm::ForcedTile()).in_place, out);
+    PutParts(gemm::PlansFor(A, B, C, M, N, K, gemm::ForcedTile()).in_place, C, N, K, out);
     return kXSchedSuccess;
 }
 
@@ -1813,9 +1857,20 @@ EXPORT_C_FUNC XResult HipGemmBf16CopyPlanOf(const void *A, const void *B, const 
 {
     if (out == nullptr || M <= 0 || N <= 0 || K <= 0) return kXSchedErrorInvalidValue;
     const gemm::CopyPlan copies = gemm::PlansFor(A, B, C, M, N, K, gemm::ForcedTile()).copies;
-    PutParts(copies.plan, out);
+    PutParts(copies.plan, C, N, K, out);
     out[8] = (int32_t)copies.a_groups;
     out[9] = (int32_t)copies.b_groups;
+    return kXSchedSuccess;
+}
+
+EXPORT_C_FUNC XResult HipGemmBf16TileRowsOf(const void *A, const void *B, const void *C, int M, int N, int K, int32_t *out)
+{
+    if (out == nullptr || M <= 0 || N <= 0 || K <= 0) return kXSchedErrorInvalidValue;
+    const gemm::Plans plans = gemm::PlansFor(A, B, C, M, N, K, gemm::ForcedTile());
+    for (int i = 0; i < 2; ++i) {
+        out[i] = i < plans.in_place.parts ? plans.in_place.part[i].tile_rows : 0;
+        out[2 + i] = i < plans.copies.plan.parts ? plans.copies.plan.part[i].tile_rows : 0;
+    }
     return kXSchedSuccess;
 }
 
