@@ -3,7 +3,7 @@
 // HBM-bound: 12 bytes of traffic per element (read x, read y, write y). The unit of
 // work is a chunk of `steps` x 1024 contiguous elements, walked by one wavefront in
 // steps of 4 x 128-bit accesses per lane and stream, lane-contiguous so that every
-// access of a wave covers 1 KiB. Loads and stores are non-temporal: nothing is reused.
+// access of a wave covers 1 KiB. Loads are non-temporal, nothing is reused; so are the stores of long arrays.
 // Because the update is in place, a chunk must be applied exactly once: the wave reads
 // the preempt word before it stores anything, and commits the chunk's byte in the
 // progress map after its last store.
@@ -49,6 +49,22 @@ typedef float float4 __attribute__((ext_vector_type(4), aligned(4)));
 __device__ __forceinline__ float4 ld_nt(const float4 *p) { return __builtin_nontemporal_load(p); }
 __device__ __forceinline__ void st_nt(float4 *p, float4 v) { __builtin_nontemporal_store(v, p); }
 
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+/// Piece u of a wave's step that begins at `first` (uniform). kThrough: the store goes through the L2 to the
+/// last-level cache (device scope, sc1). A launch over a short array otherwise ends by writing back
+/// what its stores left in the L2s.
+template <bool kThrough>
+__device__ __forceinline__ void StoreLanes(float4 *first, uint32_t lane, uint32_t u, float4 v)
+{
+    if constexpr (kThrough) {
+        const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(first, 0, 0x7fffffff, 0x00020000);
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), r, (int)(lane * 16 + u * kLanes * 16), 0, 0x10);
+    } else {
+        st_nt(first + u * kLanes + lane, v);
+    }
+}
+
 __device__ __forceinline__ float4 fma4(float a, float4 x, float4 y)
 {
     float4 r;
@@ -63,7 +79,7 @@ __device__ __forceinline__ float4 fma4(float a, float4 x, float4 y)
 // the last work-group.
 // kVecPerStep float4 per lane and stream are requested before anything is stored:
 // 4 -> steps of 1024 elements, 8 -> steps of 2048 elements.
-template <bool kGuard, uint32_t kVecPerStep>
+template <bool kGuard, uint32_t kVecPerStep, bool kThrough>
 __global__ __launch_bounds__(64)
 void AxpyVec4Kernel(float alpha, const float *x_first, float *y_first,
                     uint64_t n4, uint32_t tail, uint32_t steps, XGuardArgs g)
@@ -94,7 +110,7 @@ void AxpyVec4Kernel(float alpha, const float *x_first, float *y_first,
             }
 #pragma unroll
             for (uint32_t u = 0; u < kVecPerStep; ++u) {
-                st_nt(&y[base + u * kLanes], fma4(alpha, xv[u], yv[u]));
+                StoreLanes<kThrough>(y + wg_base + (uint64_t)s * kStepVecs, lane, u, fma4(alpha, xv[u], yv[u]));
             }
         }
     } else {
@@ -118,7 +134,7 @@ void AxpyVec4Kernel(float alpha, const float *x_first, float *y_first,
 // way and step j+kDepth is requested right behind the stores. The preempt word is read
 // in front of the first store of every chunk; a chunk that has begun is finished and
 // committed, so it is applied exactly once.
-template <uint32_t kDepth, bool kGuard>
+template <uint32_t kDepth, bool kGuard, bool kThrough>
 __global__ __launch_bounds__(64)
 void AxpyPersistentKernel(float alpha, const float *x_first, float *y_first, uint64_t n4, uint32_t tail,
                           uint32_t steps, uint32_t n_chunks, XGuardArgs g)
@@ -195,10 +211,10 @@ void AxpyPersistentKernel(float alpha, const float *x_first, float *y_first, uin
                 }
             }
             if (full && !skip) {
-                const uint64_t base = ((uint64_t)c * steps + st) * kStepVecs + lane;
+                float4 *const first = y + ((uint64_t)c * steps + st) * kStepVecs;
 #pragma unroll
                 for (uint32_t u = 0; u < kVecPerStep; ++u) {
-                    st_nt(&y[base + u * kLanes], fma4(alpha, xv[d][u], yv[d][u]));
+                    StoreLanes<kThrough>(first, lane, u, fma4(alpha, xv[d][u], yv[d][u]));
                 }
                 if (kGuard && st == steps - 1 && g.done && lane == 0) xguard_commit(g, c);
             }
@@ -233,31 +249,43 @@ protected:
     {
         if (n_ == 0) return hipSuccess;
         const hipEvent_t stop = TakeStopEvent();
+        if (n_ <= kThroughElems) Launch<true>(guarded, stop, stream, g);
+        else Launch<false>(guarded, stop, stream, g);
+        return hipGetLastError();
+    }
+
+private:
+    template <bool kThrough>
+    void Launch(bool guarded, hipEvent_t stop, hipStream_t stream, const XGuardArgs &g)
+    {
         const dim3 grid(n_wg_), block(kLanes);
         const uint32_t waves = PersistentWaves(n_wg_);
         const uint64_t n4 = n_ / 4;
         const uint32_t tail = (uint32_t)(n_ % 4);
         if (guarded && !chunk_grid_) {
             const dim3 pgrid(n_wg_ < waves ? n_wg_ : waves);
-            LaunchWithStop(stop, (AxpyPersistentKernel<3, true>), pgrid, block, stream, alpha_, x_, y_, n4, tail, steps_, n_wg_, g);
+            LaunchWithStop(stop, (AxpyPersistentKernel<3, true, kThrough>), pgrid, block, stream, alpha_, x_, y_, n4, tail, steps_, n_wg_, g);
         } else if (!guarded && !chunk_grid_ && n_wg_ >= kLongChunks) {
             // A long array: the same few long-lived waves stream it as fast as one wave per
             // chunk does and leave nearly all wave slots to whatever else runs on the device.
-            LaunchWithStop(stop, (AxpyPersistentKernel<3, false>), dim3(waves), block, stream, alpha_, x_, y_, n4, tail, steps_, n_wg_, g);
+            LaunchWithStop(stop, (AxpyPersistentKernel<3, false, kThrough>), dim3(waves), block, stream, alpha_, x_, y_, n4, tail, steps_, n_wg_, g);
         } else {
             // An even chunk is walked in steps of 2048 elements (8 accesses in flight
             // per lane and stream), an odd one in steps of 1024.
             const bool wide = (steps_ % 2) == 0;
             const uint32_t steps = wide ? steps_ / 2 : steps_;
-            if (guarded && wide)       LaunchWithStop(stop, (AxpyVec4Kernel<true, 8>), grid, block, stream, alpha_, x_, y_, n4, tail, steps, g);
-            else if (guarded)          LaunchWithStop(stop, (AxpyVec4Kernel<true, 4>), grid, block, stream, alpha_, x_, y_, n4, tail, steps, g);
-            else if (wide)             LaunchWithStop(stop, (AxpyVec4Kernel<false, 8>), grid, block, stream, alpha_, x_, y_, n4, tail, steps, g);
-            else                       LaunchWithStop(stop, (AxpyVec4Kernel<false, 4>), grid, block, stream, alpha_, x_, y_, n4, tail, steps, g);
+            if (guarded && wide)       LaunchWithStop(stop, (AxpyVec4Kernel<true, 8, kThrough>), grid, block, stream, alpha_, x_, y_, n4, tail, steps, g);
+            else if (guarded)          LaunchWithStop(stop, (AxpyVec4Kernel<true, 4, kThrough>), grid, block, stream, alpha_, x_, y_, n4, tail, steps, g);
+            else if (wide)             LaunchWithStop(stop, (AxpyVec4Kernel<false, 8, kThrough>), grid, block, stream, alpha_, x_, y_, n4, tail, steps, g);
+            else                       LaunchWithStop(stop, (AxpyVec4Kernel<false, 4, kThrough>), grid, block, stream, alpha_, x_, y_, n4, tail, steps, g);
         }
-        return hipGetLastError();
     }
 
-private:
+    /// Up to here stores go through the L2. Passes through a queue, us, three pairs of arrays in turn, non-temporal stores / these:
+    /// level 1 2^21 elements 15.3 / 13.9, 2^22 19.0 / 18.0, 2^23 27.2 / 25.7, 2^24 43.1 / 39.9, 2^25 75.5 / 75.2, 2^28 529 / 543; level 2
+    /// (long-lived waves, which wait for older stores with their loads) 2^21 15.7 / 14.4, 2^22 19.1 / 18.5, 2^23 28.0 / 27.3, 2^24 43.8 / 43.4,
+    /// 2^25 76 / 102.
+    static constexpr uint64_t kThroughElems = (uint64_t)1 << 24;
     static constexpr uint32_t kLongChunks = 8192;   // from here on a plain launch uses long-lived waves
 
     /// Long-lived waves of a launch over n_wg chunks: two per compute unit for long arrays, more
