@@ -283,15 +283,15 @@ private:
 
     /// Up to here stores go through the L2. Passes through a queue, us, three pairs of arrays in turn, non-temporal stores / these:
     /// level 1 2^21 elements 15.3 / 13.9, 2^22 19.0 / 18.0, 2^23 27.2 / 25.7, 2^24 43.1 / 39.9, 2^25 75.5 / 75.2, 2^28 529 / 543; level 2
-    /// (long-lived waves, which wait for older stores with their loads) 2^21 15.7 / 14.4, 2^22 19.1 / 18.5, 2^23 28.0 / 27.3, 2^24 43.8 / 43.4,
-    /// 2^25 76 / 102.
+    /// (long-lived waves, which wait for older stores with their loads: with these stores more of them pay) 2^21 15.7 / 14.4, 2^22 19.1 / 18.5, 2^23 28.0 / 27.2,
+    /// 2^24 43.8 / 40.7, on two waves per CU 2^25 76 / 102.
     static constexpr uint64_t kThroughElems = (uint64_t)1 << 24;
     static constexpr uint32_t kLongChunks = 8192;   // from here on a plain launch uses long-lived waves
 
     /// Long-lived waves of a launch over n_wg chunks: two per compute unit for long arrays, more
     /// while each has only a few chunks, where what counts is how many requests are out at once
-    /// (us at 2, 4, 8 waves per CU: 2^21 elements 6.8, 6.4, 5.9; 2^22 11.2, 10.3, 9.7; 2^23
-    /// 18.9, 18.1, 18.2; 2^24 34.5, 33.5, 33.9; 2^25 65.2, 65.4, 66.0; 2^28 511, 549, 557).
+    /// (us per command at level 2 and 2, 4, 8, 12 waves per CU: 2^21 elements 8.6, 8.4, 8.0, 7.5; 2^22 13.2, 11.2, 10.7, 10.3; 2^23
+    /// 25.4, 19.0, 17.7, 17.2; 2^24 49.1, 35.1, 33.3, 33.0; with non-temporal stores 2^25 69.3, 67.4, 67.3, 69.7; 2^28 513, 554, 558, 569).
     static uint32_t PersistentWaves(uint32_t n_wg)
     {
         static const uint32_t cus = []() {
@@ -305,7 +305,7 @@ private:
             return per_cu < 0 ? (int64_t)1 : per_cu > 64 ? (int64_t)64 : per_cu;
         }();
         if (asked > 0) return (uint32_t)asked * cus;
-        return (n_wg <= 16 * cus ? 8 : n_wg <= 64 * cus ? 4 : 2) * cus;
+        return (n_wg <= 64 * cus ? 8 : 2) * cus;
     }
 
     const float alpha_;
