@@ -3,7 +3,8 @@
 // HBM-bound: 12 bytes of traffic per element (read x, read y, write y). The unit of
 // work is a chunk of `steps` x 1024 contiguous elements, walked by one wavefront in
 // steps of 4 x 128-bit accesses per lane and stream, lane-contiguous so that every
-// access of a wave covers 1 KiB. Loads are non-temporal, nothing is reused; so are the stores of long arrays.
+// access of a wave covers 1 KiB. Loads are non-temporal, nothing is reused; so are the
+// stores of long arrays. Chunks begin on a line of y (HeadOf()).
 // Because the update is in place, a chunk must be applied exactly once: the wave reads
 // the preempt word before it stores anything, and commits the chunk's byte in the
 // progress map after its last store.
@@ -43,7 +44,7 @@ constexpr uint32_t kStepElems = 1024;                      // unit in which chun
 // 128-bit access unit. It is declared aligned to its elements only: a global access of 128 bits
 // takes any multiple of four bytes, so slices of larger arrays run on the same kernels. Aligned
 // arrays lose nothing by it (2^28 elements: 508 us, 511 with 16-byte alignment declared), arrays
-// four bytes off an aligned address take 3-6 % longer (2^24: 35.5 us against 34.3).
+// off their lines lose a few per cent where their stores are (HeadOf()).
 typedef float float4 __attribute__((ext_vector_type(4), aligned(4)));
 
 __device__ __forceinline__ float4 ld_nt(const float4 *p) { return __builtin_nontemporal_load(p); }
@@ -76,13 +77,13 @@ __device__ __forceinline__ float4 fma4(float a, float4 x, float4 y)
 }
 
 // n4: number of whole float4 in the arrays; tail: the 0..3 trailing scalars, done by
-// the last work-group.
+// the last work-group; head: elements in front of x_first and y_first, done with chunk 0 (HeadOf()).
 // kVecPerStep float4 per lane and stream are requested before anything is stored:
 // 4 -> steps of 1024 elements, 8 -> steps of 2048 elements.
 template <bool kGuard, uint32_t kVecPerStep, bool kThrough>
 __global__ __launch_bounds__(64)
 void AxpyVec4Kernel(float alpha, const float *x_first, float *y_first,
-                    uint64_t n4, uint32_t tail, uint32_t steps, XGuardArgs g)
+                    uint64_t n4, uint32_t tail, uint32_t head, uint32_t steps, XGuardArgs g)
 {
     const float4 *const x = (const float4 *)x_first;
     float4 *const y = (float4 *)y_first;
@@ -98,6 +99,11 @@ void AxpyVec4Kernel(float alpha, const float *x_first, float *y_first,
     // SIMD the extra round trip does not show in the bandwidth (measured).
     if (kGuard) {
         if (!guard.Enter()) return;
+    }
+    if (wg == 0 && lane < head) {
+        const float *const xs = x_first - head;
+        float *const ys = y_first - head;
+        ys[lane] = __builtin_fmaf(alpha, xs[lane], ys[lane]);
     }
     if (full) {
         for (uint32_t s = 0; s < steps; ++s) {
@@ -137,7 +143,7 @@ void AxpyVec4Kernel(float alpha, const float *x_first, float *y_first,
 template <uint32_t kDepth, bool kGuard, bool kThrough>
 __global__ __launch_bounds__(64)
 void AxpyPersistentKernel(float alpha, const float *x_first, float *y_first, uint64_t n4, uint32_t tail,
-                          uint32_t steps, uint32_t n_chunks, XGuardArgs g)
+                          uint32_t head, uint32_t steps, uint32_t n_chunks, XGuardArgs g)
 {
     const float4 *const x = (const float4 *)x_first;
     float4 *const y = (float4 *)y_first;
@@ -195,6 +201,11 @@ void AxpyPersistentKernel(float alpha, const float *x_first, float *y_first, uin
                     if (!v.run) return;
                     skip = g.resume && g.done && xguard_committed(g, c);
                 }
+                if (!skip && c == 0 && lane < head) {
+                    const float *const xs = x_first - head;
+                    float *const ys = y_first - head;
+                    ys[lane] = __builtin_fmaf(alpha, xs[lane], ys[lane]);
+                }
                 if (!skip && !full) {
                     // the last chunk of an array that does not fill it, and the 0..3 scalars behind
                     const uint64_t chunk_base = (uint64_t)c * steps * kStepVecs;
@@ -239,17 +250,33 @@ class HipAxpyCommand final : public HipGuardedCommand
 {
 public:
     /// steps: chunk size per work-group in units of 1024 elements.
-    HipAxpyCommand(float alpha, const float *x, float *y, size_t n, uint32_t steps, uint32_t n_wg,
+    /// head: HeadOf(), which the chunks do not count.
+    HipAxpyCommand(float alpha, const float *x, float *y, size_t n, uint32_t head, uint32_t steps, uint32_t n_wg,
                    int guard_mode, bool chunk_grid)
-        : HipGuardedCommand(n_wg, guard_mode), alpha_(alpha), x_(x), y_(y), n_(n), steps_(steps)
+        : HipGuardedCommand(n_wg, guard_mode), alpha_(alpha), x_(x), y_(y), n_(n), head_(head), steps_(steps)
         , chunk_grid_(chunk_grid) {}
+
+    /// Elements of y in front of its first 128-byte line. Chunks begin behind them, so that a wave's stores cover whole lines:
+    /// of an array off its lines each store of 1 KiB began and ended inside a line, which two waves then
+    /// wrote in pieces. us per command in a stream of them from an odd offset, before (non-temporal stores) and with this, on one pair of arrays and on 800 MB
+    /// in turn: level 1 2^20 elements 4.8 / 3.8 and 5.6 / 5.1, 3 x 2^20 7.3 / 5.8 and 9.2 / 8.6, 2^23 16.8 / 16.1
+    /// and 19.1 / 18.6, 2^24 33.4 / 29.9 and 35.0 / 35.0; level 2 3 x 2^20 8.0 / 7.7 and 9.4 / 9.2, 2^24 34.0 / 31.2 and 35.3 / 35.4
+    /// (2^24 with stores through the L2 and chunks off the lines: 31.4 and 39.6).
+    static uint32_t HeadOf(const float *y, size_t n)
+    {
+        const uint32_t off = (uint32_t)((uintptr_t)y & 127);
+        if (off == 0 || off % 4 != 0) return 0;
+        const uint32_t head = (128 - off) / 4;
+        return n < head ? (uint32_t)n : head;
+    }
 
 protected:
     virtual hipError_t LaunchKernel(hipStream_t stream, bool guarded, const XGuardArgs &g) override
     {
         if (n_ == 0) return hipSuccess;
         const hipEvent_t stop = TakeStopEvent();
-        if (n_ <= kThroughElems) Launch<true>(guarded, stop, stream, g);
+        const bool chunks = chunk_grid_ || (!guarded && n_wg_ < kLongChunks);   // one wave per chunk
+        if (chunks ? n_ <= kThroughChunks : n_ > kThroughFrom && n_ <= kThroughTo) Launch<true>(guarded, stop, stream, g);
         else Launch<false>(guarded, stop, stream, g);
         return hipGetLastError();
     }
@@ -259,40 +286,47 @@ private:
     void Launch(bool guarded, hipEvent_t stop, hipStream_t stream, const XGuardArgs &g)
     {
         const dim3 grid(n_wg_), block(kLanes);
-        const uint32_t waves = PersistentWaves(n_wg_);
-        const uint64_t n4 = n_ / 4;
-        const uint32_t tail = (uint32_t)(n_ % 4);
+        const uint32_t waves = PersistentWaves(n_wg_, kThrough);
+        const float *const x = x_ + head_;
+        float *const y = y_ + head_;
+        const uint64_t n4 = (n_ - head_) / 4;
+        const uint32_t tail = (uint32_t)((n_ - head_) % 4);
         if (guarded && !chunk_grid_) {
             const dim3 pgrid(n_wg_ < waves ? n_wg_ : waves);
-            LaunchWithStop(stop, (AxpyPersistentKernel<3, true, kThrough>), pgrid, block, stream, alpha_, x_, y_, n4, tail, steps_, n_wg_, g);
+            LaunchWithStop(stop, (AxpyPersistentKernel<3, true, kThrough>), pgrid, block, stream, alpha_, x, y, n4, tail, head_, steps_, n_wg_, g);
         } else if (!guarded && !chunk_grid_ && n_wg_ >= kLongChunks) {
             // A long array: the same few long-lived waves stream it as fast as one wave per
             // chunk does and leave nearly all wave slots to whatever else runs on the device.
-            LaunchWithStop(stop, (AxpyPersistentKernel<3, false, kThrough>), dim3(waves), block, stream, alpha_, x_, y_, n4, tail, steps_, n_wg_, g);
+            LaunchWithStop(stop, (AxpyPersistentKernel<3, false, kThrough>), dim3(waves), block, stream, alpha_, x, y, n4, tail, head_, steps_, n_wg_, g);
         } else {
             // An even chunk is walked in steps of 2048 elements (8 accesses in flight
             // per lane and stream), an odd one in steps of 1024.
             const bool wide = (steps_ % 2) == 0;
             const uint32_t steps = wide ? steps_ / 2 : steps_;
-            if (guarded && wide)       LaunchWithStop(stop, (AxpyVec4Kernel<true, 8, kThrough>), grid, block, stream, alpha_, x_, y_, n4, tail, steps, g);
-            else if (guarded)          LaunchWithStop(stop, (AxpyVec4Kernel<true, 4, kThrough>), grid, block, stream, alpha_, x_, y_, n4, tail, steps, g);
-            else if (wide)             LaunchWithStop(stop, (AxpyVec4Kernel<false, 8, kThrough>), grid, block, stream, alpha_, x_, y_, n4, tail, steps, g);
-            else                       LaunchWithStop(stop, (AxpyVec4Kernel<false, 4, kThrough>), grid, block, stream, alpha_, x_, y_, n4, tail, steps, g);
+            if (guarded && wide)       LaunchWithStop(stop, (AxpyVec4Kernel<true, 8, kThrough>), grid, block, stream, alpha_, x, y, n4, tail, head_, steps, g);
+            else if (guarded)          LaunchWithStop(stop, (AxpyVec4Kernel<true, 4, kThrough>), grid, block, stream, alpha_, x, y, n4, tail, head_, steps, g);
+            else if (wide)             LaunchWithStop(stop, (AxpyVec4Kernel<false, 8, kThrough>), grid, block, stream, alpha_, x, y, n4, tail, head_, steps, g);
+            else                       LaunchWithStop(stop, (AxpyVec4Kernel<false, 4, kThrough>), grid, block, stream, alpha_, x, y, n4, tail, head_, steps, g);
         }
     }
 
-    /// Up to here stores go through the L2. Passes through a queue, us, three pairs of arrays in turn, non-temporal stores / these:
-    /// level 1 2^21 elements 15.3 / 13.9, 2^22 19.0 / 18.0, 2^23 27.2 / 25.7, 2^24 43.1 / 39.9, 2^25 75.5 / 75.2, 2^28 529 / 543; level 2
-    /// (long-lived waves, which wait for older stores with their loads: with these stores more of them pay) 2^21 15.7 / 14.4, 2^22 19.1 / 18.5, 2^23 28.0 / 27.2,
-    /// 2^24 43.8 / 40.7, on two waves per CU 2^25 76 / 102.
-    static constexpr uint64_t kThroughElems = (uint64_t)1 << 24;
+    /// Arrays of up to kThroughChunks elements on one wave per chunk, and of kThroughFrom to kThroughTo on long-lived
+    /// waves, are stored through the L2. us per command in a stream of them, non-temporal stores / these, on one pair of arrays
+    /// and on pairs of 800 MB in turn (nothing is in the last-level cache then): level 1 2^22 elements 6.9 / 6.2 and 10.1 / 10.0,
+    /// 6 x 2^20 10.9 / 11.5 and 13.8 / 13.9, 2^23 15.2 / 15.8 and 17.9 / 18.7, 12 x 2^20 23.4 / 22.3 and 25.7 / 26.8, 2^24 31.1 / 29.6 and
+    /// 33.1 / 34.5; level 2 3 x 2^20 5.4 / 6.2 and 7.7 / 7.9, 2^23 15.5 / 15.6 and 18.5 / 18.7, 12 x 2^20 23.6 / 22.5 and 26.2 / 26.9,
+    /// 2^24 32.0 / 30.1 and 33.7 / 34.7. Three pairs of 2^24 in turn, a pass through a queue: level 1 43.1 / 39.9, level 2 43.8 / 40.7. Above,
+    /// these are slower (level 1 2^28 529 / 543, level 2 2^25 76 / 102).
+    static constexpr uint64_t kThroughChunks = (uint64_t)1 << 22;
+    static constexpr uint64_t kThroughFrom = (uint64_t)1 << 23, kThroughTo = (uint64_t)1 << 24;
     static constexpr uint32_t kLongChunks = 8192;   // from here on a plain launch uses long-lived waves
 
     /// Long-lived waves of a launch over n_wg chunks: two per compute unit for long arrays, more
     /// while each has only a few chunks, where what counts is how many requests are out at once
-    /// (us per command at level 2 and 2, 4, 8, 12 waves per CU: 2^21 elements 8.6, 8.4, 8.0, 7.5; 2^22 13.2, 11.2, 10.7, 10.3; 2^23
-    /// 25.4, 19.0, 17.7, 17.2; 2^24 49.1, 35.1, 33.3, 33.0; with non-temporal stores 2^25 69.3, 67.4, 67.3, 69.7; 2^28 513, 554, 558, 569).
-    static uint32_t PersistentWaves(uint32_t n_wg)
+    /// (us per command at level 2 and 2, 4, 8, 12 waves per CU: 2^21 elements 8.6, 8.4, 8.0, 7.5; 2^22 13.2, 11.2, 10.7, 10.3; with
+    /// stores through the L2, which a wave's loads wait for, 2^24 49.1, 35.1, 33.3, 33.0; with non-temporal ones 2^25
+    /// 69.3, 67.4, 67.3, 69.7; 2^28 513, 554, 558, 569).
+    static uint32_t PersistentWaves(uint32_t n_wg, bool through)
     {
         static const uint32_t cus = []() {
             int dev = 0, n = 256;
@@ -305,13 +339,14 @@ private:
             return per_cu < 0 ? (int64_t)1 : per_cu > 64 ? (int64_t)64 : per_cu;
         }();
         if (asked > 0) return (uint32_t)asked * cus;
-        return (n_wg <= 64 * cus ? 8 : 2) * cus;
+        return (n_wg <= 16 * cus ? 8 : n_wg <= 64 * cus ? through ? 8 : 4 : 2) * cus;
     }
 
     const float alpha_;
     const float *x_;
     float *y_;
     const size_t n_;
+    const uint32_t head_;
     const uint32_t steps_;
     const bool chunk_grid_;   // guarded launches keep the one-wave-per-chunk grid
 };
@@ -342,10 +377,11 @@ EXPORT_C_FUNC XResult HipAxpyCommandCreate(HwCommandHandle *cmd, float alpha, co
     if (cmd == nullptr || (n != 0 && (x == nullptr || y == nullptr)) || guard < 0 || guard > 3) {
         return kXSchedErrorInvalidValue;
     }
-    const uint32_t steps = AxpyStepsFor(n);
+    const uint32_t head = axpy::HipAxpyCommand::HeadOf((const float *)y, n);
+    const uint32_t steps = AxpyStepsFor(n - head);
     const uint64_t per_wg = (uint64_t)steps * 1024;
-    const uint32_t n_wg = n == 0 ? 1 : (uint32_t)((n + per_wg - 1) / per_wg);
+    const uint32_t n_wg = n == head ? 1 : (uint32_t)((n - head + per_wg - 1) / per_wg);
     *cmd = HwCommandManager::Add(std::make_shared<axpy::HipAxpyCommand>(
-        alpha, (const float *)x, (float *)y, n, steps, n_wg, guard, GetEnv("XSCHED_HIP_AXPY_GRID") == "chunk"));
+        alpha, (const float *)x, (float *)y, n, head, steps, n_wg, guard, GetEnv("XSCHED_HIP_AXPY_GRID") == "chunk"));
     return kXSchedSuccess;
 }
