@@ -102,8 +102,8 @@ XResult HipGemmBf16CommandCreate(HwCommandHandle *cmd, const void *A, const void
 
 /* For tests: how a GEMM of these matrices would be launched; nothing is launched or read. `out` receives
  * 8 values, four for each of at most two launches (zeroes where there is no second one):
- * rows of C, columns of a tile, kernel (0 two LDS buffers, 1 four stages, 2 any shape) and what the
- * matrices are to square tiles of that edge (0 whole tiles, 1 16-byte rows, 2 anything). No counterpart in the reference. */
+ * rows of C, columns of a tile (its rows: HipGemmBf16TileRowsOf()), kernel (0 two LDS buffers, 1 four stages, 2 any
+ * shape) and what it assumes of the matrices (0 whole tiles, 1 16-byte rows, 2 nothing). No counterpart in the reference. */
 XResult HipGemmBf16PlanOf(const void *A, const void *B, const void *C, int M, int N, int K, int32_t *out);
 
 /* For tests: the same for the launches on copies of A and B whose rows start on 16-byte boundaries. `out`

@@ -46,10 +46,11 @@ def test_what_is_copied(xs):
             if groups:
                 assert groups == -(-rows * (-(-cols // 64) * 64) // COPIED_PER_GROUP), case
         assert sum(rows for rows, *_ in parts) == M, case
-        tiles = groups_a + groups_b
-        for rows, edge, kernel, fit in parts:
-            tiles += -(-rows // edge) * -(-N // edge)
-            whole = c % 16 == 0 and N % edge == 0 and rows % edge == 0 and K % 64 == 0
+        tiles, heights = groups_a + groups_b, (c_int32 * 4)()
+        xs.check(xs.halhip().HipGemmBf16TileRowsOf(a, b, c, M, N, K, heights))
+        for (rows, edge, kernel, fit), height in zip(parts, heights[2:]):
+            tiles += -(-rows // height) * -(-N // edge)
+            whole = c % 16 == 0 and N % edge == 0 and rows % height == 0 and K % 64 == 0
             assert fit == (EXACT if whole else EDGES), case
         assert tiles <= 1 << 18, case
     assert copied > 300

@@ -16,6 +16,13 @@ def plan_of(xs, M, N, K, offset=0):
     return [tuple(out[i:i + 4]) for i in (0, 4) if out[i] != 0]
 
 
+def tile_rows_of(xs, M, N, K, offset=0):
+    """Rows of a tile, launch by launch."""
+    out = (c_int32 * 4)()
+    xs.check(xs.halhip().HipGemmBf16TileRowsOf(ADDRESS + offset, ADDRESS, ADDRESS, M, N, K, out))
+    return [rows for rows in out[:2] if rows != 0]
+
+
 @pytest.mark.parametrize("tile", [0, 64, 128, 256])
 def test_a_plan_covers_the_rows_and_assumes_only_what_holds(xs, monkeypatch, tile):
     if tile != 0:
@@ -30,16 +37,18 @@ def test_a_plan_covers_the_rows_and_assumes_only_what_holds(xs, monkeypatch, til
         aligned = offset == 0 and N % 8 == 0 and K % 8 == 0
         case = (M, N, K, offset, plan)
         assert sum(rows for rows, *_ in plan) == M, case
-        tiles = 0
-        for rows, edge, kernel, fit in plan:
-            tiles += -(-rows // edge) * -(-N // edge)
+        tiles, tile_rows = 0, tile_rows_of(xs, M, N, K, offset)
+        assert len(tile_rows) == len(plan), case
+        for (rows, edge, kernel, fit), height in zip(plan, tile_rows):
+            tiles += -(-rows // height) * -(-N // edge)
+            assert height == edge or (edge, kernel) == (256, TWO_BUFFERS) and height in (128, 192), case
             if kernel == ANY_SHAPE:
                 assert edge == 64 and len(plan) == 1, case
                 assert N < 8 or M * K < 8 or (tile == 0 and K <= 128), case
                 continue
             assert N >= 8 and M * K >= 8 and (tile != 0 or K > 32 or (aligned and N % 32 == 0)), case
             assert fit == UNALIGNED or aligned, case
-            assert (fit == EXACT) == (aligned and rows % edge == 0 and N % edge == 0 and K % 64 == 0), case
+            assert (fit == EXACT) == (aligned and rows % height == 0 and N % edge == 0 and K % 64 == 0), case
             assert kernel == FOUR_STAGES if fit == UNALIGNED else True, case
             assert (kernel, edge) in ((TWO_BUFFERS, 256), (TWO_BUFFERS, 128), (FOUR_STAGES, 128), (FOUR_STAGES, 64)), case
             assert (kernel, edge) != (TWO_BUFFERS, 128) or fit == EXACT, case
@@ -48,6 +57,19 @@ def test_a_plan_covers_the_rows_and_assumes_only_what_holds(xs, monkeypatch, til
         if taken == xs.kXSchedSuccess:
             assert tiles <= 1 << 18, case
             xs.check(xs.preempt().HwCommandDestroy(cmd.value))
+
+
+def test_what_large_tiles_of_fewer_rows_assume(xs):
+    """Whole tiles are said of the launch's own tiles, not of square ones."""
+    rng, seen = random.Random(9), set()
+    for _ in range(20000):
+        M, N, K = (max(unit, int(2 ** rng.uniform(8, 13)) // unit * unit) for unit in (rng.choice([64, 192, 256]), 256, 64))
+        plan, heights = plan_of(xs, M, N, K), tile_rows_of(xs, M, N, K)
+        for (rows, edge, kernel, fit), height in zip(plan, heights):
+            assert fit == (EXACT if rows % height == 0 and N % edge == 0 else EDGES), (M, N, K, plan, heights)
+            seen.add((height, fit, rows % edge == 0))
+    # 192 rows: whole where 256 would not be, and ragged where 256 would be whole
+    assert {(192, EXACT, False), (192, EDGES, True), (128, EDGES, False)} <= seen
 
 
 @pytest.mark.parametrize("M,N,K,want", [

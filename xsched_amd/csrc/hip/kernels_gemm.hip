@@ -1829,27 +1829,22 @@ inline uint64_t CountedTiles(const void *A, const void *B, const void *C, int M,
 
 using namespace xsched::hip;
 
-static void PutParts(const gemm::Plan &plan, const void *C, int N, int K, int32_t *out)
+static void PutParts(const gemm::Plan &plan, int32_t *out)
 {
     for (int i = 0; i < 8; ++i) out[i] = 0;
     for (int i = 0; i < plan.parts; ++i) {
         const gemm::Part &part = plan.part[i];
-        gemm::Fit fit = part.fit;
-        if (part.tile_rows != part.tile) {   // said of square tiles, whatever rows the launch's tiles have
-            const bool whole = part.rows % part.tile == 0 && N % part.tile == 0 && K % gemm::kStepK == 0 && gemm::Aligned(C, N);
-            fit = whole ? gemm::Fit::kExact : gemm::Fit::kEdges;
-        }
         out[4 * i + 0] = part.rows;
         out[4 * i + 1] = part.tile;
         out[4 * i + 2] = (int32_t)part.body;
-        out[4 * i + 3] = (int32_t)fit;
+        out[4 * i + 3] = (int32_t)part.fit;
     }
 }
 
 EXPORT_C_FUNC XResult HipGemmBf16PlanOf(const void *A, const void *B, const void *C, int M, int N, int K, int32_t *out)
 {
     if (out == nullptr || M <= 0 || N <= 0 || K <= 0) return kXSchedErrorInvalidValue;
-    PutParts(gemm::PlansFor(A, B, C, M, N, K, gemm::ForcedTile()).in_place, C, N, K, out);
+    PutParts(gemm::PlansFor(A, B, C, M, N, K, gemm::ForcedTile()).in_place, out);
     return kXSchedSuccess;
 }
 
@@ -1857,7 +1852,7 @@ EXPORT_C_FUNC XResult HipGemmBf16CopyPlanOf(const void *A, const void *B, const 
 {
     if (out == nullptr || M <= 0 || N <= 0 || K <= 0) return kXSchedErrorInvalidValue;
     const gemm::CopyPlan copies = gemm::PlansFor(A, B, C, M, N, K, gemm::ForcedTile()).copies;
-    PutParts(copies.plan, C, N, K, out);
+    PutParts(copies.plan, out);
     out[8] = (int32_t)copies.a_groups;
     out[9] = (int32_t)copies.b_groups;
     return kXSchedSuccess;
