@@ -19,9 +19,17 @@ def tile_rows_of(xs, a, b, c, M, N, K):
 
 @pytest.mark.parametrize("M,N,K,rows", [
     (4096, 4096, 4096, 256), (8192, 8192, 8192, 256), (3072, 3072, 3072, 192), (3456, 3456, 512, 192), (7451, 2632, 1232, 192),
-    (5801, 760, 3344, 128), (805, 7704, 104, 128), (1500, 5240, 592, 128), (2048, 2048, 2048, 128), (1024, 1024, 1024, 64)])
+    (5801, 760, 3344, 128), (805, 7704, 104, 128), (1500, 5240, 592, 128), (2048, 2048, 2048, 128), (1024, 1024, 1024, 64),
+    # behind a whole round, where two launches are the other way
+    (4608, 4608, 4608, 192), (4994, 6840, 456, 192), (3488, 5808, 464, 192), (7680, 3072, 3840, 192), (2624, 7296, 6400, 192)])
 def test_the_rows_that_measured_quickest_are_taken(xs, M, N, K, rows):
     assert tile_rows_of(xs, ADDRESS, ADDRESS, ADDRESS, M, N, K)[:2] == [rows, 0]
+
+
+@pytest.mark.parametrize("M,N,K", [(3840, 4608, 2048), (6896, 2448, 2816), (3199, 5120, 6848), (7024, 2792, 4160)])
+def test_two_launches_that_measured_quickest_are_kept(xs, M, N, K):
+    first, second = tile_rows_of(xs, ADDRESS, ADDRESS, ADDRESS, M, N, K)[:2]
+    assert first == 256 and second != 0
 
 
 def test_tiles_of_fewer_rows_stay_within_what_the_progress_map_holds(xs):

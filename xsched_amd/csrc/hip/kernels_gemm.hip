@@ -1684,15 +1684,15 @@ inline Plan QuickestPlan(int M, int N, int K, Rows aligned, int split_steps)
     const int64_t in_row = (N + kLargeTile - 1) / kLargeTile;                // all whole rounds of large tiles
     const int64_t whole_rounds = (int64_t)TilesOf(M, N, kLargeTile) / ComputeUnits();
     consider(whole_rounds * ComputeUnits() / in_row * kLargeTile);
-    // All of C on large tiles of fewer rows. Behind a whole round the estimates of these and of two launches are 5 % to 10 %
-    // off, each in its own direction: there they have to be quicker by more than that (4608^3 161 us in two launches and 155 on 192 rows, by the
-    // estimate 160 and 155; 4994 x 6840 x 456 58.8 and 53.9, by the estimate 45 and 44).
+    // All of C on large tiles of fewer rows. Of 140 products that are quickest in two launches otherwise, half of them ragged, 40 are quicker on these by
+    // the estimate: they take 0.94 of the time on average, 1.03 at most (3072 x 7808 x 7488 290.2 -> 297.8 us; 4608^3 161.6 -> 154.1, 4994 x 6840 x 456
+    // 58.7 -> 55.1, 3488 x 5808 x 464 36.9 -> 32.3, 2624 x 7296 x 6400 245 -> 221). Asking them to be quicker by a tenth left 31 of the 40 in two launches.
     if (aligned.inputs) {
         for (const int tile_rows : { kThreeQuarterRows, kHalfRows }) {
             const Part part = PartOf(0, M, N, K, aligned, kLargeTile, tile_rows);
             if (part.tiles > GuardState::kMaxWorkGroups) continue;
             const double us = MicrosOf(part, K);
-            if ((part.tiles <= ComputeUnits() || best.parts == 1 ? us : us / 0.9) < least) { least = us; best = Plan { { part, {} }, 1 }; }
+            if (us < least) { least = us; best = Plan { { part, {} }, 1 }; }
         }
     }
     return best;
