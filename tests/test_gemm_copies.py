@@ -76,6 +76,23 @@ def test_thin_products_of_large_matrices_are_not_copied(xs):
         assert plans_of(xs, at, at, at, *sizes)[1] != [], sizes
 
 
+def test_copies_for_tiles_of_fewer_rows_only_where_they_gain(xs):
+    """By the estimate alone all of these are quicker on copies."""
+    at = 1 << 20
+    for sizes in ((774, 6505, 1056), (1071, 3980, 1184), (1897, 3814, 1002), (897, 4134, 1120), (1440, 5114, 808), (1271, 4106, 1020)):
+        assert plans_of(xs, at, at, at, *sizes)[1] == [], sizes
+    for sizes in ((767, 5952, 1317), (1750, 4884, 336), (3207, 6144, 197), (610, 7424, 846), (817, 5008, 1301), (6754, 631, 2169)):
+        assert plans_of(xs, at, at, at, *sizes)[1] == [(sizes[0], 256, TWO_BUFFERS, EDGES)], sizes
+
+
+@pytest.mark.parametrize("M,N,K,copied", [
+    (500, 499, 4095, False), (1500, 1499, 4095, True), (1500, 1499, 2047, False), (2000, 1999, 2047, False), (2000, 1999, 3001, False),
+    (2000, 1999, 4095, True), (2500, 2501, 1001, False), (3000, 2999, 301, False), (3000, 2999, 101, False), (4000, 3999, 301, True),
+    (1000, 999, 8001, False), (128, 8191, 8191, False)])
+def test_the_way_of_the_products_that_were_timed_both_ways(xs, M, N, K, copied):
+    assert (plans_of(xs, 1 << 20, 1 << 20, 1 << 20, M, N, K)[1] != []) == copied
+
+
 def _ints(torch, gen, shape, offset):
     """Integers in [-2, 2] between NaNs, `offset` elements behind an aligned address."""
     rows, cols = shape

@@ -1531,8 +1531,9 @@ inline Part PartOf(int first_row, int rows, int N, int K, Rows aligned, int tile
 /// units it keeps busy: in proportion, or, on tiles of 192 x 256, only where few units idle (the cube: a full round runs
 /// against the power limit, and units that idle leave the others a higher clock; the rates of 256 x 256 are fitted without
 /// it, for their choice between one launch and two: with it 4992^3 is slower by 3 %). The rates are fitted to outputs of 4 to 4096 tiles of 128 x 128 at
-/// K from 128 to 8192: of 181 products, half of them ragged, each timed on every tile, what the plan takes is 0.7 % behind the
-/// quickest on average, and at most 7 % (K up to 320).
+/// K from 128 to 8192. Of 150 products drawn from 128 to 8192 in each dimension, half of them ragged, each timed on every tile, what the
+/// plan takes is 1.2 % behind the quickest on average; 14 % at most where K is not divided (272 x 7184 x 288 7.9 us, 7.0 on
+/// tiles of 128) and 28 % where it is (561 x 456 x 2312 13.6, 10.6 in more parts).
 inline double MicrosOf(const Part &part, int K, double pace = 1.0 /* of the steps */)
 {
     // us of a round, and per K step of a full round and of one with a single tile: [exact, edges, unaligned]
@@ -1700,7 +1701,8 @@ inline Plan QuickestPlan(int M, int N, int K, Rows aligned, int split_steps)
 
 constexpr size_t kMaxScratchBytes = SharedScratch::kMaxBytes;   // copies of A and B and partial sums together
 // What copies cost by the estimate, fitted to 21 products of 300 x 301 x 6001 to 4000 x 3999 x 301, each timed in place and on
-// copies: the quicker way is taken for all of them.
+// copies. It errs towards in place: of those in PlansFor()'s comment 2000 x 1999 x 3001 and 3000 x 2999 x 301 and x 101 stay there
+// though copies are quicker.
 constexpr double kCopyMicros = 8.0;                 // launch of the copying kernel and the one behind it,
 constexpr double kCopyRate = 12e6;                  // bytes per us, read and written, as long as matrices and copies stay in the last-level
 constexpr double kCachedCopyBytes = 100e6;          // cache (256 MB): up to so many bytes of copies,
@@ -1711,6 +1713,19 @@ inline double CopyMicros(const CopyPlan &p)
 {
     const double cached = std::min((double)p.CopyBytes(), kCachedCopyBytes);
     return kCopyMicros + 2.0 * cached / kCopyRate + 2.0 * ((double)p.CopyBytes() - cached) / kFarCopyRate;
+}
+
+/// What the estimate misses of copies that are multiplied on large tiles of fewer rows, in us: behind a short K they lose to
+/// in place by what was copied of B, and a little of what was of A. Of 156 products that the estimate alone takes from in place to
+/// such tiles, all timed both ways and none with more than kCachedCopyBytes of copies (for those kFarCopyRate is fitted with them), 105 stay on them with this: 0.907 of the time in place on average (1205 x 5002 x 1440 32.2 us in place,
+/// 34.6 on copies at worst; 767 x 5952 x 1317 31.8 and 25.8, 1750 x 4884 x 336 22.8 and 19.4), and 51 go back: copies took 1.017 of their
+/// time in a stream of commands and 1.046 of a pass (897 x 4134 x 1120 24.5 and 29.6, 1897 x 3814 x 1002 27.2 and 30.3,
+/// 774 x 6505 x 1056 30.8 and 33.9; but 671 x 6179 x 1661 44.2 and 39.5). No product that went on copies to tiles of 256 rows or edges of
+/// 128 changes its way (30000 drawn ones).
+inline double FewerRowsMicros(const CopyPlan &p, int K)
+{
+    const Part &part = p.plan.part[0];
+    return part.tile_rows == part.tile || K <= 7 * kStepK || (double)p.CopyBytes() > kCachedCopyBytes ? 0.0 : 0.23e-6 * (double)p.b_bytes + 0.04e-6 * (double)p.a_bytes;
 }
 
 /// Copies of A, B or both without a plan for them; without copies where they are too large.
@@ -1769,10 +1784,10 @@ inline int SplitStepsFor(int M, int N, int K)
 /// their launch and two passes over the matrices (8191^2 elements 87 us = 6.2 TB/s with what is
 /// written, 2000 x 2047 and 2047 x 1999 together 9.5). Rows of the copies are whole 128-byte lines (rows of 2000 and
 /// 2048 elements rather than of 2048: 27 us for the 2000 x 1999 x 2047 that takes 23.5). us per command,
-/// in place / on copies: 500 x 499 x 4095 23.6 / 26.5; 1500 x 1499 x 4095 44.4 / 41.0, x 2047 25.8 / 29.8; 2000 x 1999
-/// x 2047 28.4 / 31.7, x 3001 38.9 / 38.8, x 4095 51.2 / 47.2; 2500 x 2501 x 1001 32.1 / 36.3; 3000 x 2999 x 301
-/// 28.0 / 28.5, x 101 25.5 / 23.7; 4000 x 3999 x 301 38.3 / 31.4; 1000 x 999 x 8001 44.3 / 43.5; 128 x 8191 x 8191
-/// 66.8 / 76.6. Above the size of the last-level cache (copies on large tiles of any rows): 8191 x 511 x 8191 89.5 / 113, 500 x 12287 x 8191 166 / 211, 16383 x 300 x
+/// in place / on copies: 500 x 499 x 4095 13.5 / 17.9; 1500 x 1499 x 4095 44.2 / 39.6, x 2047 25.8 / 28.1; 2000 x 1999
+/// x 2047 31.0 / 31.2, x 3001 43.3 / 38.1, x 4095 56.3 / 46.5; 2500 x 2501 x 1001 32.5 / 32.1; 3000 x 2999 x 301
+/// 27.9 / 22.7, x 101 24.3 / 18.5; 4000 x 3999 x 301 38.4 / 30.1; 1000 x 999 x 8001 36.8 / 39.9; 128 x 8191 x 8191
+/// 48.9 / 82.0. Above the size of the last-level cache (copies on large tiles of any rows): 8191 x 511 x 8191 89.5 / 113, 500 x 12287 x 8191 166 / 211, 16383 x 300 x
 /// 8191 162 / 239, 512 x 16383 x 8191 216 / 247, but 8191 x 767 x 8191 165 / 151, 700 x 8191 x 8191 176 / 151, 8191 x 1023 x 8191 180 / 164, 600 x 16383 x 4095
 /// 138 / 126, 900 x 16383 x 4095 204 / 148, 8191 x 2047 x 8191 359 / 254. A pass of 8191^3 1791 / 918.
 inline Plans PlansFor(const void *A, const void *B, const void *C, int M, int N, int K, int forced)
@@ -1806,7 +1821,7 @@ inline Plans PlansFor(const void *A, const void *B, const void *C, int M, int N,
     if (copies.CopyBytes() == 0) return plans;
     copies.plan = QuickestPlan(M, N, K, Rows { true, aligned.output }, split_steps);
     if (copies.Groups() > GuardState::kMaxWorkGroups || copies.CopyBytes() + copies.plan.PartialBytes() > kMaxScratchBytes) return plans;
-    if (CopyMicros(copies) + MicrosOfPlan(copies.plan, K, kCopyPace) < MicrosOfPlan(plans.in_place, K)) plans.copies = copies;
+    if (CopyMicros(copies) + FewerRowsMicros(copies, K) + MicrosOfPlan(copies.plan, K, kCopyPace) < MicrosOfPlan(plans.in_place, K)) plans.copies = copies;
     return plans;
 }
 
