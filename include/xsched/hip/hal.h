@@ -84,6 +84,11 @@ XResult HipQueueMarkEpochFlushed(HwQueueHandle hwq);
 XResult HipAxpyCommandCreate(HwCommandHandle *cmd, float alpha, const void *x, void *y,
                              size_t n, int guard);
 
+/* For tests: how an AXPY into y would be launched on a device of so many compute units, guarded or not; nothing is launched
+ * or read. out[0] receives the number of chunks, out[1] how many long-lived waves walk them (0: a wave for each), out[2] the
+ * first chunk whose stores go through the L2 (out[0]: none do). No counterpart in the reference. */
+XResult HipAxpyPlanOf(const void *y, size_t n, int guarded, uint32_t compute_units, uint32_t *out);
+
 /* C[M,N] = A[M,K] * B[K,N]; A, B, C row-major bf16, fp32 accumulation in ascending
  * k, round-to-nearest-even on store. Any M, N, K >= 1 (at most 2^18 tiles), any alignment to
  * the element. The work is cut into tiles of C of 256x256 (N and K multiples of 8, matrices

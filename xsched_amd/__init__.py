@@ -121,6 +121,7 @@ HALHIP_API = {
     "HipQueueSetMarkerOnKernel": (XResult, [c_uint64, c_int]),
     "HipQueueMarkEpochFlushed": (XResult, [c_uint64]),
     "HipAxpyCommandCreate": (XResult, [POINTER(c_uint64), c_float, c_void_p, c_void_p, c_size_t, c_int]),
+    "HipAxpyPlanOf": (XResult, [c_void_p, c_size_t, c_int, c_uint32, POINTER(c_uint32)]),
     "HipGemmBf16CommandCreate": (XResult, [POINTER(c_uint64), c_void_p, c_void_p, c_void_p,
                                            c_int, c_int, c_int, c_int]),
     "HipGemmBf16PlanOf": (XResult, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, POINTER(c_int32)]),

@@ -270,13 +270,39 @@ public:
         return n < head ? (uint32_t)n : head;
     }
 
+    static bool WavePerChunk(bool guarded, uint32_t n_wg, bool chunk_grid) { return chunk_grid || (!guarded && n_wg < kLongChunks); }
+
+    /// Whether stores go through the L2. On one wave per chunk: arrays of up to kThroughTo elements, from a size on that depends on
+    /// whether they begin on a line. us per command in a stream of them, on one pair of arrays / on pairs of 800 MB in turn (nothing is in
+    /// the last-level cache then), and of a pass alone, on one pair / behind a fill of 640 MB, non-temporal stores -> these: on a line 2^20 elements 4.20 / 4.50, 13.0 / 16.5 ->
+    /// 4.09 / 4.53, 13.3 / 15.6 (runs differ by 0.1 to 0.3), 5 x 2^18 4.31 / 4.72, 13.6 / 16.5 -> 4.33 / 4.92, 13.6 / 16.1, 2^21 4.75 / 6.30, 14.0 / 18.1 -> 4.76 / 6.18,
+    /// 14.7 / 17.3, 5 x 2^19 5.97 / 7.67, 16.1 / 19.7 -> 5.25 / 7.43, 16.3 / 18.9, 2^22 8.40 / 10.3, 18.3 / 22.3 -> 6.57 / 10.1, 18.2 / 21.7; off a line 2^20
+    /// 4.60 / 5.39, 13.4 / 17.4 -> 4.71 / 5.19, 13.6 / 16.7, 5 x 2^18 5.21 / 5.88, 15.7 / 19.7 -> 4.81 / 5.72, 15.8 / 18.6, 2^21 5.83 / 7.21, 15.9 / 19.3 ->
+    /// 4.86 / 6.84, 15.6 / 18.5. Traced, a launch of 2^16 elements takes 2.5 us with these and 2.1 without.
+    /// Above, level 1 6 x 2^20 10.9 / 13.8 -> 11.5 / 13.9. On long-lived waves: from kThroughLongFrom to kThroughLongTo,
+    /// 12 x 2^20 23.4 / 25.7 -> 22.3 / 26.8, 2^24 31.1 / 33.1 -> 29.6 / 34.5.
+    static bool Through(size_t n, uint32_t head, bool wave_per_chunk)
+    {
+        return wave_per_chunk ? n > (head != 0 ? kThroughOffLines : kThroughOnLines) && n <= kThroughTo
+                              : n > kThroughLongFrom && n <= kThroughLongTo;
+    }
+
+    /// Long-lived waves of a launch over n_wg chunks: two per compute unit for long arrays, more
+    /// while each has only a few chunks, where what counts is how many requests are out at once
+    /// (us per command at level 2 and 2, 4, 8, 12 waves per CU: 2^21 elements 8.6, 8.4, 8.0, 7.5; 2^22 13.2, 11.2, 10.7, 10.3; with
+    /// stores through the L2, which a wave's loads wait for, 2^24 49.1, 35.1, 33.3, 33.0; with non-temporal ones 2^25
+    /// 69.3, 67.4, 67.3, 69.7; 2^28 513, 554, 558, 569).
+    static uint32_t WavesFor(uint32_t n_wg, bool through, uint32_t units)
+    {
+        return (n_wg <= 16 * units ? 8 : n_wg <= 64 * units ? through ? 8 : 4 : 2) * units;
+    }
+
 protected:
     virtual hipError_t LaunchKernel(hipStream_t stream, bool guarded, const XGuardArgs &g) override
     {
         if (n_ == 0) return hipSuccess;
         const hipEvent_t stop = TakeStopEvent();
-        const bool chunks = chunk_grid_ || (!guarded && n_wg_ < kLongChunks);   // one wave per chunk
-        if (chunks ? n_ <= kThroughChunks : n_ > kThroughFrom && n_ <= kThroughTo) Launch<true>(guarded, stop, stream, g);
+        if (Through(n_, head_, WavePerChunk(guarded, n_wg_, chunk_grid_))) Launch<true>(guarded, stop, stream, g);
         else Launch<false>(guarded, stop, stream, g);
         return hipGetLastError();
     }
@@ -310,22 +336,6 @@ private:
         }
     }
 
-    /// Arrays of up to kThroughChunks elements on one wave per chunk, and of kThroughFrom to kThroughTo on long-lived
-    /// waves, are stored through the L2. us per command in a stream of them, non-temporal stores / these, on one pair of arrays
-    /// and on pairs of 800 MB in turn (nothing is in the last-level cache then): level 1 2^22 elements 6.9 / 6.2 and 10.1 / 10.0,
-    /// 6 x 2^20 10.9 / 11.5 and 13.8 / 13.9, 2^23 15.2 / 15.8 and 17.9 / 18.7, 12 x 2^20 23.4 / 22.3 and 25.7 / 26.8, 2^24 31.1 / 29.6 and
-    /// 33.1 / 34.5; level 2 3 x 2^20 5.4 / 6.2 and 7.7 / 7.9, 2^23 15.5 / 15.6 and 18.5 / 18.7, 12 x 2^20 23.6 / 22.5 and 26.2 / 26.9,
-    /// 2^24 32.0 / 30.1 and 33.7 / 34.7. Three pairs of 2^24 in turn, a pass through a queue: level 1 43.1 / 39.9, level 2 43.8 / 40.7. Above,
-    /// these are slower (level 1 2^28 529 / 543, level 2 2^25 76 / 102).
-    static constexpr uint64_t kThroughChunks = (uint64_t)1 << 22;
-    static constexpr uint64_t kThroughFrom = (uint64_t)1 << 23, kThroughTo = (uint64_t)1 << 24;
-    static constexpr uint32_t kLongChunks = 8192;   // from here on a plain launch uses long-lived waves
-
-    /// Long-lived waves of a launch over n_wg chunks: two per compute unit for long arrays, more
-    /// while each has only a few chunks, where what counts is how many requests are out at once
-    /// (us per command at level 2 and 2, 4, 8, 12 waves per CU: 2^21 elements 8.6, 8.4, 8.0, 7.5; 2^22 13.2, 11.2, 10.7, 10.3; with
-    /// stores through the L2, which a wave's loads wait for, 2^24 49.1, 35.1, 33.3, 33.0; with non-temporal ones 2^25
-    /// 69.3, 67.4, 67.3, 69.7; 2^28 513, 554, 558, 569).
     static uint32_t PersistentWaves(uint32_t n_wg, bool through)
     {
         static const uint32_t cus = []() {
@@ -339,8 +349,12 @@ private:
             return per_cu < 0 ? (int64_t)1 : per_cu > 64 ? (int64_t)64 : per_cu;
         }();
         if (asked > 0) return (uint32_t)asked * cus;
-        return (n_wg <= 16 * cus ? 8 : n_wg <= 64 * cus ? through ? 8 : 4 : 2) * cus;
+        return WavesFor(n_wg, through, cus);
     }
+
+    static constexpr uint64_t kThroughOffLines = (uint64_t)1 << 20, kThroughOnLines = (uint64_t)1 << 21, kThroughTo = (uint64_t)1 << 22;
+    static constexpr uint64_t kThroughLongFrom = (uint64_t)1 << 23, kThroughLongTo = (uint64_t)1 << 24;
+    static constexpr uint32_t kLongChunks = 8192;   // from here on a plain launch uses long-lived waves
 
     const float alpha_;
     const float *x_;
@@ -383,5 +397,20 @@ EXPORT_C_FUNC XResult HipAxpyCommandCreate(HwCommandHandle *cmd, float alpha, co
     const uint32_t n_wg = n == head ? 1 : (uint32_t)((n - head + per_wg - 1) / per_wg);
     *cmd = HwCommandManager::Add(std::make_shared<axpy::HipAxpyCommand>(
         alpha, (const float *)x, (float *)y, n, head, steps, n_wg, guard, GetEnv("XSCHED_HIP_AXPY_GRID") == "chunk"));
+    return kXSchedSuccess;
+}
+
+EXPORT_C_FUNC XResult HipAxpyPlanOf(const void *y, size_t n, int guarded, uint32_t compute_units, uint32_t *out)
+{
+    if (out == nullptr || n == 0 || compute_units == 0) return kXSchedErrorInvalidValue;
+    using Command = axpy::HipAxpyCommand;
+    const uint32_t head = Command::HeadOf((const float *)y, n), steps = AxpyStepsFor(n - head);
+    const uint64_t per_wg = (uint64_t)steps * 1024;
+    const uint32_t chunks = n == head ? 1 : (uint32_t)((n - head + per_wg - 1) / per_wg);
+    const bool wave_per_chunk = Command::WavePerChunk(guarded != 0, chunks, GetEnv("XSCHED_HIP_AXPY_GRID") == "chunk");
+    const bool through = Command::Through(n, head, wave_per_chunk);
+    out[0] = chunks;
+    out[1] = wave_per_chunk ? 0 : Command::WavesFor(chunks, through, compute_units);
+    out[2] = through ? 0 : chunks;
     return kXSchedSuccess;
 }
