@@ -81,7 +81,8 @@ def test_copies_for_tiles_of_fewer_rows_only_where_they_gain(xs):
     at = 1 << 20
     for sizes in ((774, 6505, 1056), (1071, 3980, 1184), (1897, 3814, 1002), (897, 4134, 1120), (1440, 5114, 808), (1271, 4106, 1020)):
         assert plans_of(xs, at, at, at, *sizes)[1] == [], sizes
-    for sizes in ((767, 5952, 1317), (1750, 4884, 336), (3207, 6144, 197), (610, 7424, 846), (817, 5008, 1301), (6754, 631, 2169)):
+    for sizes in ((767, 5952, 1317), (1750, 4884, 336), (3207, 6144, 197), (610, 7424, 846), (817, 5008, 1301), (6754, 631, 2169), (640, 12001, 3801),
+                  (730, 7489, 2278), (599, 7697, 2539)):
         assert plans_of(xs, at, at, at, *sizes)[1] == [(sizes[0], 256, TWO_BUFFERS, EDGES)], sizes
 
 

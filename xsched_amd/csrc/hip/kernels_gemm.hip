@@ -1720,12 +1720,13 @@ inline double CopyMicros(const CopyPlan &p)
 /// such tiles, all timed both ways and none with more than kCachedCopyBytes of copies (for those kFarCopyRate is fitted with them), 105 stay on them with this: 0.907 of the time in place on average (1205 x 5002 x 1440 32.2 us in place,
 /// 34.6 on copies at worst; 767 x 5952 x 1317 31.8 and 25.8, 1750 x 4884 x 336 22.8 and 19.4), and 51 go back: copies took 1.017 of their
 /// time in a stream of commands and 1.046 of a pass (897 x 4134 x 1120 24.5 and 29.6, 1897 x 3814 x 1002 27.2 and 30.3,
-/// 774 x 6505 x 1056 30.8 and 33.9; but 671 x 6179 x 1661 44.2 and 39.5). No product that went on copies to tiles of 256 rows or edges of
-/// 128 changes its way (30000 drawn ones).
+/// 774 x 6505 x 1056 30.8 and 33.9; but 671 x 6179 x 1661 44.2 and 39.5). Of more than 30 MB of B or 60 of A no more than for
+/// those: 640 x 12001 x 3801 (91 MB of B) 114.4 in place and 98.9, 730 x 7489 x 2278 (35 MB) 57.8 and 53.0, but 400 x 8191 x 4001 (66 MB) 56.3 and 62.6.
+/// Of 30000 drawn products of up to 16384 x 16384 x 8192 that went on copies to other tiles one changes its way by it (11157 x 633 x 2629 65.3 in place and 69.6).
 inline double FewerRowsMicros(const CopyPlan &p, int K)
 {
     const Part &part = p.plan.part[0];
-    return part.tile_rows == part.tile || K <= 7 * kStepK || (double)p.CopyBytes() > kCachedCopyBytes ? 0.0 : 0.23e-6 * (double)p.b_bytes + 0.04e-6 * (double)p.a_bytes;
+    return part.tile_rows == part.tile || K <= 7 * kStepK || (double)p.CopyBytes() > kCachedCopyBytes ? 0.0 : 0.23e-6 * std::min((double)p.b_bytes, 30e6) + 0.04e-6 * std::min((double)p.a_bytes, 60e6);
 }
 
 /// Copies of A, B or both without a plan for them; without copies where they are too large.
