@@ -3,8 +3,8 @@
 // HBM-bound: 12 bytes of traffic per element (read x, read y, write y). The unit of
 // work is a chunk of `steps` x 1024 contiguous elements, walked by one wavefront in
 // steps of 4 x 128-bit accesses per lane and stream, lane-contiguous so that every
-// access of a wave covers 1 KiB. Loads are non-temporal, nothing is reused; so are the
-// stores of long arrays. Chunks begin on a line of y (HeadOf()).
+// access of a wave covers 1 KiB. Loads are non-temporal, nothing is reused; so are most
+// stores (ThroughFrom()). Chunks begin on a line of y (HeadOf()).
 // Because the update is in place, a chunk must be applied exactly once: the wave reads
 // the preempt word before it stores anything, and commits the chunk's byte in the
 // progress map after its last store.
@@ -140,10 +140,12 @@ void AxpyVec4Kernel(float alpha, const float *x_first, float *y_first,
 // way and step j+kDepth is requested right behind the stores. The preempt word is read
 // in front of the first store of every chunk; a chunk that has begun is finished and
 // committed, so it is applied exactly once.
+// kThrough: the chunks from `through` on are stored through the L2, which holds nothing to be
+// written back of them when the kernel ends (ThroughFrom()).
 template <uint32_t kDepth, bool kGuard, bool kThrough>
 __global__ __launch_bounds__(64)
 void AxpyPersistentKernel(float alpha, const float *x_first, float *y_first, uint64_t n4, uint32_t tail,
-                          uint32_t head, uint32_t steps, uint32_t n_chunks, XGuardArgs g)
+                          uint32_t head, uint32_t steps, uint32_t n_chunks, uint32_t through, XGuardArgs g)
 {
     const float4 *const x = (const float4 *)x_first;
     float4 *const y = (float4 *)y_first;
@@ -223,9 +225,12 @@ void AxpyPersistentKernel(float alpha, const float *x_first, float *y_first, uin
             }
             if (full && !skip) {
                 float4 *const first = y + ((uint64_t)c * steps + st) * kStepVecs;
+                if (kThrough && c >= through) {
 #pragma unroll
-                for (uint32_t u = 0; u < kVecPerStep; ++u) {
-                    StoreLanes<kThrough>(first, lane, u, fma4(alpha, xv[d][u], yv[d][u]));
+                    for (uint32_t u = 0; u < kVecPerStep; ++u) StoreLanes<true>(first, lane, u, fma4(alpha, xv[d][u], yv[d][u]));
+                } else {
+#pragma unroll
+                    for (uint32_t u = 0; u < kVecPerStep; ++u) StoreLanes<false>(first, lane, u, fma4(alpha, xv[d][u], yv[d][u]));
                 }
                 if (kGuard && st == steps - 1 && g.done && lane == 0) xguard_commit(g, c);
             }
@@ -258,10 +263,10 @@ public:
 
     /// Elements of y in front of its first 128-byte line. Chunks begin behind them, so that a wave's stores cover whole lines:
     /// of an array off its lines each store of 1 KiB began and ended inside a line, which two waves then
-    /// wrote in pieces. us per command in a stream of them from an odd offset, before (non-temporal stores) and with this, on one pair of arrays and on 800 MB
-    /// in turn: level 1 2^20 elements 4.8 / 3.8 and 5.6 / 5.1, 3 x 2^20 7.3 / 5.8 and 9.2 / 8.6, 2^23 16.8 / 16.1
-    /// and 19.1 / 18.6, 2^24 33.4 / 29.9 and 35.0 / 35.0; level 2 3 x 2^20 8.0 / 7.7 and 9.4 / 9.2, 2^24 34.0 / 31.2 and 35.3 / 35.4
-    /// (2^24 with stores through the L2 and chunks off the lines: 31.4 and 39.6).
+    /// wrote in pieces. us per command in a stream of them from an odd offset, without and with it (and with the stores of ThroughFrom()), on one pair of arrays and on 800 MB
+    /// in turn: level 1 2^20 elements 4.6 / 4.2 and 5.7 / 5.3, 3 x 2^20 7.0 / 5.6 and 9.2 / 8.5, 6 x 2^20 13.0 / 12.3 and 15.2 / 14.5, 2^23 17.2 / 16.5
+    /// and 19.1 / 18.6, 2^24 33.2 / 29.7 and 34.8 / 31.3, 2^25 67.9 / 65.9 and 68.4 / 66.2; level 2 3 x 2^20 7.6 / 7.5 and 9.4 / 9.2, 2^24 33.6 / 31.0 and 35.2 / 32.6.
+    /// (All of 2^24 through the L2 without it: 31.4 and 39.6.)
     static uint32_t HeadOf(const float *y, size_t n)
     {
         const uint32_t off = (uint32_t)((uintptr_t)y & 127);
@@ -272,29 +277,37 @@ public:
 
     static bool WavePerChunk(bool guarded, uint32_t n_wg, bool chunk_grid) { return chunk_grid || (!guarded && n_wg < kLongChunks); }
 
-    /// Whether stores go through the L2. On one wave per chunk: arrays of up to kThroughTo elements, from a size on that depends on
+    /// First chunk whose stores go through the L2 (n_wg: none). On one wave per chunk all of them, of arrays of up to kThroughTo elements, from a size on that depends on
     /// whether they begin on a line. us per command in a stream of them, on one pair of arrays / on pairs of 800 MB in turn (nothing is in
     /// the last-level cache then), and of a pass alone, on one pair / behind a fill of 640 MB, non-temporal stores -> these: on a line 2^20 elements 4.20 / 4.50, 13.0 / 16.5 ->
     /// 4.09 / 4.53, 13.3 / 15.6 (runs differ by 0.1 to 0.3), 5 x 2^18 4.31 / 4.72, 13.6 / 16.5 -> 4.33 / 4.92, 13.6 / 16.1, 2^21 4.75 / 6.30, 14.0 / 18.1 -> 4.76 / 6.18,
     /// 14.7 / 17.3, 5 x 2^19 5.97 / 7.67, 16.1 / 19.7 -> 5.25 / 7.43, 16.3 / 18.9, 2^22 8.40 / 10.3, 18.3 / 22.3 -> 6.57 / 10.1, 18.2 / 21.7; off a line 2^20
     /// 4.60 / 5.39, 13.4 / 17.4 -> 4.71 / 5.19, 13.6 / 16.7, 5 x 2^18 5.21 / 5.88, 15.7 / 19.7 -> 4.81 / 5.72, 15.8 / 18.6, 2^21 5.83 / 7.21, 15.9 / 19.3 ->
     /// 4.86 / 6.84, 15.6 / 18.5. Traced, a launch of 2^16 elements takes 2.5 us with these and 2.1 without.
-    /// Above, level 1 6 x 2^20 10.9 / 13.8 -> 11.5 / 13.9. On long-lived waves: from kThroughLongFrom to kThroughLongTo,
-    /// 12 x 2^20 23.4 / 25.7 -> 22.3 / 26.8, 2^24 31.1 / 33.1 -> 29.6 / 34.5.
-    static bool Through(size_t n, uint32_t head, bool wave_per_chunk)
+    /// Above, level 1 6 x 2^20 10.9 / 13.8 -> 11.5 / 13.9.
+    /// On long-lived waves, eight per compute unit, for more than 32768 and up to 65536 elements per unit (2^23 and 2^24 on 256): the last three
+    /// quarters of the chunks. Non-temporal -> all of them -> these, the same four figures: level 1 2^23 + 1024 elements 16.0 / 17.8, 27.5 / 28.9 -> 14.0 / 18.4, 23.7 / 28.9 ->
+    /// 15.1 / 17.9, 24.3 / 29.3; 12 x 2^20 24.3 / 25.8, 35.4 / 37.2 -> 21.0 / 26.6, 30.0 / 37.4 -> 22.1 / 24.2, 31.0 / 37.4; 2^24 31.3 / 33.1, 42.4 / 45.0 ->
+    /// 28.8 / 34.2, 38.9 / 46.1 -> 29.3 / 30.9, 38.3 / 45.4; level 2 2^23 + 1024 16.0 / 18.4, 28.4 / 29.8 -> 14.6 / 18.7, 24.7 / 29.8 -> 15.0 / 18.3, 25.6 / 29.8;
+    /// 2^24 31.4 / 33.5, 43.5 / 44.9 -> 29.1 / 34.6, 39.4 / 46.2 -> 30.7 / 32.2, 39.4 / 46.4. So arrays that are not in the last-level cache, which lost 2 % to 3 % with
+    /// all chunks through, gain up to 7 % where they follow each other, and single passes over them lose up to 1 us (runs differ by as much); a half or five
+    /// eighths of the chunks gain less in all figures but that one. 5000 elements longer it is non-temporal stores and two waves per unit: 33.5 / 35.0, 44.9 / 46.3.
+    static uint32_t ThroughFrom(size_t n, uint32_t head, uint32_t n_wg, bool wave_per_chunk, uint32_t units)
     {
-        return wave_per_chunk ? n > (head != 0 ? kThroughOffLines : kThroughOnLines) && n <= kThroughTo
-                              : n > kThroughLongFrom && n <= kThroughLongTo;
+        if (wave_per_chunk) return n > (head != 0 ? kThroughOffLines : kThroughOnLines) && n <= kThroughTo ? 0 : n_wg;
+        if (n <= (uint64_t)32 * kStepElems * units || n > (uint64_t)64 * kStepElems * units) return n_wg;
+        return n_wg / 4;
     }
 
     /// Long-lived waves of a launch over n_wg chunks: two per compute unit for long arrays, more
     /// while each has only a few chunks, where what counts is how many requests are out at once
-    /// (us per command at level 2 and 2, 4, 8, 12 waves per CU: 2^21 elements 8.6, 8.4, 8.0, 7.5; 2^22 13.2, 11.2, 10.7, 10.3; with
-    /// stores through the L2, which a wave's loads wait for, 2^24 49.1, 35.1, 33.3, 33.0; with non-temporal ones 2^25
-    /// 69.3, 67.4, 67.3, 69.7; 2^28 513, 554, 558, 569).
+    /// (us per command at level 2 in a stream of them, on one pair of arrays / on 800 MB of them, at 2, 4, 8, 12 waves per CU and with non-temporal
+    /// stores: 2^21 elements 5.7 / 7.1, 5.4 / 6.7, 5.2 / 6.3, 5.2 / 6.3; 2^22 10.2 / 11.6, 9.1 / 10.7, 8.4 / 10.3, 8.2 / 10.0; 6 x 2^20 14.4 / 15.8, 13.1 / 14.8,
+    /// 12.9 / 14.7, 12.6 / 14.6; 2^23 18.4 / 19.7, 16.9 / 18.6, 16.9 / 18.9, 16.3 / 18.1; 2^25 69.3, 67.4, 67.3, 69.7; 2^28 513, 554, 558, 569). `through`: with
+    /// stores through the L2, which the loads of a guarded launch's wave wait for, 2^24 takes 32.1 with four and 29.1 with eight.
     static uint32_t WavesFor(uint32_t n_wg, bool through, uint32_t units)
     {
-        return (n_wg <= 16 * units ? 8 : n_wg <= 64 * units ? through ? 8 : 4 : 2) * units;
+        return (through || n_wg <= 16 * units ? 8 : n_wg <= 64 * units ? 4 : 2) * units;
     }
 
 protected:
@@ -302,14 +315,15 @@ protected:
     {
         if (n_ == 0) return hipSuccess;
         const hipEvent_t stop = TakeStopEvent();
-        if (Through(n_, head_, WavePerChunk(guarded, n_wg_, chunk_grid_))) Launch<true>(guarded, stop, stream, g);
-        else Launch<false>(guarded, stop, stream, g);
+        const uint32_t through = ThroughFrom(n_, head_, n_wg_, WavePerChunk(guarded, n_wg_, chunk_grid_), ComputeUnits());
+        if (through < n_wg_) Launch<true>(guarded, stop, stream, through, g);
+        else Launch<false>(guarded, stop, stream, through, g);
         return hipGetLastError();
     }
 
 private:
     template <bool kThrough>
-    void Launch(bool guarded, hipEvent_t stop, hipStream_t stream, const XGuardArgs &g)
+    void Launch(bool guarded, hipEvent_t stop, hipStream_t stream, uint32_t through, const XGuardArgs &g)
     {
         const dim3 grid(n_wg_), block(kLanes);
         const uint32_t waves = PersistentWaves(n_wg_, kThrough);
@@ -319,11 +333,11 @@ private:
         const uint32_t tail = (uint32_t)((n_ - head_) % 4);
         if (guarded && !chunk_grid_) {
             const dim3 pgrid(n_wg_ < waves ? n_wg_ : waves);
-            LaunchWithStop(stop, (AxpyPersistentKernel<3, true, kThrough>), pgrid, block, stream, alpha_, x, y, n4, tail, head_, steps_, n_wg_, g);
+            LaunchWithStop(stop, (AxpyPersistentKernel<3, true, kThrough>), pgrid, block, stream, alpha_, x, y, n4, tail, head_, steps_, n_wg_, through, g);
         } else if (!guarded && !chunk_grid_ && n_wg_ >= kLongChunks) {
             // A long array: the same few long-lived waves stream it as fast as one wave per
             // chunk does and leave nearly all wave slots to whatever else runs on the device.
-            LaunchWithStop(stop, (AxpyPersistentKernel<3, false, kThrough>), dim3(waves), block, stream, alpha_, x, y, n4, tail, head_, steps_, n_wg_, g);
+            LaunchWithStop(stop, (AxpyPersistentKernel<3, false, kThrough>), dim3(waves), block, stream, alpha_, x, y, n4, tail, head_, steps_, n_wg_, through, g);
         } else {
             // An even chunk is walked in steps of 2048 elements (8 accesses in flight
             // per lane and stream), an odd one in steps of 1024.
@@ -336,24 +350,27 @@ private:
         }
     }
 
-    static uint32_t PersistentWaves(uint32_t n_wg, bool through)
+    static uint32_t ComputeUnits()
     {
         static const uint32_t cus = []() {
             int dev = 0, n = 256;
             if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev);
             return (uint32_t)(n > 0 ? n : 256);
         }();
+        return cus;
+    }
+
+    static uint32_t PersistentWaves(uint32_t n_wg, bool through)
+    {
         static const int64_t asked = []() {
             int64_t per_cu = 0;
             GetEnvInt64("XSCHED_HIP_AXPY_WAVES_PER_CU", per_cu);
             return per_cu < 0 ? (int64_t)1 : per_cu > 64 ? (int64_t)64 : per_cu;
         }();
-        if (asked > 0) return (uint32_t)asked * cus;
-        return WavesFor(n_wg, through, cus);
+        return asked > 0 ? (uint32_t)asked * ComputeUnits() : WavesFor(n_wg, through, ComputeUnits());
     }
 
     static constexpr uint64_t kThroughOffLines = (uint64_t)1 << 20, kThroughOnLines = (uint64_t)1 << 21, kThroughTo = (uint64_t)1 << 22;
-    static constexpr uint64_t kThroughLongFrom = (uint64_t)1 << 23, kThroughLongTo = (uint64_t)1 << 24;
     static constexpr uint32_t kLongChunks = 8192;   // from here on a plain launch uses long-lived waves
 
     const float alpha_;
@@ -408,9 +425,8 @@ EXPORT_C_FUNC XResult HipAxpyPlanOf(const void *y, size_t n, int guarded, uint32
     const uint64_t per_wg = (uint64_t)steps * 1024;
     const uint32_t chunks = n == head ? 1 : (uint32_t)((n - head + per_wg - 1) / per_wg);
     const bool wave_per_chunk = Command::WavePerChunk(guarded != 0, chunks, GetEnv("XSCHED_HIP_AXPY_GRID") == "chunk");
-    const bool through = Command::Through(n, head, wave_per_chunk);
     out[0] = chunks;
-    out[1] = wave_per_chunk ? 0 : Command::WavesFor(chunks, through, compute_units);
-    out[2] = through ? 0 : chunks;
+    out[2] = Command::ThroughFrom(n, head, chunks, wave_per_chunk, compute_units);
+    out[1] = wave_per_chunk ? 0 : Command::WavesFor(chunks, out[2] < chunks, compute_units);
     return kXSchedSuccess;
 }
