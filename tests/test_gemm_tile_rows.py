@@ -21,33 +21,49 @@ def tile_rows_of(xs, a, b, c, M, N, K):
     (4096, 4096, 4096, 256), (8192, 8192, 8192, 256), (3072, 3072, 3072, 192), (3456, 3456, 512, 192), (7451, 2632, 1232, 192),
     (5801, 760, 3344, 128), (805, 7704, 104, 128), (1500, 5240, 592, 128), (2048, 2048, 2048, 128), (1024, 1024, 1024, 64),
     # behind a whole round, where two launches are the other way
-    (4608, 4608, 4608, 192), (4994, 6840, 456, 192), (3488, 5808, 464, 192), (7680, 3072, 3840, 192), (2624, 7296, 6400, 192)])
+    (4608, 4608, 4608, 192), (4994, 6840, 456, 192), (3488, 5808, 464, 192), (7680, 3072, 3840, 192), (2624, 7296, 6400, 192), (5124, 4096, 2048, 192)])
 def test_the_rows_that_measured_quickest_are_taken(xs, M, N, K, rows):
     assert tile_rows_of(xs, ADDRESS, ADDRESS, ADDRESS, M, N, K)[:2] == [rows, 0]
 
 
-@pytest.mark.parametrize("M,N,K", [(3840, 4608, 2048), (6896, 2448, 2816), (3199, 5120, 6848), (7024, 2792, 4160)])
+@pytest.mark.parametrize("M,N,K", [(4996, 4096, 2048), (3840, 4608, 2048), (6896, 2448, 2816), (3199, 5120, 6848), (7024, 2792, 4160)])
 def test_two_launches_that_measured_quickest_are_kept(xs, M, N, K):
     first, second = tile_rows_of(xs, ADDRESS, ADDRESS, ADDRESS, M, N, K)[:2]
     assert first == 256 and second != 0
 
 
+def counted_tiles(M, N, K):
+    """By which a product of matrices on 16-byte boundaries is accepted, up to 2^18."""
+    tiles = lambda rows, edge: -(-rows // edge) * -(-N // edge)
+    whole = M // 128 * 128
+    if whole == 0 or N % 128 != 0 or K % 64 != 0:
+        return tiles(M, 64)
+    return tiles(whole, 256 if whole % 256 == 0 and N % 256 == 0 else 128) + tiles(M - whole, 64)
+
+
 def test_tiles_of_fewer_rows_stay_within_what_the_progress_map_holds(xs):
+    """And no product is refused for them."""
     rng = random.Random(3)
-    seen = set()
-    for _ in range(3000):
+    seen, too_many = set(), 0
+    for _ in range(6000):
         M, N, K = int(2 ** rng.uniform(6, 24)), int(2 ** rng.uniform(6, 14)) // 8 * 8, 64 * rng.randint(1, 64)
-        plan = (c_int32 * 8)()
+        if rng.random() < 0.3:      # about the limit, a multiple of the tiles
+            N = max(256, N // 256 * 256)
+            M = int((1 << 18) / (N // 256) * rng.uniform(0.4, 1.02)) * 256
+        plan, cmd = (c_int32 * 8)(), c_uint64()
         xs.check(xs.halhip().HipGemmBf16PlanOf(ADDRESS, ADDRESS, ADDRESS, M, N, K, plan))
         rows = tile_rows_of(xs, ADDRESS, ADDRESS, ADDRESS, M, N, K)
-        cmd = c_uint64()
-        if xs.halhip().HipGemmBf16CommandCreate(byref(cmd), ADDRESS, ADDRESS, ADDRESS, M, N, K, 1) != xs.kXSchedSuccess:
+        case = (M, N, K, list(plan), rows)
+        taken = xs.halhip().HipGemmBf16CommandCreate(byref(cmd), ADDRESS, ADDRESS, ADDRESS, M, N, K, 1) == xs.kXSchedSuccess
+        assert taken == (counted_tiles(M, N, K) <= 1 << 18), case
+        if not taken:
             continue
         xs.check(xs.preempt().HwCommandDestroy(cmd.value))
-        tiles = sum(-(-plan[4 * i] // rows[i]) * -(-N // plan[4 * i + 1]) for i in range(2) if rows[i])
-        assert tiles <= 1 << 18, (M, N, K, list(plan), rows)
+        assert sum(-(-plan[4 * i] // rows[i]) * -(-N // plan[4 * i + 1]) for i in range(2) if rows[i]) <= 1 << 18, case
         seen.update((rows[i], plan[4 * i + 1]) for i in range(2) if rows[i])
+        too_many += -(-M // 192) * -(-N // 256) > 1 << 18
     assert {(256, 256), (192, 256), (128, 256), (128, 128), (64, 64)} <= seen
+    assert too_many > 100       # 192 rows would not fit there, 256 do
 
 
 @pytest.mark.gpu
