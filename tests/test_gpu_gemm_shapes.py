@@ -1,7 +1,6 @@
 """GPU parity of the GEMM's tile kernels at the sizes where they change their ways: the number
 of K steps around the length of their pipelines and of their polls of the preempt word, the last
 step full and not, edges of tiles, and rows that start on 16-byte boundaries or do not."""
-import random
 import time
 from ctypes import byref, c_int32, c_uint64
 
@@ -9,6 +8,7 @@ import numpy as np
 import pytest
 
 import oracle
+from test_gemm_split import Busy, Moment
 from test_gpu_kernels import Queue, gemm_cmd
 from test_gpu_preempt import hip_stats
 
@@ -192,7 +192,8 @@ def test_gemm_flushed_and_replayed(xs, gpu, M, N, K, want_plan):
     """The queue is suspended at a random moment of a command until that has flushed it in the
     middle three times (C holds some tiles and not others; of two launches: all of the first one's and
     not all of the second's), then resumed each time: the replay does what is missing and nothing
-    else. Integers in [-2, 2] (K x 4 < 2^24): float32 sums are exact in any order."""
+    else. Other work keeps compute units busy: without it the 256 tiles of 4001 x 4003 x 2048 on copies all start at
+    once, and 600 rounds met two such moments. Integers in [-2, 2] (K x 4 < 2^24): float32 sums are exact in any order."""
     torch = gpu
     print(f"case gemm-flush M={M} N={N} K={K}", flush=True)
     gen = torch.Generator(device="cuda")
@@ -202,25 +203,27 @@ def test_gemm_flushed_and_replayed(xs, gpu, M, N, K, want_plan):
     plan = plan_of(xs, a, b, c, M, N, K)
     assert [(p[1], p[2]) for p in plan] == want_plan, plan
     want = (a.float() @ b.float()).to(torch.bfloat16)
-    q, p, rnd = Queue(xs, torch, 2), xs.preempt(), random.Random(M)
+    q, p, busy = Queue(xs, torch, 2), xs.preempt(), Busy(torch)
     torch.cuda.synchronize()
-    began = time.perf_counter()
-    for _ in range(4):
+    for _ in range(3):
+        began = time.perf_counter()
+        busy.begin()
         q.submit(gemm_cmd(xs, a, b, c, M, N, K, 1))
-    q.wait()
-    span = (time.perf_counter() - began) / 4
-    flushed = rounds = 0
-    while flushed < 3 and rounds < 600:
+        q.wait()
+        span = time.perf_counter() - began
+        torch.cuda.synchronize()
+    flushed, rounds, moment = 0, 0, Moment(M, span)
+    while flushed < 3 and rounds < 3000:
         rounds += 1
         c.fill_(float("nan"))
         torch.cuda.synchronize()
+        busy.begin()
         q.submit(gemm_cmd(xs, a, b, c, M, N, K, 1))
-        until = time.perf_counter() + rnd.uniform(0.0, 1.2 * span)
-        while time.perf_counter() < until:
-            pass
+        moment.wait()
         xs.check(p.XQueueSuspend(q.xq, xs.kQueueSuspendFlagSyncHwQueue))
         missing = torch.isnan(c)
         first = plan[0][0] if len(plan) == 2 else 0
+        moment.met(missing[:first].any() if first else missing, missing)
         some = bool(missing[first:].any()) and (not bool(missing[:first].any()) if first else not bool(missing.all()))
         xs.check(p.XQueueResume(q.xq, xs.kQueueResumeFlagNone))
         q.wait()
