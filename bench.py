@@ -50,6 +50,13 @@ def axpy_bytes(n):
     return 12.0 * n  # read x, read y, write y
 
 
+def axpy_kernel(n):
+    """The kernel of a plain command over n elements that begin on a 128-byte line (the last argument: stores through the L2)."""
+    if n >= 1 << 23:
+        return "AxpyPersistentKernel<3, false, %s>" % ("true" if 1 << 23 < n <= 1 << 24 else "false")
+    return "AxpyVec4Kernel<false, 4, %s>" % ("true" if 1 << 21 < n <= 1 << 22 else "false")
+
+
 def gemm_flops(n):
     return 2.0 * n * n * n
 
@@ -359,7 +366,7 @@ def config2(H, a):
                   "commands_in_latency_block": r["bg_cont_cmds"]}
     line["roofline"] = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                         "frac": achieved / HBM_PEAK_GBS, "traffic": recorded_traffic("axpy_2p28_hbm_traffic.md", bg_n == 1 << 28),
-                        "kernel": "AxpyPersistentKernel<3, false>" if bg_n >= 1 << 23 else "AxpyVec4Kernel<false, 4>",
+                        "kernel": axpy_kernel(bg_n),
                         "algorithmic_bytes_per_launch": axpy_bytes(bg_n),
                         "avg_launch_ms": per_launch_ms, "launches_timed": r["bg_cont_launches"],
                         "timed_with": "HIP events on the background stream around the contended latency block"}

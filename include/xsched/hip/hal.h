@@ -80,7 +80,7 @@ XResult HipQueueMarkEpochFlushed(HwQueueHandle hwq);
  * its entry: ~180 us of drain. */
 
 /* y[i] = fma(alpha, x[i], y[i]) in place, fp32, i < n. 128-bit loads/stores; x and y aligned
- * to their elements (16-byte alignment is worth 3-6 %). */
+ * to their elements. Fastest where y begins on a 128-byte line: 2^22 elements take 6.4 us on one and 7.3 off it, 2^25 64.3 and 65.9. */
 XResult HipAxpyCommandCreate(HwCommandHandle *cmd, float alpha, const void *x, void *y,
                              size_t n, int guard);
 
@@ -91,7 +91,7 @@ XResult HipAxpyPlanOf(const void *y, size_t n, int guarded, uint32_t compute_uni
 
 /* C[M,N] = A[M,K] * B[K,N]; A, B, C row-major bf16, fp32 accumulation in ascending
  * k, round-to-nearest-even on store. Any M, N, K >= 1 (at most 2^18 tiles), any alignment to
- * the element. The work is cut into tiles of C of 256x256 (N and K multiples of 8, matrices
+ * the element. The work is cut into tiles of C of 256x256, 192x256 or 128x256 (N and K multiples of 8, matrices
  * aligned to 16 bytes), 128x128 or 64x64, whichever is estimated to be quickest, or into two
  * launches, 256x256 for most rows and smaller ones for the rest
  * (XSCHED_HIP_GEMM_TILE=64|128|256 overrides that where the shape allows). Fastest where the rows of all three matrices start on 16-byte boundaries (N and K multiples
