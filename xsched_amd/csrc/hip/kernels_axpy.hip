@@ -290,8 +290,8 @@ public:
     /// 15.1 / 17.9, 24.3 / 29.3; 12 x 2^20 24.3 / 25.8, 35.4 / 37.2 -> 21.0 / 26.6, 30.0 / 37.4 -> 22.1 / 24.2, 31.0 / 37.4; 2^24 31.3 / 33.1, 42.4 / 45.0 ->
     /// 28.8 / 34.2, 38.9 / 46.1 -> 29.3 / 30.9, 38.3 / 45.4; level 2 2^23 + 1024 16.0 / 18.4, 28.4 / 29.8 -> 14.6 / 18.7, 24.7 / 29.8 -> 15.0 / 18.3, 25.6 / 29.8;
     /// 2^24 31.4 / 33.5, 43.5 / 44.9 -> 29.1 / 34.6, 39.4 / 46.2 -> 30.7 / 32.2, 39.4 / 46.4. So arrays that are not in the last-level cache, which lost 2 % to 3 % with
-    /// all chunks through, gain up to 7 % where they follow each other, and single passes over them lose up to 1 us (runs differ by as much); a half or five
-    /// eighths of the chunks gain less in all figures but that one. 5000 elements longer it is non-temporal stores and two waves per unit: 33.5 / 35.0, 44.9 / 46.3.
+    /// all chunks through, gain up to 7 % where they follow each other, and single passes over them lose up to 1.5 us (runs differ by 1); with a half or five
+    /// eighths of the chunks passes on one pair gain up to 2 us less. 5000 elements longer it is non-temporal stores and two waves per unit: 33.5 / 35.0, 44.9 / 46.3.
     static uint32_t ThroughFrom(size_t n, uint32_t head, uint32_t n_wg, bool wave_per_chunk, uint32_t units)
     {
         if (wave_per_chunk) return n > (head != 0 ? kThroughOffLines : kThroughOnLines) && n <= kThroughTo ? 0 : n_wg;
